@@ -32,7 +32,7 @@ def build(force=False):
     """Compile liboracle.so (and the reference basis builds when the tree exists)."""
     if force or not os.path.exists(LIB):
         subprocess.check_call(["make", "-s", "-C", HERE, "oracle"])
-    if os.path.isdir("/root/reference"):
+    if os.path.isfile("/root/reference/BLQH_without_spin/basis.cpp"):
         subprocess.check_call(["make", "-s", "-C", HERE, "ref"])
 
 
