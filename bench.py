@@ -62,7 +62,7 @@ MEASURED_SWEEP_TRAFFIC = {
 }
 # fused Lanczos K1 kernel of each SpMV variant (lanczos.hip)
 KERNEL_NAMES = {0: "k_lz1", 1: "k_pspmv<LZ=true>", 2: "k_sps<LZ=true>", 3: "k_jag<LZ=true>", 4: "k_t4<LZ=true>",
-                5: "k_jagr<LZ=true>"}
+                5: "k_jagr<LZ=true>", 6: "k_cod<LZ=true>"}
 
 WORKLOADS = {
     # name: (nspecies, nphi, nel, nel_up, J, K, d, delta_sas, label)

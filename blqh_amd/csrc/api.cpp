@@ -13,7 +13,7 @@
 
 void blqh_basis_build_impl(const blqh_sector& s, blqh_basis* B);
 void blqh_hamil_build_impl(const blqh_basis* B, const blqh_params& p, blqh_hamil* H, int terms);
-void blqh_hamil_combine_impl(const blqh_hamil* base, const blqh_hamil* tun, double dsas, blqh_hamil* H);
+void blqh_hamil_combine_impl(const blqh_hamil* base, const blqh_hamil* tun, double dsas, blqh_hamil* H, bool formats);
 void blqh_spmv_device_impl(blqh_hamil* H, const void* x, void* y);
 void blqh_lanczos_impl(blqh_hamil* H, const blqh_lanczos_opts& o, blqh_lanczos_result& r, double* psi, double* alpha,
                        double* beta);
@@ -347,7 +347,7 @@ int blqh_hamil_build_terms(const blqh_basis* b, const blqh_params* p, int32_t te
 
 int blqh_hamil_prepare(blqh_hamil* h) {
     if (!h) return fail(BLQH_EINVAL, "null hamiltonian");
-    return guarded([&] { blqh::ensure_panels(h); });
+    return guarded([&] { blqh::ensure_coded(h); });
 }
 
 int blqh_hamil_combine(const blqh_hamil* base, const blqh_hamil* tun, double delta_sas, blqh_hamil** out) {
@@ -356,7 +356,7 @@ int blqh_hamil_combine(const blqh_hamil* base, const blqh_hamil* tun, double del
     return guarded([&] {
         auto* H = new blqh_hamil;
         try {
-            blqh_hamil_combine_impl(base, tun, delta_sas, H);
+            blqh_hamil_combine_impl(base, tun, delta_sas, H, true);
         } catch (...) {
             delete H;
             throw;
@@ -398,7 +398,7 @@ int blqh_hamil_get_spmv(const blqh_hamil* h, int32_t* kind, int32_t* lanes, int3
 
 int blqh_hamil_set_spmv(blqh_hamil* h, int32_t kind, int32_t lanes, int32_t threads, int32_t wpc, int32_t rows) {
     if (!h) return fail(BLQH_EINVAL, "null hamiltonian");
-    if (kind >= 1) {  // the panel kinds need the SpMV formats
+    if (kind >= 1 && kind <= 5) {  // the panel kinds need the panels
         const int rc = guarded([&] { blqh::ensure_panels(h); });
         if (rc != BLQH_OK) return rc;
     }
@@ -417,6 +417,9 @@ int blqh_hamil_set_spmv(blqh_hamil* h, int32_t kind, int32_t lanes, int32_t thre
     if (kind == 5)
         ok = h->pan.built && (lanes == 2 || lanes == 4 || lanes == 8) && (threads == 512 || threads == 1024) &&
              wpc >= 1 && wpc <= 4 && (rows == 1 || rows == 2 || rows == 4) && lanes * rows <= 8;
+    if (kind == 6)
+        ok = lanes == 64 && (threads == 256 || threads == 512 || threads == 1024) &&
+             (rows == 1 || rows == 2 || rows == 4 || rows == 8 || rows == 16) && rows * 64 <= threads;
     if (kind == 4) {
         // the column-tile layout is built here on first use (one workgroup per CU)
         int rc = guarded([&] { ok = blqh::build_tiles(h, blqh::runtime().num_cus); });
@@ -432,7 +435,7 @@ int blqh_hamil_set_spmv(blqh_hamil* h, int32_t kind, int32_t lanes, int32_t thre
     h->spmv_kind = kind;
     h->spmv_lpr = kind < 0 ? 0 : lanes;
     h->spmv_threads = kind >= 1 ? threads : 256;
-    h->spmv_wgs_per_cu = kind >= 1 ? wpc : 0;
+    h->spmv_wgs_per_cu = kind >= 1 && kind <= 5 ? wpc : 0;
     h->spmv_rows = kind >= 1 ? rows : 0;
     return BLQH_OK;
 }

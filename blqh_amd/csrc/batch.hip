@@ -46,7 +46,7 @@ void start_vector(int64_t n, uint32_t seed, std::vector<double2>& v);
 double tridiag_lowest(int m, const double* a, const double* b, double* vec);
 double tridiag_lowest_next(int m, const double* a, const double* b, double prev, double step);
 }  // namespace blqh
-void blqh_hamil_combine_impl(const blqh_hamil* base, const blqh_hamil* tun, double dsas, blqh_hamil* H);
+void blqh_hamil_combine_impl(const blqh_hamil* base, const blqh_hamil* tun, double dsas, blqh_hamil* H, bool formats);
 
 namespace {
 
@@ -61,7 +61,8 @@ constexpr int kBTj = kSplit * 256;  // threads per workgroup of k_b1j (an item's
 struct BProb {
     int64_t n;
     int32_t npan, real;
-    const int64_t* pbase;
+    CodView c;              // k_b1j, k_b1s
+    const int64_t* pbase;   // panels: k_b1
     const uint32_t* prow;
     const uint16_t* pcol;
     const double* pvr;
@@ -199,11 +200,21 @@ __global__ void __launch_bounds__(kBT) k_b1(BState S, int jrel, const double2* _
     }
 }
 
-// Same contract as k_b1 over panels in step-major order: kSplit wavefronts
+// Workgroup's share of its XCD's work list: workgroups reach the XCDs round
+// robin (workgroup b on XCD b mod 8, grid a multiple of 8) and each takes a
+// stretch of consecutive items, so that it stays with one member's value table
+// and its XCD gathers from the x vectors of few members at a time.
+__device__ __forceinline__ void list_share(const int32_t* seg, int32_t& k0, int32_t& k1) {
+    const int32_t s0 = seg[0], cnt = seg[1] - s0, nb = (int32_t)(gridDim.x >> 3), b = (int32_t)(blockIdx.x >> 3);
+    k0 = s0 + (int32_t)((int64_t)cnt * b / nb);
+    k1 = s0 + (int32_t)((int64_t)cnt * (b + 1) / nb);
+}
+
+// Same contract as k_b1 over the coded layout: kSplit wavefronts
 // per 64-row slice of the item (waves kSplit*s .. kSplit*s + kSplit-1 own
 // slice s, one lane per row), each summing every kSplit-th step group
-// (jag_row_sum_part); the partial sums of waves 1.. go through LDS to wave 0
-// of the slice, which adds them in wave order and runs the K1 epilogue.  KIND 0 / 1 walk only the members with real / complex panel
+// (cod_run_sum); the partial sums of waves 1.. go through LDS to wave 0
+// of the slice, which adds them in wave order and runs the K1 epilogue.  KIND 0 / 1 walk only the members with real / complex
 // values, KIND 2 walks all members and branches per work item (one launch per
 // step for a mixed batch, so that the members of both kinds run side by side).
 template <bool LZ, int KIND>
@@ -211,21 +222,27 @@ __global__ void __launch_bounds__(kBTj) k_b1j(BState S, int jrel, const double2*
                                               double2* __restrict__ ys, double* __restrict__ part) {
     __shared__ double sh[kBTj / 64];
     __shared__ double2 red[kItemRows / 64][kSplit - 1][64];  // partial row sums of waves 1.. of each slice
+    extern __shared__ __align__(16) double ctab[];
     const int j = LZ ? *S.jbase + jrel : 0;
     if (LZ && j >= S.cap) return;
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int sl = wv / kSplit, par = wv % kSplit;
-    // Workgroups go to the XCDs round robin (workgroup b to XCD b mod 8, grid
-    // a multiple of 8); each XCD walks its own list of whole problems, so the
-    // x vectors it gathers from are those of the few problems its 32 CUs are
-    // working on and stay in its L2.
-    const int32_t* seg = S.xseg + KIND * 9 + (blockIdx.x & 7);
-    const int32_t kend = seg[1];
-    for (int32_t k = seg[0] + (int32_t)(blockIdx.x >> 3); k < kend; k += (int32_t)(gridDim.x >> 3)) {
+    int32_t k0, k1;
+    list_share(S.xseg + KIND * 9 + (blockIdx.x & 7), k0, k1);
+    int pt = -1;  // member whose value table is in LDS
+    for (int32_t k = k0; k < k1; ++k) {
         const int64_t it = S.xitems[k];
         const int p = S.item_prob[it];
         if (!S.active[p]) continue;  // uniform over the workgroup
         const BProb P = S.probs[p];
+        const bool real = KIND == 2 ? P.real != 0 : KIND == 0;
+        if (p != pt) {
+            __syncthreads();  // the previous member's table is no longer read
+            if (real) cod_stage<true>(P.c.tab, P.c.ntab, ctab, kBTj);
+            else cod_stage<false>(P.c.tab, P.c.ntab, ctab, kBTj);
+            __syncthreads();
+            pt = p;
+        }
         const double2* x;
         double2* y;
         const double2* Wp = nullptr;
@@ -245,18 +262,18 @@ __global__ void __launch_bounds__(kBTj) k_b1j(BState S, int jrel, const double2*
         const int64_t row0 = (it - P.item0) * kItemRows + sl * 64, myrow = row0 + lane;
         double ar = 0.0, ai = 0.0;
         if (row0 < n) {  // uniform over the wavefront
-            const int64_t rend = row0 + 64 < n ? row0 + 64 : n;
+            const int64_t slc = row0 >> 6;
             for (int pan = 0; pan < P.npan; ++pan) {
-                const uint32_t* rp = P.prow + (int64_t)pan * (n + 1);
-                const uint32_t s = myrow < n ? rp[myrow] : rp[rend];
-                const uint32_t e = myrow < n ? rp[myrow + 1] : rp[rend];
-                const int64_t run = P.pbase[pan] + (uint32_t)__builtin_amdgcn_readfirstlane((int)s);  // rp[row0]
+                const int64_t run = (int64_t)pan * P.c.nslices + slc;
                 const double2* xp = x + (int64_t)pan * kPanelWidth;
-                if (KIND == 2 ? P.real != 0 : KIND == 0)
-                    jag_row_sum_part<true, kSplit>(P.pcol + run, P.pvr + run, P.pvc + run, xp, e - s, par, ar, ai);
-                else
-                    jag_row_sum_part<false, kSplit>(P.pcol + run, P.pvr + run, P.pvc + run, xp, e - s, par, ar, ai);
+                const uint32_t len = P.c.len[run * 64 + lane];
+                if (real) cod_run_sum<true, kSplit, 4>(P.c.ent + P.c.base[run], ctab, xp, len, par, ar, ai);
+                else cod_run_sum<false, kSplit, 4>(P.c.ent + P.c.base[run], ctab, xp, len, par, ar, ai);
             }
+            const int64_t q0 = P.c.rbase[slc];
+            const uint32_t rl = P.c.rlen[myrow];
+            if (real) cod_rest_sum<true, kSplit>(P.c.rcol + q0, P.c.rval + q0, x, rl, par, ar, ai);
+            else cod_rest_sum<false, kSplit>(P.c.rcol + q0, P.c.rval + 2 * q0, x, rl, par, ar, ai);
         }
         if (par) red[sl][par - 1][lane] = make_double2(ar, ai);
         __syncthreads();
@@ -294,86 +311,117 @@ __global__ void __launch_bounds__(kBTj) k_b1j(BState S, int jrel, const double2*
 // column (a sector of at most 32,768 states, one panel), and problem g scales
 // them by s_g.  One pass over the entries serves all G problems: the column
 // and value of an entry are loaded once and gathered against G vectors.
-constexpr uint16_t kTunBit = 0x8000;
-
 struct SGroups {
     const int32_t* gitem_grp;  // group work item -> group
     const int64_t* gitem0;     // [ngroups + 1] first group item
     const double* tscale;      // [P] scale of the flagged entries, problem p
 };
 
-// jag_row_sum_part for G vectors: lane sums of row `lane` of a 64-row slice
-// over the steps of its wave (see jag_row_sum_part), entry values scaled by
-// ts[g] where the column carries kTunBit.  act[g] == false skips vector g.
-template <bool REAL, int NP, int G>
-__device__ __forceinline__ void jag_row_sum_shared(const uint16_t* __restrict__ cr, const double* __restrict__ vr,
-                                                   const double2* __restrict__ vc, const double2* const* xp,
-                                                   const double* ts, const bool* act, uint32_t len, int par,
-                                                   double* ar, double* ai) {
-    typedef double d2v_t __attribute__((ext_vector_type(2)));
-    uint32_t off = 0;
-    auto issue = [&](uint32_t t, int* c, double2* v, bool& any) {
-        uint64_t m[4];
+// cod_run_sum for G vectors: lane sums of row `lane` of a 64-row slice over the
+// step groups of its wave, entry values scaled by ts[g] where the column carries
+// kCodTun.  act[g] == false skips vector g.
+template <bool REAL, int G>
+__device__ __forceinline__ void shared_fma(uint32_t c, double2 v, const double2* const* xp, const double* ts,
+                                           const bool* act, double* ar, double* ai) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) m[u] = __ballot(t + u < len);
+    for (int g = 0; g < G; ++g)
+        if (act[g]) {
+            const double2 xv = xp[g][c & (kCodTun - 1)];
+            const double sc = (c & kCodTun) ? ts[g] : 1.0;
+            const double wr = sc * v.x;
+            if (REAL) {
+                ar[g] += wr * xv.x;
+                ai[g] += wr * xv.y;
+            } else {
+                const double wi = sc * v.y;
+                ar[g] += wr * xv.x - wi * xv.y;
+                ai[g] += wr * xv.y + wi * xv.x;
+            }
+        }
+}
+
+template <bool REAL, int NP, int G>
+__device__ __forceinline__ void cod_run_shared(const uint32_t* __restrict__ er, const double* tab,
+                                               const double2* const* xp, const double* ts, const bool* act,
+                                               uint32_t len, int par, double* ar, double* ai) {
+    constexpr int U = 4;
+    uint32_t off = 0;
+    auto issue = [&](uint32_t t, uint32_t* e, bool& any) {
+        uint64_t m[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) m[u] = __ballot(t + u < len);
         any = m[0] != 0;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < U; ++u) {
             const uint32_t q = off + lanes_below(m[u]);
             off += (uint32_t)__popcll(m[u]);
-            const bool a = t + u < len;
-            c[u] = a ? (int)__builtin_nontemporal_load(&cr[q]) : 0;
-            if (REAL) {
-                v[u] = make_double2(a ? __builtin_nontemporal_load(&vr[q]) : 0.0, 0.0);
-            } else if (a) {
-                const d2v_t w = __builtin_nontemporal_load(reinterpret_cast<const d2v_t*>(&vc[q]));
-                v[u] = make_double2(w.x, w.y);
-            } else {
-                v[u] = make_double2(0.0, 0.0);
-            }
+            e[u] = t + u < len ? __builtin_nontemporal_load(&er[q]) : 0u;
         }
     };
     auto skip = [&](uint32_t t) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) off += (uint32_t)__popcll(__ballot(t + u < len));
+        for (int u = 0; u < U; ++u) off += (uint32_t)__popcll(__ballot(t + u < len));
     };
-    int c0[4], c1[4];
-    double2 v0[4], v1[4];
+    uint32_t e0[U], e1[U];
     bool any0, any1;
-    for (int g = 0; g < par; ++g) skip(4u * g);
-    issue(4u * par, c0, v0, any0);
-    for (uint32_t t = 4u * par + 4u * NP; any0; t += 4u * NP) {
+    for (int g = 0; g < par; ++g) skip((uint32_t)(U * g));
+    uint32_t t0 = (uint32_t)(U * par);
+    issue(t0, e0, any0);
+    while (any0) {
+        const uint32_t t = t0 + (uint32_t)(U * NP);
 #pragma unroll
-        for (int g = NP - 1; g > 0; --g) skip(t - 4u * g);
-        issue(t, c1, v1, any1);
-        // one vector at a time: four gathers in flight per vector keep the
-        // register count at 144 (all G x 4 at once: 162, and measured 9 % slower)
+        for (int g = NP - 1; g > 0; --g) skip(t - (uint32_t)(U * g));
+        issue(t, e1, any1);
+        double2 v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            v[u] = REAL ? make_double2(cod_real(tab, e0[u]), 0.0)
+                        : cod_cplx(reinterpret_cast<const double2*>(tab), e0[u]);
+            if (!(t0 + u < len)) v[u] = make_double2(0.0, 0.0);
+        }
+        // one vector at a time: U gathers in flight per vector
 #pragma unroll
         for (int g = 0; g < G; ++g)
             if (act[g]) {
-                double2 xv[4];
+                double2 xv[U];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) xv[u] = xp[g][c0[u] & (kTunBit - 1)];
+                for (int u = 0; u < U; ++u) xv[u] = xp[g][e0[u] & (kCodTun - 1)];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const double sc = (c0[u] & kTunBit) ? ts[g] : 1.0;
-                    const double wr = sc * v0[u].x;
+                for (int u = 0; u < U; ++u) {
+                    const double sc = (e0[u] & kCodTun) ? ts[g] : 1.0;
+                    const double wr = sc * v[u].x;
                     if (REAL) {
                         ar[g] += wr * xv[u].x;
                         ai[g] += wr * xv[u].y;
                     } else {
-                        const double wi = sc * v0[u].y;
+                        const double wi = sc * v[u].y;
                         ar[g] += wr * xv[u].x - wi * xv[u].y;
                         ai[g] += wr * xv[u].y + wi * xv[u].x;
                     }
                 }
             }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            c0[u] = c1[u];
-            v0[u] = v1[u];
-        }
+        for (int u = 0; u < U; ++u) e0[u] = e1[u];
         any0 = any1;
+        t0 = t;
+    }
+}
+
+// the rest of a slice (cod_rest_sum) for G vectors
+template <bool REAL, int NP, int G>
+__device__ __forceinline__ void cod_rest_shared(const uint32_t* __restrict__ rc, const double* __restrict__ rv,
+                                                const double2* const* x, const double* ts, const bool* act,
+                                                uint32_t len, int par, double* ar, double* ai) {
+    uint32_t off = 0;
+    for (uint32_t t = 0;; ++t) {
+        const uint64_t m = __ballot(t < len);
+        if (m == 0) break;
+        if ((int)(t % NP) == par && t < len) {
+            const uint32_t q = off + lanes_below(m);
+            const double2 v = REAL ? make_double2(rv[q], 0.0) : reinterpret_cast<const double2*>(rv)[q];
+            shared_fma<REAL, G>(rc[q], v, x, ts, act, ar, ai);
+        }
+        off += (uint32_t)__popcll(m);
     }
 }
 
@@ -386,13 +434,15 @@ __global__ void __launch_bounds__(kBTj) k_b1s(BState S, SGroups Q, int jrel, con
                                               double2* __restrict__ ys, double* __restrict__ part) {
     __shared__ double sh[kBTj / 64];
     __shared__ double2 red[kItemRows / 64][kSplit - 1][G][64];
+    extern __shared__ __align__(16) double ctab[];
     const int j = LZ ? *S.jbase + jrel : 0;
     if (LZ && j >= S.cap) return;
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int sl = wv / kSplit, par = wv % kSplit;
-    const int32_t* seg = S.xseg + KIND * 9 + (blockIdx.x & 7);
-    const int32_t kend = seg[1];
-    for (int32_t k = seg[0] + (int32_t)(blockIdx.x >> 3); k < kend; k += (int32_t)(gridDim.x >> 3)) {
+    int32_t k0, k1;
+    list_share(S.xseg + KIND * 9 + (blockIdx.x & 7), k0, k1);
+    int qt = -1;  // sector whose value table is in LDS
+    for (int32_t k = k0; k < k1; ++k) {
         const int64_t it = S.xitems[k];
         const int q = Q.gitem_grp[it];
         const int64_t li = it - Q.gitem0[q];
@@ -406,6 +456,14 @@ __global__ void __launch_bounds__(kBTj) k_b1s(BState S, SGroups Q, int jrel, con
         if (!anyact) continue;  // uniform over the workgroup
         const BProb P0 = S.probs[q * G];
         const int64_t n = P0.n;
+        const bool real = KIND == 2 ? P0.real != 0 : KIND == 0;
+        if (q != qt) {
+            __syncthreads();  // the previous sector's table is no longer read
+            if (real) cod_stage<true>(P0.c.tab, P0.c.ntab, ctab, kBTj);
+            else cod_stage<false>(P0.c.tab, P0.c.ntab, ctab, kBTj);
+            __syncthreads();
+            qt = q;
+        }
         const double2* x[G];
         double2* y[G];
         const double2* Wp[G];
@@ -435,16 +493,15 @@ __global__ void __launch_bounds__(kBTj) k_b1s(BState S, SGroups Q, int jrel, con
 #pragma unroll
         for (int g = 0; g < G; ++g) ar[g] = ai[g] = 0.0;
         if (row0 < n) {  // uniform over the wavefront; one panel (n <= 32768)
-            const int64_t rend = row0 + 64 < n ? row0 + 64 : n;
-            const uint32_t s = myrow < n ? P0.prow[myrow] : P0.prow[rend];
-            const uint32_t e = myrow < n ? P0.prow[myrow + 1] : P0.prow[rend];
-            const int64_t run = P0.pbase[0] + (uint32_t)__builtin_amdgcn_readfirstlane((int)s);
-            if (KIND == 2 ? P0.real != 0 : KIND == 0)
-                jag_row_sum_shared<true, kSplit, G>(P0.pcol + run, P0.pvr + run, P0.pvc + run, x, ts, act, e - s,
-                                                    par, ar, ai);
-            else
-                jag_row_sum_shared<false, kSplit, G>(P0.pcol + run, P0.pvr + run, P0.pvc + run, x, ts, act, e - s,
-                                                     par, ar, ai);
+            const int64_t slc = row0 >> 6, run = P0.c.base[slc], q0 = P0.c.rbase[slc];
+            const uint32_t len = P0.c.len[myrow], rl = P0.c.rlen[myrow];
+            if (real) {
+                cod_run_shared<true, kSplit, G>(P0.c.ent + run, ctab, x, ts, act, len, par, ar, ai);
+                cod_rest_shared<true, kSplit, G>(P0.c.rcol + q0, P0.c.rval + q0, x, ts, act, rl, par, ar, ai);
+            } else {
+                cod_run_shared<false, kSplit, G>(P0.c.ent + run, ctab, x, ts, act, len, par, ar, ai);
+                cod_rest_shared<false, kSplit, G>(P0.c.rcol + q0, P0.c.rval + 2 * q0, x, ts, act, rl, par, ar, ai);
+            }
         }
         if (par) {
 #pragma unroll
@@ -481,26 +538,6 @@ __global__ void __launch_bounds__(kBTj) k_b1s(BState S, SGroups Q, int jrel, con
             if (threadIdx.x == 0) part[S.probs[q * G + g].item0 + li] = t;
         }
     }
-}
-
-// T-entry flags of a one-panel sector in row-major panel order: bit 15 of
-// the column of every entry between words of different upper-layer
-// occupation (nu, internal row order); the flagged entries are counted.
-__global__ void k_mark_tun(int64_t n, const int64_t* __restrict__ pbase, const uint32_t* __restrict__ prow,
-                           uint16_t* __restrict__ pcol, const uint8_t* __restrict__ nu, int32_t* __restrict__ cnt) {
-    int32_t c = 0;
-    for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n; r += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t b = pbase[0];
-        for (uint32_t k = prow[r]; k < prow[r + 1]; ++k) {
-            const uint16_t col = pcol[b + k];
-            if (nu[col] != nu[r]) {
-                pcol[b + k] = (uint16_t)(col | kTunBit);
-                ++c;
-            }
-        }
-    }
-    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-    if ((threadIdx.x & 63) == 0 && c) atomicAdd(cnt, c);
 }
 
 // K2: alpha_j, W_{j+1} = u - alpha_j W_j / beta_j, |W_{j+1}|^2 partials
@@ -778,7 +815,8 @@ struct blqh_batch {
     DevBuf<int32_t> item_prob;
     DevBuf<int32_t> xitems, xseg;    // per-XCD work lists of k_b1j (rebuilt by refresh_probs)
     std::vector<int32_t> h_xitems, h_xseg;
-    int lpr = 0;                 // lanes per row of k_b1 (autotuned)
+    int lpr = 0;                 // 64: k_b1j over the coded layout; else lanes per row of k_b1
+    size_t tab_bytes = 0;        // LDS for the members' largest value table
     bool has_real = false, has_complex = false;  // value kinds among the members
     int grid = 0;
     // kept between solves of the same lambda: device pools, the captured
@@ -788,6 +826,7 @@ struct blqh_batch {
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     int g_chk = -1, g_lpr = -1, g_cap = -1, g_kinds = -1;
+    size_t g_tab = 0;  // table LDS of the captured launches
     char* pin = nullptr;
     double2* psi_pin = nullptr;  // pinned staging of the ground states (b->rows entries, on first use)
     // pl.u holds every problem's ground state of the last finished solve in
@@ -828,7 +867,7 @@ std::vector<XcdMember> xcd_members(const blqh_batch* b, const std::vector<char>*
             bool on = !live;
             for (int g = 0; g < b->G && !on; ++g) on = (*live)[q * b->G + g] != 0;
             if (on)
-                mem.push_back({b->gitem0[q], b->gitem0[q + 1], b->tpl[q]->nnz * b->G, 1, b->tpl[q]->pan.real ? 1 : 0});
+                mem.push_back({b->gitem0[q], b->gitem0[q + 1], b->tpl[q]->nnz * b->G, 1, b->tpl[q]->cod.real ? 1 : 0});
         }
         return mem;
     }
@@ -836,8 +875,8 @@ std::vector<XcdMember> xcd_members(const blqh_batch* b, const std::vector<char>*
     mem.reserve(P);
     for (int p = 0; p < P; ++p)
         if (!live || (*live)[p])
-            mem.push_back({b->item0[p], b->item0[p + 1], b->hs[p]->nnz, b->hs[p]->pan.npan,
-                           b->hs[p]->pan.real ? 1 : 0});
+            mem.push_back({b->item0[p], b->item0[p + 1], b->hs[p]->nnz, b->h_probs[p].npan,
+                           b->h_probs[p].real});
     return mem;
 }
 
@@ -856,51 +895,83 @@ void build_xcd_lists(blqh_batch* b) {
     BLQH_HIP(hipStreamSynchronize(st));
 }
 
-// Row-major panel layout and current panel buffers of every member.
+// The layout that the batch's kernels read and its current buffers, of every
+// member: the coded one (lanes 64), else row-major panels.
 void refresh_probs(blqh_batch* b) {
     b->has_real = b->has_complex = false;
-    for (blqh_hamil* H : b->hs) (H->pan.real ? b->has_real : b->has_complex) = true;
-    // k_b1j reads step-major runs, k_b1 row-major ones: one relayout launch for all members
-    // plain step order: a rebind re-lays out every member at each parameter point
-    if (b->G)  // the templates, once each
-        set_panel_layouts(b->tpl.data(), (int)b->tpl.size(), true, b->relayout.get(), b->relayout.bytes(), false);
-    else
-        set_panel_layouts(b->hs.data(), (int)b->hs.size(), b->lpr == 64, b->relayout.get(), b->relayout.bytes(),
-                          false);
-    build_xcd_lists(b);
+    b->tab_bytes = 0;
+    const bool coded = b->lpr == 64;
+    if (!coded) {
+        for (blqh_hamil* H : b->hs) ensure_panels(H);
+        const size_t scratch = panel_layout_scratch_bytes(b->hs.data(), (int)b->hs.size());
+        if (scratch > b->relayout.bytes()) b->relayout.alloc(scratch);
+        set_panel_layouts(b->hs.data(), (int)b->hs.size(), false, b->relayout.get(), b->relayout.bytes(), false);
+    }
     for (size_t p = 0; p < b->hs.size(); ++p) {
         blqh_hamil* H = b->hs[p];
         BProb& d = b->h_probs[p];
-        d.pbase = H->pan.pbase.get();
-        d.prow = H->pan.prow.get();
-        d.pcol = H->pan.pcol.get();
-        d.pvr = H->pan.pvr.get();
-        d.pvc = H->pan.pvc.get();
+        if (coded) ensure_coded(H);
+        const bool real = coded ? H->cod.real : H->pan.real;
+        d.real = real ? 1 : 0;
+        (real ? b->has_real : b->has_complex) = true;
+        if (coded) {
+            d.c = cview(H->cod, H->n);
+            b->tab_bytes = std::max(b->tab_bytes, cod_lds_bytes(real, H->cod.ntab));
+        } else {
+            d.pbase = H->pan.pbase.get();
+            d.prow = H->pan.prow.get();
+            d.pcol = H->pan.pcol.get();
+            d.pvr = H->pan.pvr.get();
+            d.pvc = H->pan.pvc.get();
+        }
     }
+    build_xcd_lists(b);
+}
+
+// Kernels with the value table in dynamic LDS, raised to the largest table once.
+template <class K>
+void allow_table(K kern) {
+    BLQH_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 (int)cod_lds_bytes(false, kCodCplx)));
 }
 
 SGroups make_groups(const blqh_batch* b) {
     return SGroups{b->gitem_grp.get(), b->dgitem0.get(), b->dtscale.get()};
 }
 
+template <bool LZ, int KIND, int G>
+void launch_b1s_go(const blqh_batch* b, const BState& S, int jrel, const double2* xs, double2* ys, double* part,
+                   hipStream_t st) {
+    static const bool attr = (allow_table(k_b1s<LZ, KIND, G>), true);  // once per instantiation, thread-safe
+    (void)attr;
+    hipLaunchKernelGGL((k_b1s<LZ, KIND, G>), dim3(b->grid), dim3(kBTj), b->tab_bytes, st, S, make_groups(b), jrel, xs,
+                       ys, part);
+}
+
 template <bool LZ, int KIND>
 void launch_b1s_kind(const blqh_batch* b, const BState& S, int jrel, const double2* xs, double2* ys, double* part,
                      hipStream_t st) {
-    const dim3 g(b->grid), tj(kBTj);
-    const SGroups Q = make_groups(b);
     switch (b->G) {
-        case 1: hipLaunchKernelGGL((k_b1s<LZ, KIND, 1>), g, tj, 0, st, S, Q, jrel, xs, ys, part); break;
-        case 2: hipLaunchKernelGGL((k_b1s<LZ, KIND, 2>), g, tj, 0, st, S, Q, jrel, xs, ys, part); break;
-        case 3: hipLaunchKernelGGL((k_b1s<LZ, KIND, 3>), g, tj, 0, st, S, Q, jrel, xs, ys, part); break;
-        case 4: hipLaunchKernelGGL((k_b1s<LZ, KIND, 4>), g, tj, 0, st, S, Q, jrel, xs, ys, part); break;
+        case 1: launch_b1s_go<LZ, KIND, 1>(b, S, jrel, xs, ys, part, st); break;
+        case 2: launch_b1s_go<LZ, KIND, 2>(b, S, jrel, xs, ys, part, st); break;
+        case 3: launch_b1s_go<LZ, KIND, 3>(b, S, jrel, xs, ys, part, st); break;
+        case 4: launch_b1s_go<LZ, KIND, 4>(b, S, jrel, xs, ys, part, st); break;
         default: throw Error(BLQH_EINTERNAL, "unsupported group size");
     }
+}
+
+template <bool LZ, int KIND>
+void launch_b1j(const blqh_batch* b, const BState& S, int jrel, const double2* xs, double2* ys, double* part,
+                hipStream_t st) {
+    static const bool attr = (allow_table(k_b1j<LZ, KIND>), true);
+    (void)attr;
+    hipLaunchKernelGGL((k_b1j<LZ, KIND>), dim3(b->grid), dim3(kBTj), b->tab_bytes, st, S, jrel, xs, ys, part);
 }
 
 template <bool LZ>
 void launch_b1(const blqh_batch* b, const BState& S, int jrel, const double2* xs, double2* ys, double* part,
                hipStream_t st) {
-    const dim3 g(b->grid), t(kBT), tj(kBTj);
+    const dim3 g(b->grid), t(kBT);
     if (b->G) {  // shared-scale groups: one pass over each sector's entries for all its problems
         if (b->has_real && b->has_complex) {
             launch_b1s_kind<LZ, 2>(b, S, jrel, xs, ys, part, st);
@@ -913,11 +984,11 @@ void launch_b1(const blqh_batch* b, const BState& S, int jrel, const double2* xs
     switch (b->lpr) {
         case 64:
             if (b->has_real && b->has_complex) {  // measured faster than one launch per kind
-                hipLaunchKernelGGL((k_b1j<LZ, 2>), g, tj, 0, st, S, jrel, xs, ys, part);
+                launch_b1j<LZ, 2>(b, S, jrel, xs, ys, part, st);
                 break;
             }
-            if (b->has_real) hipLaunchKernelGGL((k_b1j<LZ, 0>), g, tj, 0, st, S, jrel, xs, ys, part);
-            if (b->has_complex) hipLaunchKernelGGL((k_b1j<LZ, 1>), g, tj, 0, st, S, jrel, xs, ys, part);
+            if (b->has_real) launch_b1j<LZ, 0>(b, S, jrel, xs, ys, part, st);
+            if (b->has_complex) launch_b1j<LZ, 1>(b, S, jrel, xs, ys, part, st);
             break;
         case 4: hipLaunchKernelGGL((k_b1<4, LZ>), g, t, 0, st, S, jrel, xs, ys, part); break;
         case 8: hipLaunchKernelGGL((k_b1<8, LZ>), g, t, 0, st, S, jrel, xs, ys, part); break;
@@ -946,44 +1017,6 @@ BState make_state(const blqh_batch* b, Pools& pl, int cap) {
     return S;
 }
 
-// time the plain batched product for each lane count and keep the fastest
-void tune_batch(blqh_batch* b) {
-    hipStream_t st = stream();
-    Pools pl;
-    const int P = (int)b->hs.size();
-    pl.probs.alloc(P);
-    pl.active.alloc(P);
-    BLQH_HIP(hipMemcpyAsync(pl.probs.get(), b->h_probs.data(), P * sizeof(BProb), hipMemcpyHostToDevice, st));
-    std::vector<int32_t> on(P, 1);
-    BLQH_HIP(hipMemcpyAsync(pl.active.get(), on.data(), P * 4, hipMemcpyHostToDevice, st));
-    DevBuf<double2> x(b->rows), y(b->rows);
-    DevBuf<double> part(b->nitems);
-    BLQH_HIP(hipMemsetAsync(x.get(), 0, b->rows * sizeof(double2), st));
-    BState S = make_state(b, pl, 1);
-    hipEvent_t e0, e1;
-    BLQH_HIP(hipEventCreate(&e0));
-    BLQH_HIP(hipEventCreate(&e1));
-    float best = 1e30f;
-    int bl = 8;
-    for (int l : {4, 8, 16, 32, 64}) {  // 64: one lane per row, step-major panels (last: one relayout)
-        b->lpr = l;
-        refresh_probs(b);
-        BLQH_HIP(hipMemcpyAsync(pl.probs.get(), b->h_probs.data(), P * sizeof(BProb), hipMemcpyHostToDevice, st));
-        launch_b1<false>(b, S, 0, x.get(), y.get(), part.get(), st);
-        BLQH_HIP(hipEventRecord(e0, st));
-        for (int r = 0; r < 3; ++r) launch_b1<false>(b, S, 0, x.get(), y.get(), part.get(), st);
-        BLQH_HIP(hipEventRecord(e1, st));
-        BLQH_HIP(hipEventSynchronize(e1));
-        float ms = 0;
-        BLQH_HIP(hipEventElapsedTime(&ms, e0, e1));
-        if (ms < best) { best = ms; bl = l; }
-    }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    b->lpr = bl;
-    refresh_probs(b);
-}
-
 }  // namespace
 
 blqh_batch* blqh_batch_create_impl(blqh_hamil* const* hs, int count, int lanes) {
@@ -998,12 +1031,10 @@ blqh_batch* blqh_batch_create_impl(blqh_hamil* const* hs, int count, int lanes) 
         for (int p = 0; p < count; ++p) {
             blqh_hamil* H = hs[p];
             BLQH_REQUIRE(H != nullptr, BLQH_EINVAL, "null hamiltonian in batch");
-            ensure_panels(H);
-            BLQH_REQUIRE(H->pan.built && H->n > 0, BLQH_EINVAL, "batched solve needs a non-empty panel layout");
+            BLQH_REQUIRE(H->n > 0, BLQH_EINVAL, "batched solve needs non-empty Hamiltonians");
             BProb d{};
             d.n = H->n;
-            d.npan = H->pan.npan;
-            d.real = H->pan.real ? 1 : 0;
+            d.npan = (int32_t)ceil_div(H->n, (int64_t)kPanelWidth);
             d.item0 = b->nitems;
             d.voff = b->rows;
             const int64_t nit = ceil_div(H->n, kItemRows);
@@ -1021,14 +1052,8 @@ blqh_batch* blqh_batch_create_impl(blqh_hamil* const* hs, int count, int lanes) 
         b->grid = (int)(8 * ceil_div(std::min<int64_t>(b->nitems, (int64_t)runtime().num_cus * 8), 8));
         b->xitems.alloc(2 * b->nitems);
         b->xseg.alloc(27);
-        b->relayout.alloc(panel_layout_scratch_bytes(b->hs.data(), count));
-        if (lanes) {
-            b->lpr = lanes;
-            refresh_probs(b);
-        } else {
-            refresh_probs(b);
-            tune_batch(b);
-        }
+        b->lpr = lanes ? lanes : 64;
+        refresh_probs(b);
     } catch (...) {
         delete b;
         throw;
@@ -1044,36 +1069,31 @@ void blqh_batch_rebind_impl(blqh_batch* b, blqh_hamil* const* hs, int count) {
     int64_t nnz = 0;
     for (int p = 0; p < count; ++p) {
         BLQH_REQUIRE(hs[p] != nullptr, BLQH_EINVAL, "null hamiltonian in batch");
-        ensure_panels(hs[p]);
-        BLQH_REQUIRE(hs[p]->n == b->h_probs[p].n && hs[p]->pan.npan == b->h_probs[p].npan, BLQH_EINVAL,
+        BLQH_REQUIRE(hs[p]->n == b->h_probs[p].n, BLQH_EINVAL,
                      "rebind needs Hamiltonians of the same sizes, in the same order");
         nnz += hs[p]->nnz;
     }
     b->nnz = nnz;
     b->hs.assign(hs, hs + count);
-    for (int p = 0; p < count; ++p) b->h_probs[p].real = hs[p]->pan.real ? 1 : 0;
-    const size_t scratch = panel_layout_scratch_bytes(b->hs.data(), count);
-    if (scratch > b->relayout.bytes()) b->relayout.alloc(scratch);
     refresh_probs(b);
 }
 
 namespace {
-// H0 + 1 T of one sector (blqh_hamil_combine) with bit 15 set on the column
-// of every T entry, in row-major panel order.  The tunnelling terms are the
+// H0 + 1 T of one sector (blqh_hamil_combine) in the coded layout, the tunnelling
+// flag set on the column of every T entry (those between words of different
+// upper-layer occupation; nu per row in the internal order).  The tunnelling terms are the
 // only ones that move an electron between the layers, so T's entries are
 // exactly those between words of different upper-layer occupation; their
 // count must equal T's.
 blqh_hamil* make_template(const blqh_hamil* base, const blqh_hamil* tun) {
     BLQH_REQUIRE(base != nullptr && tun != nullptr, BLQH_EINVAL, "null hamiltonian in batch");
     BLQH_REQUIRE(base->basis->geo.S >= 2, BLQH_EINVAL, "a shared-scale batch needs bilayer sectors");
-    BLQH_REQUIRE(base->n <= (int64_t)kTunBit, BLQH_EINVAL,
+    BLQH_REQUIRE(base->n <= (int64_t)kCodTun, BLQH_EINVAL,
                  "a shared-scale batch takes sectors of at most 32768 states");
     auto* H = new blqh_hamil;
     try {
-        blqh_hamil_combine_impl(base, tun, 1.0, H);
-        ensure_panels(H);
-        BLQH_REQUIRE(H->pan.built && H->pan.npan == 1, BLQH_EINTERNAL, "template is not a one-panel matrix");
-        set_panel_layout(H, false);  // row-major: the marking kernel walks rows
+        blqh_hamil_combine_impl(base, tun, 1.0, H, false);
+        build_order(H);
         const blqh_basis* B = H->basis;
         const int64_t n = H->n;
         const uint64_t upper = lowbits(B->geo.S * B->geo.nphi / 2);
@@ -1082,18 +1102,11 @@ blqh_hamil* make_template(const blqh_hamil* base, const blqh_hamil* tun) {
             const int64_t i = H->ord.on ? H->ord.h_iperm[r] : r;
             nu[r] = (uint8_t)popc(B->h_id[i] & upper);
         }
-        hipStream_t st = stream();
         DevBuf<uint8_t> dnu(n);
-        DevBuf<int32_t> cnt(1);
-        BLQH_HIP(hipMemcpyAsync(dnu.get(), nu.data(), n, hipMemcpyHostToDevice, st));
-        BLQH_HIP(hipMemsetAsync(cnt.get(), 0, 4, st));
-        const int g = (int)std::min<int64_t>(std::max<int64_t>(ceil_div(n, 256), 1), 4096);
-        hipLaunchKernelGGL(k_mark_tun, dim3(g), dim3(256), 0, st, n, H->pan.pbase.get(), H->pan.prow.get(),
-                           H->pan.pcol.get(), dnu.get(), cnt.get());
-        BLQH_HIP(hipGetLastError());
-        int32_t hc = 0;
-        copy_sync(&hc, cnt.get(), 4, hipMemcpyDeviceToHost);
-        BLQH_REQUIRE(hc == tun->nnz, BLQH_EINTERNAL, "the tunnelling entries are not the layer-changing entries");
+        BLQH_HIP(hipMemcpyAsync(dnu.get(), nu.data(), n, hipMemcpyHostToDevice, stream()));
+        int64_t ntun = 0;
+        build_coded(H, dnu.get(), &ntun);
+        BLQH_REQUIRE(ntun == tun->nnz, BLQH_EINTERNAL, "the tunnelling entries are not the layer-changing entries");
     } catch (...) {
         delete H;
         throw;
@@ -1164,8 +1177,7 @@ blqh_batch* blqh_batch_create_scaled_impl(const blqh_hamil* const* base, const b
                 BProb d{};
                 d.n = H->n;
                 d.npan = 1;
-                d.real = H->pan.real ? 1 : 0;
-                d.item0 = b->nitems;
+                    d.item0 = b->nitems;
                 d.voff = b->rows;
                 for (int64_t i = 0; i < nit; ++i) ip.push_back(p);
                 b->nitems += nit;
@@ -1187,7 +1199,6 @@ blqh_batch* blqh_batch_create_scaled_impl(const blqh_hamil* const* base, const b
         b->grid = (int)(8 * ceil_div(std::min<int64_t>(b->nitems, (int64_t)runtime().num_cus * 8), 8));
         b->xitems.alloc(2 * b->nitems);
         b->xseg.alloc(27);
-        b->relayout.alloc(panel_layout_scratch_bytes(b->tpl.data(), nsec));
         b->lpr = 64;
         refresh_probs(b);
     } catch (...) {
@@ -1216,11 +1227,9 @@ void blqh_batch_rebind_scaled_impl(blqh_batch* b, const blqh_hamil* const* base,
         for (int g = 0; g < b->G; ++g) {
             const int p = q * b->G + g;
             b->hs[p] = b->tpl[q];
-            b->h_probs[p].real = b->tpl[q]->pan.real ? 1 : 0;
+            b->h_probs[p].real = b->tpl[q]->cod.real ? 1 : 0;
         }
     }
-    const size_t scratch = panel_layout_scratch_bytes(b->tpl.data(), nsec);
-    if (scratch > b->relayout.bytes()) b->relayout.alloc(scratch);
     refresh_probs(b);
 }
 
@@ -1264,9 +1273,9 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
     const int chk = std::max(1, o.check_every);
     const int64_t ld = cap + 1;
 
-    // Panel pointers are re-read here: a single-problem solve or SpMV of a
-    // member Hamiltonian may have reordered its panels (new buffers) since
-    // the batch was created.
+    // Layout pointers are re-read here: a single-problem solve or SpMV of a
+    // member Hamiltonian may have reordered its panels since the batch was
+    // created, and set_lanes changes the layout.
     refresh_probs(b);
     // Krylov blocks of all problems and the per-problem scalars (kept for the
     // next solve with the same lambda)
@@ -1486,7 +1495,8 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
         }
     } evguard{ev};
     const int kinds = (b->has_real ? 2 : 0) | (b->has_complex ? 1 : 0);  // which K1 launches a step has
-    if (!timed && (b->g_chk != chk || b->g_lpr != b->lpr || b->g_cap != cap || b->g_kinds != kinds || !b->gexec)) {
+    if (!timed && (b->g_chk != chk || b->g_lpr != b->lpr || b->g_cap != cap || b->g_kinds != kinds ||
+                   b->g_tab != b->tab_bytes || !b->gexec)) {
         if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
         if (b->graph) (void)hipGraphDestroy(b->graph);
         b->gexec = nullptr;
@@ -1499,6 +1509,7 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
         b->g_lpr = b->lpr;
         b->g_cap = cap;
         b->g_kinds = kinds;
+        b->g_tab = b->tab_bytes;
     }
     hipGraphExec_t gexec = b->gexec;
     const int zero = 0;

@@ -1,0 +1,176 @@
+// coded.hpp -- the coded Hamiltonian layout of the SpMV hot loops (built in
+// coded.hip) and its per-row sums.
+//
+// A matrix element is a sum of a few Coulomb table entries times a translation
+// phase, so a sector's entries take few distinct values: the 1,024 most
+// frequent magnitudes of a real sector and the 4,096 most frequent (|re|, |im|)
+// pairs of a complex one cover 99 % of the entries and more (N_phi = 12: 99.2 /
+// 99.4 %, N_phi = 14: 99.6 / 99.5 %, N_phi = 16 at half filling: 99.7 %).  Those values sit in a table that every workgroup
+// holds in LDS, and an entry is one 32-bit word: column within its panel in the
+// low 16 bits, table index above, sign of the real (and imaginary) part on top.  The matrix stream is 4 bytes an entry instead of 10 (real) or 18
+// (complex), bit for bit the same values.  Entries whose value is not in the
+// table form the rest: 32-bit column and value, one run per 64-row slice.
+//
+// Order: columns in panels of 65,536, 64-row slices; run (panel, slice) is
+// step-major: step t holds entry t of every row with more than t entries in the
+// panel, rows in order, columns ascending in a row.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <cstdint>
+
+#include "common.hpp"
+#include "panel.hpp"
+
+namespace blqh {
+
+constexpr int kCodReal = 1024;   // table entries of a real matrix (8 KiB of LDS), at most
+constexpr int kCodCplx = 4096;   // of a complex one (64 KiB)
+constexpr uint32_t kCodTun = 0x8000u;  // tunnelling flag of a shared-scale template's columns
+
+struct Coded {
+    bool built = false;
+    bool real = false;
+    int npan = 0;
+    int ntab = 0;
+    int64_t ncod = 0, nrest = 0;
+    DevBuf<double> tab;      // [ntab] |v|, or [2 ntab] (|re|, |im|)
+    DevBuf<int64_t> base;    // [npan * nslices + 1] first word of run p * nslices + s
+    DevBuf<uint16_t> len;    // [npan][nslices * 64] words of the row in the run
+    DevBuf<uint32_t> ent;    // [ncod]
+    DevBuf<int64_t> rbase;   // [nslices + 1]
+    DevBuf<uint16_t> rlen;   // [nslices * 64]
+    DevBuf<uint32_t> rcol;   // [nrest]
+    DevBuf<double> rval;     // [nrest] or [2 nrest]
+};
+
+struct CodView {
+    int64_t n, nslices;
+    int npan, ntab;
+    const double* tab;
+    const int64_t* base;
+    const uint16_t* len;
+    const uint32_t* ent;
+    const int64_t* rbase;
+    const uint16_t* rlen;
+    const uint32_t* rcol;
+    const double* rval;
+};
+
+inline CodView cview(const Coded& C, int64_t n) {
+    return CodView{n,           (n + 63) >> 6, C.npan,        C.ntab,       C.tab.get(),  C.base.get(),
+                   C.len.get(), C.ent.get(),   C.rbase.get(), C.rlen.get(), C.rcol.get(), C.rval.get()};
+}
+
+inline size_t cod_lds_bytes(bool real, int ntab) { return (size_t)(ntab > 0 ? ntab : 1) * (real ? 8 : 16); }
+
+// The value of word e: magnitudes from the LDS table, signs from the top bits.
+__device__ __forceinline__ double cod_sign(double v, uint32_t top) {  // top: sign in bit 31
+    return __hiloint2double(__double2hiint(v) ^ (int)(top & 0x80000000u), __double2loint(v));
+}
+__device__ __forceinline__ double cod_real(const double* tab, uint32_t e) {
+    return cod_sign(tab[(e >> 16) & 0x7fffu], e);
+}
+__device__ __forceinline__ double2 cod_cplx(const double2* tab, uint32_t e) {
+    const double2 v = tab[(e >> 16) & 0x3fffu];
+    return make_double2(cod_sign(v.x, e), cod_sign(v.y, e << 1));
+}
+
+// Table to LDS (the caller synchronises the workgroup).
+template <bool REAL>
+__device__ __forceinline__ void cod_stage(const double* __restrict__ tab, int ntab, double* lds, int nthreads) {
+    if (REAL) {
+        for (int i = threadIdx.x; i < ntab; i += nthreads) lds[i] = tab[i];
+    } else {
+        const double2* t = reinterpret_cast<const double2*>(tab);
+        double2* l = reinterpret_cast<double2*>(lds);
+        for (int i = threadIdx.x; i < ntab; i += nthreads) l[i] = t[i];
+    }
+}
+
+// Row sums of one run: lane l owns row l (`len` words); the step groups (U
+// steps each) are dealt to NP wavefronts, this one taking those with g mod NP
+// == par.  The words of the next group are loaded before the x gathers of the
+// current one, so a wavefront always has loads in flight.
+template <bool REAL, int NP, int U>
+__device__ __forceinline__ void cod_run_sum(const uint32_t* __restrict__ er, const double* tab,
+                                            const double2* __restrict__ xp, uint32_t len, int par, double& ar,
+                                            double& ai) {
+    uint32_t off = 0;
+    auto issue = [&](uint32_t t, uint32_t* e, bool& any) {
+        uint64_t m[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) m[u] = __ballot(t + u < len);
+        any = m[0] != 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t q = off + lanes_below(m[u]);
+            off += (uint32_t)__popcll(m[u]);
+            e[u] = t + u < len ? __builtin_nontemporal_load(&er[q]) : 0u;
+        }
+    };
+    auto skip = [&](uint32_t t) {  // another wave's group: advance the offset only
+#pragma unroll
+        for (int u = 0; u < U; ++u) off += (uint32_t)__popcll(__ballot(t + u < len));
+    };
+    uint32_t e0[U], e1[U];
+    bool any0, any1;
+    for (int g = 0; g < par; ++g) skip((uint32_t)(U * g));
+    uint32_t t0 = (uint32_t)(U * par);
+    issue(t0, e0, any0);
+    while (any0) {
+        const uint32_t t = t0 + (uint32_t)(U * NP);
+#pragma unroll
+        for (int g = NP - 1; g > 0; --g) skip(t - (uint32_t)(U * g));
+        issue(t, e1, any1);
+        double2 xv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) xv[u] = xp[e0[u] & 0xffffu];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool act = t0 + u < len;
+            if (REAL) {
+                const double v = act ? cod_real(tab, e0[u]) : 0.0;
+                ar += v * xv[u].x;
+                ai += v * xv[u].y;
+            } else {
+                double2 v = cod_cplx(reinterpret_cast<const double2*>(tab), e0[u]);
+                if (!act) v = make_double2(0.0, 0.0);
+                ar += v.x * xv[u].x - v.y * xv[u].y;
+                ai += v.x * xv[u].y + v.y * xv[u].x;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) e0[u] = e1[u];
+        any0 = any1;
+        t0 = t;
+    }
+}
+
+// The rest of a slice: one step at a time (about one entry a row), step t to
+// the wavefront t mod NP.
+template <bool REAL, int NP>
+__device__ __forceinline__ void cod_rest_sum(const uint32_t* __restrict__ rc, const double* __restrict__ rv,
+                                             const double2* __restrict__ x, uint32_t len, int par, double& ar,
+                                             double& ai) {
+    uint32_t off = 0;
+    for (uint32_t t = 0;; ++t) {
+        const uint64_t m = __ballot(t < len);
+        if (m == 0) break;
+        if ((NP == 1 || (int)(t % NP) == par) && t < len) {
+            const uint32_t q = off + lanes_below(m);
+            const double2 xv = x[rc[q]];
+            if (REAL) {
+                const double v = rv[q];
+                ar += v * xv.x;
+                ai += v * xv.y;
+            } else {
+                const double2 v = reinterpret_cast<const double2*>(rv)[q];
+                ar += v.x * xv.x - v.y * xv.y;
+                ai += v.x * xv.y + v.y * xv.x;
+            }
+        }
+        off += (uint32_t)__popcll(m);
+    }
+}
+
+}  // namespace blqh

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "bits.hpp"
+#include "coded.hpp"
 #include "common.hpp"
 #include "panel.hpp"
 #include "rowterms.hpp"
@@ -48,13 +49,16 @@ struct blqh_hamil {
         blqh::DevBuf<int32_t> perm;      // perm[i]: internal position of reference row i
         blqh::DevBuf<int32_t> iperm;     // iperm[r]: reference row at internal position r
         std::vector<int32_t> h_iperm;
+        bool csr = false;                // the three arrays below exist (ensure_panels)
         blqh::DevBuf<int64_t> rowptr;    // the CSR in internal order, columns ascending
         blqh::DevBuf<int32_t> col;
         blqh::DevBuf<double2> val;
     } ord;
-    blqh::Panels pan;                // panel-major copy for the SpMV hot loop
+    blqh::Coded cod;                 // coded copy for the SpMV hot loops (coded.hpp)
+    blqh::Panels pan;                // panel-major copy of SpMV kinds 1 to 5 and batch lanes below 64, on demand
     blqh::Tiles til;                 // column-tile copy (SpMV kind 4), built on demand
-    int spmv_kind = -1;              // autotuned SpMV: 0 = row-major CSR, 1 = panel-major (-1 = not tuned)
+    int row_max = 0;                 // entries of the longest row (0: unknown)
+    int spmv_kind = -1;              // SpMV variant in use (-1: none chosen yet)
     int spmv_lpr = 0;                // lanes per row of the chosen kernel
     int spmv_threads = 0;            // workgroup size of the panel kernel
     int spmv_wgs_per_cu = 0;         // persistent workgroups per CU (panel kernel)
@@ -113,12 +117,16 @@ struct HostTables {
     double Ec = 0;
 };
 HostTables host_tables(const blqh_sector& s, const blqh_params& p);
-void build_panels(blqh_hamil* H);
-// The SpMV formats of H (internal-order CSR, panels): built with a full
-// Hamiltonian or a merge, on first use (or blqh_hamil_prepare) for the parts
-// of a merge (terms 1 and 2), which often only feed blqh_hamil_combine or a
-// shared-scale batch and never need them.
+// The coded SpMV layout of H: built with a full Hamiltonian or a merge, on first
+// use (or blqh_hamil_prepare) for the parts of a merge (terms 1 and 2), which often
+// only feed blqh_hamil_combine or a shared-scale batch and never need it.  nu:
+// see k_cod_rows; *ntun receives the number of flagged entries.
+void build_coded(blqh_hamil* H, const uint8_t* nu, int64_t* ntun);
+void ensure_coded(blqh_hamil* H);
+// The internal-order CSR and the panels, read by SpMV kinds 0 to 5 and the batch
+// lanes below 64 only: built when one of them is asked for.
 void ensure_panels(blqh_hamil* H);
+void launch_absmax(int64_t nnz, const double2* val, unsigned long long* out, hipStream_t st);
 // Column-tile layout for SpMV kind 4 on `G` workgroups; returns false (and
 // builds nothing) when the matrix does not fit it.
 bool build_tiles(blqh_hamil* H, int G);
@@ -139,14 +147,15 @@ void set_panel_layouts(blqh_hamil* const* hs, int count, bool jagged, void* scra
                        bool greedy, int rows = 1);
 size_t panel_layout_scratch_bytes(blqh_hamil* const* hs, int count);
 
-// The CSR that the SpMV formats are built from and the CSR kernel reads:
-// the internal order's when it is on, else the Hamiltonian's own.
+// The CSR that the panels are built from and the CSR kernel reads: the internal
+// order's when it is on (ensure_panels has built it), else the Hamiltonian's own.
 struct CsrView {
     const int64_t* rowptr;
     const int32_t* col;
     const double2* val;
 };
 inline CsrView spmv_csr(const blqh_hamil* H) {
+    BLQH_REQUIRE(!H->ord.on || H->ord.csr, BLQH_EINTERNAL, "internal-order CSR not built");
     if (H->ord.on) return CsrView{H->ord.rowptr.get(), H->ord.col.get(), H->ord.val.get()};
     return CsrView{H->rowptr.get(), H->col.get(), H->val.get()};
 }

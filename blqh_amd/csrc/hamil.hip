@@ -721,6 +721,7 @@ void blqh_hamil_build_impl(const blqh_basis* B, const blqh_params& p_in, blqh_ha
         BLQH_REQUIRE(h_ctr[1] == 0, BLQH_ERANGE, "a Hamiltonian row has more than 4096 distinct columns");
         row_max = std::max(row_max, h_ctr[3]);
     }
+    H->row_max = row_max;
     // rows of a build with the pair terms size the hash of later builds over this basis
     if (terms & 1) {
         int32_t cur = B->max_row_nnz.load();
@@ -763,9 +764,9 @@ void blqh_hamil_build_impl(const blqh_basis* B, const blqh_params& p_in, blqh_ha
     BLQH_REQUIRE((single ? e1[2] == 0 : e1[2] == novf) && e2[2] == 0, BLQH_EINTERNAL,
                  "count and fill passes disagree");
     phase(3);
-    // the SpMV formats (internal order, panels): now for a full Hamiltonian,
+    // the SpMV layout: now for a full Hamiltonian,
     // on first use for the parts of a merge, which may never need them
-    if (terms == 3) build_panels(H);
+    if (terms == 3) ensure_coded(H);
     phase(4);
     H->seconds_build = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     if (timing)
@@ -839,7 +840,7 @@ __global__ void __launch_bounds__(256) k_combine_fill(int64_t n, const int64_t* 
 
 }  // namespace
 
-void blqh_hamil_combine_impl(const blqh_hamil* base, const blqh_hamil* tun, double dsas, blqh_hamil* H) {
+void blqh_hamil_combine_impl(const blqh_hamil* base, const blqh_hamil* tun, double dsas, blqh_hamil* H, bool formats) {
     using namespace blqh;
     BLQH_REQUIRE(base->terms == 1 || (base->terms == 3 && base->par.delta_sas == 0.0), BLQH_EINVAL,
                  "the base must be built without tunnelling (Delta_SAS = 0)");
@@ -879,6 +880,7 @@ void blqh_hamil_combine_impl(const blqh_hamil* base, const blqh_hamil* tun, doub
     BLQH_HIP(hipMemcpyAsync(&herr, err.get(), sizeof(int32_t), hipMemcpyDeviceToHost, st));
     BLQH_HIP(hipStreamSynchronize(st));
     BLQH_REQUIRE(herr == 0, BLQH_EINTERNAL, "tunnelling and Coulomb entries overlap");
-    build_panels(H);
+    H->row_max = base->row_max + tun->row_max;
+    if (formats) ensure_coded(H);
     H->seconds_build = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
 }

@@ -766,6 +766,65 @@ __global__ void __launch_bounds__(kT4Threads) k_t4(TileView V, const double2* __
     if (LZ) block_partial(dacc, partials);
 }
 
+// ---- coded SpMV (kind 6) ---------------------------------------------------------------
+// The coded layout (coded.hpp): a matrix entry is 4 bytes, its value comes from
+// the table in LDS.  A team of NP wavefronts owns a 64-row slice (lane l <-> row l)
+// and shares its step groups; a workgroup holds WPB / NP teams on neighbouring
+// slices, which gather from the same lines of x.
+template <bool REAL, bool LZ, int WPB, int NP>
+__global__ void __launch_bounds__(WPB * 64) k_cod(CodView P, const double2* __restrict__ x, double2* __restrict__ out,
+                                                  const double2* __restrict__ Wp, Scal sc, int j, double* partials) {
+    extern __shared__ __align__(16) double ctab[];
+    __shared__ double2 red[NP > 1 ? WPB * 64 : 1];  // the wavefronts' shares of their rows
+    constexpr int TM = WPB / NP, U = 8;
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, par = wv % NP;
+    const int64_t n = P.n, nsl = P.nslices;
+    const int64_t sl = (int64_t)blockIdx.x * TM + wv / NP, row = sl * 64 + lane;
+    cod_stage<REAL>(P.tab, P.ntab, ctab, WPB * 64);
+    __syncthreads();
+    double2 y = make_double2(0.0, 0.0);
+    for (int p = 0; p < P.npan; ++p) {
+        if (P.npan > 1) __syncthreads();  // keep the workgroup on one panel
+        if (sl >= nsl) continue;      // uniform over the wavefront
+        const int64_t run = (int64_t)p * nsl + sl;
+        cod_run_sum<REAL, NP, U>(P.ent + P.base[run], ctab, x + (int64_t)p * kPanelWidth,
+                                 P.len[run * 64 + lane], par, y.x, y.y);
+    }
+    if (sl < nsl) {
+        const int64_t q0 = P.rbase[sl];
+        cod_rest_sum<REAL, NP>(P.rcol + q0, P.rval + q0 * (REAL ? 1 : 2), x, P.rlen[row], par, y.x, y.y);
+    }
+    if (NP > 1) {
+        red[threadIdx.x] = y;
+        __syncthreads();
+    }
+    double dacc = 0.0;
+    if (par == 0 && sl < nsl && row < n) {
+#pragma unroll
+        for (int q = 1; q < NP; ++q) {  // the team's shares in wavefront order
+            const double2 o = red[threadIdx.x + q * 64];
+            y.x += o.x;
+            y.y += o.y;
+        }
+        if (LZ) {
+            const double ib = sc.invb[j];
+            double ur = ib * y.x, ui = ib * y.y;
+            if (j > 0) {
+                const double cp = sc.beta[j] * sc.invb[j - 1];
+                const double2 q = Wp[row];
+                ur -= cp * q.x;
+                ui -= cp * q.y;
+            }
+            out[row] = make_double2(ur, ui);
+            const double2 w = x[row];
+            dacc = w.x * ur + w.y * ui;
+        } else {
+            out[row] = y;
+        }
+    }
+    if (LZ) block_partial(dacc, partials);
+}
+
 // ---- launch helpers -----------------------------------------------------------
 int vec_grid(int64_t n) {
     const int ncu = runtime().num_cus;
@@ -952,8 +1011,55 @@ void t4_dispatch(const blqh_hamil* H, const double2* x, double2* out, const doub
     throw Error(BLQH_EINTERNAL, "unsupported column-tile SpMV layout");
 }
 
+// workgroups of pl.threads / 64 wavefronts, teams of pl.rows
+int cod_grid(const blqh_hamil* H, const Plan& pl) {
+    return (int)ceil_div(ceil_div(H->n, 64), (int64_t)(pl.threads / 64 / pl.rows));
+}
+
+template <bool REAL, bool LZ, int WPB, int NP>
+void cod_go(const blqh_hamil* H, const Plan& pl, const double2* x, double2* out, const double2* Wp, const Scal& sc,
+            int j, double* partials, hipStream_t st) {
+    auto kern = k_cod<REAL, LZ, WPB, NP>;
+    static const bool attr = [&] {  // once per instantiation, thread-safe
+        BLQH_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     (int)cod_lds_bytes(REAL, REAL ? kCodReal : kCodCplx)));
+        return true;
+    }();
+    (void)attr;
+    hipLaunchKernelGGL(kern, dim3(cod_grid(H, pl)), dim3(WPB * 64), cod_lds_bytes(REAL, H->cod.ntab), st,
+                       cview(H->cod, H->n), x, out, Wp, sc, j, partials);
+}
+
+template <bool LZ>
+void cod_dispatch(const blqh_hamil* H, const Plan& pl, const double2* x, double2* out, const double2* Wp,
+                  const Scal& sc, int j, double* partials, hipStream_t st) {
+    BLQH_REQUIRE(H->cod.built, BLQH_EINTERNAL, "coded SpMV without its layout");
+#define BLQH_COD_CASE(WPB, NP)                                                                \
+    if (pl.threads == WPB * 64 && pl.rows == NP) {                                            \
+        if (H->cod.real) cod_go<true, LZ, WPB, NP>(H, pl, x, out, Wp, sc, j, partials, st);   \
+        else cod_go<false, LZ, WPB, NP>(H, pl, x, out, Wp, sc, j, partials, st);              \
+        return;                                                                               \
+    }
+    BLQH_COD_CASE(4, 1) BLQH_COD_CASE(4, 2) BLQH_COD_CASE(4, 4)
+    BLQH_COD_CASE(8, 1) BLQH_COD_CASE(8, 2) BLQH_COD_CASE(8, 4) BLQH_COD_CASE(8, 8)
+    BLQH_COD_CASE(16, 1) BLQH_COD_CASE(16, 2) BLQH_COD_CASE(16, 4) BLQH_COD_CASE(16, 8)
+    BLQH_COD_CASE(16, 16)
+#undef BLQH_COD_CASE
+    throw Error(BLQH_EINTERNAL, "unsupported coded SpMV plan");
+}
+
+// The coded plan of a matrix by its size.
+Plan coded_plan(const blqh_hamil* H) {
+    const int64_t nsl = ceil_div(H->n, 64);
+    int np = 1;
+    while (np < 8 && nsl * np * 2 <= 24576) np *= 2;
+    return Plan{6, 64, 512, 0, np};
+}
+
 void launch_spmv_plan(const blqh_hamil* H, const Plan& pl, const double2* x, double2* y, hipStream_t st) {
-    if (pl.kind == 5) {
+    if (pl.kind == 6) {
+        cod_dispatch<false>(H, pl, x, y, nullptr, Scal{}, 0, nullptr, st);
+    } else if (pl.kind == 5) {
         jagr_dispatch<false>(H, pl, x, y, nullptr, Scal{}, 0, nullptr, st);
     } else if (pl.kind == 4) {
         t4_dispatch<false>(H, x, y, nullptr, Scal{}, 0, nullptr, st);
@@ -972,6 +1078,7 @@ void launch_spmv_plan(const blqh_hamil* H, const Plan& pl, const double2* x, dou
 
 // grid size (for partial-sum buffers) of the fused K1 under a plan
 int lz1_grid(const blqh_hamil* H, const Plan& pl) {
+    if (pl.kind == 6) return cod_grid(H, pl);
     if (pl.kind == 4) return H->til.G;
     if (pl.kind == 5) return jagr_grid(H, pl);
     return pl.kind >= 2 ? sps_grid(H, pl) : pl.kind == 1 ? panel_launch(H, pl).grid : spmv_grid(H->n, pl.lpr);
@@ -979,7 +1086,9 @@ int lz1_grid(const blqh_hamil* H, const Plan& pl) {
 
 void launch_lz1(const blqh_hamil* H, const Plan& pl, const double2* W, const double2* Wp, double2* u, const Scal& sc,
                 int j, double* partials, hipStream_t st) {
-    if (pl.kind == 5) {
+    if (pl.kind == 6) {
+        cod_dispatch<true>(H, pl, W, u, Wp, sc, j, partials, st);
+    } else if (pl.kind == 5) {
         jagr_dispatch<true>(H, pl, W, u, Wp, sc, j, partials, st);
     } else if (pl.kind == 4) {
         t4_dispatch<true>(H, W, u, Wp, sc, j, partials, st);
@@ -996,67 +1105,50 @@ void launch_lz1(const blqh_hamil* H, const Plan& pl, const double2* W, const dou
     }
 }
 
-// Shape of a tuned matrix (the plan cache's key).
-struct TuneKey {
-    int npan, real, lg_n, lg_row;  // log2 of rows and of the mean row length, in quarters
-    bool operator==(const TuneKey& o) const {
-        return npan == o.npan && real == o.real && lg_n == o.lg_n && lg_row == o.lg_row;
-    }
-};
-std::mutex g_tune_mu;
-std::vector<std::pair<TuneKey, Plan>> g_tune_cache;  // most recent last, at most 64
+void set_plan(blqh_hamil* H, const Plan& p) {
+    H->spmv_kind = p.kind;
+    H->spmv_lpr = p.lpr;
+    H->spmv_threads = p.threads;
+    H->spmv_wgs_per_cu = p.wpc;
+    H->spmv_rows = p.rows;
+}
 
-// Autotuner: time every variant on this matrix (random x) and keep the fastest.
-void tune(blqh_hamil* H) {
-    // BLQH_SPMV_PLAN="kind,lanes,threads,wgs_per_cu,rows" pins a variant (profiling, reproducibility)
+// The variant of a matrix that has none pinned: the coded layout's, by size
+// (coded_plan).  BLQH_SPMV_PLAN="kind,lanes,threads,wgs_per_cu,rows" pins one
+// (profiling, reproducibility); BLQH_TUNE_ALL=1 times every kind on the matrix
+// (random x) and keeps the fastest.
+void choose_plan(blqh_hamil* H) {
     if (const char* env = std::getenv("BLQH_SPMV_PLAN")) {
         Plan p{};
-        if (std::sscanf(env, "%d,%d,%d,%d,%d", &p.kind, &p.lpr, &p.threads, &p.wpc, &p.rows) == 5 &&
-            (p.kind == 0 || H->pan.built) && (p.kind != 4 || build_tiles(H, runtime().num_cus))) {
-            H->spmv_kind = p.kind;
-            H->spmv_lpr = p.lpr;
-            H->spmv_threads = p.threads;
-            H->spmv_wgs_per_cu = p.wpc;
-            H->spmv_rows = p.rows;
-            return;
-        }
-    }
-    // A matrix of the shape of one tuned before (same panels and value kind,
-    // rows and mean row length within 19 %) takes that plan without timing:
-    // the sectors of a sweep tune once.  BLQH_TUNE_CACHE=0 times every matrix.
-    const double mean_row = H->n ? (double)H->nnz / H->n : 0;
-    const char* cenv = std::getenv("BLQH_TUNE_CACHE");
-    const bool use_cache = !(cenv && cenv[0] == '0');
-    const TuneKey key{H->pan.built ? H->pan.npan : 0, H->pan.real ? 1 : 0,
-                      (int)std::lround(4.0 * std::log2((double)std::max<int64_t>(H->n, 1))),
-                      (int)std::lround(4.0 * std::log2(std::max(mean_row, 1.0)))};
-    if (use_cache) {
-        std::lock_guard<std::mutex> lk(g_tune_mu);
-        for (const auto& e : g_tune_cache)
-            if (e.first == key && (e.second.kind == 0 || H->pan.built)) {
-                const Plan& p = e.second;
-                H->spmv_kind = p.kind;
-                H->spmv_lpr = p.lpr;
-                H->spmv_threads = p.threads;
-                H->spmv_wgs_per_cu = p.wpc;
-                H->spmv_rows = p.rows;
+        if (std::sscanf(env, "%d,%d,%d,%d,%d", &p.kind, &p.lpr, &p.threads, &p.wpc, &p.rows) == 5) {
+            if (p.kind != 6) ensure_panels(H);
+            const bool ok = p.kind != 6 || (p.rows >= 1 && p.rows * 64 <= p.threads);
+            if (ok && (p.kind != 4 || build_tiles(H, runtime().num_cus))) {
+                set_plan(H, p);
                 return;
             }
+        }
     }
+    const char* aenv = std::getenv("BLQH_TUNE_ALL");
+    if (!(aenv && aenv[0] == '1')) {
+        set_plan(H, coded_plan(H));
+        return;
+    }
+    ensure_coded(H);
+    ensure_panels(H);
+    const double mean_row = H->n ? (double)H->nnz / H->n : 0;
     hipStream_t st = stream();
     std::vector<Plan> cands;
     for (int lpr : {4, 8, 16, 32, 64})
         if (!(lpr > 4 * mean_row + 8 && lpr > 8)) cands.push_back(Plan{0, lpr, kThreads, 0, 0});
-    // Kinds 1, 2, 4 and 5 never won on any measured matrix (79 to 2.35M rows);
-    // BLQH_TUNE_ALL=1 times them too.
-    const char* aenv = std::getenv("BLQH_TUNE_ALL");
-    const bool all_kinds = aenv && aenv[0] == '1';
-    if (H->pan.built && all_kinds)
+    for (int pt : {256, 512, 1024})
+        for (int np = 1; np <= pt / 64; np *= 2) cands.push_back(Plan{6, 64, pt, 0, np});
+    if (H->pan.built)
         for (int pt : {512, 1024})
             for (int lpr : {4, 8, 16})
                 for (int wpc : {1, 2})
                     for (int u : {2, 4}) cands.push_back(Plan{1, lpr, pt, wpc, u});
-    if (H->pan.built && all_kinds)
+    if (H->pan.built)
         for (int pt : {512, 1024})
             for (int wpc : {1, 2, 4}) {
                 // slices per wavefront: the smallest supported count that covers the matrix in one round
@@ -1067,7 +1159,7 @@ void tune(blqh_hamil* H) {
                 cands.push_back(Plan{2, 64, pt, wpc, ms});
             }
     // column tiles: an x tile per LDS, worth it when x does not fit the caches
-    if (H->pan.built && all_kinds && H->n > 4 * kTileCols && build_tiles(H, runtime().num_cus))
+    if (H->pan.built && H->n > 4 * kTileCols && build_tiles(H, runtime().num_cus))
         cands.push_back(Plan{4, 64, kT4Threads, 1, H->til.R});
     if (H->pan.built)  // jagged kernel last: one layout conversion
         for (int pt : {256, 512, 1024})
@@ -1078,7 +1170,7 @@ void tune(blqh_hamil* H) {
                 while (ms < need && ms < 8) ms <<= 1;
                 cands.push_back(Plan{3, 64, pt, wpc, ms});
             }
-    if (H->pan.built && all_kinds)  // R rows per lane: one layout conversion per R
+    if (H->pan.built)  // R rows per lane: one layout conversion per R
         for (int R : {2, 4, 8})
             for (int pt : {512, 1024})
                 for (int wpc : {1, 2}) {
@@ -1115,7 +1207,7 @@ void tune(blqh_hamil* H) {
     }
     const bool log = std::getenv("BLQH_TUNE_LOG") != nullptr;  // print the timing of every variant
     for (const Plan& pl : cands) {
-        if (pl.kind >= 1) set_panel_layout(H, pl.kind == 3 || pl.kind == 5, nullptr, 0, pl.kind == 5 ? pl.lpr : 1);
+        if (pl.kind >= 1 && pl.kind <= 5) set_panel_layout(H, pl.kind == 3 || pl.kind == 5, nullptr, 0, pl.kind == 5 ? pl.lpr : 1);
         launch_spmv_plan(H, pl, x.get(), y.get(), st);  // warm
         BLQH_HIP(hipEventRecord(e0, st));
         for (int r = 0; r < reps; ++r) launch_spmv_plan(H, pl, x.get(), y.get(), st);
@@ -1133,7 +1225,7 @@ void tune(blqh_hamil* H) {
     // a whole workgroup on one panel, so bigger workgroups hold a smaller x
     // working set per CU (2.35M-state N_phi = 16 sector: 1024 x 1 moves 13.5 GB per launch where
     // 512 x 2 moves 23 GB, in the same time).
-    if (bp.kind >= 2)
+    if (bp.kind >= 2 && bp.kind <= 5)
         for (const auto& c : timed)
             if (c.first.kind == bp.kind && c.second <= best * 1.02f &&
                 (c.first.threads > bp.threads || (c.first.threads == bp.threads && c.first.wpc < bp.wpc)))
@@ -1141,25 +1233,14 @@ void tune(blqh_hamil* H) {
     BLQH_HIP(hipGetLastError());
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    H->spmv_kind = bp.kind;
-    H->spmv_lpr = bp.lpr;
-    H->spmv_threads = bp.threads;
-    H->spmv_wgs_per_cu = bp.wpc;
-    H->spmv_rows = bp.rows;
-    if (use_cache) {
-        std::lock_guard<std::mutex> lk(g_tune_mu);
-        if (g_tune_cache.size() >= 64) g_tune_cache.erase(g_tune_cache.begin());
-        g_tune_cache.push_back({key, bp});
-    }
+    set_plan(H, bp);
 }
 
-// Tunes on first use (unless a variant is pinned) and puts the panels in the
-// entry order the chosen kernel reads; the column-tile copy is released when
-// another variant won.
+// Chooses the variant on first use (unless one is pinned) and puts its layout in
+// place; the column-tile copy is released when another variant won.
 void autotune(blqh_hamil* H) {
-    ensure_panels(H);
     if (H->spmv_kind < 0) {
-        tune(H);
+        choose_plan(H);
         if (H->spmv_kind != 4 && H->til.built) {
             Tiles& T = H->til;
             T.len.release();
@@ -1171,6 +1252,8 @@ void autotune(blqh_hamil* H) {
             T.tried = false;
         }
     }
+    if (H->spmv_kind == 6) ensure_coded(H);
+    else ensure_panels(H);
     if ((H->spmv_kind >= 1 && H->spmv_kind <= 3) || H->spmv_kind == 5)
         set_panel_layout(H, H->spmv_kind == 3 || H->spmv_kind == 5, nullptr, 0, H->spmv_kind == 5 ? H->spmv_lpr : 1);
 }
@@ -1771,24 +1854,26 @@ __global__ void __launch_bounds__(1024) k_mt_start(int64_t n, uint32_t seed, dou
 }
 
 // The SpMV plan the Hamiltonian's current layout supports without any
-// conversion (the tuned one when its layout is in place, else the CSR
-// kernel, whose arrays always exist).
+// conversion: the chosen one when its layout is in place, else the coded one,
+// else (a part of a merge without formats) the CSR kernel.
 Plan noalloc_plan(const blqh_hamil* H) {
     if (H->spmv_kind >= 0) {
         const Plan p = plan_of(H);
         const Panels& P = H->pan;
         bool ok = false;
         switch (p.kind) {
-            case 0: ok = true; break;
+            case 0: ok = !H->ord.on || H->ord.csr; break;
             case 1:
             case 2: ok = P.built && !P.jagged; break;
             case 3: ok = P.built && P.jagged && P.greedy == greedy_step_order() && P.rows == 1; break;
             case 4: ok = H->til.built; break;
             case 5: ok = P.built && P.jagged && P.rows == p.lpr; break;
+            case 6: ok = H->cod.built; break;
             default: break;
         }
         if (ok) return p;
     }
+    if (H->cod.built) return coded_plan(H);
     const double mean = H->n ? (double)H->nnz / (double)H->n : 0.0;
     int lpr = 4;
     while (lpr < 64 && 4.0 * lpr < mean) lpr *= 2;

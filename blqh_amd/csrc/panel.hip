@@ -823,10 +823,10 @@ __global__ void k_ord_scatter(int64_t n, const int32_t* __restrict__ iperm, cons
 int ord_grid(int64_t n) { return (int)std::min<int64_t>(std::max<int64_t>(ceil_div(n, kBlk), 1), 65536); }
 }  // namespace
 
-// The internal CSR of H from its CSR and the basis order (no-op for the identity order).
+// Row order of H's SpMV formats from the basis order (no-op for the identity order).
 void build_order(blqh_hamil* H) {
     blqh_hamil::Order& O = H->ord;
-    O.on = false;
+    if (O.on) return;
     const std::vector<int32_t>& perm = internal_order(H->basis);
     if (perm.empty()) return;
     const int64_t n = H->n;
@@ -838,6 +838,16 @@ void build_order(blqh_hamil* H) {
     O.iperm.alloc(n);
     BLQH_HIP(hipMemcpyAsync(O.perm.get(), perm.data(), n * 4, hipMemcpyHostToDevice, st));
     BLQH_HIP(hipMemcpyAsync(O.iperm.get(), O.h_iperm.data(), n * 4, hipMemcpyHostToDevice, st));
+    O.on = true;
+}
+
+namespace {
+// The CSR of H with rows and columns in the internal order.
+void build_order_csr(blqh_hamil* H) {
+    blqh_hamil::Order& O = H->ord;
+    if (!O.on || O.csr) return;
+    hipStream_t st = stream();
+    const int64_t n = H->n;
     DevBuf<int32_t> len(n);
     DevBuf<int32_t> err(1);
     BLQH_HIP(hipMemsetAsync(err.get(), 0, 4, st));
@@ -858,8 +868,9 @@ void build_order(blqh_hamil* H) {
     BLQH_HIP(hipStreamSynchronize(st));
     BLQH_REQUIRE(herr == 0, BLQH_EINTERNAL, "a CSR row is longer than the internal-order kernel handles");
     BLQH_REQUIRE(tot == H->nnz, BLQH_EINTERNAL, "internal CSR size differs");
-    O.on = true;
+    O.csr = true;
 }
+}  // namespace
 
 void order_to_internal(const blqh_hamil* H, const double2* src, double2* dst, hipStream_t st) {
     if (!H->ord.on) {
@@ -879,12 +890,18 @@ void order_to_reference(const blqh_hamil* H, const double2* src, double2* dst, h
     BLQH_HIP(hipGetLastError());
 }
 
-void ensure_panels(blqh_hamil* H) {
-    if (!H->pan.built) build_panels(H);
+// max |re| and max |im| of the values into out[0], out[1] (bits of non-negative
+// doubles; the caller has cleared them)
+void launch_absmax(int64_t nnz, const double2* val, unsigned long long* out, hipStream_t st) {
+    const int g = (int)std::min<int64_t>(std::max<int64_t>(ceil_div(nnz, kBlk * 8), 1), 2048);
+    hipLaunchKernelGGL(k_absmax, dim3(g), dim3(kBlk), 0, st, nnz, val, out);
+    BLQH_HIP(hipGetLastError());
 }
 
-void build_panels(blqh_hamil* H) {
+void ensure_panels(blqh_hamil* H) {
+    if (H->pan.built) return;
     build_order(H);
+    build_order_csr(H);
     const CsrView A = spmv_csr(H);
     hipStream_t st = stream();
     const int64_t n = H->n;
@@ -893,8 +910,7 @@ void build_panels(blqh_hamil* H) {
     P.npan = npan;
     DevBuf<unsigned long long> mx(2);
     BLQH_HIP(hipMemsetAsync(mx.get(), 0, 16, st));
-    const int g = (int)std::min<int64_t>(std::max<int64_t>(ceil_div(H->nnz, kBlk * 8), 1), 2048);
-    hipLaunchKernelGGL(k_absmax, dim3(g), dim3(kBlk), 0, st, H->nnz, A.val, mx.get());
+    launch_absmax(H->nnz, A.val, mx.get(), st);
     unsigned long long hm[2];
     BLQH_HIP(hipMemcpyAsync(hm, mx.get(), 16, hipMemcpyDeviceToHost, st));
     BLQH_HIP(hipStreamSynchronize(st));

@@ -139,9 +139,16 @@ int blqh_spmv_device(const blqh_hamil* h, const void* x_dev, void* y_dev); /* de
  * `wgs_per_cu` 1-4, `rows` = blocks per wavefront and round with
  * R * rows <= 8.  Kind 3 orders each step greedily (lanes that read the same
  * x cache line share a step), kind 5 keeps each row's entries in order.
- * get: kind = -1 until
- * the autotuner has run (first SpMV or solve).  set: pins a variant (returns
- * BLQH_EINVAL for an unsupported one); kind = -1 re-arms the autotuner. */
+ * kind 6 (the default): the coded layout, 4 bytes per entry (16-bit column
+ * within a 65536-column panel, index of the value in a table held in LDS,
+ * signs; the few values outside the table are kept whole), lanes = 64,
+ * `threads` 256, 512 or 1024, `rows` = 1, 2, 4, 8 or 16 wavefronts sharing a
+ * 64-row slice (rows * 64 <= threads), `wgs_per_cu` unused.  The panels of
+ * kinds 1-5 are built when one of them is asked for.
+ * get: kind = -1 until the first SpMV or solve.  set: pins a variant (returns
+ * BLQH_EINVAL for an unsupported one); kind = -1 returns to the default,
+ * whose team size follows the number of rows (BLQH_TUNE_ALL=1 in the
+ * environment times every kind instead). */
 int blqh_hamil_get_spmv(const blqh_hamil* h, int32_t* kind, int32_t* lanes, int32_t* threads, int32_t* wgs_per_cu,
                         int32_t* rows);
 int blqh_hamil_set_spmv(blqh_hamil* h, int32_t kind, int32_t lanes, int32_t threads, int32_t wgs_per_cu,

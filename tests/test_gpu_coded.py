@@ -1,0 +1,69 @@
+"""The coded layout (SpMV kind 6: 4-byte entries whose values come from a table)
+against scipy's CSR product of the exported matrix, at its edges: fewer rows than
+a slice, a ragged last slice, one column panel and several, real and complex
+values, a matrix whose values the table covers badly, each team size."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+import blqh_amd
+
+pytestmark = pytest.mark.gpu
+
+PLANS = [(6, 64, t, 0, r) for t in (256, 512, 1024) for r in (1, 2, 4, 8, 16) if r * 64 <= t]
+
+# (name, (nspecies, nphi, nel, nel_up, nel_su, J, K), params)
+SECTORS = [
+    ("one_slice_real", (2, 4, 4, 2, -1, 0, 0), dict(d=1.0)),
+    ("ragged_real", (2, 8, 8, 4, -1, 4, 4), dict(d=3.0)),
+    ("ragged_complex", (2, 8, 8, -1, -1, 1, 3), dict(d=1.0, delta_sas=0.05)),
+    ("twisted_many_values", (2, 10, 10, -1, -1, 3, 2), dict(d=0.7, delta_sas=0.05, theta_x=0.3, theta_y=1.1)),
+    ("spinful_complex", (4, 6, 6, 3, 3, 0, 1), dict(d=1.0, delta_sas=0.05, delta_v=0.02, delta_z=0.01)),
+    ("panels_real", (2, 14, 14, -1, -1, 0, 0), dict(d=1.0, delta_sas=0.05)),
+    ("panels_complex", (2, 14, 14, -1, -1, 0, 3), dict(d=0.5, delta_sas=0.05)),
+]
+
+
+@pytest.fixture(scope="module", params=SECTORS, ids=[s[0] for s in SECTORS])
+def built(request):
+    name, (S, nphi, nel, nu, nsu, J, K), kw = request.param
+    B = blqh_amd.Basis(nphi, nel, nu, J, K, nspecies=S, nel_su=nsu)
+    H = blqh_amd.Hamiltonian(B, blqh_amd.params(nphi, **kw))
+    print(f"sector {name} n {H.n}", flush=True)
+    rp, col, val = H.export()
+    return name, B, H, sp.csr_matrix((val, col, rp), shape=(H.n, H.n))
+
+
+@pytest.mark.parametrize("plan", PLANS, ids=[f"t{p[2]}_np{p[4]}" for p in PLANS])
+def test_product(built, plan):
+    name, B, H, A = built
+    print(f"{name} n={H.n} plan {plan}", flush=True)
+    H.set_spmv(*plan)
+    rng = np.random.default_rng(1)
+    x = rng.normal(size=H.n) + 1j * rng.normal(size=H.n)
+    scale = np.abs(A).max() * np.abs(x).max() * np.diff(A.indptr).max()
+    np.testing.assert_allclose(H.spmv(x), A @ x, rtol=0, atol=2e-15 * scale)
+    assert H.get_spmv()[0] == 6
+
+
+def test_default_matches_csr_solver(built):
+    """The default plan's ground state is the CSR kernel's: the values are the same bits,
+    only the order of a row's sum differs."""
+    name, B, H, A = built
+    if H.n < 8:
+        pytest.skip("too few states for a set number of steps")
+    print(f"{name} n={H.n} Lanczos", flush=True)
+    H.set_spmv(-1)
+    a = H.lanczos(lam=120, seed=5)
+    assert H.get_spmv()[0] == 6
+    H.set_spmv(0, 16)
+    b = H.lanczos(lam=120, seed=5)
+    assert a["E0"] == pytest.approx(b["E0"], rel=1e-10, abs=1e-12)
+    assert a["E_rq"] == pytest.approx(b["E_rq"], rel=1e-10, abs=1e-12)
+
+
+def test_refused_plans(built):
+    name, B, H, A = built
+    for bad in ((6, 32, 512, 0, 2), (6, 64, 128, 0, 1), (6, 64, 256, 0, 8), (6, 64, 512, 0, 3), (6, 64, 512, 0, 0)):
+        with pytest.raises(blqh_amd.BlqhError):
+            H.set_spmv(*bad)
