@@ -250,7 +250,7 @@ def run_sweep(args):
         prev = batch.hams if batch is not None else None  # freed after the timed solve
         t = time.perf_counter()
         if batch is None:
-            batch = blqh_amd.Batch(hs)  # autotunes the batched SpMV once for the sweep
+            batch = blqh_amd.Batch(hs)
         else:
             batch.rebind(hs)  # same sectors, next parameter point: pools and replay kept
         dt = time.perf_counter() - t
@@ -285,7 +285,7 @@ def run_sweep(args):
                 cont["max_rel_dE0"] = max(cont["max_rel_dE0"], max(rel))
                 cont["mismatch"] += bad
         if warm and plain is None:
-            # plain single-problem solves of the same Hamiltonians (each autotuned by a first solve)
+            # plain single-problem solves of the same Hamiltonians (after a first solve)
             for i, H in enumerate(hs):
                 H.lanczos(lam=args.lam, seed=seeds[i], tol=1e-10, check_every=args.check_every, want_psi=False)
             tp = time.perf_counter()
@@ -412,8 +412,7 @@ def run_sweep(args):
             "frac": achieved / HBM_PEAK_GBS,
             "traffic": (MEASURED_SWEEP_TRAFFIC.get((args.workload, "per-point")) or (None,))[0],
             "traffic_source": (MEASURED_SWEEP_TRAFFIC.get((args.workload, "per-point")) or (None, None))[1],
-            "kernel": ("k_b1j<LZ=true> (batched fused SpMV + Lanczos K1, step-major panels, two wavefronts per "
-                       "64-row slice)" if batch.lanes == 64 else
+            "kernel": ("k_b1x<LZ=true> (batched fused SpMV + Lanczos K1, coded layout, x tiles in LDS)" if batch.lanes == 64 else
                        f"k_b1<{batch.lanes}, LZ=true> (batched fused SpMV + Lanczos K1, row-major panels)"),
             "avg_launch_ms": avg_ms,
             "launches": launches,
@@ -511,7 +510,7 @@ def run_sweep_shared(args):
                 cont["max_rel_dE0"] = max(cont["max_rel_dE0"], max(rel))
                 cont["mismatch"] += bad
         if warm and plain is None:
-            # plain single-problem solves of the same problems (each autotuned by a first solve)
+            # plain single-problem solves of the same problems (after a first solve)
             hs = [blqh_amd.Hamiltonian.combine(b, tn, x) for b, tn in zip(base, tun) for x in ds_list]
             for i, H in enumerate(hs):
                 H.lanczos(lam=args.lam, seed=seeds[i], tol=1e-10, check_every=args.check_every, want_psi=False)
@@ -641,7 +640,7 @@ def run_sweep_shared(args):
             "frac": achieved / HBM_PEAK_GBS,
             "traffic": (MEASURED_SWEEP_TRAFFIC.get((args.workload, "shared")) or (None,))[0],
             "traffic_source": (MEASURED_SWEEP_TRAFFIC.get((args.workload, "shared")) or (None, None))[1],
-            "kernel": f"k_b1s<LZ=true, G={G}> (shared-scale batched fused SpMV + Lanczos K1: each sector's "
+            "kernel": f"k_b1x<LZ=true, G={G}, shared> (shared-scale batched fused SpMV + Lanczos K1: each sector's "
                       f"entries read once for its {G} DSAS problems)",
             "avg_launch_ms": avg_ms,
             "launches": launches,
@@ -724,7 +723,7 @@ def run_warm(args):
         for s, B in bases.items():
             hs.append(ham(B, d))
             keys.append((s, d))
-    for i, H in enumerate(hs):  # autotune every matrix outside the timed regions
+    for i, H in enumerate(hs):  # a first solve of every matrix outside the timed regions
         H.lanczos(lam=args.lam, seed=1, tol=1e-10, check_every=chk, want_psi=False)
     # plain: seeded random start, one problem at a time
     t = time.perf_counter()

@@ -437,7 +437,7 @@ class Batch:
     objects are kept alive by the batch."""
 
     def __init__(self, hams, lanes=0):
-        """lanes=0 autotunes the batched SpMV; otherwise 4, 8, 16, 32 or 64."""
+        """lanes of the batched SpMV: 0 is the default (64, the coded layout); otherwise 4, 8, 16 or 32 (panels)."""
         self.hams = list(hams)
         self._lib = lib()
         arr = (C.c_void_p * len(self.hams))(*[H.h.value for H in self.hams])

@@ -24,6 +24,7 @@
 // on the device in the reference row order as the start of a continuation
 // solve at the next parameter point (k_bcont).
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -57,11 +58,23 @@ constexpr int kBT = 256;        // threads per workgroup
 constexpr int kSplit = 2;       // k_b1j: wavefronts per 64-row slice (measured: 2 beats 1 and 4)
 constexpr int kBTj = kSplit * 256;  // threads per workgroup of k_b1j (an item's four slices)
 
+// A one-panel coded layout regrouped for k_b1x: by 64-row slice, then column tile of
+// tw columns, then groups of four steps; a group holds four words of every lane
+// (ent[group * 64 + lane]), rows shorter than the slice's longest in that tile
+// padded with words of value zero.  Tile t of slice s is groups goff[s nt + t] ..
+// goff[s nt + t + 1).
+struct ColTiles {
+    int tw, nt;
+    const uint4* ent;
+    const int64_t* goff;
+};
+
 // device descriptor of one problem
 struct BProb {
     int64_t n;
     int32_t npan, real;
-    CodView c;              // k_b1j, k_b1s
+    CodView c;              // coded layout: k_b1x, k_b1j
+    ColTiles t;            // its column tiles: k_b1x
     const int64_t* pbase;   // panels: k_b1
     const uint32_t* prow;
     const uint16_t* pcol;
@@ -77,7 +90,7 @@ struct BState {
     const BProb* probs;
     const int32_t* item_prob;  // work item -> problem
     int64_t nitems;
-    const int32_t* xitems;     // k_b1j work lists: items grouped per XCD (real, complex, all members)
+    const int32_t* xitems;     // work lists of k_b1j (items) and k_b1x (units) per XCD (real, complex, all members)
     const int32_t* xseg;       // [3][9] list offsets: kind (real, complex, all) x XCD
     const int32_t* active;     // [P]
     int32_t* jbase;            // step of the first kernel in a replay (advanced by k_bnext)
@@ -285,6 +298,9 @@ __global__ void __launch_bounds__(kBTj) k_b1j(BState S, int jrel, const double2*
                 ar += o.x;
                 ai += o.y;
             }
+            const double2 w = x[myrow], dg = cod_diag(P.c, real, myrow);
+            ar += dg.x * w.x - dg.y * w.y;
+            ai += dg.x * w.y + dg.y * w.x;
             double ur = ar, ui = ai;
             if (LZ) {
                 ur = ib * ar;
@@ -296,7 +312,6 @@ __global__ void __launch_bounds__(kBTj) k_b1j(BState S, int jrel, const double2*
                 }
             }
             y[myrow] = make_double2(ur, ui);
-            const double2 w = x[myrow];
             acc = w.x * ur + w.y * ui;
         }
         const double t = block_sum<kBTj>(acc, sh);
@@ -304,238 +319,401 @@ __global__ void __launch_bounds__(kBTj) k_b1j(BState S, int jrel, const double2*
     }
 }
 
-// ---- shared-scale groups ----------------------------------------------------
-// G problems of one sector whose Hamiltonians are H0 + s_g T (the Delta_SAS
-// points of one d) share one panel layout of H0 + T: the entries of T (those
-// between words of different upper-layer occupation) carry bit 15 of their
-// column (a sector of at most 32,768 states, one panel), and problem g scales
-// them by s_g.  One pass over the entries serves all G problems: the column
-// and value of an entry are loaded once and gathered against G vectors.
-struct SGroups {
-    const int32_t* gitem_grp;  // group work item -> group
-    const int64_t* gitem0;     // [ngroups + 1] first group item
-    const double* tscale;      // [P] scale of the flagged entries, problem p
-};
+// ---- K1 with x in LDS -------------------------------------------------------
+// For members of one panel.  The x gathers bound k_b1j: the vector memory path
+// serves about one 16-byte lane address per clock and CU (0.75 measured), LDS a
+// wavefront's 64 in about 20 clocks.  So a workgroup of 16 wavefronts (one per CU:
+// it takes the whole LDS) owns a unit of 16 slices, stages x tile by tile beside the
+// value table and sums its slices' words of that tile from LDS.  The tiles are as
+// wide as the LDS allows (8,192 columns of one vector at most), so a unit of an
+// 18.8k-row member stages 300 KB for 158k entries.  With x in LDS the address
+// arithmetic counts: a word's fields are LDS byte offsets (one mask each), rows are
+// padded to their slice's longest (no lane masks or prefix sums) and a lane loads
+// four words at once.
+//
+// Shared-scale groups (SH): G problems of one sector whose Hamiltonians are
+// H0 + s_g T (the Delta_SAS points of one d) share one coded layout of H0 + T: the
+// entries of T (those between words of different upper-layer occupation) carry the
+// tunnelling flag (a sector of at most 32,768 states), and problem
+// g scales them by s_g.  One pass over the entries serves all G problems: an
+// entry's word and value are read once and multiplied with G tiles.
+//
+// Bound by vector-ALU work per padded word (decode, sign, two to four 64-bit
+// multiply-adds) and, in sweeps, by the staging of x and the barrier around it (about
+// half at G = 3); bank conflicts cost nothing measurable (a conflict-free order of
+// the words took the same time).  K1 with every member live, jagged panels gathering
+// x -> this: 64 spinful N_phi = 8 sectors 446 -> 193 us, N_phi = 12 sweep, 144 sectors
+// at three scales, 2,393 -> 1,203 us.
+//
+// Word: bit 31 / 30 sign of the real / imaginary part, bits 17..28 index of the
+// value in the LDS table (0: the value zero), bits 4..16 column in the tile, bit 0
+// the tunnelling flag.
+constexpr int kUnit = 16;              // slices of a unit, one per wavefront
+constexpr int kBTx = kUnit * 64;
+constexpr int kUnitItems = kUnit * 64 / kItemRows;
+constexpr size_t kLdsMax = 160 * 1024 - 1024;  // dynamic LDS; the rest is k_b1x's static part
+constexpr int kTileMax = 8192;         // columns of a tile (13 bits)
 
-// cod_run_sum for G vectors: lane sums of row `lane` of a 64-row slice over the
-// step groups of its wave, entry values scaled by ts[g] where the column carries
-// kCodTun.  act[g] == false skips vector g.
-template <bool REAL, int G>
-__device__ __forceinline__ void shared_fma(uint32_t c, double2 v, const double2* const* xp, const double* ts,
-                                           const bool* act, double* ar, double* ai) {
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-        if (act[g]) {
-            const double2 xv = xp[g][c & (kCodTun - 1)];
-            const double sc = (c & kCodTun) ? ts[g] : 1.0;
-            const double wr = sc * v.x;
-            if (REAL) {
-                ar[g] += wr * xv.x;
-                ai[g] += wr * xv.y;
-            } else {
-                const double wi = sc * v.y;
-                ar[g] += wr * xv.x - wi * xv.y;
-                ai[g] += wr * xv.y + wi * xv.x;
-            }
-        }
+// An element of k_b1x's work list names an owner (a problem; SH: a group) and, counted
+// in elements, the place in it: owner << kElemBits | element.  An element is `span`
+// (S.xseg[27], 1 or 2) consecutive units.
+constexpr int kElemBits = 7;  // at most 64 units of a one-panel member
+
+// LDS bytes of the table: the value zero, then the layout's values
+__host__ __device__ inline size_t tile_tab_bytes(bool real, int ntab) {
+    return ((size_t)(ntab + 1) * (real ? 8 : 16) + 15) / 16 * 16;
 }
 
-template <bool REAL, int NP, int G>
-__device__ __forceinline__ void cod_run_shared(const uint32_t* __restrict__ er, const double* tab,
-                                               const double2* const* xp, const double* ts, const bool* act,
-                                               uint32_t len, int par, double* ar, double* ai) {
+__device__ __forceinline__ double with_sign(double mag, uint32_t top) {  // mag >= 0, sign in bit 31
+    return __hiloint2double((int)((uint32_t)__double2hiint(mag) | (top & 0x80000000u)), __double2loint(mag));
+}
+
+// (ar, ai) += (wr, wi) xv in four multiply-adds
+__device__ __forceinline__ void cfma(double wr, double wi, double2 xv, double& ar, double& ai) {
+    ar = fma(wr, xv.x, ar);
+    ai = fma(wr, xv.y, ai);
+    ar = fma(-wi, xv.y, ar);
+    ai = fma(wi, xv.x, ai);
+}
+
+// the rest of a slice, x in global memory; four steps of loads in flight
+template <bool REAL, int G, bool SH>
+__device__ __forceinline__ void tile_rest_sum(const uint32_t* __restrict__ rc, const double* __restrict__ rv,
+                                              const double2* const* x, const double* ts, uint32_t len, double* ar,
+                                              double* ai) {
     constexpr int U = 4;
     uint32_t off = 0;
-    auto issue = [&](uint32_t t, uint32_t* e, bool& any) {
-        uint64_t m[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) m[u] = __ballot(t + u < len);
-        any = m[0] != 0;
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const uint32_t q = off + lanes_below(m[u]);
-            off += (uint32_t)__popcll(m[u]);
-            e[u] = t + u < len ? __builtin_nontemporal_load(&er[q]) : 0u;
-        }
-    };
-    auto skip = [&](uint32_t t) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) off += (uint32_t)__popcll(__ballot(t + u < len));
-    };
-    uint32_t e0[U], e1[U];
-    bool any0, any1;
-    for (int g = 0; g < par; ++g) skip((uint32_t)(U * g));
-    uint32_t t0 = (uint32_t)(U * par);
-    issue(t0, e0, any0);
-    while (any0) {
-        const uint32_t t = t0 + (uint32_t)(U * NP);
-#pragma unroll
-        for (int g = NP - 1; g > 0; --g) skip(t - (uint32_t)(U * g));
-        issue(t, e1, any1);
+    for (uint32_t t = 0; __ballot(t < len) != 0; t += U) {
+        uint32_t c[U];
         double2 v[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            v[u] = REAL ? make_double2(cod_real(tab, e0[u]), 0.0)
-                        : cod_cplx(reinterpret_cast<const double2*>(tab), e0[u]);
-            if (!(t0 + u < len)) v[u] = make_double2(0.0, 0.0);
+            const uint64_t m = __ballot(t + u < len);
+            const uint32_t q = off + lanes_below(m);
+            off += (uint32_t)__popcll(m);
+            c[u] = 0;
+            v[u] = make_double2(0.0, 0.0);
+            if (t + u < len) {
+                c[u] = rc[q];
+                v[u] = REAL ? make_double2(rv[q], 0.0) : reinterpret_cast<const double2*>(rv)[q];
+            }
         }
-        // one vector at a time: U gathers in flight per vector
 #pragma unroll
-        for (int g = 0; g < G; ++g)
-            if (act[g]) {
-                double2 xv[U];
+        for (int g = 0; g < G; ++g) {
+            double2 xv[U];
 #pragma unroll
-                for (int u = 0; u < U; ++u) xv[u] = xp[g][e0[u] & (kCodTun - 1)];
+            for (int u = 0; u < U; ++u) xv[u] = x[g][SH ? c[u] & (kCodTun - 1) : c[u]];
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const double sc = (e0[u] & kCodTun) ? ts[g] : 1.0;
-                    const double wr = sc * v[u].x;
-                    if (REAL) {
-                        ar[g] += wr * xv[u].x;
-                        ai[g] += wr * xv[u].y;
-                    } else {
-                        const double wi = sc * v[u].y;
-                        ar[g] += wr * xv[u].x - wi * xv[u].y;
-                        ai[g] += wr * xv[u].y + wi * xv[u].x;
-                    }
+            for (int u = 0; u < U; ++u) {
+                if (!(t + u < len)) continue;
+                const double sc = SH && (c[u] & kCodTun) ? ts[g] : 1.0;
+                if (REAL) {
+                    ar[g] = fma(sc * v[u].x, xv[u].x, ar[g]);
+                    ai[g] = fma(sc * v[u].x, xv[u].y, ai[g]);
+                } else {
+                    cfma(sc * v[u].x, sc * v[u].y, xv[u], ar[g], ai[g]);
                 }
             }
-#pragma unroll
-        for (int u = 0; u < U; ++u) e0[u] = e1[u];
-        any0 = any1;
-        t0 = t;
-    }
-}
-
-// the rest of a slice (cod_rest_sum) for G vectors
-template <bool REAL, int NP, int G>
-__device__ __forceinline__ void cod_rest_shared(const uint32_t* __restrict__ rc, const double* __restrict__ rv,
-                                                const double2* const* x, const double* ts, const bool* act,
-                                                uint32_t len, int par, double* ar, double* ai) {
-    uint32_t off = 0;
-    for (uint32_t t = 0;; ++t) {
-        const uint64_t m = __ballot(t < len);
-        if (m == 0) break;
-        if ((int)(t % NP) == par && t < len) {
-            const uint32_t q = off + lanes_below(m);
-            const double2 v = REAL ? make_double2(rv[q], 0.0) : reinterpret_cast<const double2*>(rv)[q];
-            shared_fma<REAL, G>(rc[q], v, x, ts, act, ar, ai);
         }
-        off += (uint32_t)__popcll(m);
     }
 }
 
-// k_b1j for shared-scale groups: the work lists hold group items (256 rows
-// of a sector); problems q G .. q G + G - 1 of group q share the sector's
-// panels and own their vectors, scalars and partial sums (problem p's item
-// li is item0 + li, as in k_b2 / k_b3).
-template <bool LZ, int KIND, int G>
-__global__ void __launch_bounds__(kBTj) k_b1s(BState S, SGroups Q, int jrel, const double2* __restrict__ xs,
-                                              double2* __restrict__ ys, double* __restrict__ part) {
-    __shared__ double sh[kBTj / 64];
-    __shared__ double2 red[kItemRows / 64][kSplit - 1][G][64];
+// SC: some lane's word carries the tunnelling flag
+template <bool REAL, int G, bool SC>
+__device__ __forceinline__ void tile_fma(uint32_t e, const char* lds, uint32_t xbase, uint32_t xstep, const double* ts,
+                                         double* ar, double* ai) {
+    double vr, vi = 0.0;
+    if (REAL) {
+        vr = with_sign(*reinterpret_cast<const double*>(lds + ((e >> 14) & 0x7ff8u)), e);
+    } else {
+        const double2 v = *reinterpret_cast<const double2*>(lds + ((e >> 13) & 0xfff0u));
+        vr = with_sign(v.x, e);
+        vi = with_sign(v.y, e << 1);
+    }
+    const char* xp = lds + xbase + (e & 0x1fff0u);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const double2 xv = *reinterpret_cast<const double2*>(xp + (uint32_t)g * xstep);
+        double wr = vr, wi = vi;
+        if (SC) {
+            const double sc = (e & 1u) ? ts[g] : 1.0;
+            wr *= sc;
+            wi *= sc;
+        }
+        if (REAL) {
+            ar[g] = fma(wr, xv.x, ar[g]);
+            ai[g] = fma(wr, xv.y, ai[g]);
+        } else {
+            cfma(wr, wi, xv, ar[g], ai[g]);
+        }
+    }
+}
+
+// A wavefront's words of one tile: K groups from ent, two groups loaded ahead (a0 and
+// a1 hold the first two).  A row's flagged words come first, so most groups have none.
+template <bool REAL, int G, bool SH>
+__device__ __forceinline__ void tile_sum(const uint4* __restrict__ ent, uint32_t K, uint4 a0, uint4 a1, const char* lds,
+                                         uint32_t xbase, uint32_t xstep, const double* ts, double* ar, double* ai) {
+    for (uint32_t k = 0; k < K; ++k) {
+        const uint4 e = a0;
+        a0 = a1;
+        if (k + 2 < K) a1 = ent[(k + 2) * 64];
+        if (SH && __ballot(((e.x | e.y | e.z | e.w) & 1u) != 0)) {
+            tile_fma<REAL, G, true>(e.x, lds, xbase, xstep, ts, ar, ai);
+            tile_fma<REAL, G, true>(e.y, lds, xbase, xstep, ts, ar, ai);
+            if (G > 1) __builtin_amdgcn_sched_barrier(0);  // two words' LDS reads in flight: no spills
+            tile_fma<REAL, G, true>(e.z, lds, xbase, xstep, ts, ar, ai);
+            tile_fma<REAL, G, true>(e.w, lds, xbase, xstep, ts, ar, ai);
+        } else {
+            tile_fma<REAL, G, false>(e.x, lds, xbase, xstep, ts, ar, ai);
+            tile_fma<REAL, G, false>(e.y, lds, xbase, xstep, ts, ar, ai);
+            if (G > 1) __builtin_amdgcn_sched_barrier(0);
+            tile_fma<REAL, G, false>(e.z, lds, xbase, xstep, ts, ar, ai);
+            tile_fma<REAL, G, false>(e.w, lds, xbase, xstep, ts, ar, ai);
+        }
+    }
+}
+
+// 16 bytes a lane from global memory straight to LDS, lane l to dst + l; complete
+// after wait_vmem.  dst: uniform over the wavefront.
+__device__ __forceinline__ void load_lds16(const double2* src, double2* dst) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+__device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Values that are the same on every lane, into scalar registers (the kernel writes
+// memory, so the compiler keeps what it loads per owner in vector ones).
+__device__ __forceinline__ int sgpr(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ int64_t sgpr(int64_t v) {
+    return (int64_t)((uint64_t)(uint32_t)sgpr((int)(v >> 32)) << 32 | (uint32_t)sgpr((int)v));
+}
+__device__ __forceinline__ double sgpr(double v) { return __longlong_as_double(sgpr((int64_t)__double_as_longlong(v))); }
+template <class T>
+__device__ __forceinline__ T* sgpr(T* p) {
+    return reinterpret_cast<T*>(sgpr((int64_t)reinterpret_cast<uintptr_t>(p)));
+}
+
+// Problem p0 + g, g < G, of an owner (SH: p0 = owner G; else G = 1, p0 = owner);
+// problem p's item li is item0 + li, as in k_b2 / k_b3.  A stopped problem of a
+// live group is summed along and not written.
+template <bool LZ, int G, bool SH>
+__global__ void __launch_bounds__(kBTx) k_b1x(BState S, const double* __restrict__ tscale, int jrel,
+                                              const double2* __restrict__ xs, double2* __restrict__ ys,
+                                              double* __restrict__ part) {
     extern __shared__ __align__(16) double ctab[];
+    __shared__ double red[2][G][kUnit];
     const int j = LZ ? *S.jbase + jrel : 0;
     if (LZ && j >= S.cap) return;
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int sl = wv / kSplit, par = wv % kSplit;
-    int32_t k0, k1;
-    list_share(S.xseg + KIND * 9 + (blockIdx.x & 7), k0, k1);
-    int qt = -1;  // sector whose value table is in LDS
-    for (int32_t k = k0; k < k1; ++k) {
-        const int64_t it = S.xitems[k];
-        const int q = Q.gitem_grp[it];
-        const int64_t li = it - Q.gitem0[q];
-        bool act[G];
-        bool anyact = false;
+    const char* lds = reinterpret_cast<const char*>(ctab);
+    // The XCD's workgroups walk its list side by side (unlike k_b1j's stretches):
+    // they stage the x of the same one or two owners, out of the L2.
+    const int32_t* seg = S.xseg + 2 * 9 + (blockIdx.x & 7);
+    const int span = sgpr(S.xseg[27]);
+    int ot = -1;  // owner whose value table is in LDS
+    for (int32_t k = seg[0] + (int32_t)(blockIdx.x >> 3), k1 = seg[1]; k < k1; k += (int32_t)(gridDim.x >> 3)) {
+        const int32_t id = sgpr(S.xitems[k]);
+        const int o = id >> kElemBits, p0 = SH ? o * G : o;
+        bool act[G], any = false;
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            act[g] = S.active[q * G + g] != 0;
-            anyact = anyact || act[g];
+            act[g] = sgpr(S.active[p0 + g]) != 0;
+            any = any || act[g];
         }
-        if (!anyact) continue;  // uniform over the workgroup
-        const BProb P0 = S.probs[q * G];
-        const int64_t n = P0.n;
-        const bool real = KIND == 2 ? P0.real != 0 : KIND == 0;
-        if (q != qt) {
-            __syncthreads();  // the previous sector's table is no longer read
-            if (real) cod_stage<true>(P0.c.tab, P0.c.ntab, ctab, kBTj);
-            else cod_stage<false>(P0.c.tab, P0.c.ntab, ctab, kBTj);
-            __syncthreads();
-            qt = q;
-        }
+        if (!any) continue;  // uniform over the workgroup
+        const BProb& P = S.probs[p0];
+        const int64_t n = sgpr(P.n), nsl = (n + 63) >> 6;
+        const bool real = sgpr(P.real) != 0;
+        const int ntab = sgpr(P.c.ntab), tw = sgpr(P.t.tw), nt = sgpr(P.t.nt);
+        const uint4* tent = sgpr(P.t.ent);
+        const int64_t* goff = sgpr(P.t.goff);
+        const uint32_t xbase = (uint32_t)tile_tab_bytes(real, ntab), xstep = (uint32_t)tw * 16u;
+        double2* xt = reinterpret_cast<double2*>(reinterpret_cast<char*>(ctab) + xbase);
         const double2* x[G];
-        double2* y[G];
-        const double2* Wp[G];
-        double ib[G], cp[G], ts[G];
+        double ts[G], ar[2][G], ai[2][G];
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            const BProb& Pg = S.probs[q * G + g];
-            ts[g] = Q.tscale[q * G + g];
-            ib[g] = 1.0;
-            cp[g] = 0.0;
-            if (LZ) {
-                const int64_t ld = S.cap + 1;
-                const int p = q * G + g;
-                ib[g] = S.invb[p * ld + j];
-                cp[g] = j > 0 ? S.beta[p * ld + j] * S.invb[p * ld + j - 1] : 0.0;
-                x[g] = Pg.W + (int64_t)j * n;
-                Wp[g] = j > 0 ? x[g] - n : x[g];
-                y[g] = S.u + Pg.voff;
-            } else {
-                x[g] = xs + Pg.voff;
-                Wp[g] = x[g];
-                y[g] = ys + Pg.voff;
+            const BProb& Pg = S.probs[p0 + g];
+            x[g] = sgpr(LZ ? Pg.W + (int64_t)j * n : xs + Pg.voff);
+            ts[g] = SH ? sgpr(tscale[p0 + g]) : 1.0;
+            ar[0][g] = ai[0][g] = ar[1][g] = ai[1][g] = 0.0;
+        }
+        const int32_t u0 = (id & ((1 << kElemBits) - 1)) * span;  // the element's first unit
+        const int64_t sl0 = (int64_t)u0 * kUnit + wv;             // this wavefront's slices: sl0, sl0 + kUnit
+        for (int t = 0; t < nt; ++t) {
+            // the first words are on their way while the tile is staged
+            uint32_t K[2];
+            const uint4* ent[2];
+            uint4 a0[2], a1[2];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int64_t sl = sl0 + q * kUnit;
+                const bool mine = q < span && sl < nsl;  // uniform over the wavefront
+                const int64_t g0 = mine ? goff[sl * nt + t] : 0;
+                K[q] = mine ? (uint32_t)(goff[sl * nt + t + 1] - g0) : 0u;
+                ent[q] = tent + g0 * 64 + lane;
+                a0[q] = a1[q] = make_uint4(0, 0, 0, 0);
+                if (K[q] > 0) a0[q] = ent[q][0];
+                if (K[q] > 1) a1[q] = ent[q][64];
+            }
+            __syncthreads();  // the previous tile (and table) is no longer read
+            if (o != ot) {
+                if (real) {
+                    for (int i = threadIdx.x; i <= ntab; i += kBTx) ctab[i] = i ? P.c.tab[i - 1] : 0.0;
+                } else {
+                    const double2* t2 = reinterpret_cast<const double2*>(P.c.tab);
+                    double2* l2 = reinterpret_cast<double2*>(ctab);
+                    for (int i = threadIdx.x; i <= ntab; i += kBTx) l2[i] = i ? t2[i - 1] : make_double2(0.0, 0.0);
+                }
+                ot = o;
+            }
+            const int64_t c0 = (int64_t)t * tw;
+            const int w = (int)(n - c0 < tw ? n - c0 : tw);
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+                for (int i = threadIdx.x; i < w; i += kBTx)
+                    load_lds16(&x[g][c0 + i], xt + g * tw + (i - lane));
+            wait_vmem();
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                if (real) tile_sum<true, G, SH>(ent[q], K[q], a0[q], a1[q], lds, xbase, xstep, ts, ar[q], ai[q]);
+                else tile_sum<false, G, SH>(ent[q], K[q], a0[q], a1[q], lds, xbase, xstep, ts, ar[q], ai[q]);
             }
         }
-        const int64_t row0 = li * kItemRows + sl * 64, myrow = row0 + lane;
-        double ar[G], ai[G];
 #pragma unroll
-        for (int g = 0; g < G; ++g) ar[g] = ai[g] = 0.0;
-        if (row0 < n) {  // uniform over the wavefront; one panel (n <= 32768)
-            const int64_t slc = row0 >> 6, run = P0.c.base[slc], q0 = P0.c.rbase[slc];
-            const uint32_t len = P0.c.len[myrow], rl = P0.c.rlen[myrow];
-            if (real) {
-                cod_run_shared<true, kSplit, G>(P0.c.ent + run, ctab, x, ts, act, len, par, ar, ai);
-                cod_rest_shared<true, kSplit, G>(P0.c.rcol + q0, P0.c.rval + q0, x, ts, act, rl, par, ar, ai);
-            } else {
-                cod_run_shared<false, kSplit, G>(P0.c.ent + run, ctab, x, ts, act, len, par, ar, ai);
-                cod_rest_shared<false, kSplit, G>(P0.c.rcol + q0, P0.c.rval + 2 * q0, x, ts, act, rl, par, ar, ai);
+        for (int q = 0; q < 2; ++q) {
+            const int64_t sl = sl0 + q * kUnit, row = sl * 64 + lane;
+            const bool mine = q < span && sl < nsl && row < n;
+            if (q < span && sl < nsl) {
+                const int64_t q0 = P.c.rbase[sl];
+                const uint32_t rl = P.c.rlen[row];
+                if (real) tile_rest_sum<true, G, SH>(P.c.rcol + q0, P.c.rval + q0, x, ts, rl, ar[q], ai[q]);
+                else tile_rest_sum<false, G, SH>(P.c.rcol + q0, P.c.rval + 2 * q0, x, ts, rl, ar[q], ai[q]);
             }
-        }
-        if (par) {
+            const double2 dg = mine ? cod_diag(P.c, real, row) : make_double2(0.0, 0.0);
 #pragma unroll
-            for (int g = 0; g < G; ++g) red[sl][par - 1][g][lane] = make_double2(ar[g], ai[g]);
+            for (int g = 0; g < G; ++g) {
+                double acc = 0.0;
+                if (act[g] && mine) {
+                    double2* y = (LZ ? S.u : ys) + S.probs[p0 + g].voff;
+                    double yr = ar[q][g], yi = ai[q][g];
+                    const double2 w = x[g][row];
+                    cfma(dg.x, dg.y, w, yr, yi);
+                    if (LZ) {
+                        const int64_t ld = S.cap + 1;
+                        const int p = p0 + g;
+                        const double ib = S.invb[p * ld + j];
+                        yr *= ib;
+                        yi *= ib;
+                        if (j > 0) {
+                            const double cp = S.beta[p * ld + j] * S.invb[p * ld + j - 1];
+                            const double2 wp = x[g][row - n];  // W_{j-1}
+                            yr -= cp * wp.x;
+                            yi -= cp * wp.y;
+                        }
+                    }
+                    y[row] = make_double2(yr, yi);
+                    acc = w.x * yr + w.y * yi;
+                }
+                for (int d = 32; d > 0; d >>= 1) acc += __shfl_xor(acc, d, 64);
+                if (lane == 0) red[q][g][wv] = acc;
+            }
         }
         __syncthreads();
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            if (!act[g]) continue;  // uniform over the workgroup
-            double acc = 0.0;
-            if (!par && myrow < n) {
-                double sr = ar[g], si = ai[g];
-#pragma unroll
-                for (int w = 0; w < kSplit - 1; ++w) {
-                    const double2 o = red[sl][w][g][lane];
-                    sr += o.x;
-                    si += o.y;
-                }
-                double ur = sr, ui = si;
-                if (LZ) {
-                    ur = ib[g] * sr;
-                    ui = ib[g] * si;
-                    if (j > 0) {
-                        const double2 qv = Wp[g][myrow];
-                        ur -= cp[g] * qv.x;
-                        ui -= cp[g] * qv.y;
-                    }
-                }
-                y[g][myrow] = make_double2(ur, ui);
-                const double2 w = x[g][myrow];
-                acc = w.x * ur + w.y * ui;
+        if (threadIdx.x < 2 * G * kUnitItems) {  // item partials: its four slices in order
+            const int q = threadIdx.x / (G * kUnitItems), g = threadIdx.x / kUnitItems % G, m = threadIdx.x % kUnitItems;
+            const int64_t li = (int64_t)(u0 + q) * kUnitItems + m;
+            if (q < span && S.active[p0 + g] && li * kItemRows < n) {
+                double t = 0;
+                for (int i = 0; i < kItemRows / 64; ++i) t += red[q][g][m * (kItemRows / 64) + i];
+                part[S.probs[p0 + g].item0 + li] = t;
             }
-            const double t = block_sum<kBTj>(acc, sh);
-            if (threadIdx.x == 0) part[S.probs[q * G + g].item0 + li] = t;
+        }
+    }
+}
+
+// Coded words of one-panel members regrouped into ColTiles, one wavefront per slice,
+// grid.y = member: first (FILL false) each tile's groups into cnt, then the words
+// (goff: the scanned counts of all members).  LDS: words per tile and lane, and
+// per step of the slice its first word and the lanes that hold one.
+struct TileJob {
+    CodView c;
+    int tw, nt;
+    int real;
+    uint32_t cmask;  // column bits of a coded word
+    int64_t goff0;   // this member's first (slice, tile)
+};
+
+template <bool FILL>
+__global__ void __launch_bounds__(64) k_tiles(const TileJob* __restrict__ jobs, int maxrow, int maxnt,
+                                              int32_t* __restrict__ cnt, const int64_t* __restrict__ goff,
+                                              uint4* __restrict__ ent) {
+    extern __shared__ uint64_t lds_tiles[];
+    uint64_t* mk = lds_tiles;
+    uint32_t* so = reinterpret_cast<uint32_t*>(mk + (FILL ? maxrow : 0));
+    uint16_t* tc = reinterpret_cast<uint16_t*>(so + (FILL ? maxrow : 0));  // [maxnt][64]
+    const TileJob J = jobs[blockIdx.y];
+    const int lane = threadIdx.x;
+    const uint64_t below = lane ? ~0ull >> (64 - lane) : 0;
+    const int64_t nsl = J.c.nslices;
+    for (int64_t sl = blockIdx.x; sl < nsl; sl += gridDim.x) {
+        const uint32_t len = J.c.len[sl * 64 + lane];
+        const uint32_t* src = J.c.ent + J.c.base[sl];
+        __syncthreads();  // the previous slice's steps are read
+        uint32_t off = 0, nw = 0, end = (uint32_t)J.tw;
+        int cur = 0;
+        for (uint32_t i = 0; i < (uint32_t)maxrow; ++i) {
+            const uint64_t m = __ballot(i < len);
+            if (m == 0) break;
+            if (FILL && lane == 0) {
+                mk[i] = m;
+                so[i] = off;
+            }
+            if (i < len) {
+                const uint32_t c = src[off + (uint32_t)__popcll(m & below)] & J.cmask;
+                for (; c >= end && cur < J.nt - 1; ++cur) {
+                    tc[cur * 64 + lane] = (uint16_t)nw;
+                    nw = 0;
+                    end += (uint32_t)J.tw;
+                }
+                ++nw;
+            }
+            off += (uint32_t)__popcll(m);
+        }
+        for (; cur < J.nt; ++cur) {
+            tc[cur * 64 + lane] = (uint16_t)nw;
+            nw = 0;
+        }
+        __syncthreads();
+        uint32_t first = 0;
+        for (int t = 0; t < J.nt; ++t) {
+            const uint32_t ln = tc[t * 64 + lane];
+            const int64_t at = J.goff0 + sl * J.nt + t;
+            if (!FILL) {
+                uint32_t mx = ln;
+                for (int o = 32; o > 0; o >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o, 64));
+                if (lane == 0) cnt[at] = (int32_t)((mx + 3) / 4);
+                continue;
+            }
+            const int64_t g0 = goff[at], K = goff[at + 1] - g0;
+            const uint32_t sub = (uint32_t)t * (uint32_t)J.tw;
+            uint32_t* out = reinterpret_cast<uint32_t*>(ent + g0 * 64 + lane);  // word k: out[(k / 4) * 256 + k % 4]
+            auto word = [&](uint32_t i) { return src[so[i] + (uint32_t)__popcll(mk[i] & below)]; };
+            uint32_t nt = 0, pt = 0;  // flagged words of the lane, and those placed
+            for (uint32_t i = 0; i < ln; ++i) nt += (word(first + i) & ~J.cmask & kCodTun) != 0;
+            for (uint32_t i = 0; i < ln; ++i) {
+                const uint32_t w = word(first + i);
+                const bool tun = (w & ~J.cmask & kCodTun) != 0;
+                const uint32_t id = ((w >> 16) & (J.real ? 0x7fffu : 0x3fffu)) + 1;
+                const uint32_t k = tun ? pt : nt + i - pt;
+                pt += tun;
+                out[(k >> 2) * 256 + (k & 3)] = (w & (J.real ? 0x80000000u : 0xc0000000u)) | id << 17 |
+                                                ((w & J.cmask) - sub) << 4 | (uint32_t)tun;
+            }
+            for (uint32_t k = ln; k < (uint32_t)K * 4; ++k) out[(k >> 2) * 256 + (k & 3)] = 0;
+            first += ln;
         }
     }
 }
@@ -826,7 +1004,7 @@ struct blqh_batch {
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     int g_chk = -1, g_lpr = -1, g_cap = -1, g_kinds = -1;
-    size_t g_tab = 0;  // table LDS of the captured launches
+    std::array<size_t, 2> g_tab{};  // launch shape of the captured K1 (k1_shape)
     char* pin = nullptr;
     double2* psi_pin = nullptr;  // pinned staging of the ground states (b->rows entries, on first use)
     // pl.u holds every problem's ground state of the last finished solve in
@@ -839,11 +1017,16 @@ struct blqh_batch {
     int G = 0;
     std::vector<blqh_hamil*> tpl;
     std::vector<double> tscale;   // [P]
-    std::vector<int64_t> gitem0;  // [nsector + 1] group work items
-    int64_t ngitems = 0;
-    DevBuf<int32_t> gitem_grp;
-    DevBuf<int64_t> dgitem0;
     DevBuf<double> dtscale;
+    // k_b1x (members of one panel, lanes 64): every owner's (problem's, or group of
+    // G's) column tiles, made when the members change
+    bool one_panel = false;
+    bool tiles_ok = false;
+    std::vector<ColTiles> tiles;
+    DevBuf<uint4> tent;
+    DevBuf<int64_t> tgoff;
+    size_t x_bytes = 0;           // k_b1x's dynamic LDS
+    int x_grid = 0;
     std::unique_ptr<HostPool> hpool;  // convergence-test threads (batches of 32 or more problems)
     ~blqh_batch() {
         if (gexec) (void)hipGraphExecDestroy(gexec);
@@ -856,34 +1039,101 @@ struct blqh_batch {
 
 namespace {
 
-// Planner view of the members (all, or those with live[p] set); with
-// shared-scale groups, of the groups (live when one of their problems is).
-std::vector<XcdMember> xcd_members(const blqh_batch* b, const std::vector<char>* live = nullptr) {
+bool use_tiles(const blqh_batch* b) { return b->lpr == 64 && b->one_panel; }
+
+// What the captured K1 launches depend on beside the lanes and the value kinds.
+std::array<size_t, 2> k1_shape(const blqh_batch* b) {
+    if (!use_tiles(b)) return {0, b->tab_bytes};
+    return {(size_t)b->x_grid, b->x_bytes};
+}
+
+// Work lists (xcd_lists) over the members (all, or those with live[p] set); with
+// shared-scale groups over the groups (live when one of their problems is).  k_b1x:
+// elements of two units while that leaves every workgroup at least four (an element
+// stages the owner's whole x), else of one; seg[27] = units per element.
+void work_lists(const blqh_batch* b, const std::vector<char>* live, std::vector<int32_t>& items,
+                std::vector<int32_t>& seg) {
     std::vector<XcdMember> mem;
-    if (b->G) {
-        const int ns = (int)b->tpl.size();
-        mem.reserve(ns);
-        for (int q = 0; q < ns; ++q) {
-            bool on = !live;
-            for (int g = 0; g < b->G && !on; ++g) on = (*live)[q * b->G + g] != 0;
-            if (on)
-                mem.push_back({b->gitem0[q], b->gitem0[q + 1], b->tpl[q]->nnz * b->G, 1, b->tpl[q]->cod.real ? 1 : 0});
-        }
-        return mem;
+    const int per = b->G ? b->G : 1, no = (int)b->hs.size() / per;
+    mem.reserve(no);
+    std::vector<int> on;
+    int64_t units = 0;
+    for (int o = 0; o < no; ++o) {
+        bool l = !live;
+        for (int g = 0; g < per && !l; ++g) l = (*live)[o * per + g] != 0;
+        if (!l) continue;
+        on.push_back(o);
+        units += ceil_div(b->h_probs[o * per].n, (int64_t)kUnit * 64);
     }
-    const int P = (int)b->hs.size();
-    mem.reserve(P);
-    for (int p = 0; p < P; ++p)
-        if (!live || (*live)[p])
-            mem.push_back({b->item0[p], b->item0[p + 1], b->hs[p]->nnz, b->h_probs[p].npan,
-                           b->h_probs[p].real});
-    return mem;
+    const bool tiled = use_tiles(b);
+    const int span = tiled && units >= 8 * (int64_t)b->x_grid ? 2 : 1;
+    for (int o : on) {
+        const BProb& d = b->h_probs[o * per];
+        if (tiled) {
+            const int64_t e0 = (int64_t)o << kElemBits;
+            mem.push_back({e0, e0 + ceil_div(d.n, (int64_t)kUnit * 64 * span), b->hs[o * per]->nnz * per, 1, d.real});
+        } else {
+            mem.push_back({b->item0[o], b->item0[o + 1], b->hs[o]->nnz, d.npan, d.real});
+        }
+    }
+    xcd_lists(mem, items, seg);
+    seg.push_back(span);
+}
+
+// Column tiles of every owner's coded layout, as wide as the LDS beside its value
+// table allows.
+void make_tiles(blqh_batch* b) {
+    hipStream_t st = stream();
+    const int per = b->G ? b->G : 1, no = (int)b->hs.size() / per;
+    std::vector<TileJob> jobs(no);
+    int64_t runs = 0, smax = 1;
+    int rmax = 64, ntmax = 1;
+    b->x_bytes = 0;
+    for (int o = 0; o < no; ++o) {
+        const blqh_hamil* H = b->hs[o * per];
+        const size_t tabb = tile_tab_bytes(H->cod.real, H->cod.ntab);
+        const int64_t most = std::min<int64_t>(kTileMax, (int64_t)((kLdsMax - tabb) / (sizeof(double2) * per)));
+        const int nt = (int)ceil_div(H->n, most), tw = (int)ceil_div(H->n, (int64_t)nt);
+        const int64_t nsl = ceil_div(H->n, (int64_t)64);
+        jobs[o] = TileJob{cview(H->cod, H->n), tw, nt, H->cod.real ? 1 : 0, b->G ? kCodTun - 1 : 0xffffu, runs};
+        runs += nsl * nt;
+        smax = std::max(smax, nsl);
+        ntmax = std::max(ntmax, nt);
+        rmax = std::max(rmax, std::min(H->row_max > 0 ? H->row_max : 4096, 4096));
+        b->x_bytes = std::max(b->x_bytes, tabb + sizeof(double2) * per * (size_t)tw);
+    }
+    DevBuf<TileJob> dj(no);
+    DevBuf<int32_t> cnt(runs);
+    if ((int64_t)b->tgoff.n < runs + 1) b->tgoff.alloc(runs + 1);
+    BLQH_HIP(hipMemcpyAsync(dj.get(), jobs.data(), no * sizeof(TileJob), hipMemcpyHostToDevice, st));
+    auto launch = [&](auto kern, bool fill) {
+        for (int o = 0; o < no; o += 65535)
+            hipLaunchKernelGGL(kern, dim3((unsigned)std::min<int64_t>(smax, 4096), (unsigned)std::min(65535, no - o)),
+                               dim3(64), (fill ? (size_t)rmax * 12 : 0) + (size_t)ntmax * 128, st, dj.get() + o, rmax,
+                               ntmax, cnt.get(), b->tgoff.get(), b->tent.get());
+        BLQH_HIP(hipGetLastError());
+    };
+    launch(k_tiles<false>, false);
+    exclusive_scan(cnt.get(), b->tgoff.get(), runs, st);
+    int64_t groups = 0;
+    copy_sync(&groups, b->tgoff.get() + runs, 8, hipMemcpyDeviceToHost);
+    if ((int64_t)b->tent.n < groups * 64) b->tent.alloc(std::max<int64_t>(groups * 64, 1));
+    launch(k_tiles<true>, true);
+    BLQH_HIP(hipStreamSynchronize(st));
+    b->tiles.resize(no);
+    for (int o = 0; o < no; ++o)
+        b->tiles[o] = ColTiles{jobs[o].tw, jobs[o].nt, b->tent.get(), b->tgoff.get() + jobs[o].goff0};
+    int64_t units = 0;
+    for (int o = 0; o < no; ++o) units += ceil_div(jobs[o].c.n, (int64_t)kUnit * 64);
+    const int wpc = b->x_bytes <= 79 * 1024 ? 2 : 1;  // workgroups of 1024 threads that share a CU's LDS
+    b->x_grid = (int)(8 * ceil_div(std::min<int64_t>(units, (int64_t)runtime().num_cus * wpc), 8));
+    b->tiles_ok = true;
 }
 
 // Work lists of k_b1j (xcd_lists), uploaded when they change.
 void build_xcd_lists(blqh_batch* b) {
     std::vector<int32_t> items, seg;
-    xcd_lists(xcd_members(b), items, seg);
+    work_lists(b, nullptr, items, seg);
     if (items == b->h_xitems && seg == b->h_xseg) return;
     b->h_xitems.swap(items);
     b->h_xseg.swap(seg);
@@ -891,7 +1141,7 @@ void build_xcd_lists(blqh_batch* b) {
     // touched again before the copies have completed
     hipStream_t st = stream();
     BLQH_HIP(hipMemcpyAsync(b->xitems.get(), b->h_xitems.data(), b->h_xitems.size() * 4, hipMemcpyHostToDevice, st));
-    BLQH_HIP(hipMemcpyAsync(b->xseg.get(), b->h_xseg.data(), 27 * 4, hipMemcpyHostToDevice, st));
+    BLQH_HIP(hipMemcpyAsync(b->xseg.get(), b->h_xseg.data(), 28 * 4, hipMemcpyHostToDevice, st));
     BLQH_HIP(hipStreamSynchronize(st));
 }
 
@@ -925,45 +1175,32 @@ void refresh_probs(blqh_batch* b) {
             d.pvc = H->pan.pvc.get();
         }
     }
+    if (use_tiles(b)) {
+        if (!b->tiles_ok) make_tiles(b);
+        for (size_t p = 0; p < b->hs.size(); ++p) b->h_probs[p].t = b->tiles[p / (b->G ? b->G : 1)];
+    }
     build_xcd_lists(b);
 }
 
-// Kernels with the value table in dynamic LDS, raised to the largest table once.
+// Dynamic LDS above the default, allowed once per kernel.
 template <class K>
-void allow_table(K kern) {
-    BLQH_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 (int)cod_lds_bytes(false, kCodCplx)));
+void allow_lds(K kern, size_t bytes) {
+    BLQH_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
 }
 
-SGroups make_groups(const blqh_batch* b) {
-    return SGroups{b->gitem_grp.get(), b->dgitem0.get(), b->dtscale.get()};
-}
-
-template <bool LZ, int KIND, int G>
-void launch_b1s_go(const blqh_batch* b, const BState& S, int jrel, const double2* xs, double2* ys, double* part,
-                   hipStream_t st) {
-    static const bool attr = (allow_table(k_b1s<LZ, KIND, G>), true);  // once per instantiation, thread-safe
+template <bool LZ, int G, bool SH>
+void launch_b1x(const blqh_batch* b, const BState& S, int jrel, const double2* xs, double2* ys, double* part,
+                hipStream_t st) {
+    static const bool attr = (allow_lds(k_b1x<LZ, G, SH>, kLdsMax), true);  // once per instantiation, thread-safe
     (void)attr;
-    hipLaunchKernelGGL((k_b1s<LZ, KIND, G>), dim3(b->grid), dim3(kBTj), b->tab_bytes, st, S, make_groups(b), jrel, xs,
+    hipLaunchKernelGGL((k_b1x<LZ, G, SH>), dim3(b->x_grid), dim3(kBTx), b->x_bytes, st, S, b->dtscale.get(), jrel, xs,
                        ys, part);
-}
-
-template <bool LZ, int KIND>
-void launch_b1s_kind(const blqh_batch* b, const BState& S, int jrel, const double2* xs, double2* ys, double* part,
-                     hipStream_t st) {
-    switch (b->G) {
-        case 1: launch_b1s_go<LZ, KIND, 1>(b, S, jrel, xs, ys, part, st); break;
-        case 2: launch_b1s_go<LZ, KIND, 2>(b, S, jrel, xs, ys, part, st); break;
-        case 3: launch_b1s_go<LZ, KIND, 3>(b, S, jrel, xs, ys, part, st); break;
-        case 4: launch_b1s_go<LZ, KIND, 4>(b, S, jrel, xs, ys, part, st); break;
-        default: throw Error(BLQH_EINTERNAL, "unsupported group size");
-    }
 }
 
 template <bool LZ, int KIND>
 void launch_b1j(const blqh_batch* b, const BState& S, int jrel, const double2* xs, double2* ys, double* part,
                 hipStream_t st) {
-    static const bool attr = (allow_table(k_b1j<LZ, KIND>), true);
+    static const bool attr = (allow_lds(k_b1j<LZ, KIND>, cod_lds_bytes(false, kCodCplx)), true);
     (void)attr;
     hipLaunchKernelGGL((k_b1j<LZ, KIND>), dim3(b->grid), dim3(kBTj), b->tab_bytes, st, S, jrel, xs, ys, part);
 }
@@ -972,13 +1209,16 @@ template <bool LZ>
 void launch_b1(const blqh_batch* b, const BState& S, int jrel, const double2* xs, double2* ys, double* part,
                hipStream_t st) {
     const dim3 g(b->grid), t(kBT);
-    if (b->G) {  // shared-scale groups: one pass over each sector's entries for all its problems
-        if (b->has_real && b->has_complex) {
-            launch_b1s_kind<LZ, 2>(b, S, jrel, xs, ys, part, st);
-        } else {
-            if (b->has_real) launch_b1s_kind<LZ, 0>(b, S, jrel, xs, ys, part, st);
-            if (b->has_complex) launch_b1s_kind<LZ, 1>(b, S, jrel, xs, ys, part, st);
-        }
+    switch (b->G) {  // shared-scale groups: one pass over each sector's entries for all its problems
+        case 0: break;
+        case 1: launch_b1x<LZ, 1, true>(b, S, jrel, xs, ys, part, st); return;
+        case 2: launch_b1x<LZ, 2, true>(b, S, jrel, xs, ys, part, st); return;
+        case 3: launch_b1x<LZ, 3, true>(b, S, jrel, xs, ys, part, st); return;
+        case 4: launch_b1x<LZ, 4, true>(b, S, jrel, xs, ys, part, st); return;
+        default: throw Error(BLQH_EINTERNAL, "unsupported group size");
+    }
+    if (use_tiles(b)) {
+        launch_b1x<LZ, 1, false>(b, S, jrel, xs, ys, part, st);
         return;
     }
     switch (b->lpr) {
@@ -1051,7 +1291,9 @@ blqh_batch* blqh_batch_create_impl(blqh_hamil* const* hs, int count, int lanes) 
         // a multiple of 8 (one share per XCD in k_b1j)
         b->grid = (int)(8 * ceil_div(std::min<int64_t>(b->nitems, (int64_t)runtime().num_cus * 8), 8));
         b->xitems.alloc(2 * b->nitems);
-        b->xseg.alloc(27);
+        b->xseg.alloc(28);
+        b->one_panel = b->hs.size() < ((size_t)1 << (31 - kElemBits));
+        for (const BProb& d : b->h_probs) b->one_panel = b->one_panel && d.npan == 1;
         b->lpr = lanes ? lanes : 64;
         refresh_probs(b);
     } catch (...) {
@@ -1075,6 +1317,7 @@ void blqh_batch_rebind_impl(blqh_batch* b, blqh_hamil* const* hs, int count) {
     }
     b->nnz = nnz;
     b->hs.assign(hs, hs + count);
+    b->tiles_ok = false;
     refresh_probs(b);
 }
 
@@ -1161,14 +1404,11 @@ blqh_batch* blqh_batch_create_scaled_impl(const blqh_hamil* const* base, const b
         const int P = nsec * G;
         b->hs.resize(P);
         b->item0.assign(P + 1, 0);
-        b->gitem0.assign(nsec + 1, 0);
         b->tscale.resize(P);
-        std::vector<int32_t> ip, gp;
+        std::vector<int32_t> ip;
         for (int q = 0; q < nsec; ++q) {
             blqh_hamil* H = b->tpl[q];
             const int64_t nit = ceil_div(H->n, kItemRows);
-            b->gitem0[q + 1] = b->gitem0[q] + nit;
-            for (int64_t i = 0; i < nit; ++i) gp.push_back(q);
             b->nnz += H->nnz;
             for (int g = 0; g < G; ++g) {
                 const int p = q * G + g;
@@ -1186,20 +1426,17 @@ blqh_batch* blqh_batch_create_scaled_impl(const blqh_hamil* const* base, const b
                 b->h_probs.push_back(d);
             }
         }
-        b->ngitems = b->gitem0[nsec];
         BLQH_REQUIRE(b->nitems < (int64_t)1 << 31, BLQH_ERANGE, "batch too large");
         b->item_prob.alloc(ip.size());
         copy_sync(b->item_prob.get(), ip.data(), ip.size() * 4, hipMemcpyHostToDevice);
-        b->gitem_grp.alloc(gp.size());
-        copy_sync(b->gitem_grp.get(), gp.data(), gp.size() * 4, hipMemcpyHostToDevice);
-        b->dgitem0.alloc(nsec + 1);
-        copy_sync(b->dgitem0.get(), b->gitem0.data(), (nsec + 1) * 8, hipMemcpyHostToDevice);
         b->dtscale.alloc(P);
         copy_sync(b->dtscale.get(), b->tscale.data(), P * 8, hipMemcpyHostToDevice);
         b->grid = (int)(8 * ceil_div(std::min<int64_t>(b->nitems, (int64_t)runtime().num_cus * 8), 8));
         b->xitems.alloc(2 * b->nitems);
-        b->xseg.alloc(27);
+        b->xseg.alloc(28);
         b->lpr = 64;
+        b->one_panel = b->hs.size() < ((size_t)1 << (31 - kElemBits));
+        for (const BProb& d : b->h_probs) b->one_panel = b->one_panel && d.npan == 1;
         refresh_probs(b);
     } catch (...) {
         delete b;
@@ -1224,12 +1461,9 @@ void blqh_batch_rebind_scaled_impl(blqh_batch* b, const blqh_hamil* const* base,
     b->nnz = 0;
     for (int q = 0; q < nsec; ++q) {
         b->nnz += b->tpl[q]->nnz;
-        for (int g = 0; g < b->G; ++g) {
-            const int p = q * b->G + g;
-            b->hs[p] = b->tpl[q];
-            b->h_probs[p].real = b->tpl[q]->cod.real ? 1 : 0;
-        }
+        for (int g = 0; g < b->G; ++g) b->hs[q * b->G + g] = b->tpl[q];
     }
+    b->tiles_ok = false;
     refresh_probs(b);
 }
 
@@ -1310,7 +1544,7 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
         b->pin = nullptr;
         // alpha, beta, two slots of active flags, two slots of live work lists
         const size_t pin_bytes = ((size_t)P * cap + (size_t)P * ld) * 8 + 2 * (size_t)P * 4 +
-                                 2 * (2 * (size_t)b->nitems + 27) * 4;
+                                 2 * (2 * (size_t)b->nitems + 28) * 4;
         BLQH_HIP(hipHostMalloc((void**)&b->pin, pin_bytes, hipHostMallocDefault));
         b->pool_cap = cap;
     }
@@ -1496,7 +1730,7 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
     } evguard{ev};
     const int kinds = (b->has_real ? 2 : 0) | (b->has_complex ? 1 : 0);  // which K1 launches a step has
     if (!timed && (b->g_chk != chk || b->g_lpr != b->lpr || b->g_cap != cap || b->g_kinds != kinds ||
-                   b->g_tab != b->tab_bytes || !b->gexec)) {
+                   b->g_tab != k1_shape(b) || !b->gexec)) {
         if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
         if (b->graph) (void)hipGraphDestroy(b->graph);
         b->gexec = nullptr;
@@ -1509,7 +1743,7 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
         b->g_lpr = b->lpr;
         b->g_cap = cap;
         b->g_kinds = kinds;
-        b->g_tab = b->tab_bytes;
+        b->g_tab = k1_shape(b);
     }
     hipGraphExec_t gexec = b->gexec;
     const int zero = 0;
@@ -1527,7 +1761,7 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
     // Every item's sums keep their owner and order, so results do not depend
     // on the lists.  Two pinned slots, as for the active flags.
     int32_t* listpin = actpin + 2 * (size_t)P;
-    const size_t list_slot = 2 * (size_t)b->nitems + 27;
+    const size_t list_slot = 2 * (size_t)b->nitems + 28;
     int lslot = 0;
     bool lists_live = false;
     hipEvent_t evc;
@@ -1637,12 +1871,12 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
             slot ^= 1;
             if (b->lpr == 64) {  // k_b1j walks the lists
                 std::vector<int32_t> items, seg;
-                xcd_lists(xcd_members(b, &live), items, seg);
+                work_lists(b, &live, items, seg);
                 int32_t* lp = listpin + (size_t)lslot * list_slot;
                 std::copy(items.begin(), items.end(), lp);
                 std::copy(seg.begin(), seg.end(), lp + 2 * b->nitems);
                 BLQH_HIP(hipMemcpyAsync(b->xitems.get(), lp, items.size() * 4, hipMemcpyHostToDevice, st));
-                BLQH_HIP(hipMemcpyAsync(b->xseg.get(), lp + 2 * b->nitems, 27 * 4, hipMemcpyHostToDevice, st));
+                BLQH_HIP(hipMemcpyAsync(b->xseg.get(), lp + 2 * b->nitems, 28 * 4, hipMemcpyHostToDevice, st));
                 lslot ^= 1;
                 lists_live = true;
             }
@@ -1652,7 +1886,7 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
     BLQH_HIP(hipStreamSynchronize(st));  // a speculative replay may still run
     if (lists_live) {  // every member takes part in the final products again
         copy_sync(b->xitems.get(), b->h_xitems.data(), b->h_xitems.size() * 4, hipMemcpyHostToDevice);
-        copy_sync(b->xseg.get(), b->h_xseg.data(), 27 * 4, hipMemcpyHostToDevice);
+        copy_sync(b->xseg.get(), b->h_xseg.data(), 28 * 4, hipMemcpyHostToDevice);
     }
 
     phase("iterate");

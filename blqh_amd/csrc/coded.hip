@@ -173,8 +173,9 @@ __global__ void __launch_bounds__(kHist) k_dict_select(const uint64_t* __restric
 }
 
 // A wavefront per internal row r (reference row iperm[r]): key = rest flag and
-// internal column in the high word, code and source index in the low one; sorted,
-// so the coded entries come first, columns ascending, then the rest.  skey is
+// internal column in the high word, code, flag and source index in the low one; sorted,
+// so the coded entries come first, columns ascending, then the rest, then (marked
+// kNoKey) the diagonal, which goes to diag.  skey is
 // indexed as the CSR (row iperm[r]'s place).  nu (a shared-scale template): upper-
 // layer occupation per internal row; an entry between different ones carries the
 // tunnelling flag and is counted.
@@ -184,12 +185,13 @@ __global__ void __launch_bounds__(64) k_cod_rows(int64_t n, int64_t npadrows, in
                                                  const double2* __restrict__ val, DictHash L,
                                                  const int32_t* __restrict__ info, const uint8_t* __restrict__ nu,
                                                  uint64_t* __restrict__ skey, uint16_t* __restrict__ len,
-                                                 uint16_t* __restrict__ rlen, int32_t* __restrict__ ctr) {
+                                                 uint16_t* __restrict__ rlen, double* __restrict__ diag,
+                                                 int32_t* __restrict__ ctr) {
     extern __shared__ uint64_t key[];
     const int lane = threadIdx.x;
     const bool real = info[1] != 0;
     const uint32_t lmask = real ? L.mask_real : L.mask_cplx;
-    int ntun = 0;
+    int ntun = 0, dtot = 0;
     for (int64_t r = blockIdx.x; r < npadrows; r += gridDim.x) {
         if (r >= n) {  // padding rows of the last slice
             for (int p = lane; p < npan; p += 64) len[(int64_t)p * npadrows + r] = 0;
@@ -205,14 +207,25 @@ __global__ void __launch_bounds__(64) k_cod_rows(int64_t n, int64_t npadrows, in
         }
         int P = 64;
         while (P < m) P <<= 1;
-        int nrest = 0;
+        int nrest = 0, ndiag = 0;
+        if (lane == 0) {
+            diag[real ? r : 2 * r] = 0.0;
+            if (!real) diag[2 * r + 1] = 0.0;
+        }
         __syncthreads();
         for (int k = lane; k < P; k += 64) {
             uint64_t w = kNoKey;
             if (k < m) {
                 const int32_t c0 = col[s + k];
-                uint32_t c = (uint32_t)(perm ? perm[c0] : c0);
+                const uint32_t c = (uint32_t)(perm ? perm[c0] : c0);
                 const double2 v = val[s + k];
+                if (c0 == o) {
+                    diag[real ? r : 2 * r] = v.x;
+                    if (!real) diag[2 * r + 1] = v.y;
+                    ++ndiag;
+                    key[k] = kNoKey;
+                    continue;
+                }
                 const uint64_t br = (uint64_t)__double_as_longlong(v.x), bi = (uint64_t)__double_as_longlong(v.y);
                 const uint64_t kr = br & kAbs, ki = real ? 0 : bi & kAbs;
                 uint32_t h = dict_hash(kr, ki) & lmask;
@@ -231,15 +244,16 @@ __global__ void __launch_bounds__(64) k_cod_rows(int64_t n, int64_t npadrows, in
                     code = (uint32_t)id | (uint32_t)((br >> 63) << 15) | (real ? 0u : (uint32_t)((bi >> 63) << 14));
                 else
                     ++nrest;
-                if (nu && nu[c] != nu[r]) {
-                    ++ntun;
-                    c |= kCodTun;  // columns below 2^15: order kept within each kind
-                }
-                w = (uint64_t)(id < 0) << 63 | (uint64_t)c << 32 | code << 16 | (uint32_t)k;
+                const bool tun = nu && nu[c] != nu[r];
+                ntun += tun;
+                w = (uint64_t)(id < 0) << 63 | (uint64_t)c << 32 | code << 16 | (tun ? kCodTun : 0u) | (uint32_t)k;
             }
             key[k] = w;
         }
-        for (int q = 32; q > 0; q >>= 1) nrest += __shfl_xor(nrest, q, 64);
+        for (int q = 32; q > 0; q >>= 1) {
+            nrest += __shfl_xor(nrest, q, 64);
+            ndiag += __shfl_xor(ndiag, q, 64);
+        }
         __syncthreads();
         for (int k = 2; k <= P; k <<= 1)
             for (int j = k >> 1; j > 0; j >>= 1) {
@@ -254,7 +268,8 @@ __global__ void __launch_bounds__(64) k_cod_rows(int64_t n, int64_t npadrows, in
                 __syncthreads();
             }
         for (int k = lane; k < m; k += 64) skey[s + k] = key[k];
-        const int nc = m - nrest;
+        const int nc = m - nrest - ndiag;
+        dtot += ndiag;
         for (int p = lane; p < npan; p += 64) {  // entries of panel p: between two lower bounds
             const uint64_t a = (uint64_t)p << 48, b = (uint64_t)(p + 1) << 48;
             int lo = 0, hi = nc;
@@ -272,6 +287,7 @@ __global__ void __launch_bounds__(64) k_cod_rows(int64_t n, int64_t npadrows, in
         }
         if (lane == 0) rlen[r] = (uint16_t)nrest;
     }
+    if (lane == 0 && dtot) atomicAdd(&ctr[2], dtot);
     if (nu) {
         for (int q = 32; q > 0; q >>= 1) ntun += __shfl_xor(ntun, q, 64);
         if (lane == 0 && ntun) atomicAdd(&ctr[1], ntun);
@@ -314,7 +330,7 @@ __global__ void __launch_bounds__(kBlk) k_cod_fill(int64_t n, int64_t nslices, i
                     const uint64_t m = __ballot(t + u < ln);
                     if (t + u < ln)
                         out[off + lanes_below(m)] = ((uint32_t)(w[u] >> 32) & 0xffffu) |
-                                                    ((uint32_t)w[u] & 0xffff0000u);
+                                                    ((uint32_t)w[u] & (0xffff0000u | kCodTun));
                     off += (uint32_t)__popcll(m);
                 }
             }
@@ -324,10 +340,11 @@ __global__ void __launch_bounds__(kBlk) k_cod_fill(int64_t n, int64_t nslices, i
 }
 
 // A wavefront per slice: its rest (32-bit column, value), step-major.
-__global__ void __launch_bounds__(kBlk) k_cod_rest(int64_t n, int64_t nslices, int real,
+__global__ void __launch_bounds__(kBlk) k_cod_rest(int64_t n, int64_t nslices, int npan, int real,
                                                    const int32_t* __restrict__ iperm,
                                                    const int64_t* __restrict__ rowptr,
                                                    const double2* __restrict__ val, const uint64_t* __restrict__ skey,
+                                                   const uint16_t* __restrict__ len,
                                                    const uint16_t* __restrict__ rlen,
                                                    const int64_t* __restrict__ rbase, uint32_t* __restrict__ rcol,
                                                    double* __restrict__ rval) {
@@ -337,16 +354,18 @@ __global__ void __launch_bounds__(kBlk) k_cod_rest(int64_t n, int64_t nslices, i
         const int64_t row = sl * 64 + lane;
         const uint32_t ln = rlen[row];
         const int64_t o = row < n ? (iperm ? iperm[row] : row) : 0;
-        const int64_t s = row < n ? rowptr[o] : 0, e = row < n ? rowptr[o + 1] : 0;
+        const int64_t s = row < n ? rowptr[o] : 0;
+        int64_t f = s;  // the row's first rest entry: behind its coded ones
+        for (int p = 0; p < npan; ++p) f += len[((int64_t)p * nslices + sl) * 64 + lane];
         int64_t off = rbase[sl];
         for (uint32_t t = 0;; ++t) {
             const uint64_t m = __ballot(t < ln);
             if (m == 0) break;
             if (t < ln) {
-                const uint64_t w = skey[e - ln + t];
+                const uint64_t w = skey[f + t];
                 const int64_t to = off + lanes_below(m);
-                const double2 v = val[s + (int64_t)(w & 0xffffu)];
-                rcol[to] = (uint32_t)(w >> 32) & 0x7fffffffu;
+                const double2 v = val[s + (int64_t)(w & (kMaxRow - 1))];
+                rcol[to] = ((uint32_t)(w >> 32) & 0x7fffffffu) | ((uint32_t)w & kCodTun);
                 if (real) {
                     rval[to] = v.x;
                 } else {
@@ -384,7 +403,7 @@ void build_coded(blqh_hamil* H, const uint8_t* nu, int64_t* ntun) {
     const int64_t samples = std::min<int64_t>(nnz, 1 << 16);
     uint32_t slots = 1024;
     while (slots < 2 * samples) slots <<= 1;
-    constexpr uint32_t kLook = 2 * kCodCplx;
+    constexpr uint32_t kLook = 2 * (kCodCplx + 1);
     // one block: maxima (2 words), info and counters (4 + 4 ints), histogram, the
     // sample's hash, the lookup hash
     constexpr size_t kHead = 8 + kHist;
@@ -398,7 +417,7 @@ void build_coded(blqh_hamil* H, const uint8_t* nu, int64_t* ntun) {
     uint64_t* ski = skr + slots;
     int32_t* cnt = (int32_t*)(ski + slots);
     uint64_t* look = ski + slots + slots / 2;
-    const DictHash L{look, look + kLook, (int32_t*)(look + 2 * kLook), 2 * kCodReal - 1, kLook - 1};
+    const DictHash L{look, look + kLook, (int32_t*)(look + 2 * kLook), 2 * (kCodReal + 1) - 1, kLook - 1};
     DevBuf<double> tab(2 * kCodCplx);
     auto fill = [&](void* p, int64_t words, uint64_t v) {
         hipLaunchKernelGGL(k_fill64, dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>(ceil_div(words, kBlk), 2048))),
@@ -419,6 +438,7 @@ void build_coded(blqh_hamil* H, const uint8_t* nu, int64_t* ntun) {
     DevBuf<uint64_t> skey(std::max<int64_t>(nnz, 1));
     C.len.alloc((size_t)runs * 64);
     C.rlen.alloc((size_t)nsl * 64);
+    C.diag.alloc(2 * (size_t)std::max<int64_t>(n, 1));
     const int64_t rows = nsl * 64;
     const int gr = (int)std::min<int64_t>(rows, (int64_t)runtime().num_cus * 40);
     int P = 64;  // LDS for the longest row the build can have kept
@@ -426,7 +446,7 @@ void build_coded(blqh_hamil* H, const uint8_t* nu, int64_t* ntun) {
     while (P < rmax) P <<= 1;
     hipLaunchKernelGGL(k_cod_rows, dim3(gr), dim3(64), (size_t)P * 8, st, n, rows, C.npan, P, iperm, perm,
                        H->rowptr.get(), H->col.get(), H->val.get(), L, info, nu, skey.get(), C.len.get(),
-                       C.rlen.get(), ctr);
+                       C.rlen.get(), C.diag.get(), ctr);
     BLQH_HIP(hipGetLastError());
     DevBuf<int32_t> tot(runs + nsl);
     hipLaunchKernelGGL(k_cod_runs, dim3(grid_waves(runs)), dim3(kBlk), 0, st, runs, C.len.get(), tot.get());
@@ -444,7 +464,7 @@ void build_coded(blqh_hamil* H, const uint8_t* nu, int64_t* ntun) {
     C.ntab = hw[0];
     C.real = hw[1] != 0;
     BLQH_REQUIRE(hw[4] == 0, BLQH_EINTERNAL, "a CSR row is longer than the coded layout handles");
-    BLQH_REQUIRE(C.ncod + C.nrest == nnz, BLQH_EINTERNAL, "coded layout lost entries");
+    BLQH_REQUIRE(C.ncod + C.nrest + hw[6] == nnz, BLQH_EINTERNAL, "coded layout lost entries");
     if (ntun) *ntun = hw[5];
     C.ent.alloc(std::max<int64_t>(C.ncod, 1));
     C.rcol.alloc(std::max<int64_t>(C.nrest, 1));
@@ -454,8 +474,8 @@ void build_coded(blqh_hamil* H, const uint8_t* nu, int64_t* ntun) {
     hipLaunchKernelGGL(k_cod_fill, dim3(grid_waves(nsl)), dim3(kBlk), 0, st, n, nsl, C.npan, iperm,
                        H->rowptr.get(), skey.get(), C.len.get(), C.base.get(), C.ent.get());
     if (C.nrest > 0)
-        hipLaunchKernelGGL(k_cod_rest, dim3(grid_waves(nsl)), dim3(kBlk), 0, st, n, nsl, C.real ? 1 : 0, iperm,
-                           H->rowptr.get(), H->val.get(), skey.get(), C.rlen.get(), C.rbase.get(), C.rcol.get(),
+        hipLaunchKernelGGL(k_cod_rest, dim3(grid_waves(nsl)), dim3(kBlk), 0, st, n, nsl, C.npan,
+                           C.real ? 1 : 0, iperm, H->rowptr.get(), H->val.get(), skey.get(), C.len.get(), C.rlen.get(), C.rbase.get(), C.rcol.get(),
                            C.rval.get());
     BLQH_HIP(hipGetLastError());
     BLQH_HIP(hipStreamSynchronize(st));  // complete for solves on other threads' streams

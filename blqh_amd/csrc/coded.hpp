@@ -2,14 +2,15 @@
 // coded.hip) and its per-row sums.
 //
 // A matrix element is a sum of a few Coulomb table entries times a translation
-// phase, so a sector's entries take few distinct values: the 1,024 most
-// frequent magnitudes of a real sector and the 4,096 most frequent (|re|, |im|)
+// phase, so a sector's entries take few distinct values: the 1,023 most
+// frequent magnitudes of a real sector and the 4,095 most frequent (|re|, |im|)
 // pairs of a complex one cover 99 % of the entries and more (N_phi = 12: 99.2 /
 // 99.4 %, N_phi = 14: 99.6 / 99.5 %, N_phi = 16 at half filling: 99.7 %).  Those values sit in a table that every workgroup
 // holds in LDS, and an entry is one 32-bit word: column within its panel in the
 // low 16 bits, table index above, sign of the real (and imaginary) part on top.  The matrix stream is 4 bytes an entry instead of 10 (real) or 18
 // (complex), bit for bit the same values.  Entries whose value is not in the
-// table form the rest: 32-bit column and value, one run per 64-row slice.
+// table form the rest: 32-bit column and value, one run per 64-row slice.  The
+// diagonal, whose values are nearly all different, is an array of its own.
 //
 // Order: columns in panels of 65,536, 64-row slices; run (panel, slice) is
 // step-major: step t holds entry t of every row with more than t entries in the
@@ -23,8 +24,8 @@
 
 namespace blqh {
 
-constexpr int kCodReal = 1024;   // table entries of a real matrix (8 KiB of LDS), at most
-constexpr int kCodCplx = 4096;   // of a complex one (64 KiB)
+constexpr int kCodReal = 1023;   // table entries of a real matrix (8 KiB of LDS), at most
+constexpr int kCodCplx = 4095;   // of a complex one (64 KiB)
 constexpr uint32_t kCodTun = 0x8000u;  // tunnelling flag of a shared-scale template's columns
 
 struct Coded {
@@ -41,6 +42,7 @@ struct Coded {
     DevBuf<uint16_t> rlen;   // [nslices * 64]
     DevBuf<uint32_t> rcol;   // [nrest]
     DevBuf<double> rval;     // [nrest] or [2 nrest]
+    DevBuf<double> diag;     // [n] or [2 n]
 };
 
 struct CodView {
@@ -54,11 +56,13 @@ struct CodView {
     const uint16_t* rlen;
     const uint32_t* rcol;
     const double* rval;
+    const double* diag;
 };
 
 inline CodView cview(const Coded& C, int64_t n) {
     return CodView{n,           (n + 63) >> 6, C.npan,        C.ntab,       C.tab.get(),  C.base.get(),
-                   C.len.get(), C.ent.get(),   C.rbase.get(), C.rlen.get(), C.rcol.get(), C.rval.get()};
+                   C.len.get(), C.ent.get(),   C.rbase.get(), C.rlen.get(), C.rcol.get(), C.rval.get(),
+                   C.diag.get()};
 }
 
 inline size_t cod_lds_bytes(bool real, int ntab) { return (size_t)(ntab > 0 ? ntab : 1) * (real ? 8 : 16); }
@@ -73,6 +77,11 @@ __device__ __forceinline__ double cod_real(const double* tab, uint32_t e) {
 __device__ __forceinline__ double2 cod_cplx(const double2* tab, uint32_t e) {
     const double2 v = tab[(e >> 16) & 0x3fffu];
     return make_double2(cod_sign(v.x, e), cod_sign(v.y, e << 1));
+}
+
+// diagonal element of a row
+__device__ __forceinline__ double2 cod_diag(const CodView& C, bool real, int64_t row) {
+    return real ? make_double2(C.diag[row], 0.0) : reinterpret_cast<const double2*>(C.diag)[row];
 }
 
 // Table to LDS (the caller synchronises the workgroup).

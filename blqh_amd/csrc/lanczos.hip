@@ -771,6 +771,16 @@ __global__ void __launch_bounds__(kT4Threads) k_t4(TileView V, const double2* __
 // the table in LDS.  A team of NP wavefronts owns a 64-row slice (lane l <-> row l)
 // and shares its step groups; a workgroup holds WPB / NP teams on neighbouring
 // slices, which gather from the same lines of x.
+//
+// Bound by the vector L1's rate of x gathers, not by the stream: 0.75 lane gathers
+// per clock and CU at N_phi = 16 (831M entries; 3.3 GB of words read at 1.8 TB/s).
+// What measured best there: 512 threads, the whole workgroup kept on one panel by
+// the barrier (2,100 us without it, 1,880 with), eight steps in flight per wavefront
+// (four: 2,050 us).  Wider panels, 4 or 16 wavefronts a workgroup and persistent
+// grids gave nothing.  Step of one Lanczos iteration, K1 only, against the
+// jagged panels of 10 (real) or 18 (complex) bytes an entry: N_phi = 16 all
+// densities 2,907 -> 1,880 us, nel_up = 8 811 -> 475, N_phi = 14 real 209 -> 131 and
+// complex 265 -> 155, N_phi = 12 complex 24 -> 17.5.
 template <bool REAL, bool LZ, int WPB, int NP>
 __global__ void __launch_bounds__(WPB * 64) k_cod(CodView P, const double2* __restrict__ x, double2* __restrict__ out,
                                                   const double2* __restrict__ Wp, Scal sc, int j, double* partials) {
@@ -806,6 +816,9 @@ __global__ void __launch_bounds__(WPB * 64) k_cod(CodView P, const double2* __re
             y.x += o.x;
             y.y += o.y;
         }
+        const double2 w = x[row], dg = cod_diag(P, REAL, row);
+        y.x += dg.x * w.x - dg.y * w.y;
+        y.y += dg.x * w.y + dg.y * w.x;
         if (LZ) {
             const double ib = sc.invb[j];
             double ur = ib * y.x, ui = ib * y.y;
@@ -816,7 +829,6 @@ __global__ void __launch_bounds__(WPB * 64) k_cod(CodView P, const double2* __re
                 ui -= cp * q.y;
             }
             out[row] = make_double2(ur, ui);
-            const double2 w = x[row];
             dacc = w.x * ur + w.y * ui;
         } else {
             out[row] = y;
@@ -1048,7 +1060,12 @@ void cod_dispatch(const blqh_hamil* H, const Plan& pl, const double2* x, double2
     throw Error(BLQH_EINTERNAL, "unsupported coded SpMV plan");
 }
 
-// The coded plan of a matrix by its size.
+// The coded plan of a matrix by its size.  A team of NP wavefronts per slice splits
+// the slice's chain of steps, which a small matrix needs to fill 256 CUs with 32
+// wavefronts each (N_phi = 12, 295 slices: 27 us at NP = 1, 17.5 at 8); at 24,576
+// wavefronts the chip is full and the team's sum costs more than it gives (N_phi =
+// 14, 3,200 slices: NP = 4 131 us, 8 151 us; N_phi = 16, nel_up = 8, 9,300 slices: NP =
+// 2 475 us, 1 497 us, 4 490 us).
 Plan coded_plan(const blqh_hamil* H) {
     const int64_t nsl = ceil_div(H->n, 64);
     int np = 1;

@@ -241,8 +241,7 @@ int blqh_lanczos_reconstruct(const blqh_hamil* h, int32_t m, uint32_t seed, cons
  * start vectors (NULL array or NULL entry: seeded); psi: per-problem outputs
  * (2*nrows doubles; NULL array or entry: not copied); res[count]. ---- */
 typedef struct blqh_batch blqh_batch;
-/* lanes: 0 = autotune the batched SpMV on this batch, else as blqh_batch_set_lanes
- * (a sweep tunes its first batch and passes the choice to the next ones). */
+/* lanes: 0 = the default (64), else as blqh_batch_set_lanes. */
 int blqh_batch_create(blqh_hamil* const* hs, int32_t count, int32_t lanes, blqh_batch** out);
 /* Replace the members by Hamiltonians of the same sizes in the same order (the
  * next point of a parameter sweep); device pools, the captured replay and the
@@ -266,7 +265,7 @@ int blqh_batch_lanczos(blqh_batch* b, const blqh_lanczos_opts* o, const uint32_t
 int blqh_batch_lanczos_continue(blqh_batch* b, const blqh_lanczos_opts* o, const uint32_t* seeds,
                                 double excited_mix, blqh_lanczos_result* res, double* const* psi);
 /* Lanes per row of the batched SpMV (4, 8, 16 or 32 over row-major panels;
- * 64: one lane per row over step-major panels; autotuned at create). */
+ * 64, the default: one lane per row over the coded layout). */
 int blqh_batch_get_lanes(const blqh_batch* b, int32_t* lanes);
 int blqh_batch_set_lanes(blqh_batch* b, int32_t lanes);
 /* Shared-scale batch: the Delta_SAS points of one d, the inner loop of

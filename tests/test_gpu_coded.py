@@ -67,3 +67,53 @@ def test_refused_plans(built):
     for bad in ((6, 32, 512, 0, 2), (6, 64, 128, 0, 1), (6, 64, 256, 0, 8), (6, 64, 512, 0, 3), (6, 64, 512, 0, 0)):
         with pytest.raises(blqh_amd.BlqhError):
             H.set_spmv(*bad)
+
+
+# Batches of one-panel members take x through LDS by column tiles; a member of more than
+# 65536 rows moves the whole batch to the gathering kernel.
+BATCHES = {
+    "tiny": [(2, 4, 4, 2, -1, 0, 0), (2, 6, 6, 3, -1, 1, 2), (2, 8, 8, 4, -1, 4, 4)],
+    "mixed_kinds": [(2, 8, 8, -1, -1, 1, 3), (2, 10, 10, 5, -1, 0, 0), (4, 6, 6, 3, 3, 0, 1)],
+    "one_and_many_tiles": [(2, 12, 12, -1, -1, 0, 0), (2, 6, 6, 3, -1, 0, 0), (2, 13, 13, -1, -1, 1, 0)],
+    "several_panels": [(2, 14, 14, -1, -1, 0, 0), (2, 8, 8, 4, -1, 4, 4)],
+}
+
+
+@pytest.mark.parametrize("name", BATCHES)
+def test_batch_against_panel_kernel(name):
+    """lanes = 64 (coded layout) against lanes = 16 (CSR-valued panels): a set number of
+    steps, so that both run the same recurrence; energies to 1e-11 of the scale."""
+    hams = []
+    for S, nphi, nel, nu, nsu, J, K in BATCHES[name]:
+        B = blqh_amd.Basis(nphi, nel, nu, J, K, nspecies=S, nel_su=nsu)
+        hams.append(blqh_amd.Hamiltonian(B, blqh_amd.params(nphi, d=0.9, delta_sas=0.05 if nu < 0 else 0.0)))
+    print(f"{name} rows {[h.n for h in hams]}", flush=True)
+    seeds = list(range(3, 3 + len(hams)))
+    batch = blqh_amd.Batch(hams)
+    assert batch.lanes == 64
+    steps = dict(lam=8, seeds=seeds, tol=0.0, res_tol=0.0, check_every=3)
+    a = batch.lanczos(**steps)
+    batch.lanes = 16
+    b = batch.lanczos(**steps)
+    for h, u, v in zip(hams, a, b):
+        assert u["E0"] == pytest.approx(v["E0"], rel=1e-11, abs=1e-11)
+        if h.n > 8:  # with fewer states than steps the recurrence has run out of vectors
+            np.testing.assert_allclose(u["psi"], v["psi"], rtol=0, atol=1e-9)
+
+
+@pytest.mark.parametrize("G", [1, 2, 3, 4])
+@pytest.mark.parametrize("sector", [(12, 0, 6), (12, 1, 5), (8, 1, 3)], ids=["real_tiles", "complex_tiles", "one_tile"])
+def test_shared_scales_against_combined(sector, G):
+    """G scales on one base and tunnelling part against the G combined matrices, eight steps."""
+    nphi, J, K = sector
+    scales = [0.05, 0.1, 0.2, 0.0][:G]
+    B = blqh_amd.Basis(nphi, nphi, -1, J, K)
+    par = blqh_amd.params(nphi, d=0.6)
+    h0, t = blqh_amd.Hamiltonian(B, par, terms=1), blqh_amd.Hamiltonian(B, par, terms=2)
+    print(f"sector {sector} n {h0.n} G {G}", flush=True)
+    steps = dict(lam=8, tol=0.0, res_tol=0.0)
+    r = blqh_amd.Batch.scaled([h0], [t], scales).lanczos(seeds=[7] * G, check_every=3, **steps)
+    for s, u in zip(scales, r):
+        one = blqh_amd.Hamiltonian.combine(h0, t, s).lanczos(seed=7, **steps)
+        assert u["E0"] == pytest.approx(one["E0"], rel=1e-11, abs=1e-11)
+        np.testing.assert_allclose(u["psi"], one["psi"], rtol=0, atol=1e-9)
