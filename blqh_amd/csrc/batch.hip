@@ -1835,6 +1835,8 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
                 }
                 if (o.tol > 0 && j > 0 && dE[p] < o.tol) {
                     if (o.res_tol <= 0) { conv[p] = 1; break; }
+                    resid[p] = INFINITY;
+                    if (residual_exceeds(j + 1, a, bb + 1, ritz[p][j], bb[j + 1], o.res_tol)) continue;
                     (void)tridiag_lowest(j + 1, a, bb + 1, svec.data());
                     resid[p] = bb[j + 1] * std::fabs(svec[j]);
                     if (resid[p] < o.res_tol) { conv[p] = 1; break; }
@@ -1846,7 +1848,8 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
             for (int p = 0; p < P; ++p)
                 if (live[p]) live_ids.push_back(p);
             const int nl = (int)live_ids.size();
-            const int nt = std::min(nthr, (nl + 3) / 4);  // at least four problems per thread
+            // a test of m steps takes about 0.1 m us; waking a thread, some 20 us
+            const int nt = std::min({nthr, nl, 1 + nl * (upto - done) * upto / 400});
             if (nt <= 1) {
                 for (int p : live_ids) test(p, svecs[0]);
             } else {

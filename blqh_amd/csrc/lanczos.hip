@@ -26,6 +26,7 @@
 
 #include "engine.hpp"
 #include "mtstart.hpp"
+#include "ritz.hpp"
 
 namespace {
 
@@ -186,14 +187,37 @@ __global__ void __launch_bounds__(kThreads) k_lz2(int64_t n, const double2* __re
     block_partial(acc, part2);
 }
 
-// K3: beta[j+1] = sqrt(sum of K2's partials), invb[j+1]; one workgroup
-__global__ void __launch_bounds__(kThreads) k_lz3(Scal sc, int j, const double* __restrict__ part2, int npart2) {
+// Mailbox of a solve in pinned host memory: K3 of step j leaves alpha_j and beta_{j+1}
+// in entry j mod kMail and then its tag (solve number, step), which the host polls.
+// A copy and a stream synchronisation per convergence test cost 31 us of an idle GPU.
+struct alignas(64) StepMail {
+    double alpha, beta;
+    uint64_t tag;
+};
+constexpr int kMail = 64;
+
+// K3: beta[j+1] = sqrt(sum of K2's partials), invb[j+1]; one workgroup.  mail: null in a
+// replay.
+__global__ void __launch_bounds__(kThreads) k_lz3(Scal sc, int j, const double* __restrict__ part2, int npart2,
+                                                  StepMail* mail, uint64_t tag) {
     const double t = block_total(part2, npart2);
     if (threadIdx.x == 0) {
         const double b = sqrt(t);
         sc.beta[j + 1] = b;
         sc.invb[j + 1] = 1.0 / b;
+        if (mail) {
+            StepMail* e = mail + (j & (kMail - 1));
+            e->alpha = sc.alpha[j];
+            e->beta = b;
+            __hip_atomic_store(&e->tag, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     }
+}
+
+// beta[0] = 1/beta[0] = 1
+__global__ void k_lz_init(Scal sc) {
+    sc.beta[0] = 1.0;
+    sc.invb[0] = 1.0;
 }
 
 // *out = sum of part[0 .. cnt); one workgroup
@@ -1348,19 +1372,6 @@ void start_vector(int64_t n, uint32_t seed, std::vector<double2>& v) {
     for (int64_t i = 0; i < n; ++i) { v[i].x /= nrm; v[i].y /= nrm; }
 }
 
-// Number of eigenvalues of T below x (Sturm sequence of the LDL^T pivots).
-static int sturm_count(int m, const double* a, const double* b, double x) {
-    int c = 0;
-    double q = 1.0;
-    for (int i = 0; i < m; ++i) {
-        const double bb = i ? b[i - 1] * b[i - 1] : 0.0;
-        q = a[i] - x - (i ? bb / q : 0.0);
-        if (q == 0.0) q = -1e-300;
-        if (q < 0) ++c;
-    }
-    return c;
-}
-
 // Lowest eigenvalue by bisection, eigenvector by inverse iteration, with
 // caller work space: ws holds 8 m doubles, piv m ints (both used only when
 // vec is given).
@@ -1371,12 +1382,7 @@ double tridiag_lowest_ws(int m, const double* a, const double* b, double* vec, d
         lo = std::min(lo, a[i] - r);
         hi = std::max(hi, a[i] + r);
     }
-    for (int it = 0; it < 200; ++it) {
-        const double mid = 0.5 * (lo + hi);
-        if (mid <= lo || mid >= hi) break;
-        if (sturm_count(m, a, b, mid) >= 1) hi = mid; else lo = mid;
-    }
-    const double e = 0.5 * (lo + hi);
+    const double e = lowest_in(m, a, b, lo, hi);
     if (!vec) return e;
     // inverse iteration: (T - e I) x = y with partial pivoting (Gaussian elimination on the band)
     double* x = ws;
@@ -1444,36 +1450,22 @@ double tridiag_lowest_ws(int m, const double* a, const double* b, double* vec, d
 
 // The lowest eigenvalue of T_m when `prev`, that of T_{m-1}, and `step`, the
 // last change of the sequence, are known (the Ritz values of pass 1): by
-// interlacing the eigenvalue lies at or below prev, so the bisection starts
-// from [prev - w, prev + 1e-13 |prev|] with w = 4 step, widened 16-fold while
-// the lower end is not below the eigenvalue (checked by Sturm counts), down to
-// the Gershgorin bound.  About 25 bisection steps instead of 52 once the
-// sequence settles.  Falls back to the full bracket without a usable prev.
+// interlacing the eigenvalue lies at or below prev, so the search starts from
+// [prev - w, prev + 1e-13 |prev|], w the smallest of 4 step 16^k, k = 0..6, that
+// holds it (one pass of eight Sturm sequences).  Falls back to the full bracket
+// without a usable prev or if it is outside.
 double tridiag_lowest_next(int m, const double* a, const double* b, double prev, double step) {
     if (m < 3 || !std::isfinite(prev) || !std::isfinite(step))
         return tridiag_lowest_ws(m, a, b, nullptr, nullptr, nullptr);
-    double glo = a[0];
-    for (int i = 0; i < m; ++i) {
-        const double r = (i ? std::fabs(b[i - 1]) : 0.0) + (i + 1 < m ? std::fabs(b[i]) : 0.0);
-        glo = std::min(glo, a[i] - r);
-    }
     const double scale = std::max(1.0, std::fabs(prev));
-    const double hi0 = prev + 1e-13 * scale;
-    if (sturm_count(m, a, b, hi0) < 1) return tridiag_lowest_ws(m, a, b, nullptr, nullptr, nullptr);
-    double w = std::max(4.0 * step, 1e-12 * scale);
-    double lo = prev - w;
-    while (lo > glo && sturm_count(m, a, b, lo) >= 1) {
-        w *= 16.0;
-        lo = prev - w;
-    }
-    if (lo < glo) lo = glo;
-    double hi = hi0;
-    for (int it = 0; it < 200; ++it) {
-        const double mid = 0.5 * (lo + hi);
-        if (mid <= lo || mid >= hi) break;
-        if (sturm_count(m, a, b, mid) >= 1) hi = mid; else lo = mid;
-    }
-    return 0.5 * (lo + hi);
+    double x[8], w = std::max(4.0 * step, 1e-12 * scale);
+    x[0] = prev + 1e-13 * scale;
+    for (int k = 1; k < 8; ++k, w *= 16.0) x[k] = prev - w;
+    const unsigned r = sturm_any8(m, a, b, x);
+    int k = 0;
+    while (k < 8 && (r >> k & 1)) ++k;  // x falls: x[k] is the first with no eigenvalue below
+    if (k == 0 || k == 8) return tridiag_lowest_ws(m, a, b, nullptr, nullptr, nullptr);
+    return lowest_in(m, a, b, x[k], x[k - 1]);
 }
 
 double tridiag_lowest(int m, const double* a, const double* b, double* vec) {
@@ -1606,11 +1598,11 @@ struct DevWork {
 // K2 and K3 of one step after the K1 launched with grid `g1` wrote part1.
 void launch_lz23(int64_t n, const double2* u, const double2* W, double2* Wn, const Scal& sc, int j, int ns,
                  double2* psi, const double* coef, int ldc, const double* part1, int g1, double* part2,
-                 hipStream_t st) {
+                 hipStream_t st, StepMail* mail = nullptr, uint64_t tag = 0) {
     const int gv = vec_grid(n);
     hipLaunchKernelGGL(k_lz2, dim3(gv), dim3(kThreads), 0, st, n, u, W, Wn, sc, j, ns, psi, coef, ldc, part1, g1,
                        part2);
-    hipLaunchKernelGGL(k_lz3, dim3(1), dim3(kThreads), 0, st, sc, j, part2, gv);
+    hipLaunchKernelGGL(k_lz3, dim3(1), dim3(kThreads), 0, st, sc, j, part2, gv, mail, tag);
 }
 
 // *out = |x|^2 and *out = Re<x|y>: block partials, then one wavefront sums them
@@ -1624,9 +1616,77 @@ void reduce_redot(int64_t n, const double2* x, const double2* y, double* out, do
     hipLaunchKernelGGL(k_redot, dim3(gv), dim3(kThreads), 0, st, n, x, y, part);
     hipLaunchKernelGGL(k_psum, dim3(1), dim3(kThreads), 0, st, part, gv, out);
 }
+// Mailboxes (pinned, kMail entries): one per host thread, taken on its first solve and
+// handed back when it ends; never freed, since an abandoned solve's kernels may still
+// write there.  `solve` numbers the solves that used it, so a tag is never met twice.
+struct Mailbox {
+    StepMail* m = nullptr;
+    uint64_t solve = 0;
+};
+Mailbox* new_mailbox() {
+    auto* b = new Mailbox;
+    if (hipHostMalloc((void**)&b->m, kMail * sizeof(StepMail), hipHostMallocCoherent | hipHostMallocMapped) !=
+        hipSuccess) {
+        delete b;
+        throw Error(BLQH_ENOMEM, "pinned memory for the solver's mailbox");
+    }
+    for (int i = 0; i < kMail; ++i) b->m[i].tag = 0;
+    return b;
+}
+std::mutex g_mail_mu;
+std::vector<Mailbox*>* g_free_mail = new std::vector<Mailbox*>;  // never destroyed
+struct ThreadMailbox {
+    Mailbox* b = nullptr;
+    ~ThreadMailbox() {
+        if (!b) return;
+        std::lock_guard<std::mutex> lk(g_mail_mu);
+        g_free_mail->push_back(b);
+    }
+};
+thread_local ThreadMailbox t_mail;
+Mailbox* thread_mailbox() {
+    if (t_mail.b) return t_mail.b;
+    std::lock_guard<std::mutex> lk(g_mail_mu);
+    if (!g_free_mail->empty()) {
+        t_mail.b = g_free_mail->back();
+        g_free_mail->pop_back();
+    } else {
+        t_mail.b = new_mailbox();
+    }
+    return t_mail.b;
+}
+
+// Waits for the entry's tag; a stream that ends (or fails) without it is an error.
+void wait_mail(const StepMail* e, uint64_t tag, hipStream_t st) {
+    for (uint32_t spin = 1;; ++spin) {
+        if (__atomic_load_n(&e->tag, __ATOMIC_ACQUIRE) == tag) return;
+        if ((spin & 0x3fff) == 0) {
+            const hipError_t q = hipStreamQuery(st);
+            if (q == hipErrorNotReady) continue;
+            BLQH_HIP(q);
+            BLQH_REQUIRE(__atomic_load_n(&e->tag, __ATOMIC_ACQUIRE) == tag, BLQH_EINTERNAL,
+                         "Lanczos step ended without its coefficients");
+            return;
+        }
+        __builtin_ia32_pause();
+    }
+}
+
+// Steps queued ahead of the one that the host waits for, so that the GPU works through
+// the wait, the test and the launches (about 30 us a test).  The queued steps of a solve
+// that has converged are wasted, so they must cost less than the idle time of its
+// tests: about 60 steps, 60 / chk tests.  Step time: 12 us of launches, then 400,000
+// entries per us (measured: N_phi = 12 16 us, N_phi = 14 140 us, N_phi = 16 2.2 ms).
+int steps_ahead(int64_t nnz, int chk) {
+    const double t = 12.0 + (double)nnz / 4e5;
+    const int d = std::max(1, std::min(8, (int)std::ceil(30.0 / t)));
+    return d * t < 0.5 * (60.0 / chk) * 30.0 ? d : 0;
+}
+
 struct HostWork {
     double *ha, *hb, *ritz, *svec, *c, *aux, *aux2, *tri;
     int* piv;
+    Mailbox* mail;
 };
 
 // Passes 1-3 and the Rayleigh quotient of blqh_lanczos on given work areas.
@@ -1646,9 +1706,7 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
                  "partial-sum buffer smaller than the grid");
     const int g1 = lz1_grid(H, plan);  // K1's partials, summed by K2
     Scal sc{D.sc, D.sc + cap, D.sc + 2 * cap + 2};
-    const double one = 1.0;
-    BLQH_HIP(hipMemcpyAsync(sc.beta, &one, 8, hipMemcpyHostToDevice, st));
-    BLQH_HIP(hipMemcpyAsync(sc.invb, &one, 8, hipMemcpyHostToDevice, st));
+    hipLaunchKernelGGL(k_lz_init, dim3(1), dim3(1), 0, st, sc);
 
     auto slot = [&](int j) -> double2* { return D.Wb + (size_t)(store ? j : j % 3) * n; };
     if (H->ord.on) {  // start vector in the reference order, the recurrence in the internal one
@@ -1662,6 +1720,7 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
     Profile& prof = profile();
     const bool prof_on = timed && prof.on;
     int ntimed = 0;
+    const uint64_t tag0 = ++hw.mail->solve << 32;
     auto step = [&](int j, double2* psi_acc, const double* cf) {
         double2* W = slot(j);
         double2* Wp = j > 0 ? slot(j - 1) : slot(j);
@@ -1676,7 +1735,7 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
         launch_lz1(H, plan, W, Wp, D.u, sc, j, D.partials, st);
         if (prof_on) BLQH_HIP(hipEventRecord(prof.ev[2 * ntimed++ + 1], st));
         launch_lz23(n, D.u, W, slot(j + 1), sc, j, psi_acc ? 1 : 0, psi_acc, cf, cap, D.partials, g1, D.partials2,
-                    st);
+                    st, psi_acc ? nullptr : hw.mail->m, tag0 | (uint32_t)(j + 1));
     };
     auto account = [&]() {
         if (!prof_on) return;
@@ -1695,14 +1754,26 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
     int m = 0;  // Krylov vectors in use
     bool conv = false;
     double dE = INFINITY, resid = INFINITY;
-    int done = 0;
+    int done = 0, queued = 0;
+    const int ahead = steps_ahead(H->nnz, chk);
+    hb[0] = 1.0;
     while (done < cap && !conv) {
         const int upto = std::min(cap, done + chk);
-        for (int j = done; j < upto; ++j) step(j, nullptr, nullptr);
+        int got = done;  // coefficients read
+        auto read_to = [&](int e) {
+            for (; got < e; ++got) {
+                const StepMail* q = hw.mail->m + (got & (kMail - 1));
+                wait_mail(q, tag0 | (uint32_t)(got + 1), st);
+                ha[got] = q->alpha;
+                hb[got + 1] = q->beta;
+            }
+        };
+        for (; queued < std::min(cap, upto + ahead); ++queued) {
+            read_to(std::min(upto, queued - kMail + 1));  // the entry's last tenant has been read
+            step(queued, nullptr, nullptr);
+        }
         BLQH_HIP(hipGetLastError());
-        BLQH_HIP(hipMemcpyAsync(ha, sc.alpha, upto * 8, hipMemcpyDeviceToHost, st));
-        BLQH_HIP(hipMemcpyAsync(hb, sc.beta, (upto + 1) * 8, hipMemcpyDeviceToHost, st));
-        BLQH_HIP(hipStreamSynchronize(st));
+        read_to(upto);
         for (int j = done; j < upto; ++j) {
             // T_{j+1}: alpha[0..j], off-diagonal beta[1..j]
             hw.ritz[j] = j == 0 ? tridiag_lowest_ws(1, ha, hb + 1, nullptr, nullptr, nullptr)
@@ -1719,6 +1790,8 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
             if (o.tol > 0 && j > 0 && dE < o.tol) {
                 if (o.res_tol <= 0) { conv = true; break; }
                 // residual of the Ritz pair: |H y - theta y| = beta_{j+1} |s_j|
+                resid = INFINITY;
+                if (residual_exceeds(j + 1, ha, hb + 1, hw.ritz[j], hb[j + 1], o.res_tol)) continue;
                 (void)tridiag_lowest_ws(j + 1, ha, hb + 1, hw.svec, hw.tri, hw.piv);
                 resid = hb[j + 1] * std::fabs(hw.svec[j]);
                 if (resid < o.res_tol) { conv = true; break; }
@@ -1748,10 +1821,8 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
     }
     // pass 3
     if (store) {
-        double* invb = hw.aux;
-        copy_sync(invb, sc.invb, m * 8, hipMemcpyDeviceToHost);
         double* w = hw.aux2;
-        for (int l = 0; l < m; ++l) w[l] = c[l] * invb[l];
+        for (int l = 0; l < m; ++l) w[l] = c[l] * (1.0 / hb[l]);  // invb as K3 rounds it
         BLQH_HIP(hipMemcpyAsync(D.coef, w, m * 8, hipMemcpyHostToDevice, st));
         hipLaunchKernelGGL(k_combine, dim3(gv), dim3(kThreads), 0, st, n, m, D.Wb, n, D.coef, D.psi);
         res.passes = 2;
@@ -1824,7 +1895,8 @@ void blqh_lanczos_impl(blqh_hamil* H, const blqh_lanczos_opts& o, blqh_lanczos_r
     std::vector<int> piv(cap);
     double* hp = hbuf.data();
     const size_t L = (size_t)cap + 1;
-    const HostWork hw{hp, hp + L, hp + 2 * L, hp + 3 * L, hp + 4 * L, hp + 5 * L, hp + 6 * L, hp + 7 * L, piv.data()};
+    const HostWork hw{hp, hp + L, hp + 2 * L, hp + 3 * L, hp + 4 * L, hp + 5 * L, hp + 6 * L, hp + 7 * L, piv.data(),
+                      thread_mailbox()};
     const DevWork D{Wb.get(), u.get(), psi.get(), v0.get(), sc_buf.get(), coef.get(), red.get(), partials.get(),
                     partials.get() + gmax, gmax};
     lanczos_core(H, plan, o, store, D, hw,
@@ -1859,6 +1931,7 @@ static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
 namespace {
 std::mutex g_noalloc_mu;
+Mailbox* g_noalloc_mail = nullptr;  // used under g_noalloc_mu
 void* g_scratch_ptr[kMaxDevices] = {};
 // host work arrays of the allocation-free solve (used under g_noalloc_mu)
 double g_noalloc_host[7 * (kNoAllocMaxLambda + 1) + 8 * kNoAllocMaxLambda];
@@ -1908,6 +1981,7 @@ void noalloc_setup(int device) {
     BLQH_REQUIRE(p != nullptr, BLQH_EDEVICE, "no device address for the solver's static scratch array");
     std::lock_guard<std::mutex> lk(g_noalloc_mu);
     g_scratch_ptr[device] = p;
+    if (!g_noalloc_mail) g_noalloc_mail = new_mailbox();
 }
 }  // namespace blqh
 
@@ -1939,7 +2013,7 @@ void blqh_lanczos_noalloc_impl(blqh_hamil* H, const blqh_lanczos_opts& o, blqh_l
     double* hp = g_noalloc_host;
     const size_t L = (size_t)cap + 1;
     const HostWork hw{hp, hp + L, hp + 2 * L, hp + 3 * L, hp + 4 * L, hp + 5 * L, hp + 6 * L, hp + 7 * L,
-                      g_noalloc_piv};
+                      g_noalloc_piv, g_noalloc_mail};
     auto start = [&](double2* dst) {
         double s = 0;
         if (o.start) {

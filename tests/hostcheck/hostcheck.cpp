@@ -315,6 +315,20 @@ void hc_tridiag_vector_k(int m, const double* a, const double* b, int k, double*
     tridiag_vector_k(m, a, b, k, x);
 }
 
+// the solvers' convergence test (ritz.hpp)
+double hc_lowest_in(int m, const double* a, const double* b, double lo, double hi) { return lowest_in(m, a, b, lo, hi); }
+double hc_lowest_bisected(int m, const double* a, const double* b, double lo, double hi) {
+    for (int it = 0; it < 200; ++it) {
+        const double mid = 0.5 * (lo + hi);
+        if (mid <= lo || mid >= hi) break;
+        if (sturm_below(m, a, b, mid) >= 1) hi = mid; else lo = mid;
+    }
+    return 0.5 * (lo + hi);
+}
+int hc_residual_exceeds(int m, const double* a, const double* b, double theta, double beta_m, double res_tol) {
+    return residual_exceeds(m, a, b, theta, beta_m, res_tol);
+}
+
 void hc_excited_mix(int m, const double* a, const double* b, const double* c0, double* out) {
     excited_mix(m, a, b, c0, out);
 }

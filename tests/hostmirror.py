@@ -28,6 +28,10 @@ def lib():
         _L.hc_internal_order.argtypes = [C.POINTER(blqh_amd.Sector), C.c_void_p, C.c_int64, C.c_void_p]
         _L.hc_hash_order_check.restype = C.c_int
         _L.hc_hash_order_check.argtypes = [C.POINTER(blqh_amd.Sector), C.POINTER(C.c_int64)]
+        for f in (_L.hc_lowest_in, _L.hc_lowest_bisected):
+            f.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_double, C.c_double]
+            f.restype = C.c_double
+        _L.hc_residual_exceeds.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_double, C.c_double, C.c_double]
         _L.hc_tridiag_vector_k.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p]
         _L.hc_excited_mix.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
         _L.hc_hash_order_levels_check.restype = C.c_int
@@ -119,6 +123,15 @@ def hash_order_levels_check(sec):
     n = C.c_int64()
     ok = lib().hc_hash_order_levels_check(C.byref(sec), C.byref(n))
     return bool(ok), n.value
+
+
+def lowest_in(a, b, lo, hi):
+    """Lowest tridiagonal eigenvalue: (nine-way search of the solvers, bisection)."""
+    return tuple(f(a.size, a.ctypes.data, b.ctypes.data, lo, hi) for f in (lib().hc_lowest_in, lib().hc_lowest_bisected))
+
+
+def residual_exceeds(a, b, theta, beta_m, res_tol):
+    return bool(lib().hc_residual_exceeds(a.size, a.ctypes.data, b.ctypes.data, theta, beta_m, res_tol))
 
 
 def tridiag_vector_k(a, b, k):

@@ -247,3 +247,30 @@ def test_low_ritz_vectors_match_lapack(m, seed):
         c = np.abs(V[:, 1:3].T @ xm)
         assert np.allclose(c, 1 / np.sqrt(2), atol=1e-9), c
     assert np.all(hostmirror.excited_mix(a[:1], b[:0], c0[:1]) == 0)
+
+
+@pytest.mark.parametrize("m", [1, 2, 3, 17, 60, 200])
+def test_convergence_test_routines(m):
+    """The nine-way search ends on the bisection's bits; a Ritz pair is only said to be
+    above ten times the tolerance if LAPACK's eigenvector says so."""
+    from scipy.linalg import eigh_tridiagonal
+    rng = np.random.default_rng(m)
+    for rep in range(20):
+        a = rng.normal(size=m) * 10.0 ** rng.uniform(-1, 2)
+        b = np.abs(rng.normal(size=m)) + 0.1  # b[m-1] is the coupling to the next vector
+        if rep == 3 and m > 2:
+            b[m // 2] = 0.0  # two blocks
+        r = np.abs(a).max() + 2 * np.abs(b).max() + 1
+        e, ref = hostmirror.lowest_in(a, b, -r, r)
+        assert e == ref
+        w, V = eigh_tridiagonal(a, b[:-1])
+        res = b[-1] * abs(V[-1, 0])
+        for tol in (1e-3, 1e-7, 1e-10):
+            if hostmirror.residual_exceeds(a, b, e, b[-1], tol):
+                assert res > 9 * tol, (m, rep, tol)
+    # a uniform chain: residual 0.5 sqrt(2 / (m + 1)) sin(pi / (m + 1)), 8e-4 at m = 200
+    a, b = np.zeros(m), np.full(m, 0.5)
+    e, ref = hostmirror.lowest_in(a, b, -2.0, 2.0)
+    assert e == ref
+    assert hostmirror.residual_exceeds(a, b, e, 0.5, 1e-7)
+    assert not hostmirror.residual_exceeds(a, b, e, 0.5, 0.5)
