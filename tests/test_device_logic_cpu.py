@@ -269,8 +269,8 @@ def test_convergence_test_routines(m):
             if hostmirror.residual_exceeds(a, b, e, b[-1], tol):
                 assert res > 9 * tol, (m, rep, tol)
     # a uniform chain: residual 0.5 sqrt(2 / (m + 1)) sin(pi / (m + 1)), 8e-4 at m = 200
-    a, b = np.zeros(m), np.full(m, 0.5)
-    e, ref = hostmirror.lowest_in(a, b, -2.0, 2.0)
+    a, b = np.full(m, 2.0), np.full(m, 0.5)
+    e, ref = hostmirror.lowest_in(a, b, 0.0, 4.0)
     assert e == ref
     assert hostmirror.residual_exceeds(a, b, e, 0.5, 1e-7)
     assert not hostmirror.residual_exceeds(a, b, e, 0.5, 0.5)
