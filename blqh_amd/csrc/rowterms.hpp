@@ -23,6 +23,7 @@ struct RowCtx {
     int spinless;   // operand order of the reference's spinless / spinful expressions
     int twist_sel;  // 1: spinless interlayer pairs, 2: spinful (0,3)/(1,2) pairs
     int mono_odd;   // monolayer with odd nphi: the pair sign counts occupied orbitals (below)
+    int uniform;    // no twist and no theta_B phases: H commutes with the translations
     const int16_t* period;
     const int32_t* lut;
     const uint32_t* cnt;
@@ -30,6 +31,16 @@ struct RowCtx {
     const double2* FT;   // [2 nphi - 1]: FT[ql - qr + nphi - 1] = exp(2 pi i (ql - qr) K / order)
     const double2* tw;   // [2 nphi - 1] twist phase per t
 };
+
+// True if the translated images of a term between full orbits are equal (a pair hop's up
+// to image_count's signs): a translation
+// carries the term of ql on to that of ql + 1 with the same element (the Coulomb table is
+// symmetric under dm -> nphi - dm, and the signs and phases of a full turn cancel, each
+// electron crossing its block's end once).  Rows or targets of shorter period, whose
+// phases need not cancel, are summed image by image.
+BLQH_HD bool images_equal(const RowCtx& c, int Dl, int Dr) {
+    return c.uniform && c.K >= 0 && Dl == c.g.order() && Dr == Dl;
+}
 
 BLQH_HD double2 cmul(double2 a, double2 b) { return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
 
@@ -140,10 +151,11 @@ BLQH_HD bool pair_hop(int nphi, uint64_t L, int n, int m, int t, PairHop& h) {
 }
 
 // Two-body element of the open pair hop h of L (pair n < m, shift t) whose
-// target lies in the orbit of row j (sector-table shift q1, period Dr).
+// target lies in the orbit of row j (sector-table shift q1, period Dr).  fold (t >= 0, no
+// twist): with that of shift t - nphi, which has the same target.
 // BLQH_without_spin/lanczos_hamiltonian.cpp:109-292, BLQH_with_spin/lanczos_hamiltonian.cpp:109-712.
 BLQH_HD void pair_value(const RowCtx& c, uint64_t L, int signl, int Dl, int ql, int n, int m, int t, const PairHop& h,
-                        int q1, int Dr, double& re, double& im) {
+                        int q1, int Dr, double& re, double& im, bool fold = false) {
     const int nphi = c.g.nphi;
     const int a = h.a, b = h.b, n0 = h.n0, xm = h.xm, nt = h.nt, mt = h.mt;
     int qr = 0, sr = 1;
@@ -161,7 +173,8 @@ BLQH_HD void pair_value(const RowCtx& c, uint64_t L, int signl, int Dl, int ql, 
     int dm = xm - n0;
     dm = dm < 0 ? -dm : dm;
     const int at = t < 0 ? -t : t;
-    const double Cv = c.C[alpha * nphi * nphi + dm * nphi + at];
+    const double* Cm = c.C + alpha * nphi * nphi + dm * nphi;
+    const double Cv = fold && t ? Cm[at] + Cm[nphi - at] : Cm[at];
     double2 ft = c.FT[ql - qr + nphi - 1];
     const bool twisted = c.twist_sel == 1 ? (a != b) : (c.twist_sel == 2 && ((a == 0 && b == 3) || (a == 1 && b == 2)));
     if (twisted) ft = cmul(ft, c.tw[t + nphi - 1]);
@@ -199,6 +212,24 @@ BLQH_HD int rot_in_block(int nphi, int x, int k) {
     return a * nphi + y;
 }
 
+// Sum of the signs of the Dl = nphi / step equal images of an open pair hop, the first one's
+// taken as +1.  In the bilayers the reference's pair sign counts empty orbitals (sign2), which
+// for odd nphi turns with each image in which exactly one of the two electrons wraps around
+// its block: n in the t rotations that bring it to the block's last t orbitals, m
+// in those that bring it to the first t.  (t - nphi: both complements, the same images.)
+BLQH_HD int image_count(const RowCtx& c, int Dl, int n, int m, int t, const PairHop& h) {
+    const int nphi = c.g.nphi;
+    if (c.g.S == 1 || !(nphi & 1)) return Dl;
+    const int tt = t < 0 ? t + nphi : t;
+    const uint32_t full = (uint32_t)lowbits(nphi), first = (uint32_t)lowbits(tt), last = first << (nphi - tt);
+    const int m0 = m - h.b * nphi;
+    // bit k: rotation by k (the orbital x moves to (x + k) mod nphi)
+    const uint32_t wn = ((last >> h.n0) | (last << (nphi - h.n0))) & full;
+    const uint32_t wm = ((first >> m0) | (first << (nphi - m0))) & full;
+    const int one = popc((uint64_t)(wn ^ wm));
+    return h.wn != h.wm ? 2 * one - Dl : Dl - 2 * one;
+}
+
 // The pair hop (n0 < m0 of the row word L0 = Ls[0], shift t) and its images
 // in the translated words Ls[ql] = translate(L0, ql) (signs sgl[ql]), ql < Dl.
 // A translation maps the open hops of L0 one to one onto those of Ls[ql] (the
@@ -209,43 +240,51 @@ BLQH_HD int rot_in_block(int nphi, int x, int k) {
 // image's term in Ls[ql]; false when the hop is blocked or its target has no
 // representative.
 BLQH_HD bool pair_orbit_sum(const RowCtx& c, const uint64_t* Ls, const int* sgl, int Dl, int n0, int m0, int t, int& j,
-                            double& re, double& im) {
+                            double& re, double& im, bool fold = false) {
     const int nphi = c.g.nphi;
     PairHop h;
     if (!pair_hop(nphi, Ls[0], n0, m0, t, h)) return false;
     int q1, Dr;
     if (!locate_word(c, h.word, j, q1, Dr)) return false;
+    if (images_equal(c, Dl, Dr)) {
+        pair_value(c, Ls[0], sgl[0], Dl, 0, n0, m0, t, h, q1, Dr, re, im, fold);
+        const double cnt = image_count(c, Dl, n0, m0, t, h);
+        re *= cnt;
+        im *= cnt;
+        return true;
+    }
     re = 0.0;
     im = 0.0;
-    for (int ql = 0; ql < Dl; ++ql) {
-        const int k = ql * c.g.step;
-        int n = rot_in_block(nphi, n0, k), m = rot_in_block(nphi, m0, k), tq = t;
-        if (n > m) {
-            const int x = n;
-            n = m;
-            m = x;
-            tq = -t;
+    for (int f = 0; f < (fold && t ? 2 : 1); ++f)
+        for (int ql = 0; ql < Dl; ++ql) {
+            const int k = ql * c.g.step;
+            int n = rot_in_block(nphi, n0, k), m = rot_in_block(nphi, m0, k), tq = t - f * nphi;
+            if (n > m) {
+                const int x = n;
+                n = m;
+                m = x;
+                tq = -tq;
+            }
+            (void)pair_hop(nphi, Ls[ql], n, m, tq, h);  // open: the image of an open hop
+            double r, i;
+            pair_value(c, Ls[ql], sgl[ql], Dl, ql, n, m, tq, h, q1, Dr, r, i);
+            re += r;
+            im += i;
         }
-        if (ql) (void)pair_hop(nphi, Ls[ql], n, m, tq, h);  // open: the image of an open hop
-        double r, i;
-        pair_value(c, Ls[ql], sgl[ql], Dl, ql, n, m, tq, h, q1, Dr, r, i);
-        re += r;
-        im += i;
-    }
     return true;
 }
 
 // One-body tunnelling term.  BLQH_without_spin/lanczos_hamiltonian.cpp:295-322,
 // BLQH_with_spin/lanczos_hamiltonian.cpp:718-898.
-BLQH_HD bool hop_term(const RowCtx& c, uint64_t L, int signl, int Dl, int ql, const HopTerm& h, int& j, double& re,
-                      double& im) {
+BLQH_HD bool hop_term(const RowCtx& c, uint64_t L, int signl, int Dl, int ql, const HopTerm& h, int& j, int& Dr,
+                      double& re, double& im) {
     const uint64_t mask = (1ULL << h.n) | (1ULL << h.nt);
     const uint64_t kn = L & mask;
     if (kn == 0 || kn == mask) return false;
     const uint64_t R0 = L ^ mask;
     if (c.spec.maskA && popc(R0 & c.spec.maskA) != c.spec.nA) return false;
     if (c.spec.maskB && popc(R0 & c.spec.maskB) != c.spec.nB) return false;
-    int qr, Dr, sr;
+    int qr, sr;
     if (!locate(c, R0, ql, j, qr, Dr, sr)) return false;
     const int sign = sign1(L, h.lo, h.hi) * signl * sr;
     const int nphi = c.g.nphi;
@@ -256,6 +295,35 @@ BLQH_HD bool hop_term(const RowCtx& c, uint64_t L, int signl, int Dl, int ql, co
     const double sq = sqrt((double)(Dl * Dr));
     re = v.x / sq;
     im = v.y / sq;
+    return true;
+}
+
+// The hop h of the row word L0 and its images in translate(L0, ql), ql < Dl (the hops of the
+// rotated orbitals), summed; their targets lie in one orbit, row j.  For hop lists that
+// the translations map onto themselves (c.uniform): summed over the list it is the sum of
+// hop_term over list and ql.
+BLQH_HD bool hop_orbit_sum(const RowCtx& c, uint64_t L0, int Dl, const HopTerm& h, int& j, double& re, double& im) {
+    int Dr;
+    if (!hop_term(c, L0, 1, Dl, 0, h, j, Dr, re, im)) return false;
+    if (images_equal(c, Dl, Dr)) {
+        re *= Dl;
+        im *= Dl;
+        return true;
+    }
+    for (int ql = 1; ql < Dl; ++ql) {
+        const int k = ql * c.g.step;
+        HopTerm x = h;
+        x.n = rot_in_block(c.g.nphi, h.n, k);
+        x.nt = rot_in_block(c.g.nphi, h.nt, k);
+        x.lo = x.n < x.nt ? x.n : x.nt;
+        x.hi = x.n < x.nt ? x.nt : x.n;
+        int s, jq;
+        const uint64_t L = translate(c.g, L0, ql, s);
+        double r, i;
+        if (!hop_term(c, L, s, Dl, ql, x, jq, Dr, r, i)) continue;  // unreachable: the image of an open hop
+        re += r;
+        im += i;
+    }
     return true;
 }
 

@@ -9,6 +9,7 @@
 // GPU tests.
 #include <algorithm>
 #include <cstring>
+#include <array>
 #include <map>
 #include <vector>
 
@@ -173,7 +174,7 @@ int hc_sign1(uint64_t c, int n, int nt) { return sign1(c, n, nt); }
 // Full Hamiltonian through the mirror.  Returns nnz (or -nnz when cap is too
 // small).  ql_major = 0: the build kernel's order (each open pair hop of the
 // row word with its translated images summed by pair_orbit_sum, then the
-// tunnelling hops per translation, then the diagonal); 1: the reference's
+// tunnelling hops with theirs (per translation with a twist), then the diagonal); 1: the reference's
 // loop order (translation, then pair and shift, through pair_term), which
 // checks that regrouping.
 static int64_t hamil_mirror(const blqh_sector* s, const blqh_params* p, int64_t* rowptr, int64_t* col, double* val,
@@ -193,6 +194,7 @@ static int64_t hamil_mirror(const blqh_sector* s, const blqh_params* p, int64_t*
     c.C = T.C.data();
     c.FT = T.FT.data();
     c.tw = T.tw.data();
+    c.uniform = p->theta_x == 0 && p->theta_y == 0 && p->theta_b == 0;
     const int nphi = s->nphi, nel = s->nel, Tn = 2 * nphi - 1;
     const int npairs = nel * (nel - 1) / 2;
     const int64_t n = (int64_t)B.id.size();
@@ -226,26 +228,30 @@ static int64_t hamil_mirror(const blqh_sector* s, const blqh_params* p, int64_t*
                     if (pair_term(c, Ls[ql], sgl[ql], Dl, ql, occ[pw & 0xff], occ[pw >> 8], t, j, re, im)) add(j, re, im);
                 }
                 for (const HopTerm& h : T.hops) {
-                    int j;
+                    int j, Dr;
                     double re, im;
-                    if (hop_term(c, Ls[ql], sgl[ql], Dl, ql, h, j, re, im)) add(j, re, im);
+                    if (hop_term(c, Ls[ql], sgl[ql], Dl, ql, h, j, Dr, re, im)) add(j, re, im);
                 }
             }
         } else {
             int occ[64];
             occ_of(L0, occ);
-            for (int cnd = 0; cnd < npairs * Tn; ++cnd) {
-                const int pr = cnd / Tn, t = cnd - pr * Tn - (nphi - 1);
+            const bool fold = c.uniform != 0;  // t and t - nphi as one candidate
+            const int Tc = fold ? nphi : Tn, tmin = fold ? 0 : 1 - nphi;
+            for (int cnd = 0; cnd < npairs * Tc; ++cnd) {
+                const int pr = cnd / Tc, t = cnd - pr * Tc + tmin;
                 const unsigned short pw = pair_decode(nel, pr);
                 int j;
                 double re, im;
-                if (pair_orbit_sum(c, Ls, sgl, Dl, occ[pw & 0xff], occ[pw >> 8], t, j, re, im)) add(j, re, im);
+                if (pair_orbit_sum(c, Ls, sgl, Dl, occ[pw & 0xff], occ[pw >> 8], t, j, re, im, fold)) add(j, re, im);
             }
-            for (int ql = 0; ql < Dl; ++ql)
+            for (int ql = 0; ql < (fold ? 1 : Dl); ++ql)
                 for (const HopTerm& h : T.hops) {
-                    int j;
+                    int j, Dr;
                     double re, im;
-                    if (hop_term(c, Ls[ql], sgl[ql], Dl, ql, h, j, re, im)) add(j, re, im);
+                    if (fold ? hop_orbit_sum(c, L0, Dl, h, j, re, im)
+                             : hop_term(c, Ls[ql], sgl[ql], Dl, ql, h, j, Dr, re, im))
+                        add(j, re, im);
                 }
         }
         acc[(int)i].first += diag_term(c.g, c.spinless != 0, L0, T.Ec * nel, p->d, p->delta_v, p->delta_z);
@@ -308,6 +314,56 @@ int hc_hash_order_levels_check(const blqh_sector* s, int64_t* n) {
 // with a given reciprocal r of d.
 void hc_mod_by_rcp(int n, int d, float r, int32_t* out) {
     for (int s = 0; s < n; ++s) out[s] = mod_by_rcp(s, d, r);
+}
+
+// Largest difference, over the elements of the layer-exchanging hops n <-> n + nphi (n <
+// nphi, coefficient 1/2), between the sum over translations and hops (hop_term) and the sum
+// over hops with their images (hop_orbit_sum); relative to the largest element.
+double hc_hop_images(const blqh_sector* s) {
+    HostBasis B;
+    build(*s, B);
+    blqh_params p{};
+    p.lx = p.ly = std::sqrt(2.0 * M_PI * s->nphi);
+    HostTables T = host_tables(*s, p);
+    RowCtx c{};
+    c.g = B.g;
+    c.spec = B.spec;
+    c.M = B.M;
+    c.K = s->K;
+    set_row_species(c, *s);
+    c.period = B.period.data();
+    c.lut = B.lut.data();
+    c.cnt = B.cnt.data();
+    c.FT = T.FT.data();
+    c.uniform = 1;
+    double diff = 0, top = 0;
+    for (int64_t i = 0; i < (int64_t)B.id.size(); ++i) {
+        std::map<int, std::array<double, 4>> acc;
+        const int Dl = c.K < 0 ? 1 : B.period[i];
+        const int f = s->nphi, d = s->nspecies == 4 ? 2 * f : f;
+        for (int n = 0; n < f; ++n) {
+            const HopTerm h{n, n + d, n, n + d, 0.5, 1.0, 0.0, 0};
+            int j, Dr;
+            double re, im;
+            if (hop_orbit_sum(c, B.id[i], Dl, h, j, re, im)) {
+                acc[j][0] += re;
+                acc[j][1] += im;
+            }
+            for (int ql = 0; ql < Dl; ++ql) {
+                int sg;
+                const uint64_t L = translate(c.g, B.id[i], ql, sg);
+                if (hop_term(c, L, sg, Dl, ql, h, j, Dr, re, im)) {
+                    acc[j][2] += re;
+                    acc[j][3] += im;
+                }
+            }
+        }
+        for (const auto& e : acc) {
+            diff = std::max(diff, std::hypot(e.second[0] - e.second[2], e.second[1] - e.second[3]));
+            top = std::max(top, std::hypot(e.second[2], e.second[3]));
+        }
+    }
+    return top > 0 ? diff / top : -1.0;
 }
 
 // the batched solver's low Ritz vectors (ritz.hpp)

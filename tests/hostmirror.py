@@ -31,6 +31,8 @@ def lib():
         for f in (_L.hc_lowest_in, _L.hc_lowest_bisected):
             f.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_double, C.c_double]
             f.restype = C.c_double
+        _L.hc_hop_images.argtypes = [C.POINTER(blqh_amd.Sector)]
+        _L.hc_hop_images.restype = C.c_double
         _L.hc_residual_exceeds.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_double, C.c_double, C.c_double]
         _L.hc_tridiag_vector_k.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p]
         _L.hc_excited_mix.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
@@ -123,6 +125,11 @@ def hash_order_levels_check(sec):
     n = C.c_int64()
     ok = lib().hc_hash_order_levels_check(C.byref(sec), C.byref(n))
     return bool(ok), n.value
+
+
+def hop_images(sec):
+    """Largest relative difference of the two ways to sum a hop list over the translations."""
+    return lib().hc_hop_images(C.byref(sec))
 
 
 def lowest_in(a, b, lo, hi):

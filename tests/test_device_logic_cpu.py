@@ -274,3 +274,28 @@ def test_convergence_test_routines(m):
     assert e == ref
     assert hostmirror.residual_exceeds(a, b, e, 0.5, 1e-7)
     assert not hostmirror.residual_exceeds(a, b, e, 0.5, 0.5)
+
+
+# no twist: the images of a hop are equal, up to the signs of odd N_phi
+UNIFORM = [(2, 7, 7, -1, -1, 2, 3), (2, 9, 6, -1, -1, 2, 1), (2, 9, 9, 4, -1, 0, 3), (2, 8, 6, -1, -1, 4, 2),
+           (2, 8, 8, -1, -1, 0, 4), (2, 8, 4, 2, -1, 2, 1), (2, 6, 6, -1, -1, 3, -1), (2, 5, 4, -1, -1, 1, 2),
+           (4, 5, 4, -1, -1, 2, 1), (4, 6, 6, 3, -1, 3, 2), (4, 4, 4, -1, -1, 0, 2), (4, 7, 3, -1, -1, 1, 0),
+           (1, 9, 3, -1, -1, 3, 1), (1, 15, 5, -1, -1, 5, 2), (1, 12, 6, -1, -1, 6, 4), (1, 10, 4, -1, -1, 2, 1)]
+
+
+@pytest.mark.parametrize("case", UNIFORM, ids=lambda c: "_".join(map(str, c)))
+def test_equal_images_against_reference_loop_order(case):
+    """Without a twist one element stands for all images of a term between full orbits, and
+    the shifts t and t - nphi are taken together; rows and targets of shorter period (even
+    N_phi at these J) are summed image by image.  Against the reference's loop order."""
+    sec = blqh_amd.Sector(*case)
+    par = blqh_amd.params(case[1], **({} if case[0] == 1 else dict(d=0.7, delta_sas=0.1, delta_v=0.05)))
+    ids, per = hostmirror.basis(sec)
+    cap = 600 * len(ids) + 64
+    rp, col, val = hostmirror.hamil(sec, par, len(ids), cap)
+    rp2, col2, val2 = hostmirror.hamil_ql_major(sec, par, len(ids), cap)
+    np.testing.assert_array_equal(rp, rp2)
+    np.testing.assert_array_equal(col, col2)
+    np.testing.assert_allclose(val, val2, rtol=0, atol=1e-13 * np.abs(val2).max())
+    if case[0] > 1 and case[3] < 0:
+        assert 0 <= hostmirror.hop_images(sec) < 1e-13
