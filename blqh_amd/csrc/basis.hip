@@ -153,8 +153,6 @@ __global__ void k_block_scan(const int32_t* __restrict__ in, int64_t n, const in
     if (i < n) out[i] = offs[blockIdx.x] + sh[threadIdx.x] - v;
 }
 
-__global__ void k_copy_total(const int64_t* __restrict__ tot, int64_t* __restrict__ dst) { *dst = *tot; }
-
 // ---- basis kernels -----------------------------------------------------------
 
 // flags[r] = 1 when word r is the orbit member latest in the hash order (or
@@ -461,15 +459,17 @@ std::vector<std::pair<int64_t, uint64_t>> hash_levels(int64_t n) {
     return lv;
 }
 
-void exclusive_scan(const int32_t* in, int64_t* out, int64_t n, hipStream_t st) {
-    const int64_t nb = std::max<int64_t>(1, ceil_div(n, kScanBlock));
-    DevBuf<int64_t> sums(nb + 1);
-    hipLaunchKernelGGL(k_block_sums, dim3((unsigned)nb), dim3(kScanBlock), 0, st, in, n, sums.get());
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanBlock), 0, st, sums.get(), nb, sums.get() + nb);
-    hipLaunchKernelGGL(k_block_scan, dim3((unsigned)nb), dim3(kScanBlock), 0, st, in, n, sums.get(), out);
-    hipLaunchKernelGGL(k_copy_total, dim3(1), dim3(1), 0, st, sums.get() + nb, out + n);
+int64_t scan_scratch(int64_t n) { return std::max<int64_t>(1, ceil_div(n, kScanBlock)) + 1; }
+
+void exclusive_scan(const int32_t* in, int64_t* out, int64_t n, hipStream_t st, int64_t* scratch) {
+    const int64_t nb = scan_scratch(n) - 1;
+    DevBuf<int64_t> own(scratch ? 0 : nb + 1);
+    int64_t* sums = scratch ? scratch : own.get();
+    hipLaunchKernelGGL(k_block_sums, dim3((unsigned)nb), dim3(kScanBlock), 0, st, in, n, sums);
+    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanBlock), 0, st, sums, nb, out + n);
+    hipLaunchKernelGGL(k_block_scan, dim3((unsigned)nb), dim3(kScanBlock), 0, st, in, n, sums, out);
     BLQH_HIP(hipGetLastError());
-    BLQH_HIP(hipStreamSynchronize(st));  // sums is freed on return
+    if (!scratch) BLQH_HIP(hipStreamSynchronize(st));  // own is freed on return
 }
 
 // posOf[rank(w)] = position of sector word w in the map's iteration order
@@ -491,7 +491,7 @@ void map_positions(const blqh_sector& s, const RankSpec& smap, const uint32_t* c
     DevBuf<uint64_t> key(M);
     DevBuf<uint32_t> tau(M), tau2(M), bucket(M), members(M), gmin(mmax);
     DevBuf<int32_t> gcount(mmax), first_sz(M);
-    DevBuf<int64_t> goff(mmax + 1), later(M + 1);
+    DevBuf<int64_t> goff(mmax + 1), later(M + 1), sums(scan_scratch(std::max<int64_t>((int64_t)mmax, M)));
     hipLaunchKernelGGL(k_dfs_keys, dim3(grid_for(M)), dim3(kBlock), 0, st, M, srev, dtrev.get(), smap.nbits,
                        key.get());
     hipLaunchKernelGGL(k_fill_i32, dim3(grid_for((int64_t)mmax)), dim3(kBlock), 0, st, gcount.get(), (int64_t)mmax, 0);
@@ -507,11 +507,11 @@ void map_positions(const blqh_sector& s, const RankSpec& smap, const uint32_t* c
         hipLaunchKernelGGL(k_hl_bucket, dim3(grid_for(en)), dim3(kBlock), 0, st, st_r, en, m, key.get(), cur,
                            bucket.get(), gcount.get(), gmin.get());
         BLQH_HIP(hipGetLastError());
-        exclusive_scan(gcount.get(), goff.get(), (int64_t)m, st);
+        exclusive_scan(gcount.get(), goff.get(), (int64_t)m, st, sums.get());
         hipLaunchKernelGGL(k_hl_members, dim3(grid_for(en)), dim3(kBlock), 0, st, en, cur, bucket.get(), goff.get(),
                            gcount.get(), gmin.get(), members.get(), first_sz.get());
         BLQH_HIP(hipGetLastError());
-        exclusive_scan(first_sz.get(), later.get(), en, st);
+        exclusive_scan(first_sz.get(), later.get(), en, st, sums.get());
         hipLaunchKernelGGL(k_hl_pos, dim3(grid_for(en)), dim3(kBlock), 0, st, en, cur, bucket.get(), goff.get(),
                            gmin.get(), members.get(), later.get(), nxt);
         BLQH_HIP(hipGetLastError());

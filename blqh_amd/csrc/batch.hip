@@ -1341,8 +1341,9 @@ blqh_hamil* make_template(const blqh_hamil* base, const blqh_hamil* tun) {
         const int64_t n = H->n;
         const uint64_t upper = lowbits(B->geo.S * B->geo.nphi / 2);
         std::vector<uint8_t> nu(n);
+        const int32_t* ip = H->ord.on ? host_iperm(H).data() : nullptr;
         for (int64_t r = 0; r < n; ++r) {
-            const int64_t i = H->ord.on ? H->ord.h_iperm[r] : r;
+            const int64_t i = ip ? ip[r] : r;
             nu[r] = (uint8_t)popc(B->h_id[i] & upper);
         }
         DevBuf<uint8_t> dnu(n);
@@ -1645,7 +1646,10 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
             }
         };
         int ncaller = 0;
-        for (int p = 0; p < P; ++p) ncaller += seeded[p] ? 0 : 1;
+        for (int p = 0; p < P; ++p) {
+            ncaller += seeded[p] ? 0 : 1;
+            if (!seeded[p] && b->hs[p]->ord.on) (void)host_iperm(b->hs[p]);  // for the threads below
+        }
         if (ncaller > 0) {
             const int nt = std::max(1, std::min<int>(ncaller, (int)std::min(16u, std::max(1u, std::thread::hardware_concurrency()))));
             std::vector<std::thread> th;

@@ -32,6 +32,10 @@ struct blqh_basis {
     mutable std::mutex ord_mu;
     mutable bool ord_done = false;
     mutable std::vector<int32_t> h_order;  // h_order[i] = internal position of row i (empty: identity)
+    // the same on the device (device_order): d_perm[i] = internal position of row i, d_iperm its inverse
+    mutable std::mutex dord_mu;
+    mutable bool dord_done = false;
+    mutable blqh::DevBuf<int32_t> d_perm, d_iperm;
 };
 
 struct blqh_hamil {
@@ -48,7 +52,7 @@ struct blqh_hamil {
         bool on = false;
         blqh::DevBuf<int32_t> perm;      // perm[i]: internal position of reference row i
         blqh::DevBuf<int32_t> iperm;     // iperm[r]: reference row at internal position r
-        std::vector<int32_t> h_iperm;
+        mutable std::vector<int32_t> h_iperm;  // on the host, once something asked (host_iperm)
         bool csr = false;                // the three arrays below exist (ensure_panels)
         blqh::DevBuf<int64_t> rowptr;    // the CSR in internal order, columns ascending
         blqh::DevBuf<int32_t> col;
@@ -92,7 +96,10 @@ inline void set_row_species(RowCtx& c, const blqh_sector& s) {
 
 RankSpec make_rank_spec(const blqh_sector& s, bool with_spin_constraint);
 std::vector<uint32_t> make_rank_table(const RankSpec& spec, int64_t* total);
-void exclusive_scan(const int32_t* in, int64_t* out, int64_t n, hipStream_t st);  // out has n+1 entries
+// out has n+1 entries.  scratch: scan_scratch(n) entries in use on st until the scan is
+// done; null: taken here, and the call waits for the stream.
+void exclusive_scan(const int32_t* in, int64_t* out, int64_t n, hipStream_t st, int64_t* scratch = nullptr);
+int64_t scan_scratch(int64_t n);
 std::vector<uint64_t> hash_iteration_order(const blqh_sector& s);
 std::vector<uint64_t> hash_iteration_order_map(const blqh_sector& s);  // from a real std::unordered_map
 // rehash schedule of the map over n inserts: (first insert after the rehash, buckets)
@@ -163,6 +170,8 @@ inline CsrView spmv_csr(const blqh_hamil* H) {
 // moves of vectors between the reference order and the internal one.
 const std::vector<int32_t>& internal_order(const blqh_basis* B);
 void build_order(blqh_hamil* H);
+bool device_order(const blqh_basis* B);
+const std::vector<int32_t>& host_iperm(const blqh_hamil* H);
 void order_to_internal(const blqh_hamil* H, const double2* src, double2* dst, hipStream_t st);
 void order_to_reference(const blqh_hamil* H, const double2* src, double2* dst, hipStream_t st);
 

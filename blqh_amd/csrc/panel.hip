@@ -715,6 +715,9 @@ size_t panel_layout_scratch_bytes(const blqh_hamil* H) {
 // the distinct x cache lines a step gathers from.  The Lanczos recurrence is
 // invariant under a permutation of the basis, so only the start vector and
 // the returned states move between the orders.
+//
+// This is the sequential form, for keys of more than 64 bits and the CPU tests;
+// device_order (order.hip) computes the same order.
 const std::vector<int32_t>& internal_order(const blqh_basis* B) {
     std::lock_guard<std::mutex> lk(B->ord_mu);
     if (B->ord_done) return B->h_order;
@@ -822,24 +825,6 @@ __global__ void k_ord_scatter(int64_t n, const int32_t* __restrict__ iperm, cons
 
 int ord_grid(int64_t n) { return (int)std::min<int64_t>(std::max<int64_t>(ceil_div(n, kBlk), 1), 65536); }
 }  // namespace
-
-// Row order of H's SpMV formats from the basis order (no-op for the identity order).
-void build_order(blqh_hamil* H) {
-    blqh_hamil::Order& O = H->ord;
-    if (O.on) return;
-    const std::vector<int32_t>& perm = internal_order(H->basis);
-    if (perm.empty()) return;
-    const int64_t n = H->n;
-    BLQH_REQUIRE((int64_t)perm.size() == n, BLQH_EINTERNAL, "internal order and Hamiltonian sizes differ");
-    hipStream_t st = stream();
-    O.h_iperm.assign(n, 0);
-    for (int64_t i = 0; i < n; ++i) O.h_iperm[perm[i]] = (int32_t)i;
-    O.perm.alloc(n);
-    O.iperm.alloc(n);
-    BLQH_HIP(hipMemcpyAsync(O.perm.get(), perm.data(), n * 4, hipMemcpyHostToDevice, st));
-    BLQH_HIP(hipMemcpyAsync(O.iperm.get(), O.h_iperm.data(), n * 4, hipMemcpyHostToDevice, st));
-    O.on = true;
-}
 
 namespace {
 // The CSR of H with rows and columns in the internal order.

@@ -293,6 +293,20 @@ void hc_internal_order(const blqh_sector* s, const uint64_t* ids, int64_t n, int
     for (int64_t i = 0; i < n; ++i) out[i] = o.empty() ? -1 : o[i];
 }
 
+// The order computed on the device for a basis handle against the sequential one: rows that
+// differ (GPU); -1: identity on both sides.
+int64_t hc_device_order_diff(const blqh_basis* B) {
+    const std::vector<int32_t>& o = internal_order(B);
+    if (!device_order(B)) return o.empty() ? -1 : (int64_t)o.size();
+    if ((int64_t)o.size() != B->n) return B->n;
+    std::vector<int32_t> p(B->n), ip(B->n);
+    copy_sync(p.data(), B->d_perm.get(), B->n * 4, hipMemcpyDeviceToHost);
+    copy_sync(ip.data(), B->d_iperm.get(), B->n * 4, hipMemcpyDeviceToHost);
+    int64_t bad = 0;
+    for (int64_t i = 0; i < B->n; ++i) bad += p[i] != o[i] || ip[o[i]] != i;
+    return bad;
+}
+
 // 1 when the replayed hash-map iteration order (basis.hip) equals the order
 // of a real std::unordered_map filled the same way; *n = words.
 int hc_hash_order_check(const blqh_sector* s, int64_t* n) {

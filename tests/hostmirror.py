@@ -31,6 +31,8 @@ def lib():
         for f in (_L.hc_lowest_in, _L.hc_lowest_bisected):
             f.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_double, C.c_double]
             f.restype = C.c_double
+        _L.hc_device_order_diff.argtypes = [C.c_void_p]
+        _L.hc_device_order_diff.restype = C.c_int64
         _L.hc_hop_images.argtypes = [C.POINTER(blqh_amd.Sector)]
         _L.hc_hop_images.restype = C.c_double
         _L.hc_residual_exceeds.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_double, C.c_double, C.c_double]
@@ -103,6 +105,11 @@ def mod_by_rcp(n, d, r):
     out = np.empty(n, np.int32)
     lib().hc_mod_by_rcp(n, d, float(np.float32(r)), _p(out))
     return out
+
+
+def device_order_diff(basis):
+    """Rows of a GPU basis whose internal order differs between device and host (-1: no order)."""
+    return lib().hc_device_order_diff(basis.h)
 
 
 def internal_order(sec, ids):

@@ -59,3 +59,18 @@ def test_internal_order_changes_nothing(case, kw):
     c = Ho.lanczos(lam=300, seed=5, store_basis=0)
     assert c["passes"] == 3 and c["E0"] == a["E0"]
     assert abs(np.vdot(a["psi"], c["psi"])) >= 1 - 1e-12
+
+
+@pytest.mark.parametrize("case", [(2, 4, 4, 2, -1, 0, 0), (2, 6, 6, -1, -1, 3, 3), (2, 8, 8, -1, -1, 0, 4),
+                                  (2, 9, 6, -1, -1, 2, 1), (2, 12, 12, -1, -1, 0, 6), (2, 14, 14, 7, -1, 7, 7),
+                                  (4, 6, 6, 3, 3, 0, 1), (4, 8, 8, 4, 4, 4, 0), (4, 16, 3, -1, -1, 3, 1),
+                                  (4, 14, 4, 2, -1, 1, 2), (2, 8, 8, -1, -1, 0, -1), (1, 12, 4, -1, -1, 0, 2)],
+                         ids=lambda c: "_".join(map(str, c)))
+def test_device_order_equals_sequential_order(case):
+    """The radix-sorted row order against the comparison sort: one tile and several, orbits of
+    short period, keys of 13 to 61 bits, keys too long for the device, sectors without an order."""
+    from tests import hostmirror
+    S, nphi, nel, nu, nsu, J, K = case
+    B = blqh_amd.Basis(nphi, nel, nu, J, K, nspecies=S, nel_su=nsu)
+    print(f"order {case} n {len(B)}", flush=True)
+    assert hostmirror.device_order_diff(B) == (-1 if K < 0 or S < 2 else 0)
