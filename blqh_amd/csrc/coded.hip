@@ -18,6 +18,7 @@
 
 #include "coded.hpp"
 #include "engine.hpp"
+#include "wavesort.hpp"
 
 namespace {
 
@@ -255,18 +256,29 @@ __global__ void __launch_bounds__(64) k_cod_rows(int64_t n, int64_t npadrows, in
             ndiag += __shfl_xor(ndiag, q, 64);
         }
         __syncthreads();
-        for (int k = 2; k <= P; k <<= 1)
-            for (int j = k >> 1; j > 0; j >>= 1) {
-                for (int i = lane; i < P / 2; i += 64) {
-                    const int lo = 2 * i - (i & (j - 1)), hi = lo + j;
-                    const uint64_t a = key[lo], b = key[hi];
-                    if ((a > b) == ((lo & k) == 0)) {
-                        key[lo] = b;
-                        key[hi] = a;
+        if (P <= 64) {
+            sort_lds<1>(key);
+        } else if (P == 128) {
+            sort_lds<2>(key);
+        } else if (P == 256) {
+            sort_lds<4>(key);
+        } else if (P == 512) {
+            sort_lds<8>(key);
+        } else {
+            for (int k = 2; k <= P; k <<= 1)
+                for (int j = k >> 1; j > 0; j >>= 1) {
+                    for (int i = lane; i < P / 2; i += 64) {
+                        const int lo = 2 * i - (i & (j - 1)), hi = lo + j;
+                        const uint64_t a = key[lo], b = key[hi];
+                        if ((a > b) == ((lo & k) == 0)) {
+                            key[lo] = b;
+                            key[hi] = a;
+                        }
                     }
+                    __syncthreads();
                 }
-                __syncthreads();
-            }
+        }
+        __syncthreads();
         for (int k = lane; k < m; k += 64) skey[s + k] = key[k];
         const int nc = m - nrest - ndiag;
         dtot += ndiag;

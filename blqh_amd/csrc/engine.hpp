@@ -19,6 +19,8 @@ struct blqh_basis {
     blqh::Geo geo{};
     blqh::RankSpec spec{};           // the sector (with the spin-up constraint)
     blqh::DevBuf<uint32_t> cnt;      // rank table of spec
+    blqh::DevBuf<uint32_t> rsplit;   // rank shares of the word halves (sector_rank); empty above 32 bits
+    int rbits = 0;                   // bits of the lower half
     int64_t M = 0;                   // sector words
     int64_t n = 0;                   // basis states (orbit representatives)
     blqh::DevBuf<uint64_t> id;       // representatives, ascending
@@ -186,6 +188,8 @@ inline RowCtx make_row_ctx(const blqh_basis* B) {
     c.period = B->period.get();
     c.lut = B->lut.get();
     c.cnt = B->cnt.get();
+    c.rsplit = B->rsplit.get();
+    c.rbits = B->rbits;
     return c;
 }
 

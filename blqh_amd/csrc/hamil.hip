@@ -18,7 +18,7 @@
 //   whose sum is inserted once.  Without a twist the images between full orbits are
 //   one element times a count, and the shifts t and t - nphi, which share their target,
 //   one candidate: a row costs its lookups, not D_l times its elements (N_phi = 16,
-//   nel_up = 8, 3.3e5 rows: 132 ms -> 41 ms).  Tunnelling terms are one-body hops between
+//   nel_up = 8, 6.5e5 rows: 132 ms -> 41 ms).  Tunnelling terms are one-body hops between
 //   the layers; the diagonal (background, charging, bias, Zeeman) comes last.
 // Entries with |h_ij| > 1e-10 are kept, columns ascending.
 //
@@ -43,6 +43,7 @@
 
 #include "engine.hpp"
 #include "rowterms.hpp"
+#include "wavesort.hpp"
 
 namespace blqh {
 
@@ -240,6 +241,7 @@ struct BuildArgs {
     int32_t* col;
     double2* val;
     int32_t* row_counter;
+    int claim;                // rows a workgroup takes from the counter at a time; 0: every gridDim-th
     int32_t* ovf_count;
     int32_t* ovf_rows;
     int32_t* err;             // fill/count mismatch counter
@@ -250,10 +252,14 @@ struct BuildArgs {
     int terms;                // bit 0: pair terms and diagonal; tunnelling hops come with the hop list
 };
 
+// |v| > 1e-10 (squares that underflow belong to dropped entries)
+__device__ __forceinline__ bool kept(double re, double im) { return re * re + im * im > 1e-20; }
+
 template <int CAP>
 __device__ __forceinline__ bool hash_add(int* keys, double* vre, double* vim, int j, double re, double im) {
     constexpr int LOG = __builtin_ctz(CAP);
     unsigned h = ((unsigned)j * 2654435761u) >> (32 - LOG);
+    const unsigned step = (((unsigned)j * 2246822519u) >> (32 - LOG)) | 1u;  // odd: visits every slot
     for (int probe = 0; probe < CAP; ++probe) {
         int k = __atomic_load_n(&keys[h], __ATOMIC_RELAXED);
         if (k == -1) {
@@ -265,20 +271,48 @@ __device__ __forceinline__ bool hash_add(int* keys, double* vre, double* vim, in
             atomicAdd(&vim[h], im);
             return true;
         }
-        h = (h + 1) & (CAP - 1);
+        h = (h + step) & (CAP - 1);
     }
     return false;
 }
 
-// MODE 0: count, MODE 1: fill
-template <int CAP, int MODE>
+// The row's kept entries, kk[u] the column in slot lane CAP / 64 + u or -1, as keys column
+// << log2(CAP) | slot in buf[0, E), ascending.  w: the lane's first place.  In registers
+// (wavesort.hpp): with the entries moved through LDS step by step, values and all, the
+// sort took 16 of the 41 ms of a build at N_phi = 16, nel_up = 8.
+template <int CAP, class K>
+__device__ __forceinline__ void sort_row(const int* kk, int w, int E, K* buf) {
+    constexpr int CH = CAP / 64, LOG = __builtin_ctz(CAP);
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int u = 0; u < CH; ++u)
+        if (kk[u] >= 0) buf[w++] = (K)kk[u] << LOG | (K)(lane * CH + u);
+    const int R = E <= 64 ? 1 : E <= 128 ? 2 : E <= 256 ? 4 : 8;
+    for (int x = E + lane; x < 64 * R; x += 64) buf[x] = ~(K)0;
+    __syncthreads();
+    if (R == 1) sort_lds<1, K>(buf);
+    else if (R == 2) sort_lds<2, K>(buf);
+    else if (R == 4) sort_lds<4, K>(buf);
+    else if constexpr (CAP >= 512) sort_lds<8, K>(buf);
+    __syncthreads();
+}
+
+// Bound by latency: a row is a chain of table reads (rank, lookup table, period) and LDS
+// atomics on one wavefront, and the LDS of its hash and tables leaves nine wavefronts a
+// CU.  Hence ranks from two table reads, two hops a lane in flight, a hash that
+// probes by a second hash (rows of 370 entries in 512 slots), the sort in registers and no
+// square roots: N_phi = 16, nel_up = 8 (6.5e5 rows, 2.4e8 entries) 41 -> 15.3 ms, N_phi =
+// 14 (2.0e5 rows) 8.3 -> 3.7 ms, N_phi = 12 (1.9e4 rows) 0.78 -> 0.45 ms.
+// MODE 0: count, MODE 1: fill, MODE 2: single pass.  K: sort key of the small hashes,
+// 32 bits while a column and a slot fit (build_key64).
+template <int CAP, int MODE, class K>
 __global__ void __launch_bounds__(64) k_build(BuildArgs A) {
     extern __shared__ double smem[];
     __shared__ int keys[CAP];
     __shared__ double vre[CAP], vim[CAP];
-    __shared__ unsigned long long sbuf[MODE >= 1 && CAP > 512 ? CAP : 1];
+    __shared__ unsigned long long sbuf[MODE >= 1 && (CAP > 512 || sizeof(K) == 8) ? CAP : 1];
     __shared__ int occ[64];
-    __shared__ int sQ[128];  // open pair hops awaiting evaluation
+    __shared__ int sQ[192];  // open pair hops awaiting evaluation
     __shared__ uint64_t sLw[32];  // translate(L0, ql)
     __shared__ int sLs[32];       // and its sign
     __shared__ int s_row, s_ovf;
@@ -304,11 +338,20 @@ __global__ void __launch_bounds__(64) k_build(BuildArgs A) {
     ctx.tw = sTW;
     __syncthreads();
 
-    for (;;) {
-        if (lane == 0) s_row = atomicAdd(A.row_counter, 1);
-        __syncthreads();
-        const int64_t r = s_row;
-        if (r >= A.nrows) break;
+    int64_t r = 0, r1 = 0;  // claimed rows
+    for (;; ++r) {
+        if (r == r1) {
+            if (A.claim > 0) {
+                if (lane == 0) s_row = atomicAdd(A.row_counter, A.claim);
+                __syncthreads();
+                r = s_row;
+                r1 = r + A.claim < A.nrows ? r + A.claim : A.nrows;
+            } else {
+                r = r1 == 0 ? blockIdx.x : r - 1 + gridDim.x;
+                r1 = r + 1;
+            }
+            if (r >= A.nrows) break;
+        }
         const int64_t i = A.row_list ? A.row_list[r] : r;
         for (int x = lane; x < CAP; x += 64) { keys[x] = -1; vre[x] = 0.0; vim[x] = 0.0; }
         if (lane == 0) s_ovf = 0;
@@ -333,7 +376,8 @@ __global__ void __launch_bounds__(64) k_build(BuildArgs A) {
             // the candidates are open and a wavefront evaluating them in place
             // would run the lookup for nearly every group of 64, so the open
             // ones are first queued in candidate order (sQ, packed
-            // pr << 8 | tt) and evaluated 64 at a time.
+            // pr << 8 | tt) and evaluated two a lane, whose table and period
+            // reads (latency bounds the kernel) are in flight together.
             // Without a twist the shifts t and t - nphi are one candidate (fold).
             const int Tc = fold ? nphi : T, tmin = fold ? 0 : 1 - nphi;
             const int ncand = (A.terms & 1) ? npairs * Tc : 0;
@@ -341,7 +385,7 @@ __global__ void __launch_bounds__(64) k_build(BuildArgs A) {
             int pr = lane / Tc, tt = lane % Tc;
             int next = 0, qn = 0;
             for (;;) {
-                while (qn < 64 && next < ncand) {
+                while (qn < 128 && next < ncand) {
                     bool open = false;
                     if (next + lane < ncand) {
                         const unsigned short pw = sPair[pr];
@@ -364,20 +408,45 @@ __global__ void __launch_bounds__(64) k_build(BuildArgs A) {
                 }
                 if (qn == 0) break;
                 __syncthreads();  // queue entries written by other lanes
-                const int take = qn < 64 ? qn : 64;
-                const int e = lane < take ? sQ[lane] : -1;
-                const int carry = lane + 64 < qn ? sQ[lane + 64] : 0;
+                const int take = qn < 128 ? qn : 128;
+                int e[2];
+                e[0] = lane < take ? sQ[lane] : -1;
+                e[1] = lane + 64 < take ? sQ[lane + 64] : -1;
+                const int carry = lane + 128 < qn ? sQ[lane + 128] : 0;
                 __syncthreads();  // every entry read before the carried ones move to the front
-                if (lane + 64 < qn) sQ[lane] = carry;
+                if (lane + 128 < qn) sQ[lane] = carry;
                 qn -= take;
-                if (e >= 0) {
-                    const unsigned short pw = sPair[e >> 8];
-                    int j;
-                    double re, im;
-                    if (pair_orbit_sum(ctx, sLw, sLs, Dl, occ[pw & 0xff], occ[pw >> 8], (e & 0xff) + tmin, j, re,
-                                       im, fold))
-                        if (!hash_add<CAP>(keys, vre, vim, j, re, im)) ovf = true;
+                PairHop h[2];
+                int n0[2], m0[2], t[2], j[2], Dr[2];
+                int64_t rk[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int x = e[u] < 0 ? 0 : e[u];
+                    const unsigned short pw = sPair[x >> 8];
+                    n0[u] = occ[pw & 0xff];
+                    m0[u] = occ[pw >> 8];
+                    t[u] = (x & 0xff) + tmin;
+                    (void)pair_hop(nphi, L0, n0[u], m0[u], t[u], h[u]);
+                    // a lane without a hop looks its row's own word up
+                    rk[u] = sector_rank(ctx, e[u] < 0 ? L0 : h[u].word);
                 }
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    if (rk[u] < 0 || rk[u] >= ctx.M) {  // defensive: unreachable for sector words
+                        rk[u] = 0;
+                        e[u] = -1;
+                    }
+                    j[u] = ctx.lut[rk[u]];
+                }
+#pragma unroll
+                for (int u = 0; u < 2; ++u) Dr[u] = ctx.K < 0 ? 1 : ctx.period[j[u] < 0 ? 0 : j[u] >> 5];
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+                    if (e[u] >= 0 && j[u] >= 0) {
+                        double re, im;
+                        pair_orbit_value(ctx, sLw, sLs, Dl, n0[u], m0[u], t[u], h[u], j[u] & 31, Dr[u], fold, re, im);
+                        if (!hash_add<CAP>(keys, vre, vim, j[u] >> 5, re, im)) ovf = true;
+                    }
             }
         }
         for (int ql = 0; ql < (fold ? 1 : Dl); ++ql)
@@ -410,26 +479,23 @@ __global__ void __launch_bounds__(64) k_build(BuildArgs A) {
         if (MODE == 0) {
             int c = 0;
             for (int x = lane; x < CAP; x += 64)
-                if (keys[x] >= 0 && hypot(vre[x], vim[x]) > 1e-10) ++c;
+                if (keys[x] >= 0 && kept(vre[x], vim[x])) ++c;
             for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
             if (lane == 0) {
                 A.nnz_out[i] = c;
                 atomicMax(A.row_max, c);
             }
         } else if constexpr (CAP <= 512) {
-            // compact the kept (column, value) entries to the front of the
-            // hash arrays (lane owns a contiguous chunk of slots, read into
-            // registers first), then sort them by column in place
-            constexpr int CH = CAP / 64;
+            // kept entries as (column, slot) keys, compacted over the key array (lane owns
+            // a contiguous chunk of slots, read into registers first), sorted by column in
+            // registers; the values stay in their slots
+            constexpr int CH = CAP / 64, LOG = __builtin_ctz(CAP);
             int kk[CH];
-            double rr[CH], ii[CH];
             int c = 0;
 #pragma unroll
             for (int u = 0; u < CH; ++u) {
                 const int x = lane * CH + u;
-                rr[u] = vre[x];
-                ii[u] = vim[x];
-                kk[u] = keys[x] >= 0 && hypot(rr[u], ii[u]) > 1e-10 ? keys[x] : -1;
+                kk[u] = keys[x] >= 0 && kept(vre[x], vim[x]) ? keys[x] : -1;
                 c += kk[u] >= 0;
             }
             int pre = c;  // inclusive scan over lanes
@@ -438,47 +504,17 @@ __global__ void __launch_bounds__(64) k_build(BuildArgs A) {
                 if (lane >= o) pre += y;
             }
             const int E = __shfl(pre, 63, 64);
-            __syncthreads();  // every slot read before the front is overwritten
-            int w = pre - c;
-#pragma unroll
-            for (int u = 0; u < CH; ++u)
-                if (kk[u] >= 0) {
-                    keys[w] = kk[u];
-                    vre[w] = rr[u];
-                    vim[w] = ii[u];
-                    ++w;
-                }
-            int P = 1;
-            while (P < E) P <<= 1;
-            for (int x = E + lane; x < P; x += 64) keys[x] = 0x7fffffff;  // columns are < 2^31 - 1
-            __syncthreads();
-            // bitonic sort of keys[0, P) (distinct columns), values moved along
-            for (int k = 2; k <= P; k <<= 1)
-                for (int jj = k >> 1; jj > 0; jj >>= 1) {
-                    for (int x = lane; x < P; x += 64) {
-                        const int y = x ^ jj;
-                        if (y > x) {
-                            const int u = keys[x], v = keys[y];
-                            const bool up = (x & k) == 0;
-                            if ((u > v) == up) {
-                                keys[x] = v;
-                                keys[y] = u;
-                                const double a = vre[x], b = vim[x];
-                                vre[x] = vre[y];
-                                vim[x] = vim[y];
-                                vre[y] = a;
-                                vim[y] = b;
-                            }
-                        }
-                    }
-                    __syncthreads();
-                }
+            __syncthreads();  // every slot read before the keys are overwritten
+            K* key = sizeof(K) == 4 ? reinterpret_cast<K*>(keys) : reinterpret_cast<K*>(sbuf);
+            sort_row<CAP, K>(kk, pre - c, E, key);
             if (MODE == 2) {
                 // single pass: the sorted row goes to its staging slot (E <= CAP)
                 const int64_t base = i * (int64_t)CAP;
                 for (int x = lane; x < E; x += 64) {
-                    A.stage_col[base + x] = keys[x];
-                    A.stage_val[base + x] = make_double2(vre[x], vim[x]);
+                    const K k = key[x];
+                    const int slot = (int)(k & (CAP - 1));
+                    A.stage_col[base + x] = (int32_t)(k >> LOG);
+                    A.stage_val[base + x] = make_double2(vre[slot], vim[slot]);
                 }
                 if (lane == 0) {
                     A.nnz_out[i] = E;
@@ -492,8 +528,10 @@ __global__ void __launch_bounds__(64) k_build(BuildArgs A) {
                     if (lane == 0) atomicAdd(A.err, 1);
                 } else {
                     for (int x = lane; x < E; x += 64) {
-                        A.col[base + x] = keys[x];
-                        A.val[base + x] = make_double2(vre[x], vim[x]);
+                        const K k = key[x];
+                        const int slot = (int)(k & (CAP - 1));
+                        A.col[base + x] = (int32_t)(k >> LOG);
+                        A.val[base + x] = make_double2(vre[slot], vim[slot]);
                     }
                 }
             }
@@ -502,7 +540,7 @@ __global__ void __launch_bounds__(64) k_build(BuildArgs A) {
             constexpr int CH = CAP / 64;
             int c = 0;
             for (int x = lane * CH; x < lane * CH + CH; ++x)
-                if (keys[x] >= 0 && hypot(vre[x], vim[x]) > 1e-10) ++c;
+                if (keys[x] >= 0 && kept(vre[x], vim[x])) ++c;
             int pre = c;  // inclusive scan over lanes
             for (int o = 1; o < 64; o <<= 1) {
                 const int y = __shfl_up(pre, o, 64);
@@ -511,7 +549,7 @@ __global__ void __launch_bounds__(64) k_build(BuildArgs A) {
             const int E = __shfl(pre, 63, 64);
             int w = pre - c;
             for (int x = lane * CH; x < lane * CH + CH; ++x)
-                if (keys[x] >= 0 && hypot(vre[x], vim[x]) > 1e-10)
+                if (keys[x] >= 0 && kept(vre[x], vim[x]))
                     sbuf[w++] = ((unsigned long long)(unsigned)keys[x] << 32) | (unsigned)x;
             int P = 1;
             while (P < E) P <<= 1;
@@ -601,21 +639,50 @@ T* upload(DevBuf<T>& buf, const std::vector<T>& v, hipStream_t st) {
     return buf.get();
 }
 
+// 64-bit sort keys: a column and a slot no longer fit in 32 bits (BLQH_BUILD_KEY64=1: always, for tests)
+bool build_key64(int64_t n, int cap) {
+    return n > ((int64_t)1 << (32 - __builtin_ctz(cap))) || std::getenv("BLQH_BUILD_KEY64") != nullptr;
+}
+
 template <int CAP, int MODE>
-void launch_build(const BuildArgs& A, int64_t rows, size_t smem, hipStream_t st, int ncu) {
+void launch_build(const BuildArgs& A, int64_t n, int64_t rows, size_t smem, hipStream_t st, int ncu) {
     if (rows <= 0) return;
-    const int64_t blocks = std::min<int64_t>(rows, (int64_t)ncu * 32);  // rows are claimed by a counter
+    // As many workgroups as fit at once (each stages the tables).  From 32 rows each on they
+    // claim rows from a counter, 16 at a time: single rows wait for each other's atomics
+    // (2.05e5 rows 5.0 ms, in sixteens 3.7), fixed shares leave the slower CUs behind (5.5).
+    // Fewer rows are dealt out: 1.9e4 rows 0.44 ms, claimed singly 0.63, in pairs 0.58.
+    BuildArgs a = A;
+    auto blocks_of = [&](const void* kern) {
+        int per = 0;
+        BLQH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, 64, smem));
+        const int64_t g = std::min<int64_t>(rows, (int64_t)ncu * std::max(per, 1));
+        a.claim = rows >= 32 * g ? 16 : 0;
+        return dim3((unsigned)g);
+    };
     BLQH_HIP(hipMemsetAsync(A.row_counter, 0, sizeof(int32_t), st));
-    hipLaunchKernelGGL((k_build<CAP, MODE>), dim3((unsigned)blocks), dim3(64), smem, st, A);
+    bool wide = true;
+    if constexpr (CAP <= 512) {
+        wide = build_key64(n, CAP);
+        auto* kern = k_build<CAP, MODE, uint32_t>;
+        if (!wide) {
+            const dim3 g = blocks_of((const void*)kern);
+            hipLaunchKernelGGL(kern, g, dim3(64), smem, st, a);
+        }
+    }
+    auto* kern = k_build<CAP, MODE, uint64_t>;
+    if (wide) {
+        const dim3 g = blocks_of((const void*)kern);
+        hipLaunchKernelGGL(kern, g, dim3(64), smem, st, a);
+    }
     BLQH_HIP(hipGetLastError());
 }
 
 template <int MODE>
-void launch_first(int cap, const BuildArgs& A, int64_t rows, size_t smem, hipStream_t st, int ncu) {
+void launch_first(int cap, const BuildArgs& A, int64_t n, int64_t rows, size_t smem, hipStream_t st, int ncu) {
     if (cap == kSmaller)
-        launch_build<kSmaller, MODE>(A, rows, smem, st, ncu);
+        launch_build<kSmaller, MODE>(A, n, rows, smem, st, ncu);
     else
-        launch_build<kSmall, MODE>(A, rows, smem, st, ncu);
+        launch_build<kSmall, MODE>(A, n, rows, smem, st, ncu);
 }
 
 }  // namespace
@@ -701,10 +768,10 @@ void blqh_hamil_build_impl(const blqh_basis* B, const blqh_params& p_in, blqh_ha
         A.stage_col = scol.get();
         A.stage_val = sval.get();
         A.stage_ok = sok.get();
-        launch_first<2>(cap, A, B->n, smem, st, ncu);
+        launch_first<2>(cap, A, B->n, B->n, smem, st, ncu);
     } else {
         // count
-        launch_first<0>(cap, A, B->n, smem, st, ncu);
+        launch_first<0>(cap, A, B->n, B->n, smem, st, ncu);
     }
     int32_t h_ctr[4];
     BLQH_HIP(hipMemcpyAsync(h_ctr, ctr.get(), sizeof(h_ctr), hipMemcpyDeviceToHost, st));
@@ -723,7 +790,7 @@ void blqh_hamil_build_impl(const blqh_basis* B, const blqh_params& p_in, blqh_ha
         Ao.err = ctr2.get() + 2;
         Ao.row_max = ctr2.get() + 3;
         Ao.ovf_rows = ovf2.get();
-        launch_build<kLarge, 0>(Ao, novf, smem, st, ncu);
+        launch_build<kLarge, 0>(Ao, B->n, novf, smem, st, ncu);
         BLQH_HIP(hipMemcpyAsync(h_ctr, ctr2.get(), sizeof(h_ctr), hipMemcpyDeviceToHost, st));
         BLQH_HIP(hipStreamSynchronize(st));
         BLQH_REQUIRE(h_ctr[1] == 0, BLQH_ERANGE, "a Hamiltonian row has more than 4096 distinct columns");
@@ -758,11 +825,11 @@ void blqh_hamil_build_impl(const blqh_basis* B, const blqh_params& p_in, blqh_ha
                                sok.get(), H->rowptr.get(), H->col.get(), H->val.get());
         BLQH_HIP(hipGetLastError());
     } else {
-        launch_first<1>(cap, A, B->n, smem, st, ncu);  // overflow rows are skipped (counted in err)
+        launch_first<1>(cap, A, B->n, B->n, smem, st, ncu);  // overflow rows are skipped (counted in err)
     }
     if (novf > 0) {
         BLQH_HIP(hipMemsetAsync(ctr2.get(), 0, 4 * sizeof(int32_t), st));
-        launch_build<kLarge, 1>(Ao, novf, smem, st, ncu);
+        launch_build<kLarge, 1>(Ao, B->n, novf, smem, st, ncu);
     }
     int32_t e1[4] = {0, 0, 0, 0}, e2[4] = {0, 0, 0, 0};
     BLQH_HIP(hipMemcpyAsync(e1, ctr.get(), sizeof(e1), hipMemcpyDeviceToHost, st));

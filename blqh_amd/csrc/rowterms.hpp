@@ -27,6 +27,8 @@ struct RowCtx {
     const int16_t* period;
     const int32_t* lut;
     const uint32_t* cnt;
+    const uint32_t* rsplit;  // rank shares of a word's halves, null: rank_word (sector_rank)
+    int rbits;
     const double* C;     // [2][nphi][nphi] Coulomb table V[alpha][|dm|][|t|]
     const double2* FT;   // [2 nphi - 1]: FT[ql - qr + nphi - 1] = exp(2 pi i (ql - qr) K / order)
     const double2* tw;   // [2 nphi - 1] twist phase per t
@@ -85,10 +87,51 @@ BLQH_HD bool is_survivor(const Geo& g, const RankSpec& s, const T* cnt, const in
 // shift q with inv_translate(y, q) == id[j] as a word.
 BLQH_HD int32_t lut_pack(int64_t j, int q) { return (int32_t)((j << 5) | q); }
 
+// rank_word of a sector word.  What the walk over the set bits adds for the upper half
+// depends on that half alone, and the state it leaves for the lower one is fixed by the
+// lower half itself (its electrons, residual and counts, since the whole is in the sector):
+// rank = shares of the two halves, one table entry each (rsplit: the lower half's 2^rbits
+// entries, then the upper's), in place of nel dependent steps of some 35 instructions.
+BLQH_HD int64_t sector_rank(const RowCtx& c, uint64_t w) {
+    if (!c.rsplit) return rank_word(c.spec, c.cnt, w);
+    const uint32_t lo = (uint32_t)(w & lowbits(c.rbits)), hi = (uint32_t)(w >> c.rbits) + (1u << c.rbits);
+    return (int64_t)c.rsplit[lo] + (int64_t)c.rsplit[hi];
+}
+
+// Entry x of rsplit.
+BLQH_HD uint32_t rank_share(const RankSpec& s, const uint32_t* cnt, int rbits, uint32_t x) {
+    const bool upper = x >> rbits;
+    uint64_t w = upper ? (uint64_t)(x - (1u << rbits)) << rbits : (uint64_t)x;
+    int k = s.nel, r = s.Jt, a = s.nA, b = s.nB;
+    if (!upper) {  // the state that a sector word's upper half leaves
+        k = popc(w);
+        a = s.maskA ? popc(w & s.maskA) : s.nA;
+        b = s.maskB ? popc(w & s.maskB) : s.nB;
+        r = 0;
+        for (int p = 0; p < rbits; ++p)
+            if (w >> p & 1) r += p % s.nphi;
+        r %= s.R;
+        if (k > s.nel || a > s.nA || b > s.nB) return 0;  // in no sector word
+    }
+    uint32_t rk = 0;
+    for (; w; --k) {
+        if (k <= 0 || a < 0 || b < 0) return 0;  // in no sector word
+        const int p = top_bit(w);
+        w ^= 1ULL << p;
+        rk += cnt[rs_index(s, p, k, r, a, b)];
+        r -= p % s.nphi;
+        if (r < 0) r += s.R;
+        if (s.R == 1) r = 0;
+        a -= (int)((s.maskA >> p) & 1ULL);
+        b -= (int)((s.maskB >> p) & 1ULL);
+    }
+    return rk;
+}
+
 // Row j of the orbit of sector word Rs, the table's shift q1
 // (inv_translate(Rs, q1) == id[j]) and j's period Dr.
 BLQH_HD bool locate_word(const RowCtx& c, uint64_t Rs, int& j, int& q1, int& Dr) {
-    const int64_t rk = rank_word(c.spec, c.cnt, Rs);
+    const int64_t rk = sector_rank(c, Rs);
     if (rk < 0 || rk >= c.M) return false;  // defensive: unreachable for sector words
     const int32_t e = c.lut[rk];
     if (e < 0) return false;
@@ -151,11 +194,10 @@ BLQH_HD bool pair_hop(int nphi, uint64_t L, int n, int m, int t, PairHop& h) {
 }
 
 // Two-body element of the open pair hop h of L (pair n < m, shift t) whose
-// target lies in the orbit of row j (sector-table shift q1, period Dr).  fold (t >= 0, no
-// twist): with that of shift t - nphi, which has the same target.
+// target lies in the orbit of row j (sector-table shift q1, period Dr).
 // BLQH_without_spin/lanczos_hamiltonian.cpp:109-292, BLQH_with_spin/lanczos_hamiltonian.cpp:109-712.
 BLQH_HD void pair_value(const RowCtx& c, uint64_t L, int signl, int Dl, int ql, int n, int m, int t, const PairHop& h,
-                        int q1, int Dr, double& re, double& im, bool fold = false) {
+                        int q1, int Dr, double& re, double& im) {
     const int nphi = c.g.nphi;
     const int a = h.a, b = h.b, n0 = h.n0, xm = h.xm, nt = h.nt, mt = h.mt;
     int qr = 0, sr = 1;
@@ -173,8 +215,7 @@ BLQH_HD void pair_value(const RowCtx& c, uint64_t L, int signl, int Dl, int ql, 
     int dm = xm - n0;
     dm = dm < 0 ? -dm : dm;
     const int at = t < 0 ? -t : t;
-    const double* Cm = c.C + alpha * nphi * nphi + dm * nphi;
-    const double Cv = fold && t ? Cm[at] + Cm[nphi - at] : Cm[at];
+    const double Cv = c.C[alpha * nphi * nphi + dm * nphi + at];
     double2 ft = c.FT[ql - qr + nphi - 1];
     const bool twisted = c.twist_sel == 1 ? (a != b) : (c.twist_sel == 2 && ((a == 0 && b == 3) || (a == 1 && b == 2)));
     if (twisted) ft = cmul(ft, c.tw[t + nphi - 1]);
@@ -230,28 +271,33 @@ BLQH_HD int image_count(const RowCtx& c, int Dl, int n, int m, int t, const Pair
     return h.wn != h.wm ? 2 * one - Dl : Dl - 2 * one;
 }
 
-// The pair hop (n0 < m0 of the row word L0 = Ls[0], shift t) and its images
+// The pair hop h (n0 < m0 of the row word L0 = Ls[0], shift t) and its images
 // in the translated words Ls[ql] = translate(L0, ql) (signs sgl[ql]), ql < Dl.
 // A translation maps the open hops of L0 one to one onto those of Ls[ql] (the
 // image moves the rotated orbitals; when the rotation swaps their order the
 // image is the pair (m, n) with shift -t), and maps every hop target onto the
-// same orbit, so the target is located once.  Returns the row j and the sum
-// of the Dl elements, ql ascending, each computed as pair_term computes the
-// image's term in Ls[ql]; false when the hop is blocked or its target has no
-// representative.
-BLQH_HD bool pair_orbit_sum(const RowCtx& c, const uint64_t* Ls, const int* sgl, int Dl, int n0, int m0, int t, int& j,
-                            double& re, double& im, bool fold = false) {
+// same orbit, so the target (q1, Dr as locate_word gives them) is located once.  Returns
+// the sum of the Dl elements, ql ascending, each computed as pair_term computes the
+// image's term in Ls[ql]; where the images are equal (images_equal), one element with
+// FT / sqrt(Dl Dr) taken Dl times, that is FT.  fold (0 <= t): with the hop of shift
+// t - nphi, which has the same target.
+BLQH_HD void pair_orbit_value(const RowCtx& c, const uint64_t* Ls, const int* sgl, int Dl, int n0, int m0, int t,
+                              PairHop h, int q1, int Dr, bool fold, double& re, double& im) {
     const int nphi = c.g.nphi;
-    PairHop h;
-    if (!pair_hop(nphi, Ls[0], n0, m0, t, h)) return false;
-    int q1, Dr;
-    if (!locate_word(c, h.word, j, q1, Dr)) return false;
     if (images_equal(c, Dl, Dr)) {
-        pair_value(c, Ls[0], sgl[0], Dl, 0, n0, m0, t, h, q1, Dr, re, im, fold);
-        const double cnt = image_count(c, Dl, n0, m0, t, h);
-        re *= cnt;
-        im *= cnt;
-        return true;
+        int sr;
+        (void)inv_translate(c.g, h.word, q1, sr);
+        const int sign = sign2(Ls[0], n0, m0, h.nt, h.mt) * sr * (c.mono_odd && h.wn != h.wm ? -1 : 1);
+        const int sh = c.g.S == 4 ? 1 : 0;
+        const int dm = h.xm < h.n0 ? h.n0 - h.xm : h.xm - h.n0, at = t < 0 ? -t : t;
+        const double* Cm = c.C + (((h.a >> sh) != (h.b >> sh) ? nphi : 0) + dm) * nphi;
+        const double Cv = fold && t ? Cm[at] + Cm[nphi - at] : Cm[at];
+        const int cnt = image_count(c, Dl, n0, m0, t, h);
+        const double f = cnt == Dl ? (double)sign : sign * ((double)cnt / Dl);
+        const double2 ft = c.FT[nphi - 1 - q1];
+        re = ft.x * Cv * f;
+        im = ft.y * Cv * f;
+        return;
     }
     re = 0.0;
     im = 0.0;
@@ -271,6 +317,17 @@ BLQH_HD bool pair_orbit_sum(const RowCtx& c, const uint64_t* Ls, const int* sgl,
             re += r;
             im += i;
         }
+}
+
+// pair_orbit_value of the hop of n0 < m0 by t; the row j of its target.  False when the
+// hop is blocked or its target has no representative.
+BLQH_HD bool pair_orbit_sum(const RowCtx& c, const uint64_t* Ls, const int* sgl, int Dl, int n0, int m0, int t, int& j,
+                            double& re, double& im, bool fold = false) {
+    PairHop h;
+    if (!pair_hop(c.g.nphi, Ls[0], n0, m0, t, h)) return false;
+    int q1, Dr;
+    if (!locate_word(c, h.word, j, q1, Dr)) return false;
+    pair_orbit_value(c, Ls, sgl, Dl, n0, m0, t, h, q1, Dr, fold, re, im);
     return true;
 }
 

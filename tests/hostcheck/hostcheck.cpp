@@ -385,6 +385,23 @@ void hc_tridiag_vector_k(int m, const double* a, const double* b, int k, double*
     tridiag_vector_k(m, a, b, k, x);
 }
 
+// Largest difference between the split ranks (rank_share) and rank_word over a sector's words.
+int64_t hc_split_rank_diff(const blqh_sector* s) {
+    const RankSpec sp = make_rank_spec(*s, true);
+    int64_t M = 0;
+    const std::vector<uint32_t> t = make_rank_table(sp, &M);
+    RowCtx c{};
+    c.spec = sp;
+    c.rbits = sp.nbits / 2;
+    std::vector<uint32_t> split((1u << c.rbits) + (1u << (sp.nbits - c.rbits)));
+    for (uint32_t x = 0; x < split.size(); ++x) split[x] = rank_share(sp, t.data(), c.rbits, x);
+    c.rsplit = split.data();
+    int64_t diff = 0;
+    for (int64_t r = 0; r < M; ++r)
+        diff = std::max<int64_t>(diff, std::abs(sector_rank(c, unrank_word(sp, t.data(), r)) - r));
+    return diff;
+}
+
 // the solvers' convergence test (ritz.hpp)
 double hc_lowest_in(int m, const double* a, const double* b, double lo, double hi) { return lowest_in(m, a, b, lo, hi); }
 double hc_lowest_bisected(int m, const double* a, const double* b, double lo, double hi) {

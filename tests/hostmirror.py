@@ -33,6 +33,8 @@ def lib():
             f.restype = C.c_double
         _L.hc_device_order_diff.argtypes = [C.c_void_p]
         _L.hc_device_order_diff.restype = C.c_int64
+        _L.hc_split_rank_diff.argtypes = [C.POINTER(blqh_amd.Sector)]
+        _L.hc_split_rank_diff.restype = C.c_int64
         _L.hc_hop_images.argtypes = [C.POINTER(blqh_amd.Sector)]
         _L.hc_hop_images.restype = C.c_double
         _L.hc_residual_exceeds.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_double, C.c_double, C.c_double]
@@ -105,6 +107,11 @@ def mod_by_rcp(n, d, r):
     out = np.empty(n, np.int32)
     lib().hc_mod_by_rcp(n, d, float(np.float32(r)), _p(out))
     return out
+
+
+def split_rank_diff(sec):
+    """Largest difference of a sector word's rank from its halves' shares to the walk's."""
+    return lib().hc_split_rank_diff(C.byref(sec))
 
 
 def device_order_diff(basis):

@@ -299,3 +299,13 @@ def test_equal_images_against_reference_loop_order(case):
     np.testing.assert_allclose(val, val2, rtol=0, atol=1e-13 * np.abs(val2).max())
     if case[0] > 1 and case[3] < 0:
         assert 0 <= hostmirror.hop_images(sec) < 1e-13
+
+
+@pytest.mark.parametrize("case", [(2, 8, 8, -1, -1, 3, 0), (2, 8, 8, 4, -1, -1, -1), (2, 2, 1, -1, -1, 0, 0),
+                                  (2, 7, 5, -1, -1, 6, 0), (2, 12, 12, 6, -1, 1, 2), (4, 6, 6, 3, 3, 5, 0),
+                                  (4, 6, 6, 3, -1, 2, 0), (4, 5, 7, -1, 4, -1, -1), (4, 8, 4, -1, 2, 1, 0),
+                                  (1, 12, 4, -1, -1, 3, 3), (1, 9, 3, -1, -1, -1, -1), (1, 11, 4, -1, -1, 5, 0)],
+                         ids=lambda c: "_".join(map(str, c)))
+def test_split_rank_equals_walk(case):
+    """Every word of the sector: the halves' table entries add up to the rank."""
+    assert hostmirror.split_rank_diff(blqh_amd.Sector(*case)) == 0

@@ -57,3 +57,23 @@ def test_row_hash_capacities_agree(name, args, kw, bkw):
     again = blqh_amd.Hamiltonian(B, p).export()
     for a, b in zip(first, again):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("name,args,kw,bkw", CASES, ids=[c[0] for c in CASES])
+def test_row_sort_key_widths_agree(name, args, kw, bkw):
+    """Rows are sorted by 32-bit keys while a column and its slot fit, by 64-bit keys beyond
+    (8.4M rows at 512 slots; forced here), in both hashes and both schemes."""
+    print(name, flush=True)
+    B = blqh_amd.Basis(*args, **bkw)
+    p = blqh_amd.params(args[0], **kw)
+    first = blqh_amd.Hamiltonian(B, p).export()
+    for more in ({}, {"BLQH_BUILD_CAP": "256"}, {"BLQH_BUILD_TWO_PASS": "1"}):
+        env = dict(more, BLQH_BUILD_KEY64="1")
+        os.environ.update(env)
+        try:
+            wide = blqh_amd.Hamiltonian(B, p).export()
+        finally:
+            for k in env:
+                del os.environ[k]
+        for a, b in zip(first, wide):
+            assert np.array_equal(a, b), more
