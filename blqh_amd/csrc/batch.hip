@@ -40,6 +40,7 @@
 #include "ritz.hpp"
 #include "engine.hpp"
 #include "mtstart.hpp"
+#include "small.hpp"
 #include "xcdplan.hpp"
 
 namespace blqh {
@@ -718,6 +719,24 @@ __global__ void __launch_bounds__(64) k_tiles(const TileJob* __restrict__ jobs, 
     }
 }
 
+// ---- steps of small members ----------------------------------------------------
+// Steps j0 .. j1 - 1 of every live problem, a workgroup each (small.hpp).
+template <bool RES>
+__global__ void __launch_bounds__(kSmallT) k_bsmall(BState S, int j0, int j1) {
+    extern __shared__ __align__(16) double ctab[];
+    const int p = blockIdx.x;
+    if (!S.active[p]) return;
+    const BProb& P = S.probs[p];
+    double *alpha = S.alpha + (int64_t)p * S.cap, *beta = S.beta + (int64_t)p * (S.cap + 1),
+           *invb = S.invb + (int64_t)p * (S.cap + 1);
+    const int nsl = (int)((P.n + 63) >> 6);
+    const int64_t ncod = P.c.base[nsl], nrest = P.c.rbase[nsl];
+    if (P.real)
+        small_steps<true, true, RES>(P.c, ncod, nrest, P.W, alpha, beta, invb, j0, j1, nullptr, 0, ctab);
+    else
+        small_steps<false, true, RES>(P.c, ncod, nrest, P.W, alpha, beta, invb, j0, j1, nullptr, 0, ctab);
+}
+
 // K2: alpha_j, W_{j+1} = u - alpha_j W_j / beta_j, |W_{j+1}|^2 partials
 __global__ void __launch_bounds__(kBT) k_b2(BState S, int jrel) {
     __shared__ double sh[kBT / 64];
@@ -1040,6 +1059,27 @@ struct blqh_batch {
 namespace {
 
 bool use_tiles(const blqh_batch* b) { return b->lpr == 64 && b->one_panel; }
+
+// Batches whose members a workgroup each steps through (k_bsmall): lanes 64, own matrices, none
+// above kSmallRows rows and kSmallWords entries.  lds: its dynamic LDS (0: another batch),
+// res: with every matrix in LDS.
+constexpr int64_t kSmallWords = 1 << 16;
+constexpr int kSmallSteps = 8;  // steps a launch, at least
+struct SmallShape {
+    size_t lds = 0;
+    bool res = false;
+};
+SmallShape small_shape(const blqh_batch* b) {
+    if (b->lpr != 64 || b->G) return {};
+    size_t vec = 0, all = 0;
+    for (const blqh_hamil* H : b->hs) {
+        if (H->n > kSmallRows || H->nnz > kSmallWords || !H->cod.built) return {};
+        const Coded& C = H->cod;
+        vec = std::max(vec, small_lds_bytes(C.real, C.ntab, H->n));
+        all = std::max(all, small_lds_bytes(C.real, C.ntab, H->n, C.ncod, C.nrest));
+    }
+    return all <= kSmallLdsMax ? SmallShape{all, true} : vec <= kSmallLdsMax ? SmallShape{vec, false} : SmallShape{};
+}
 
 // What the captured K1 launches depend on beside the lanes and the value kinds.
 std::array<size_t, 2> k1_shape(const blqh_batch* b) {
@@ -1733,7 +1773,13 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
         }
     } evguard{ev};
     const int kinds = (b->has_real ? 2 : 0) | (b->has_complex ? 1 : 0);  // which K1 launches a step has
-    if (!timed && (b->g_chk != chk || b->g_lpr != b->lpr || b->g_cap != cap || b->g_kinds != kinds ||
+    const SmallShape shape = timed ? SmallShape{} : small_shape(b);
+    const bool small = shape.lds > 0;  // k_bsmall takes the steps
+    if (small) {
+        static const bool attr = (allow_lds(k_bsmall<true>, kSmallLdsMax), allow_lds(k_bsmall<false>, kSmallLdsMax), true);
+        (void)attr;
+    }
+    if (!timed && !small && (b->g_chk != chk || b->g_lpr != b->lpr || b->g_cap != cap || b->g_kinds != kinds ||
                    b->g_tab != k1_shape(b) || !b->gexec)) {
         if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
         if (b->graph) (void)hipGraphDestroy(b->graph);
@@ -1750,6 +1796,7 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
         b->g_tab = k1_shape(b);
     }
     hipGraphExec_t gexec = b->gexec;
+    const int stride = small ? std::max(chk, kSmallSteps) : chk;  // steps queued at a time
     const int zero = 0;
     copy_sync(pl.jbase.get(), &zero, 4, hipMemcpyHostToDevice);
 
@@ -1794,14 +1841,18 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
     // replays go ahead of each test.
     int queued = 0;  // steps queued so far
     auto enqueue = [&](int first) {
-        if (timed) chunk(true, first);
+        if (small)
+            for (int j = first; j < std::min(cap, first + stride); j += kSmallLaunch)
+                hipLaunchKernelGGL(shape.res ? k_bsmall<true> : k_bsmall<false>, dim3(P), dim3(kSmallT), shape.lds, st, S, j,
+                                   std::min({cap, first + stride, j + kSmallLaunch}));
+        else if (timed) chunk(true, first);
         else BLQH_HIP(hipGraphLaunch(gexec, st));
         BLQH_HIP(hipGetLastError());
     };
     auto enqueue_n = [&](int r) {
         for (int i = 0; i < r && queued < cap; ++i) {
             enqueue(queued);
-            queued += chk;
+            queued += stride;
         }
     };
     auto readback = [&]() {
@@ -1876,7 +1927,7 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
             for (int p = 0; p < P; ++p) dst[p] = live[p];
             BLQH_HIP(hipMemcpyAsync(pl.active.get(), dst, P * 4, hipMemcpyHostToDevice, st));
             slot ^= 1;
-            if (b->lpr == 64) {  // k_b1j walks the lists
+            if (b->lpr == 64 && !small) {  // k_b1j and k_b1x walk the lists
                 std::vector<int32_t> items, seg;
                 work_lists(b, &live, items, seg);
                 int32_t* lp = listpin + (size_t)lslot * list_slot;

@@ -79,6 +79,15 @@ __device__ __forceinline__ double2 cod_cplx(const double2* tab, uint32_t e) {
     return make_double2(cod_sign(v.x, e), cod_sign(v.y, e << 1));
 }
 
+// (ar, ai) += v x in four multiply-adds, in this order wherever a sum has to have the same
+// bits in two kernels
+__device__ __forceinline__ void cmac(double2 v, double2 x, double& ar, double& ai) {
+    ar = fma(v.x, x.x, ar);
+    ai = fma(v.x, x.y, ai);
+    ar = fma(-v.y, x.y, ar);
+    ai = fma(v.y, x.x, ai);
+}
+
 // diagonal element of a row
 __device__ __forceinline__ double2 cod_diag(const CodView& C, bool real, int64_t row) {
     return real ? make_double2(C.diag[row], 0.0) : reinterpret_cast<const double2*>(C.diag)[row];
@@ -100,7 +109,8 @@ __device__ __forceinline__ void cod_stage(const double* __restrict__ tab, int nt
 // steps each) are dealt to NP wavefronts, this one taking those with g mod NP
 // == par.  The words of the next group are loaded before the x gathers of the
 // current one, so a wavefront always has loads in flight.
-template <bool REAL, int NP, int U>
+// KEEP: the words are read again soon (small.hpp), leave them in the caches.
+template <bool REAL, int NP, int U, bool KEEP = false>
 __device__ __forceinline__ void cod_run_sum(const uint32_t* __restrict__ er, const double* tab,
                                             const double2* __restrict__ xp, uint32_t len, int par, double& ar,
                                             double& ai) {
@@ -114,7 +124,7 @@ __device__ __forceinline__ void cod_run_sum(const uint32_t* __restrict__ er, con
         for (int u = 0; u < U; ++u) {
             const uint32_t q = off + lanes_below(m[u]);
             off += (uint32_t)__popcll(m[u]);
-            e[u] = t + u < len ? __builtin_nontemporal_load(&er[q]) : 0u;
+            e[u] = t + u < len ? (KEEP ? er[q] : __builtin_nontemporal_load(&er[q])) : 0u;
         }
     };
     auto skip = [&](uint32_t t) {  // another wave's group: advance the offset only
@@ -139,13 +149,12 @@ __device__ __forceinline__ void cod_run_sum(const uint32_t* __restrict__ er, con
             const bool act = t0 + u < len;
             if (REAL) {
                 const double v = act ? cod_real(tab, e0[u]) : 0.0;
-                ar += v * xv[u].x;
-                ai += v * xv[u].y;
+                ar = fma(v, xv[u].x, ar);
+                ai = fma(v, xv[u].y, ai);
             } else {
                 double2 v = cod_cplx(reinterpret_cast<const double2*>(tab), e0[u]);
                 if (!act) v = make_double2(0.0, 0.0);
-                ar += v.x * xv[u].x - v.y * xv[u].y;
-                ai += v.x * xv[u].y + v.y * xv[u].x;
+                cmac(v, xv[u], ar, ai);
             }
         }
 #pragma unroll
@@ -153,6 +162,25 @@ __device__ __forceinline__ void cod_run_sum(const uint32_t* __restrict__ er, con
         any0 = any1;
         t0 = t;
     }
+}
+
+// Epilogue of a Lanczos row: u = y / beta_j - c q from its product's row y (the diagonal added
+// here) and the previous vector's q (c = beta_j / beta_{j-1}; prev false at j = 0).
+__device__ __forceinline__ double2 lz_row(double2 y, double2 dg, double2 w, double ib, bool prev, double c, double2 q) {
+    cmac(dg, w, y.x, y.y);
+    double ur = ib * y.x, ui = ib * y.y;
+    if (prev) {
+        ur = fma(-c, q.x, ur);
+        ui = fma(-c, q.y, ui);
+    }
+    return make_double2(ur, ui);
+}
+__device__ __forceinline__ double re_dot(double2 a, double2 b) { return fma(a.x, b.x, a.y * b.y); }
+// u - a w, and its |.|^2 added to acc
+__device__ __forceinline__ double2 lz_next(double2 u, double a, double2 w, double& acc) {
+    const double2 r = make_double2(fma(-a, w.x, u.x), fma(-a, w.y, u.y));
+    acc = fma(r.x, r.x, fma(r.y, r.y, acc));
+    return r;
 }
 
 // The rest of a slice: one step at a time (about one entry a row), step t to
@@ -170,12 +198,10 @@ __device__ __forceinline__ void cod_rest_sum(const uint32_t* __restrict__ rc, co
             const double2 xv = x[rc[q]];
             if (REAL) {
                 const double v = rv[q];
-                ar += v * xv.x;
-                ai += v * xv.y;
+                ar = fma(v, xv.x, ar);
+                ai = fma(v, xv.y, ai);
             } else {
-                const double2 v = reinterpret_cast<const double2*>(rv)[q];
-                ar += v.x * xv.x - v.y * xv.y;
-                ai += v.x * xv.y + v.y * xv.x;
+                cmac(reinterpret_cast<const double2*>(rv)[q], xv, ar, ai);
             }
         }
         off += (uint32_t)__popcll(m);

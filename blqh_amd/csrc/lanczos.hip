@@ -27,6 +27,7 @@
 #include "engine.hpp"
 #include "mtstart.hpp"
 #include "ritz.hpp"
+#include "small.hpp"
 
 namespace {
 
@@ -173,9 +174,7 @@ __global__ void __launch_bounds__(kThreads) k_lz2(int64_t n, const double2* __re
     double acc = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) {
         const double2 w = W[i], x = u[i];
-        const double2 r = make_double2(x.x - a * w.x, x.y - a * w.y);
-        Wn[i] = r;
-        acc += r.x * r.x + r.y * r.y;
+        Wn[i] = lz_next(x, a, w, acc);
         for (int s = 0; s < ns; ++s) {
             const double cj = coef[(int64_t)s * ldc + j] * sc.invb[j];
             double2 p = psi[(int64_t)s * n + i];
@@ -187,15 +186,6 @@ __global__ void __launch_bounds__(kThreads) k_lz2(int64_t n, const double2* __re
     block_partial(acc, part2);
 }
 
-// Mailbox of a solve in pinned host memory: K3 of step j leaves alpha_j and beta_{j+1}
-// in entry j mod kMail and then its tag (solve number, step), which the host polls.
-// A copy and a stream synchronisation per convergence test cost 31 us of an idle GPU.
-struct alignas(64) StepMail {
-    double alpha, beta;
-    uint64_t tag;
-};
-constexpr int kMail = 64;
-
 // K3: beta[j+1] = sqrt(sum of K2's partials), invb[j+1]; one workgroup.  mail: null in a
 // replay.
 __global__ void __launch_bounds__(kThreads) k_lz3(Scal sc, int j, const double* __restrict__ part2, int npart2,
@@ -205,12 +195,7 @@ __global__ void __launch_bounds__(kThreads) k_lz3(Scal sc, int j, const double* 
         const double b = sqrt(t);
         sc.beta[j + 1] = b;
         sc.invb[j + 1] = 1.0 / b;
-        if (mail) {
-            StepMail* e = mail + (j & (kMail - 1));
-            e->alpha = sc.alpha[j];
-            e->beta = b;
-            __hip_atomic_store(&e->tag, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
+        if (mail) post_mail(mail, j, sc.alpha[j], b, tag);
     }
 }
 
@@ -841,24 +826,25 @@ __global__ void __launch_bounds__(WPB * 64) k_cod(CodView P, const double2* __re
             y.y += o.y;
         }
         const double2 w = x[row], dg = cod_diag(P, REAL, row);
-        y.x += dg.x * w.x - dg.y * w.y;
-        y.y += dg.x * w.y + dg.y * w.x;
         if (LZ) {
-            const double ib = sc.invb[j];
-            double ur = ib * y.x, ui = ib * y.y;
-            if (j > 0) {
-                const double cp = sc.beta[j] * sc.invb[j - 1];
-                const double2 q = Wp[row];
-                ur -= cp * q.x;
-                ui -= cp * q.y;
-            }
-            out[row] = make_double2(ur, ui);
-            dacc = w.x * ur + w.y * ui;
+            const double c = j > 0 ? sc.beta[j] * sc.invb[j - 1] : 0.0;
+            const double2 u = lz_row(y, dg, w, sc.invb[j], j > 0, c, j > 0 ? Wp[row] : w);
+            out[row] = u;
+            dacc = re_dot(w, u);
         } else {
+            cmac(dg, w, y.x, y.y);
             out[row] = y;
         }
     }
     if (LZ) block_partial(dacc, partials);
+}
+
+// Steps j0 .. j1 - 1 of a small matrix in one workgroup (small.hpp).
+template <bool REAL, bool RES>
+__global__ void __launch_bounds__(kSmallT) k_small(CodView P, int64_t ncod, int64_t nrest, double2* W, Scal sc, int j0,
+                                                   int j1, StepMail* mail, uint64_t tag0) {
+    extern __shared__ __align__(16) double ctab[];
+    small_steps<REAL, false, RES>(P, ncod, nrest, W, sc.alpha, sc.beta, sc.invb, j0, j1, mail, tag0, ctab);
 }
 
 // ---- launch helpers -----------------------------------------------------------
@@ -1064,6 +1050,38 @@ void cod_go(const blqh_hamil* H, const Plan& pl, const double2* x, double2* out,
     (void)attr;
     hipLaunchKernelGGL(kern, dim3(cod_grid(H, pl)), dim3(WPB * 64), cod_lds_bytes(REAL, H->cod.ntab), st,
                        cview(H->cod, H->n), x, out, Wp, sc, j, partials);
+}
+
+// A matrix whose steps one workgroup runs (k_small): up to kSmallSingle rows under the default
+// plan, whose order of sums it keeps.
+constexpr int kSmallSingle = 1024;
+constexpr int kSmallChunk = 8;  // steps a launch
+bool small_plan(const blqh_hamil* H, const Plan& pl) {
+    return pl.kind == 6 && pl.threads == 512 && pl.rows == kSmallTeam && H->cod.built && H->n <= kSmallSingle;
+}
+
+template <bool REAL, bool RES>
+void small_go(const blqh_hamil* H, size_t lds, double2* W, const Scal& sc, int j0, int j1, StepMail* mail,
+              uint64_t tag0, hipStream_t st) {
+    auto kern = k_small<REAL, RES>;
+    static const bool attr = [&] {  // once per instantiation, thread-safe
+        BLQH_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLdsMax));
+        return true;
+    }();
+    (void)attr;
+    hipLaunchKernelGGL(kern, dim3(1), dim3(kSmallT), lds, st, cview(H->cod, H->n), H->cod.ncod, H->cod.nrest, W, sc,
+                       j0, j1, mail, tag0);
+}
+
+void launch_small(const blqh_hamil* H, double2* W, const Scal& sc, int j0, int j1, StepMail* mail, uint64_t tag0,
+                  hipStream_t st) {
+    const Coded& C = H->cod;
+    const size_t all = small_lds_bytes(C.real, C.ntab, H->n, C.ncod, C.nrest), vec = small_lds_bytes(C.real, C.ntab, H->n);
+    const bool res = all <= kSmallLdsMax;
+    if (C.real && res) small_go<true, true>(H, all, W, sc, j0, j1, mail, tag0, st);
+    else if (C.real) small_go<true, false>(H, vec, W, sc, j0, j1, mail, tag0, st);
+    else if (res) small_go<false, true>(H, all, W, sc, j0, j1, mail, tag0, st);
+    else small_go<false, false>(H, vec, W, sc, j0, j1, mail, tag0, st);
 }
 
 template <bool LZ>
@@ -1755,7 +1773,8 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
     bool conv = false;
     double dE = INFINITY, resid = INFINITY;
     int done = 0, queued = 0;
-    const int ahead = steps_ahead(H->nnz, chk);
+    const bool small = store && !prof_on && small_plan(H, plan);
+    const int ahead = small ? kSmallChunk : steps_ahead(H->nnz, chk);
     hb[0] = 1.0;
     while (done < cap && !conv) {
         const int upto = std::min(cap, done + chk);
@@ -1768,9 +1787,12 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
                 hb[got + 1] = q->beta;
             }
         };
-        for (; queued < std::min(cap, upto + ahead); ++queued) {
-            read_to(std::min(upto, queued - kMail + 1));  // the entry's last tenant has been read
-            step(queued, nullptr, nullptr);
+        while (queued < std::min(cap, upto + ahead)) {
+            const int to = small ? std::min(cap, queued + kSmallChunk) : queued + 1;
+            read_to(std::min(upto, to - kMail));  // the entries' last tenants have been read
+            if (!small) step(queued, nullptr, nullptr);
+            else launch_small(H, D.Wb, sc, queued, to, hw.mail->m, tag0, st);
+            queued = to;
         }
         BLQH_HIP(hipGetLastError());
         read_to(upto);

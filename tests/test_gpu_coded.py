@@ -117,3 +117,24 @@ def test_shared_scales_against_combined(sector, G):
         one = blqh_amd.Hamiltonian.combine(h0, t, s).lanczos(seed=7, **steps)
         assert u["E0"] == pytest.approx(one["E0"], rel=1e-11, abs=1e-11)
         np.testing.assert_allclose(u["psi"], one["psi"], rtol=0, atol=1e-9)
+
+
+@pytest.mark.parametrize("case", [(2, 4, 4, 2, -1, 0, 0), (2, 6, 6, 3, -1, 1, 2), (2, 8, 8, 4, -1, 4, 4),
+                                  (2, 8, 8, -1, -1, 1, 3), (1, 18, 6, -1, -1, 3, 1), (4, 6, 6, 3, 3, 0, 1),
+                                  (2, 9, 9, -1, -1, 0, 0), (2, 9, 9, -1, -1, 2, 1), (2, 10, 10, 5, -1, 3, 2)],
+                         ids=lambda c: "_".join(map(str, c)))
+def test_one_workgroup_steps_equal_kernel_steps(case):
+    """Up to 1,024 rows one workgroup runs the steps (Krylov vectors kept); the three kernels
+    run them when the vectors are replayed.  Same order of sums: the same bits."""
+    S, nphi, nel, nu, nsu, J, K = case
+    B = blqh_amd.Basis(nphi, nel, nu, J, K, nspecies=S, nel_su=nsu)
+    par = blqh_amd.params(nphi) if S == 1 else blqh_amd.params(nphi, d=0.8, delta_sas=0.05)
+    H = blqh_amd.Hamiltonian(B, par)
+    print(f"{case} n {H.n}", flush=True)
+    for chk in (1, 5, 70):
+        steps = dict(lam=min(100, H.n), tol=0.0, res_tol=0.0, seed=3, check_every=chk)
+        a, b = H.lanczos(store_basis=1, **steps), H.lanczos(store_basis=0, **steps)
+        assert a["iterations"] == b["iterations"]
+        np.testing.assert_array_equal(a["alpha"], b["alpha"])
+        np.testing.assert_array_equal(a["beta"], b["beta"])
+        assert a["E0"] == b["E0"]
