@@ -721,8 +721,8 @@ __global__ void __launch_bounds__(64) k_tiles(const TileJob* __restrict__ jobs, 
 
 // ---- steps of small members ----------------------------------------------------
 // Steps j0 .. j1 - 1 of every live problem, a workgroup each (small.hpp).
-template <bool RES>
-__global__ void __launch_bounds__(kSmallT) k_bsmall(BState S, int j0, int j1) {
+template <bool RES, bool SH>
+__global__ void __launch_bounds__(kSmallT) k_bsmall(BState S, const double* __restrict__ tscale, int j0, int j1) {
     extern __shared__ __align__(16) double ctab[];
     const int p = blockIdx.x;
     if (!S.active[p]) return;
@@ -731,10 +731,11 @@ __global__ void __launch_bounds__(kSmallT) k_bsmall(BState S, int j0, int j1) {
            *invb = S.invb + (int64_t)p * (S.cap + 1);
     const int nsl = (int)((P.n + 63) >> 6);
     const int64_t ncod = P.c.base[nsl], nrest = P.c.rbase[nsl];
+    const double ts = SH ? tscale[p] : 1.0;
     if (P.real)
-        small_steps<true, true, RES>(P.c, ncod, nrest, P.W, alpha, beta, invb, j0, j1, nullptr, 0, ctab);
+        small_steps<true, true, RES, SH>(P.c, ncod, nrest, P.W, alpha, beta, invb, j0, j1, nullptr, 0, ctab, ts);
     else
-        small_steps<false, true, RES>(P.c, ncod, nrest, P.W, alpha, beta, invb, j0, j1, nullptr, 0, ctab);
+        small_steps<false, true, RES, SH>(P.c, ncod, nrest, P.W, alpha, beta, invb, j0, j1, nullptr, 0, ctab, ts);
 }
 
 // K2: alpha_j, W_{j+1} = u - alpha_j W_j / beta_j, |W_{j+1}|^2 partials
@@ -1060,7 +1061,7 @@ namespace {
 
 bool use_tiles(const blqh_batch* b) { return b->lpr == 64 && b->one_panel; }
 
-// Batches whose members a workgroup each steps through (k_bsmall): lanes 64, own matrices, none
+// Batches whose members a workgroup each steps through (k_bsmall): lanes 64, no member
 // above kSmallRows rows and kSmallWords entries.  lds: its dynamic LDS (0: another batch),
 // res: with every matrix in LDS.
 constexpr int64_t kSmallWords = 1 << 16;
@@ -1070,7 +1071,7 @@ struct SmallShape {
     bool res = false;
 };
 SmallShape small_shape(const blqh_batch* b) {
-    if (b->lpr != 64 || b->G) return {};
+    if (b->lpr != 64) return {};
     size_t vec = 0, all = 0;
     for (const blqh_hamil* H : b->hs) {
         if (H->n > kSmallRows || H->nnz > kSmallWords || !H->cod.built) return {};
@@ -1775,8 +1776,12 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
     const int kinds = (b->has_real ? 2 : 0) | (b->has_complex ? 1 : 0);  // which K1 launches a step has
     const SmallShape shape = timed ? SmallShape{} : small_shape(b);
     const bool small = shape.lds > 0;  // k_bsmall takes the steps
+    void (*const bsmall)(BState, const double*, int, int) = b->G ? (shape.res ? k_bsmall<true, true> : k_bsmall<false, true>)
+                                                                 : (shape.res ? k_bsmall<true, false> : k_bsmall<false, false>);
     if (small) {
-        static const bool attr = (allow_lds(k_bsmall<true>, kSmallLdsMax), allow_lds(k_bsmall<false>, kSmallLdsMax), true);
+        static const bool attr = (allow_lds(k_bsmall<true, true>, kSmallLdsMax), allow_lds(k_bsmall<false, true>, kSmallLdsMax),
+                                  allow_lds(k_bsmall<true, false>, kSmallLdsMax),
+                                  allow_lds(k_bsmall<false, false>, kSmallLdsMax), true);
         (void)attr;
     }
     if (!timed && !small && (b->g_chk != chk || b->g_lpr != b->lpr || b->g_cap != cap || b->g_kinds != kinds ||
@@ -1843,7 +1848,7 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
     auto enqueue = [&](int first) {
         if (small)
             for (int j = first; j < std::min(cap, first + stride); j += kSmallLaunch)
-                hipLaunchKernelGGL(shape.res ? k_bsmall<true> : k_bsmall<false>, dim3(P), dim3(kSmallT), shape.lds, st, S, j,
+                hipLaunchKernelGGL(bsmall, dim3(P), dim3(kSmallT), shape.lds, st, S, b->dtscale.get(), j,
                                    std::min({cap, first + stride, j + kSmallLaunch}));
         else if (timed) chunk(true, first);
         else BLQH_HIP(hipGraphLaunch(gexec, st));

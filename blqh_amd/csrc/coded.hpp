@@ -109,11 +109,12 @@ __device__ __forceinline__ void cod_stage(const double* __restrict__ tab, int nt
 // steps each) are dealt to NP wavefronts, this one taking those with g mod NP
 // == par.  The words of the next group are loaded before the x gathers of the
 // current one, so a wavefront always has loads in flight.
-// KEEP: the words are read again soon (small.hpp), leave them in the caches.
-template <bool REAL, int NP, int U, bool KEEP = false>
+// KEEP: the words are read again soon (small.hpp), leave them in the caches.  SH: values of
+// words with the tunnelling flag are scaled by ts (columns have 15 bits).
+template <bool REAL, int NP, int U, bool KEEP = false, bool SH = false>
 __device__ __forceinline__ void cod_run_sum(const uint32_t* __restrict__ er, const double* tab,
                                             const double2* __restrict__ xp, uint32_t len, int par, double& ar,
-                                            double& ai) {
+                                            double& ai, double ts = 1.0) {
     uint32_t off = 0;
     auto issue = [&](uint32_t t, uint32_t* e, bool& any) {
         uint64_t m[U];
@@ -143,17 +144,19 @@ __device__ __forceinline__ void cod_run_sum(const uint32_t* __restrict__ er, con
         issue(t, e1, any1);
         double2 xv[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) xv[u] = xp[e0[u] & 0xffffu];
+        for (int u = 0; u < U; ++u) xv[u] = xp[e0[u] & (SH ? kCodTun - 1 : 0xffffu)];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const bool act = t0 + u < len;
             if (REAL) {
-                const double v = act ? cod_real(tab, e0[u]) : 0.0;
+                double v = act ? cod_real(tab, e0[u]) : 0.0;
+                if (SH && (e0[u] & kCodTun)) v *= ts;
                 ar = fma(v, xv[u].x, ar);
                 ai = fma(v, xv[u].y, ai);
             } else {
                 double2 v = cod_cplx(reinterpret_cast<const double2*>(tab), e0[u]);
                 if (!act) v = make_double2(0.0, 0.0);
+                if (SH && (e0[u] & kCodTun)) v = make_double2(ts * v.x, ts * v.y);
                 cmac(v, xv[u], ar, ai);
             }
         }
@@ -185,23 +188,27 @@ __device__ __forceinline__ double2 lz_next(double2 u, double a, double2 w, doubl
 
 // The rest of a slice: one step at a time (about one entry a row), step t to
 // the wavefront t mod NP.
-template <bool REAL, int NP>
+template <bool REAL, int NP, bool SH = false>
 __device__ __forceinline__ void cod_rest_sum(const uint32_t* __restrict__ rc, const double* __restrict__ rv,
                                              const double2* __restrict__ x, uint32_t len, int par, double& ar,
-                                             double& ai) {
+                                             double& ai, double ts = 1.0) {
     uint32_t off = 0;
     for (uint32_t t = 0;; ++t) {
         const uint64_t m = __ballot(t < len);
         if (m == 0) break;
         if ((NP == 1 || (int)(t % NP) == par) && t < len) {
             const uint32_t q = off + lanes_below(m);
-            const double2 xv = x[rc[q]];
+            const uint32_t c = rc[q];
+            const double2 xv = x[SH ? c & (kCodTun - 1) : c];
+            const double s = SH && (c & kCodTun) ? ts : 1.0;
             if (REAL) {
-                const double v = rv[q];
+                const double v = SH ? s * rv[q] : rv[q];
                 ar = fma(v, xv.x, ar);
                 ai = fma(v, xv.y, ai);
             } else {
-                cmac(reinterpret_cast<const double2*>(rv)[q], xv, ar, ai);
+                double2 v = reinterpret_cast<const double2*>(rv)[q];
+                if (SH) v = make_double2(s * v.x, s * v.y);
+                cmac(v, xv, ar, ai);
             }
         }
         off += (uint32_t)__popcll(m);

@@ -844,7 +844,7 @@ template <bool REAL, bool RES>
 __global__ void __launch_bounds__(kSmallT) k_small(CodView P, int64_t ncod, int64_t nrest, double2* W, Scal sc, int j0,
                                                    int j1, StepMail* mail, uint64_t tag0) {
     extern __shared__ __align__(16) double ctab[];
-    small_steps<REAL, false, RES>(P, ncod, nrest, W, sc.alpha, sc.beta, sc.invb, j0, j1, mail, tag0, ctab);
+    small_steps<REAL, false, RES, false>(P, ncod, nrest, W, sc.alpha, sc.beta, sc.invb, j0, j1, mail, tag0, ctab, 1.0);
 }
 
 // ---- launch helpers -----------------------------------------------------------

@@ -77,11 +77,12 @@ __device__ __forceinline__ double wave_total(double v) {
 // Steps j0 .. j1 - 1 of one problem by the whole workgroup (kSmallT threads): W holds the
 // vectors, W_j at j n, up to W_j0; alpha[j], beta[j + 1] and invb[j + 1] are written, and to
 // mail, if any, with tags tag0 | j + 1.  ZERO: 1/0 is 0 (the batch's convention).  RES: the
-// matrix fits in LDS beside the vectors and is staged there.
-template <bool REAL, bool ZERO, bool RES>
+// matrix fits in LDS beside the vectors and is staged there.  SH: a shared-scale template,
+// flagged entries scaled by ts.
+template <bool REAL, bool ZERO, bool RES, bool SH>
 __device__ __forceinline__ void small_steps(const CodView& P, int64_t ncod, int64_t nrest, double2* W, double* alpha,
                                             double* beta, double* invb, int j0, int j1, StepMail* mail, uint64_t tag0,
-                                            double* lds) {
+                                            double* lds, double ts) {
     __shared__ double part[kSmallSlices], nrm[kSmallSlices];  // a slice's shares of the two sums
     __shared__ int32_t sbase[kSmallSlices], srbase[kSmallSlices];
     __shared__ double sal[kSmallLaunch], sbe[kSmallLaunch];
@@ -134,9 +135,10 @@ __device__ __forceinline__ void small_steps(const CodView& P, int64_t ncod, int6
             double2 y = make_double2(0.0, 0.0);
             if (sl < nsl) {  // uniform over the wavefront
                 const uint32_t ln = slen[sl * 64 + lane];
-                cod_run_sum<REAL, kSmallTeam, 8, true>(ent + sbase[sl], lds, xs, ln & 0xffff, par, y.x, y.y);
+                cod_run_sum<REAL, kSmallTeam, 8, true, SH>(ent + sbase[sl], lds, xs, ln & 0xffff, par, y.x, y.y, ts);
                 const int q0 = srbase[sl];
-                cod_rest_sum<REAL, kSmallTeam>(rcol + q0, rval + q0 * (REAL ? 1 : 2), xs, ln >> 16, par, y.x, y.y);
+                cod_rest_sum<REAL, kSmallTeam, SH>(rcol + q0, rval + q0 * (REAL ? 1 : 2), xs, ln >> 16, par, y.x, y.y,
+                                                   ts);
             }
             red[tid] = y;
             __syncthreads();
