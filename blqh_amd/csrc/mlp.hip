@@ -17,9 +17,8 @@
 //     L = mean_s [ (o0_s - log|psi_s|)^2 + softplus(o1_s) - sign01_s o1_s ]
 // weighs configurations by their weight in the ground state.
 // Step kernels: k_sample (draw the minibatch), k_fwd_bwd (a workgroup per tile
-// of 64 states: forward, loss, back-propagation and the tile's gradient sums,
-// all in LDS), k_grad_sum (per parameter, tiles summed in order:
-// deterministic), k_adam.
+// of 16 states: forward, loss, back-propagation and gradient sums), k_grad_sum (per
+// parameter, workgroups summed in order: deterministic), k_adam.
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -185,97 +184,222 @@ __global__ void __launch_bounds__(kT) k_sample(int B, uint64_t key, int nsets, c
     S.ys[s] = ys[lo];
 }
 
-// Forward, loss, back-propagation and the tile's parameter-gradient sums
-// (part[tile][param], summed over tiles by k_grad_sum in tile order).
+// value of lane i of the wavefront, the same for all of it
+__device__ __forceinline__ float lane_value(float v, int i) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), i));
+}
+
+// a word that is the same on every lane, in scalar registers
+__device__ __forceinline__ uint64_t scalar(uint64_t w) {
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(w >> 32)) << 32 |
+           (uint32_t)__builtin_amdgcn_readfirstlane((int)w);
+}
+
+// Forward, loss, back-propagation and the parameter-gradient sums of the workgroup's tiles
+// of kSt states (part[workgroup][param], summed by k_grad_sum in order).
+//
+// A wavefront takes kSw states, lane = unit: activations and deltas stay in registers and
+// reach the other units by lane reads, so a weight read serves kSw states and the LDS
+// holds only W2 (padded: the backward pass reads it across) and what the gradient sums
+// share.  Bound by latency: a minibatch of 4,096 states is 256 tiles, one for each CU;
+// with tiles of 64 states, every product through LDS and a quarter of the CUs busy the
+// forward and backward of that took 66 us, 46 now, and the sums 16, 4 now.  Past kMaxWgs tiles a workgroup takes
+// several and keeps their sums in registers.
+constexpr int kSt = 16, kSw = kSt / (kT / 64), kMaxWgs = 512;
+constexpr int kR1 = (kMaxIn + kT / 64 - 1) / (kT / 64);  // rows of W1 a wavefront sums
+
 __global__ void __launch_bounds__(kT) k_fwd_bwd(Dims D, const float* __restrict__ P, int B, Samples S,
                                                 float* __restrict__ part) {
-    __shared__ Lds L;
-    __shared__ float G[kTile * 2];  // dL/do per state
-    stage_params(D, P, L);
-    const int t0 = blockIdx.x * kTile;
-    const int nt = B - t0 < kTile ? B - t0 : kTile;
-    __syncthreads();
-    tile_forward(D, L, S.word + t0, S.pd + t0, S.ps + t0, nt);
-    // loss and output deltas (states beyond nt get zero deltas)
-    if (threadIdx.x < kTile) {
-        const int s = threadIdx.x;
-        float g0 = 0.0f, g1 = 0.0f;
-        if (s < nt) {
-            const float o0 = L.O[2 * s], o1 = L.O[2 * s + 1];
-            const float ea = o0 - S.ya[t0 + s];
-            const float y = S.ys[t0 + s];
-            const float sp = o1 > 0.0f ? o1 + log1pf(expf(-o1)) : log1pf(expf(o1));  // softplus
-            S.loss[t0 + s] = ea * ea + sp - y * o1;
-            g0 = 2.0f * ea;
-            g1 = 1.0f / (1.0f + expf(-o1)) - y;
+    __shared__ float W2[kH * kLd], H1[kSt * kH], D2[kSt * kH], D1[kSt * kH];
+    __shared__ uint64_t sw[kSt];
+    __shared__ float sd[kSt], ss[kSt], sa[kSt], sy[kSt];
+    __shared__ float red[kT / 64][4][kH + 1];  // the wavefronts' sums of W3's columns and the biases
+    const int j = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int ntiles = (B + kSt - 1) / kSt;
+    for (int i = threadIdx.x; i < kH * kH; i += kT) W2[(i / kH) * kLd + i % kH] = P[D.oW2 + i];
+    const float b1 = P[D.ob1 + j], b2 = P[D.ob2 + j], w30 = P[D.oW3 + 2 * j], w31 = P[D.oW3 + 2 * j + 1];
+    const float b30 = P[D.ob3], b31 = P[D.ob3 + 1];
+    float g2[kH / 4], g1[kR1];  // sums of rows wv kH/4 + i of W2, wv + 4 i of W1
+    float g30 = 0.0f, g31 = 0.0f, gb1 = 0.0f, gb2 = 0.0f, gb30 = 0.0f, gb31 = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kH / 4; ++i) g2[i] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kR1; ++i) g1[i] = 0.0f;
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const int t0 = tile * kSt;
+        __syncthreads();  // W2 staged / the previous tile's sums done
+        if (threadIdx.x < kSt) {
+            const int s = threadIdx.x;
+            const bool on = t0 + s < B;
+            sw[s] = on ? S.word[t0 + s] : 0;
+            sd[s] = on ? S.pd[t0 + s] * (1.0f / 3.0f) : 0.0f;
+            ss[s] = on ? S.ps[t0 + s] * 10.0f : 0.0f;
+            sa[s] = on ? S.ya[t0 + s] : 0.0f;
+            sy[s] = on ? S.ys[t0 + s] : 0.0f;
         }
-        G[2 * s] = g0;
-        G[2 * s + 1] = g1;
-    }
-    __syncthreads();
-    const int j = threadIdx.x % kH;
-    // delta of layer 2: D2 = (1 - H2^2) (W3 G)
-    for (int s = threadIdx.x / kH; s < kTile; s += kT / kH) {
-        const float h = L.H2[s * kLd + j];
-        L.D2[s * kLd + j] = (1.0f - h * h) * (L.W3[2 * j] * G[2 * s] + L.W3[2 * j + 1] * G[2 * s + 1]);
-    }
-    __syncthreads();
-    float* out = part + (int64_t)blockIdx.x * D.n;
-    // W3, b3 (H2 is read here for the last time)
-    if (threadIdx.x < 2 * kH + 2) {
-        const int p = threadIdx.x;
-        float acc = 0.0f;
-        if (p < 2 * kH) {
-            const int i = p / 2, c = p % 2;
-            for (int s = 0; s < kTile; ++s) acc += L.H2[s * kLd + i] * G[2 * s + c];
-        } else {
-            for (int s = 0; s < kTile; ++s) acc += G[2 * s + p - 2 * kH];
+        __syncthreads();
+        uint64_t w[kSw];
+        float h1[kSw], h2[kSw], z[kSw];
+#pragma unroll
+        for (int q = 0; q < kSw; ++q) {
+            w[q] = scalar(sw[wv * kSw + q]);
+            z[q] = b1;
         }
-        out[D.oW3 + p] = acc;  // oW3 .. ob3+1 are contiguous
-    }
-    __syncthreads();
-    // delta of layer 1 into the H2 slot: D1 = (1 - H1^2) (W2 D2)
-    for (int s = threadIdx.x / kH; s < kTile; s += kT / kH) {
-        float acc = 0.0f;
 #pragma unroll 8
-        for (int i = 0; i < kH; ++i) acc += L.W2[j * kLd + i] * L.D2[s * kLd + i];
-        const float h = L.H1[s * kLd + j];
-        L.H2[s * kLd + j] = (1.0f - h * h) * acc;
+        for (int k = 0; k < D.nbits; ++k) {
+            const float wt = P[D.oW1 + k * kH + j];
+#pragma unroll
+            for (int q = 0; q < kSw; ++q) z[q] += (w[q] >> k & 1ull) ? wt : -wt;
+        }
+        {
+            const float wd = P[D.oW1 + D.nbits * kH + j], ws = P[D.oW1 + (D.nbits + 1) * kH + j];
+#pragma unroll
+            for (int q = 0; q < kSw; ++q) {
+                z[q] += sd[wv * kSw + q] * wd;
+                z[q] += ss[wv * kSw + q] * ws;
+                h1[q] = tanhf(z[q]);
+                z[q] = b2;
+            }
+        }
+#pragma unroll 16
+        for (int i = 0; i < kH; ++i) {
+            const float wt = W2[i * kLd + j];
+#pragma unroll
+            for (int q = 0; q < kSw; ++q) z[q] += lane_value(h1[q], i) * wt;
+        }
+        float d2[kSw], d1[kSw], o0 = 0.0f, o1 = 0.0f;
+#pragma unroll
+        for (int q = 0; q < kSw; ++q) {
+            h2[q] = tanhf(z[q]);
+            float a0 = h2[q] * w30, a1 = h2[q] * w31;
+            for (int o = 32; o > 0; o >>= 1) {
+                a0 += __shfl_xor(a0, o, 64);
+                a1 += __shfl_xor(a1, o, 64);
+            }
+            if (j == q) {
+                o0 = a0 + b30;
+                o1 = a1 + b31;
+            }
+        }
+        // loss and dL/do of the wavefront's states, one a lane (past B: none)
+        float e0 = 0.0f, e1 = 0.0f;
+        {
+            const int s = wv * kSw + (j & (kSw - 1));
+            const float ea = o0 - sa[s], y = sy[s], ex = expf(o1 > 0.0f ? -o1 : o1);
+            const float sp = (o1 > 0.0f ? o1 : 0.0f) + log1pf(ex);  // softplus
+            if (j < kSw && t0 + s < B) {
+                S.loss[t0 + s] = ea * ea + sp - y * o1;
+                e0 = 2.0f * ea;
+                e1 = 1.0f / (1.0f + expf(-o1)) - y;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < kSw; ++q) {
+            const float f0 = lane_value(e0, q), f1 = lane_value(e1, q);
+            d2[q] = (1.0f - h2[q] * h2[q]) * (w30 * f0 + w31 * f1);
+            g30 += h2[q] * f0;
+            g31 += h2[q] * f1;
+            gb30 += f0;
+            gb31 += f1;
+            gb2 += d2[q];
+            d1[q] = 0.0f;
+        }
+#pragma unroll 16
+        for (int i = 0; i < kH; ++i) {
+            const float wt = W2[j * kLd + i];
+#pragma unroll
+            for (int q = 0; q < kSw; ++q) d1[q] += wt * lane_value(d2[q], i);
+        }
+#pragma unroll
+        for (int q = 0; q < kSw; ++q) {
+            const int s = wv * kSw + q;
+            d1[q] *= 1.0f - h1[q] * h1[q];
+            gb1 += d1[q];
+            H1[s * kH + j] = h1[q];
+            D2[s * kH + j] = d2[q];
+            D1[s * kH + j] = d1[q];
+        }
+        __syncthreads();
+        // W2: sum_s H1[s][i] D2[s][j];  W1: sum_s x[s][k] D1[s][j]
+        for (int s = 0; s < kSt; ++s) {
+            const float e2 = D2[s * kH + j], e1 = D1[s * kH + j];
+            const uint64_t word = scalar(sw[s]);
+#pragma unroll
+            for (int i = 0; i < kH / 4; ++i) g2[i] += H1[s * kH + wv * (kH / 4) + i] * e2;
+#pragma unroll
+            for (int i = 0; i < kR1; ++i) {
+                const int k = wv + 4 * i;
+                if (k < D.nbits) g1[i] += (word >> k & 1ull) ? e1 : -e1;
+                else if (k == D.nbits) g1[i] += sd[s] * e1;
+                else if (k == D.nbits + 1) g1[i] += ss[s] * e1;
+            }
+        }
+    }
+    float* out = part + (int64_t)blockIdx.x * D.n;
+#pragma unroll
+    for (int i = 0; i < kH / 4; ++i) out[D.oW2 + (wv * (kH / 4) + i) * kH + j] = g2[i];
+#pragma unroll
+    for (int i = 0; i < kR1; ++i)
+        if (wv + 4 * i < D.nin) out[D.oW1 + (wv + 4 * i) * kH + j] = g1[i];
+    red[wv][0][j] = g30;
+    red[wv][1][j] = g31;
+    red[wv][2][j] = gb1;
+    red[wv][3][j] = gb2;
+    if (j == 0) {
+        red[wv][0][kH] = gb30;
+        red[wv][1][kH] = gb31;
     }
     __syncthreads();
-    // W2, b2: sum_s H1[s][i] D2[s][j]
-    for (int p = threadIdx.x; p < kH * kH + kH; p += kT) {
-        float acc = 0.0f;
-        if (p < kH * kH) {
-            const int i = p / kH, jj = p % kH;
-            for (int s = 0; s < kTile; ++s) acc += L.H1[s * kLd + i] * L.D2[s * kLd + jj];
-        } else {
-            for (int s = 0; s < kTile; ++s) acc += L.D2[s * kLd + p - kH * kH];
+    if (wv < 4) {  // a wavefront per kind, the wavefronts' shares in order
+        float t = 0.0f;
+        for (int q = 0; q < kT / 64; ++q) t += red[q][wv][j];
+        out[wv < 2 ? D.oW3 + 2 * j + wv : (wv == 2 ? D.ob1 : D.ob2) + j] = t;
+        if (j == 0 && wv < 2) {
+            t = 0.0f;
+            for (int q = 0; q < kT / 64; ++q) t += red[q][wv][kH];
+            out[D.ob3 + wv] = t;
         }
-        out[D.oW2 + p] = acc;  // oW2 .. ob2+63 are contiguous
-    }
-    // W1, b1: sum_s X[s][k] D1[s][j]
-    const int ldx = D.nin + 1;
-    for (int p = threadIdx.x; p < D.nin * kH + kH; p += kT) {
-        float acc = 0.0f;
-        if (p < D.nin * kH) {
-            const int k = p / kH, jj = p % kH;
-            for (int s = 0; s < kTile; ++s) acc += L.X[s * ldx + k] * L.H2[s * kLd + jj];
-        } else {
-            for (int s = 0; s < kTile; ++s) acc += L.H2[s * kLd + p - D.nin * kH];
-        }
-        out[D.oW1 + p] = acc;  // oW1 .. ob1+63 are contiguous
     }
 }
 
-// grad = (sum over tiles of part) / B, tiles in order
-__global__ void __launch_bounds__(kT) k_grad_sum(int n, int ntiles, int B, const float* __restrict__ part,
-                                                 float* __restrict__ grad) {
-    const int p = blockIdx.x * kT + threadIdx.x;
-    if (p >= n) return;
+// grad = (sum over the workgroups of k_fwd_bwd) / B: 64 parameters a workgroup, its 16
+// wavefronts sum a sixteenth of the partials each, added in order.  The last workgroup
+// sums the losses (fixed order), if wanted.
+constexpr int kGs = 1024;
+__device__ void loss_total(int B, const float* __restrict__ loss, double* sh, int nt, double* out) {
+    double a = 0.0;
+    for (int s = threadIdx.x; s < B; s += nt) a += loss[s];
+    sh[threadIdx.x] = a;
+    __syncthreads();
+    for (int o = nt / 2; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *out = sh[0] / B;
+}
+__global__ void __launch_bounds__(kGs) k_grad_sum(int n, int nparts, int B, const float* __restrict__ part,
+                                                  float* __restrict__ grad, const float* __restrict__ loss,
+                                                  double* __restrict__ out) {
+    __shared__ double sh[kGs];
+    if ((int)blockIdx.x == (n + 63) / 64) {
+        loss_total(B, loss, sh, kGs, out);
+        return;
+    }
+    float* f = reinterpret_cast<float*>(sh);
+    const int p = blockIdx.x * 64 + (threadIdx.x & 63), wv = threadIdx.x >> 6, per = (nparts + 15) / 16;
+    const int t1 = (wv + 1) * per < nparts ? (wv + 1) * per : nparts;
     float acc = 0.0f;
-    for (int t = 0; t < ntiles; ++t) acc += part[(int64_t)t * n + p];
-    grad[p] = acc / (float)B;
+    if (p < n) {
+#pragma unroll 8
+        for (int t = wv * per; t < t1; ++t) acc += part[(int64_t)t * n + p];
+    }
+    f[threadIdx.x] = acc;
+    __syncthreads();
+    if (wv == 0 && p < n) {
+        float t = 0.0f;
+        for (int q = 0; q < 16; ++q) t += f[q * 64 + threadIdx.x];
+        grad[p] = t / (float)B;
+    }
 }
 
 __global__ void __launch_bounds__(kT) k_adam(int n, float* __restrict__ P, const float* __restrict__ g,
@@ -292,18 +416,25 @@ __global__ void __launch_bounds__(kT) k_adam(int n, float* __restrict__ P, const
     P[i] -= lr * (mi / (1.0f - b1t)) / (sqrtf(vi / (1.0f - b2t)) + eps);
 }
 
-// sum of the minibatch losses (one block, fixed order)
-__global__ void __launch_bounds__(kT) k_loss_sum(int B, const float* __restrict__ loss, double* __restrict__ out) {
-    __shared__ double sh[kT];
-    double a = 0.0;
-    for (int s = threadIdx.x; s < B; s += kT) a += loss[s];
-    sh[threadIdx.x] = a;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int i = 0; i < kT; ++i) t += sh[i];
-        *out = t / B;
-    }
+// mean of the minibatch losses alone
+__global__ void __launch_bounds__(kGs) k_loss_sum(int B, const float* __restrict__ loss, double* __restrict__ out) {
+    __shared__ double sh[kGs];
+    loss_total(B, loss, sh, kGs, out);
+}
+
+int fb_grid(int B) { return (int)std::min<int64_t>(ceil_div(B, kSt), kMaxWgs); }
+
+void launch_grad(const Dims& D, const float* P, int B, const Samples& S, float* part, float* grad, double* loss,
+                 hipStream_t st) {
+    hipLaunchKernelGGL(k_fwd_bwd, dim3(fb_grid(B)), dim3(kT), 0, st, D, P, B, S, part);
+    hipLaunchKernelGGL(k_grad_sum, dim3((D.n + 63) / 64 + (loss ? 1 : 0)), dim3(kGs), 0, st, D.n, fb_grid(B), B, part,
+                       grad, S.loss, loss);
+}
+
+// B samples in one block at p: words, then pd, ps, ya, ys
+Samples packed(char* p, int B, float* loss) {
+    float* f = (float*)(p + (size_t)B * 8);
+    return Samples{(uint64_t*)p, f, f + B, f + 2 * (size_t)B, f + 3 * (size_t)B, loss};
 }
 
 struct Buffers {
@@ -318,10 +449,34 @@ struct Buffers {
         ya.alloc(B);
         ys.alloc(B);
         loss.alloc(B);
-        part.alloc((size_t)ceil_div(B, kTile) * nparams);
+        part.alloc((size_t)fb_grid(B) * nparams);
         cap = B;
     }
     Samples view() { return Samples{word.get(), pd.get(), ps.get(), ya.get(), ys.get(), loss.get()}; }
+};
+
+// Pinned host memory of a network's explicit minibatches of up to kPinned states: samples,
+// gradient, loss (grow-only, freed with the network).
+constexpr int kPinned = 1 << 16;
+struct Pinned {
+    char* p = nullptr;
+    int cap = 0;
+    float* grad = nullptr;
+    double* lsum = nullptr;
+    ~Pinned() {
+        if (p) (void)hipHostFree(p);
+    }
+    void ensure(int B, int nparams) {
+        if (B <= cap) return;
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        cap = 0;
+        const int c = std::min(kPinned, std::max(B, 4096));
+        BLQH_HIP(hipHostMalloc((void**)&p, 64 + (size_t)c * 24 + (size_t)nparams * 4, hipHostMallocDefault));
+        cap = c;
+        lsum = (double*)p;
+        grad = (float*)(p + 64 + (size_t)c * 24);
+    }
 };
 
 }  // namespace
@@ -332,6 +487,7 @@ struct blqh_mlp {
     int64_t adam_t = 0;
     Buffers buf;
     DevBuf<double> lsum;
+    Pinned pin;
 };
 
 blqh_mlp* blqh_mlp_create_impl(int nbits, uint32_t seed) {
@@ -390,18 +546,32 @@ void blqh_mlp_loss_grad_impl(blqh_mlp* M, int64_t ns, const uint64_t* words, con
     const int B = (int)ns;
     M->buf.ensure(B, M->D.n);
     Samples S = M->buf.view();
-    BLQH_HIP(hipMemcpyAsync(S.word, words, B * 8, hipMemcpyHostToDevice, st));
-    BLQH_HIP(hipMemcpyAsync(S.pd, pd, B * 4, hipMemcpyHostToDevice, st));
-    BLQH_HIP(hipMemcpyAsync(S.ps, ps, B * 4, hipMemcpyHostToDevice, st));
-    BLQH_HIP(hipMemcpyAsync(S.ya, ya, B * 4, hipMemcpyHostToDevice, st));
-    BLQH_HIP(hipMemcpyAsync(S.ys, ys, B * 4, hipMemcpyHostToDevice, st));
-    const int nt = (int)ceil_div(B, kTile);
-    hipLaunchKernelGGL(k_fwd_bwd, dim3(nt), dim3(kT), 0, st, M->D, M->P.get(), B, S, M->buf.part.get());
-    hipLaunchKernelGGL(k_grad_sum, dim3(ceil_div(M->D.n, kT)), dim3(kT), 0, st, M->D.n, nt, B, M->buf.part.get(),
-                       M->g.get());
-    hipLaunchKernelGGL(k_loss_sum, dim3(1), dim3(kT), 0, st, B, S.loss, M->lsum.get());
+    const int n = M->D.n;
+    if (B <= kPinned) {
+        // the kernels read the samples, each once, from pinned host memory and leave gradient
+        // and loss there: seven copies of 8 us each otherwise (one copy of all: 6 us more)
+        M->pin.ensure(B, n);
+        const Samples H = packed(M->pin.p + 64, B, S.loss);
+        std::memcpy(H.word, words, (size_t)B * 8);
+        std::memcpy(H.pd, pd, (size_t)B * 4);
+        std::memcpy(H.ps, ps, (size_t)B * 4);
+        std::memcpy(H.ya, ya, (size_t)B * 4);
+        std::memcpy(H.ys, ys, (size_t)B * 4);
+        launch_grad(M->D, M->P.get(), B, H, M->buf.part.get(), M->pin.grad, M->pin.lsum, st);
+        BLQH_HIP(hipGetLastError());
+        BLQH_HIP(hipStreamSynchronize(st));
+        if (grad) std::memcpy(grad, M->pin.grad, (size_t)n * 4);
+        if (loss) *loss = *M->pin.lsum;
+        return;
+    }
+    BLQH_HIP(hipMemcpyAsync(S.word, words, (size_t)B * 8, hipMemcpyHostToDevice, st));
+    BLQH_HIP(hipMemcpyAsync(S.pd, pd, (size_t)B * 4, hipMemcpyHostToDevice, st));
+    BLQH_HIP(hipMemcpyAsync(S.ps, ps, (size_t)B * 4, hipMemcpyHostToDevice, st));
+    BLQH_HIP(hipMemcpyAsync(S.ya, ya, (size_t)B * 4, hipMemcpyHostToDevice, st));
+    BLQH_HIP(hipMemcpyAsync(S.ys, ys, (size_t)B * 4, hipMemcpyHostToDevice, st));
+    launch_grad(M->D, M->P.get(), B, S, M->buf.part.get(), M->g.get(), M->lsum.get(), st);
     BLQH_HIP(hipGetLastError());
-    if (grad) BLQH_HIP(hipMemcpyAsync(grad, M->g.get(), M->D.n * 4, hipMemcpyDeviceToHost, st));
+    if (grad) BLQH_HIP(hipMemcpyAsync(grad, M->g.get(), n * 4, hipMemcpyDeviceToHost, st));
     double l = 0;
     BLQH_HIP(hipMemcpyAsync(&l, M->lsum.get(), 8, hipMemcpyDeviceToHost, st));
     BLQH_HIP(hipStreamSynchronize(st));
@@ -469,11 +639,11 @@ void blqh_mlp_train_impl(blqh_mlp* M, int nsets, const blqh_basis* const* bases,
     const int B = o.batch;
     M->buf.ensure(B, M->D.n);
     Samples S = M->buf.view();
-    const int gb = (int)ceil_div(B, kT), gp = (int)ceil_div(M->D.n, kT), ntile = (int)ceil_div(B, kTile);
+    const int gb = (int)ceil_div(B, kT), gp = (int)ceil_div(M->D.n, kT);
     const double b1 = 0.9, b2 = 0.999;
     std::vector<double> losses;
     auto record = [&]() {
-        hipLaunchKernelGGL(k_loss_sum, dim3(1), dim3(kT), 0, st, B, S.loss, M->lsum.get());
+        hipLaunchKernelGGL(k_loss_sum, dim3(1), dim3(kGs), 0, st, B, S.loss, M->lsum.get());
         double l = 0;
         BLQH_HIP(hipMemcpyAsync(&l, M->lsum.get(), 8, hipMemcpyDeviceToHost, st));
         BLQH_HIP(hipStreamSynchronize(st));
@@ -485,13 +655,12 @@ void blqh_mlp_train_impl(blqh_mlp* M, int nsets, const blqh_basis* const* bases,
         const uint64_t key = ((uint64_t)o.seed << 32) ^ (uint64_t)(M->adam_t + 1) * 0x9E3779B97F4A7C15ull;
         hipLaunchKernelGGL(k_sample, dim3(gb), dim3(kT), 0, st, B, key, nsets, dset0.get(), dcdf.get(),
                            dwords.get(), dya.get(), dys.get(), dsd.get(), dss.get(), S);
-        hipLaunchKernelGGL(k_fwd_bwd, dim3(ntile), dim3(kT), 0, st, M->D, M->P.get(), B, S, M->buf.part.get());
+        launch_grad(M->D, M->P.get(), B, S, M->buf.part.get(), M->g.get(), nullptr, st);
         if (step == 0) record();
         if (step >= o.steps - tail) {
             record();
             last += losses.back();
         }
-        hipLaunchKernelGGL(k_grad_sum, dim3(gp), dim3(kT), 0, st, M->D.n, ntile, B, M->buf.part.get(), M->g.get());
         ++M->adam_t;
         const float lr = o.lr * (o.lr_final > 0 ? (float)std::pow(o.lr_final / o.lr, (double)step / std::max(1, o.steps - 1)) : 1.0f);
         hipLaunchKernelGGL(k_adam, dim3(gp), dim3(kT), 0, st, M->D.n, M->P.get(), M->g.get(), M->m.get(),

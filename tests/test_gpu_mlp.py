@@ -39,6 +39,22 @@ def test_loss_and_gradient_match_oracle(nbits, n):
     np.testing.assert_allclose(g, gr, rtol=0, atol=2e-5 * np.abs(gr).max())
 
 
+@pytest.mark.parametrize("nbits,n", [(1, 1), (2, 15), (28, 16), (33, 17), (64, 100), (62, 8192), (12, 8193),
+                                     (28, 65536), (28, 65537)])
+def test_loss_and_gradient_at_tile_edges(nbits, n):
+    """One state, tiles of 16 full and not, one tile a workgroup and several, the widest
+    network, the largest minibatch read from host memory and the first that is copied."""
+    print(f"nbits {nbits} samples {n}", flush=True)
+    net = blqh_amd.Mlp(nbits, seed=4)
+    theta = net.params
+    data = _data(min(nbits, 63), n, 6)
+    L, g = net.loss_grad(*data)
+    Lr, gr = M.loss_grad(theta.astype(np.float64), nbits, *[np.asarray(a, np.float64) if a.dtype != np.uint64 else a
+                                                             for a in data])
+    assert L == pytest.approx(Lr, rel=1e-5)
+    np.testing.assert_allclose(g, gr, rtol=0, atol=2e-5 * np.abs(gr).max())
+
+
 def test_inference_matches_oracle():
     B = blqh_amd.Basis(8, 8, -1, 0, 0)
     net = blqh_amd.Mlp(16, seed=9)
