@@ -353,6 +353,7 @@ constexpr int kUnit = 16;              // slices of a unit, one per wavefront
 constexpr int kBTx = kUnit * 64;
 constexpr int kUnitItems = kUnit * 64 / kItemRows;
 constexpr size_t kLdsMax = 160 * 1024 - 1024;  // dynamic LDS; the rest is k_b1x's static part
+constexpr size_t kLdsHalf = 79 * 1024;
 constexpr int kTileMax = 8192;         // columns of a tile (13 bits)
 
 // An element of k_b1x's work list names an owner (a problem; SH: a group) and, counted
@@ -1166,7 +1167,9 @@ void make_tiles(blqh_batch* b) {
         b->tiles[o] = ColTiles{jobs[o].tw, jobs[o].nt, b->tent.get(), b->tgoff.get() + jobs[o].goff0};
     int64_t units = 0;
     for (int o = 0; o < no; ++o) units += ceil_div(jobs[o].c.n, (int64_t)kUnit * 64);
-    const int wpc = b->x_bytes <= 79 * 1024 ? 2 : 1;  // workgroups of 1024 threads that share a CU's LDS
+    const int wpc = b->x_bytes <= kLdsHalf ? 2 : 1;  // workgroups of 1024 threads that share a CU's LDS
+    // one of two sizes, so that the next point's tables leave the captured launches as they are
+    b->x_bytes = wpc == 2 ? kLdsHalf : kLdsMax;
     b->x_grid = (int)(8 * ceil_div(std::min<int64_t>(units, (int64_t)runtime().num_cus * wpc), 8));
     b->tiles_ok = true;
 }
@@ -1220,6 +1223,9 @@ void refresh_probs(blqh_batch* b) {
         if (!b->tiles_ok) make_tiles(b);
         for (size_t p = 0; p < b->hs.size(); ++p) b->h_probs[p].t = b->tiles[p / (b->G ? b->G : 1)];
     }
+    // one of three sizes (as x_bytes)
+    const size_t small = cod_lds_bytes(true, kCodReal), half = cod_lds_bytes(false, kCodCplx / 2);
+    b->tab_bytes = b->tab_bytes <= small ? small : b->tab_bytes <= half ? half : cod_lds_bytes(false, kCodCplx);
     build_xcd_lists(b);
 }
 
@@ -1792,8 +1798,12 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
         b->graph = nullptr;
         BLQH_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         chunk(false, 0);
-        BLQH_HIP(hipStreamEndCapture(st, &b->graph));
-        BLQH_HIP(hipGraphInstantiate(&b->gexec, b->graph, nullptr, nullptr, 0));
+        if (hipStreamEndCapture(st, &b->graph) == hipSuccess) {
+            BLQH_HIP(hipGraphInstantiate(&b->gexec, b->graph, nullptr, nullptr, 0));
+        } else {  // another thread's call broke the capture: plain launches for this solve
+            (void)hipGetLastError();
+            b->graph = nullptr;
+        }
         b->g_chk = chk;
         b->g_lpr = b->lpr;
         b->g_cap = cap;
@@ -1850,7 +1860,7 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
             for (int j = first; j < std::min(cap, first + stride); j += kSmallLaunch)
                 hipLaunchKernelGGL(bsmall, dim3(P), dim3(kSmallT), shape.lds, st, S, b->dtscale.get(), j,
                                    std::min({cap, first + stride, j + kSmallLaunch}));
-        else if (timed) chunk(true, first);
+        else if (timed || !gexec) chunk(timed, first);
         else BLQH_HIP(hipGraphLaunch(gexec, st));
         BLQH_HIP(hipGetLastError());
     };
