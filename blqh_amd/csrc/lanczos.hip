@@ -49,7 +49,7 @@ __device__ __forceinline__ double2 ntload(const double2* p) {
 // device-scope fences, whose cost grows with the number of workgroups (a
 // ticket taken by each of 4,700 workgroups made the fused step of an
 // 18.8k-row matrix ten times slower than its product).
-__device__ __forceinline__ void block_partial(double v, double* partials) {
+__device__ __forceinline__ void block_partial(double v, double* partials, int64_t at = blockIdx.x) {
     __shared__ double sh[16];  // up to 1024 threads
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
@@ -57,7 +57,7 @@ __device__ __forceinline__ void block_partial(double v, double* partials) {
     if (threadIdx.x == 0) {
         double t = 0;
         for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += sh[w];
-        partials[blockIdx.x] = t;
+        partials[at] = t;
     }
 }
 
@@ -781,15 +781,15 @@ __global__ void __launch_bounds__(kT4Threads) k_t4(TileView V, const double2* __
 // and shares its step groups; a workgroup holds WPB / NP teams on neighbouring
 // slices, which gather from the same lines of x.
 //
-// Bound by the vector L1's rate of x gathers, not by the stream: 0.75 lane gathers
-// per clock and CU at N_phi = 16 (831M entries; 3.3 GB of words read at 1.8 TB/s).
+// Bound by the x gathers: 0.75 lane gathers per clock and CU at N_phi = 16 (831M entries),
+// and 8.8 GB fetched a launch (4.7 TB/s), 5.4 of them lines of x that miss the L2.
 // What measured best there: 512 threads, the whole workgroup kept on one panel by
 // the barrier (2,100 us without it, 1,880 with), eight steps in flight per wavefront
 // (four: 2,050 us).  Wider panels, 4 or 16 wavefronts a workgroup and persistent
 // grids gave nothing.  Step of one Lanczos iteration, K1 only, against the
 // jagged panels of 10 (real) or 18 (complex) bytes an entry: N_phi = 16 all
-// densities 2,907 -> 1,880 us, nel_up = 8 811 -> 475, N_phi = 14 real 209 -> 131 and
-// complex 265 -> 155, N_phi = 12 complex 24 -> 17.5.
+// densities 2,907 -> 1,880 us, nel_up = 8 811 -> 475, N_phi = 14 real 209 -> 124 and
+// complex 265 -> 140, N_phi = 12 complex 24 -> 17.
 template <bool REAL, bool LZ, int WPB, int NP>
 __global__ void __launch_bounds__(WPB * 64) k_cod(CodView P, const double2* __restrict__ x, double2* __restrict__ out,
                                                   const double2* __restrict__ Wp, Scal sc, int j, double* partials) {
@@ -798,7 +798,12 @@ __global__ void __launch_bounds__(WPB * 64) k_cod(CodView P, const double2* __re
     constexpr int TM = WPB / NP, U = 8;
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, par = wv % NP;
     const int64_t n = P.n, nsl = P.nslices;
-    const int64_t sl = (int64_t)blockIdx.x * TM + wv / NP, row = sl * 64 + lane;
+    // workgroup b runs on XCD b mod 8: each XCD gets a stretch of neighbouring slices, which
+    // gather from the same lines of x, and so its own part of x in its L2 (the grid is a
+    // multiple of 8).  N_phi = 13 49 -> 39.6 us, 14 real 131 -> 124, complex 155 -> 140; not for
+    // the largest (NP = 1), whose x is far beyond the L2s: N_phi = 16 1,880 -> 1,895.
+    const int64_t blk = NP > 1 ? (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+    const int64_t sl = blk * TM + wv / NP, row = sl * 64 + lane;
     cod_stage<REAL>(P.tab, P.ntab, ctab, WPB * 64);
     __syncthreads();
     double2 y = make_double2(0.0, 0.0);
@@ -836,7 +841,7 @@ __global__ void __launch_bounds__(WPB * 64) k_cod(CodView P, const double2* __re
             out[row] = y;
         }
     }
-    if (LZ) block_partial(dacc, partials);
+    if (LZ) block_partial(dacc, partials, blk);
 }
 
 // Steps j0 .. j1 - 1 of a small matrix in one workgroup (small.hpp).
@@ -1033,9 +1038,9 @@ void t4_dispatch(const blqh_hamil* H, const double2* x, double2* out, const doub
     throw Error(BLQH_EINTERNAL, "unsupported column-tile SpMV layout");
 }
 
-// workgroups of pl.threads / 64 wavefronts, teams of pl.rows
+// workgroups of pl.threads / 64 wavefronts, teams of pl.rows, a multiple of 8 (one stretch an XCD)
 int cod_grid(const blqh_hamil* H, const Plan& pl) {
-    return (int)ceil_div(ceil_div(H->n, 64), (int64_t)(pl.threads / 64 / pl.rows));
+    return (int)(8 * ceil_div(ceil_div(H->n, 64), (int64_t)(8 * (pl.threads / 64 / pl.rows))));
 }
 
 template <bool REAL, bool LZ, int WPB, int NP>
