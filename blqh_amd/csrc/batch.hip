@@ -1237,45 +1237,48 @@ void allow_lds(K kern, size_t bytes) {
 
 template <bool LZ, int G, bool SH>
 void launch_b1x(const blqh_batch* b, const BState& S, int jrel, const double2* xs, double2* ys, double* part,
-                hipStream_t st) {
+                hipStream_t st, bool go) {
     static const bool attr = (allow_lds(k_b1x<LZ, G, SH>, kLdsMax), true);  // once per instantiation, thread-safe
     (void)attr;
+    if (!go) return;
     hipLaunchKernelGGL((k_b1x<LZ, G, SH>), dim3(b->x_grid), dim3(kBTx), b->x_bytes, st, S, b->dtscale.get(), jrel, xs,
                        ys, part);
 }
 
 template <bool LZ, int KIND>
 void launch_b1j(const blqh_batch* b, const BState& S, int jrel, const double2* xs, double2* ys, double* part,
-                hipStream_t st) {
+                hipStream_t st, bool go) {
     static const bool attr = (allow_lds(k_b1j<LZ, KIND>, cod_lds_bytes(false, kCodCplx)), true);
     (void)attr;
+    if (!go) return;
     hipLaunchKernelGGL((k_b1j<LZ, KIND>), dim3(b->grid), dim3(kBTj), b->tab_bytes, st, S, jrel, xs, ys, part);
 }
 
+// go false (lanes 64): only the kernel's attributes are set, which a capture is not to do.
 template <bool LZ>
 void launch_b1(const blqh_batch* b, const BState& S, int jrel, const double2* xs, double2* ys, double* part,
-               hipStream_t st) {
+               hipStream_t st, bool go = true) {
     const dim3 g(b->grid), t(kBT);
     switch (b->G) {  // shared-scale groups: one pass over each sector's entries for all its problems
         case 0: break;
-        case 1: launch_b1x<LZ, 1, true>(b, S, jrel, xs, ys, part, st); return;
-        case 2: launch_b1x<LZ, 2, true>(b, S, jrel, xs, ys, part, st); return;
-        case 3: launch_b1x<LZ, 3, true>(b, S, jrel, xs, ys, part, st); return;
-        case 4: launch_b1x<LZ, 4, true>(b, S, jrel, xs, ys, part, st); return;
+        case 1: launch_b1x<LZ, 1, true>(b, S, jrel, xs, ys, part, st, go); return;
+        case 2: launch_b1x<LZ, 2, true>(b, S, jrel, xs, ys, part, st, go); return;
+        case 3: launch_b1x<LZ, 3, true>(b, S, jrel, xs, ys, part, st, go); return;
+        case 4: launch_b1x<LZ, 4, true>(b, S, jrel, xs, ys, part, st, go); return;
         default: throw Error(BLQH_EINTERNAL, "unsupported group size");
     }
     if (use_tiles(b)) {
-        launch_b1x<LZ, 1, false>(b, S, jrel, xs, ys, part, st);
+        launch_b1x<LZ, 1, false>(b, S, jrel, xs, ys, part, st, go);
         return;
     }
     switch (b->lpr) {
         case 64:
             if (b->has_real && b->has_complex) {  // measured faster than one launch per kind
-                launch_b1j<LZ, 2>(b, S, jrel, xs, ys, part, st);
+                launch_b1j<LZ, 2>(b, S, jrel, xs, ys, part, st, go);
                 break;
             }
-            if (b->has_real) launch_b1j<LZ, 0>(b, S, jrel, xs, ys, part, st);
-            if (b->has_complex) launch_b1j<LZ, 1>(b, S, jrel, xs, ys, part, st);
+            if (b->has_real) launch_b1j<LZ, 0>(b, S, jrel, xs, ys, part, st, go);
+            if (b->has_complex) launch_b1j<LZ, 1>(b, S, jrel, xs, ys, part, st, go);
             break;
         case 4: hipLaunchKernelGGL((k_b1<4, LZ>), g, t, 0, st, S, jrel, xs, ys, part); break;
         case 8: hipLaunchKernelGGL((k_b1<8, LZ>), g, t, 0, st, S, jrel, xs, ys, part); break;
@@ -1796,6 +1799,7 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
         if (b->graph) (void)hipGraphDestroy(b->graph);
         b->gexec = nullptr;
         b->graph = nullptr;
+        if (b->lpr == 64) launch_b1<true>(b, S, 0, nullptr, nullptr, pl.part1.get(), st, false);
         BLQH_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         chunk(false, 0);
         if (hipStreamEndCapture(st, &b->graph) == hipSuccess) {
