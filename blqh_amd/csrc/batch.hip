@@ -22,7 +22,8 @@
 // state is one weighted sum per problem afterwards (no replay pass); the same
 // pass forms the excited mix (second and third Ritz vectors), and both stay
 // on the device in the reference row order as the start of a continuation
-// solve at the next parameter point (k_bcont).
+// solve at the next parameter point (k_bcont).  A batch of small members only
+// takes its steps in one workgroup per problem instead (k_bsmall, small.hpp).
 #include <algorithm>
 #include <array>
 #include <chrono>

@@ -4,10 +4,12 @@
 // coeff_explicit_update / diag / eigenstates_reconstruction /
 // ground_state_energy (BLQH_without_spin/lanczos_hamiltonian.cpp:453-656).
 //
-// Vectors are kept unnormalised: v_j = W_j / beta_j.  One Lanczos step is two
+// Vectors are kept unnormalised: v_j = W_j / beta_j.  One Lanczos step is three
 // kernels:
 //   K1  u = (H W_j)/beta_j - beta_j W_{j-1}/beta_{j-1},  alpha_j = Re<v_j|u>
-//   K2  W_{j+1} = u - alpha_j v_j,  beta_{j+1} = |W_{j+1}|
+//   K2  W_{j+1} = u - alpha_j v_j
+//   K3  beta_{j+1} = |W_{j+1}|, alpha_j and beta_{j+1} to the host's mailbox
+// or, for up to 1,024 rows, a share of one workgroup's launch (small.hpp).
 // Both reduce through per-block partials summed in block order by the last
 // block to finish, so every scalar is bit-reproducible: a replayed pass 3
 // regenerates exactly the pass-1 vectors.  When the Krylov vectors fit in
