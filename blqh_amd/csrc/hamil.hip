@@ -451,10 +451,10 @@ __global__ void __launch_bounds__(64) k_build(BuildArgs A) {
         }
         for (int ql = 0; ql < (fold ? 1 : Dl); ++ql)
             for (int h = lane; h < A.nhop; h += 64) {
-                int j, Dr;
+                int j;
                 double re, im;
                 if (fold ? hop_orbit_sum(ctx, L0, Dl, A.hops[h], j, re, im)
-                         : hop_term(ctx, sLw[ql], sLs[ql], Dl, ql, A.hops[h], j, Dr, re, im))
+                         : hop_term(ctx, sLw[ql], sLs[ql], Dl, ql, A.hops[h], j, re, im))
                     if (!hash_add<CAP>(keys, vre, vim, j, re, im)) ovf = true;
             }
         __syncthreads();

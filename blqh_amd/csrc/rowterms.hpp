@@ -355,6 +355,13 @@ BLQH_HD bool hop_term(const RowCtx& c, uint64_t L, int signl, int Dl, int ql, co
     return true;
 }
 
+// The same where the target's period is not asked for.
+BLQH_HD bool hop_term(const RowCtx& c, uint64_t L, int signl, int Dl, int ql, const HopTerm& h, int& j, double& re,
+                      double& im) {
+    int Dr;
+    return hop_term(c, L, signl, Dl, ql, h, j, Dr, re, im);
+}
+
 // The hop h of the row word L0 and its images in translate(L0, ql), ql < Dl (the hops of the
 // rotated orbitals), summed; their targets lie in one orbit, row j.  For hop lists that
 // the translations map onto themselves (c.uniform): summed over the list it is the sum of

@@ -385,6 +385,42 @@ void hc_tridiag_vector_k(int m, const double* a, const double* b, int k, double*
     tridiag_vector_k(m, a, b, k, x);
 }
 
+// The two forms of hop_term, with the target's period and without, over a sector's
+// layer-exchanging hops: calls whose return value, row or element differ.
+int64_t hc_hop_forms_diff(const blqh_sector* s) {
+    HostBasis B;
+    build(*s, B);
+    blqh_params p{};
+    p.lx = p.ly = std::sqrt(2.0 * M_PI * s->nphi);
+    HostTables T = host_tables(*s, p);
+    RowCtx c{};
+    c.g = B.g;
+    c.spec = B.spec;
+    c.M = B.M;
+    c.K = s->K;
+    set_row_species(c, *s);
+    c.period = B.period.data();
+    c.lut = B.lut.data();
+    c.cnt = B.cnt.data();
+    c.FT = T.FT.data();
+    int64_t bad = 0;
+    for (int64_t i = 0; i < (int64_t)B.id.size(); ++i) {
+        const int Dl = c.K < 0 ? 1 : B.period[i];
+        const int f = s->nphi, d = s->nspecies == 4 ? 2 * f : f;
+        for (int n = 0; n < f; ++n)
+            for (int ql = 0; ql < Dl; ++ql) {
+                const HopTerm h{n, n + d, n, n + d, 0.5, 1.0, 0.0, 0};
+                int sg, ja = -1, jb = -1, Dr;
+                const uint64_t L = translate(c.g, B.id[i], ql, sg);
+                double ra = 0, ia = 0, rb = 0, ib = 0;
+                const bool a = hop_term(c, L, sg, Dl, ql, h, ja, Dr, ra, ia);
+                const bool b = hop_term(c, L, sg, Dl, ql, h, jb, rb, ib);
+                bad += a != b || (a && (ja != jb || ra != rb || ia != ib || Dr != (c.K < 0 ? 1 : B.period[ja])));
+            }
+    }
+    return bad;
+}
+
 // Largest difference between the split ranks (rank_share) and rank_word over a sector's words.
 int64_t hc_split_rank_diff(const blqh_sector* s) {
     const RankSpec sp = make_rank_spec(*s, true);

@@ -35,6 +35,8 @@ def lib():
         _L.hc_device_order_diff.restype = C.c_int64
         _L.hc_split_rank_diff.argtypes = [C.POINTER(blqh_amd.Sector)]
         _L.hc_split_rank_diff.restype = C.c_int64
+        _L.hc_hop_forms_diff.argtypes = [C.POINTER(blqh_amd.Sector)]
+        _L.hc_hop_forms_diff.restype = C.c_int64
         _L.hc_hop_images.argtypes = [C.POINTER(blqh_amd.Sector)]
         _L.hc_hop_images.restype = C.c_double
         _L.hc_residual_exceeds.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_double, C.c_double, C.c_double]
@@ -139,6 +141,11 @@ def hash_order_levels_check(sec):
     n = C.c_int64()
     ok = lib().hc_hash_order_levels_check(C.byref(sec), C.byref(n))
     return bool(ok), n.value
+
+
+def hop_forms_diff(sec):
+    """Calls of hop_term that differ between its forms with and without the target's period."""
+    return lib().hc_hop_forms_diff(C.byref(sec))
 
 
 def hop_images(sec):

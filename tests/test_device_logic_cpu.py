@@ -309,3 +309,11 @@ def test_equal_images_against_reference_loop_order(case):
 def test_split_rank_equals_walk(case):
     """Every word of the sector: the halves' table entries add up to the rank."""
     assert hostmirror.split_rank_diff(blqh_amd.Sector(*case)) == 0
+
+
+@pytest.mark.parametrize("case", [(2, 8, 8, -1, -1, 0, 4), (2, 7, 7, -1, -1, 2, 3), (2, 6, 6, -1, -1, 3, -1),
+                                  (4, 4, 4, -1, -1, 0, 2)], ids=lambda c: "_".join(map(str, c)))
+def test_hop_term_with_and_without_the_period(case):
+    """Both forms of the hop element (the mirror calls both, so both have to be there): the same
+    row and bits, and the period is the target's."""
+    assert hostmirror.hop_forms_diff(blqh_amd.Sector(*case)) == 0
