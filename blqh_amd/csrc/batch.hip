@@ -1063,10 +1063,9 @@ namespace {
 
 bool use_tiles(const blqh_batch* b) { return b->lpr == 64 && b->one_panel; }
 
-// Batches whose members a workgroup each steps through (k_bsmall): lanes 64, no member
-// above kSmallRows rows and kSmallWords entries.  lds: its dynamic LDS (0: another batch),
+// Batches whose members a workgroup each steps through (k_bsmall): lanes 64, small members
+// only (small_matrix).  lds: its dynamic LDS (0: another batch),
 // res: with every matrix in LDS.
-constexpr int64_t kSmallWords = 1 << 16;
 constexpr int kSmallSteps = 8;  // steps a launch, at least
 struct SmallShape {
     size_t lds = 0;
@@ -1076,7 +1075,7 @@ SmallShape small_shape(const blqh_batch* b) {
     if (b->lpr != 64) return {};
     size_t vec = 0, all = 0;
     for (const blqh_hamil* H : b->hs) {
-        if (H->n > kSmallRows || H->nnz > kSmallWords || !H->cod.built) return {};
+        if (!small_matrix(H->n, H->nnz) || !H->cod.built) return {};
         const Coded& C = H->cod;
         vec = std::max(vec, small_lds_bytes(C.real, C.ntab, H->n));
         all = std::max(all, small_lds_bytes(C.real, C.ntab, H->n, C.ncod, C.nrest));

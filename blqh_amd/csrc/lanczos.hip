@@ -9,7 +9,7 @@
 //   K1  u = (H W_j)/beta_j - beta_j W_{j-1}/beta_{j-1},  alpha_j = Re<v_j|u>
 //   K2  W_{j+1} = u - alpha_j v_j
 //   K3  beta_{j+1} = |W_{j+1}|, alpha_j and beta_{j+1} to the host's mailbox
-// or, for up to 1,024 rows, a share of one workgroup's launch (small.hpp).
+// or, for a small matrix, a share of one workgroup's launch (small.hpp).
 // Both reduce through per-block partials summed in block order by the last
 // block to finish, so every scalar is bit-reproducible: a replayed pass 3
 // regenerates exactly the pass-1 vectors.  When the Krylov vectors fit in
@@ -1059,12 +1059,13 @@ void cod_go(const blqh_hamil* H, const Plan& pl, const double2* x, double2* out,
                        cview(H->cod, H->n), x, out, Wp, sc, j, partials);
 }
 
-// A matrix whose steps one workgroup runs (k_small): up to kSmallSingle rows under the default
-// plan, whose order of sums it keeps.
+// A matrix whose steps one workgroup runs (k_small): a small one of up to kSmallSingle rows
+// under the default plan, whose order of sums it keeps.
 constexpr int kSmallSingle = 1024;
 constexpr int kSmallChunk = 8;  // steps a launch
 bool small_plan(const blqh_hamil* H, const Plan& pl) {
-    return pl.kind == 6 && pl.threads == 512 && pl.rows == kSmallTeam && H->cod.built && H->n <= kSmallSingle;
+    return pl.kind == 6 && pl.threads == 512 && pl.rows == kSmallTeam && H->cod.built && H->n <= kSmallSingle &&
+           small_matrix(H->n, H->nnz);
 }
 
 template <bool REAL, bool RES>

@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "../../blqh_amd/csrc/engine.hpp"
+#include "../../blqh_amd/csrc/small.hpp"
 #include "../../blqh_amd/csrc/xcdplan.hpp"
 #include "../../blqh_amd/csrc/ritz.hpp"
 
@@ -420,6 +421,9 @@ int64_t hc_hop_forms_diff(const blqh_sector* s) {
     }
     return bad;
 }
+
+// Whether one workgroup steps a matrix of n rows and nnz entries.
+int hc_small_matrix(int64_t n, int64_t nnz) { return small_matrix(n, nnz) ? 1 : 0; }
 
 // Largest difference between the split ranks (rank_share) and rank_word over a sector's words.
 int64_t hc_split_rank_diff(const blqh_sector* s) {

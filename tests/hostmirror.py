@@ -35,6 +35,7 @@ def lib():
         _L.hc_device_order_diff.restype = C.c_int64
         _L.hc_split_rank_diff.argtypes = [C.POINTER(blqh_amd.Sector)]
         _L.hc_split_rank_diff.restype = C.c_int64
+        _L.hc_small_matrix.argtypes = [C.c_int64, C.c_int64]
         _L.hc_hop_forms_diff.argtypes = [C.POINTER(blqh_amd.Sector)]
         _L.hc_hop_forms_diff.restype = C.c_int64
         _L.hc_hop_images.argtypes = [C.POINTER(blqh_amd.Sector)]
@@ -146,6 +147,11 @@ def hash_order_levels_check(sec):
 def hop_forms_diff(sec):
     """Calls of hop_term that differ between its forms with and without the target's period."""
     return lib().hc_hop_forms_diff(C.byref(sec))
+
+
+def small_matrix(n, nnz):
+    """Whether one workgroup steps a matrix of n rows and nnz entries."""
+    return bool(lib().hc_small_matrix(n, nnz))
 
 
 def hop_images(sec):
