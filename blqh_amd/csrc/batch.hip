@@ -325,8 +325,9 @@ __global__ void __launch_bounds__(kBTj) k_b1j(BState S, int jrel, const double2*
 // For members of one panel.  The x gathers bound k_b1j: the vector memory path
 // serves about one 16-byte lane address per clock and CU (0.75 measured), LDS a
 // wavefront's 64 in about 20 clocks.  So a workgroup of 16 wavefronts (one per CU:
-// it takes the whole LDS) owns a unit of 16 slices, stages x tile by tile beside the
-// value table and sums its slices' words of that tile from LDS.  The tiles are as
+// it takes the whole LDS) owns a unit of 16 slices (fewer in batches of few members,
+// batch_team), stages x tile by tile beside the value table and sums its slices' words of
+// that tile from LDS.  The tiles are as
 // wide as the LDS allows (8,192 columns of one vector at most), so a unit of an
 // 18.8k-row member stages 300 KB for 158k entries.  With x in LDS the address
 // arithmetic counts: a word's fields are LDS byte offsets (one mask each), rows are
@@ -350,7 +351,6 @@ __global__ void __launch_bounds__(kBTj) k_b1j(BState S, int jrel, const double2*
 // Word: bit 31 / 30 sign of the real / imaginary part, bits 17..28 index of the
 // value in the LDS table (0: the value zero), bits 4..16 column in the tile, bit 0
 // the tunnelling flag.
-constexpr int kUnit = 16;              // slices of a unit, one per wavefront
 constexpr int kBTx = kUnit * 64;
 constexpr int kUnitItems = kUnit * 64 / kItemRows;
 constexpr size_t kLdsMax = 160 * 1024 - 1024;  // dynamic LDS; the rest is k_b1x's static part
@@ -359,8 +359,11 @@ constexpr int kTileMax = 8192;         // columns of a tile (13 bits)
 
 // An element of k_b1x's work list names an owner (a problem; SH: a group) and, counted
 // in elements, the place in it: owner << kElemBits | element.  An element is `span`
-// (S.xseg[27], 1 or 2) consecutive units.
-constexpr int kElemBits = 7;  // at most 64 units of a one-panel member
+// (S.xseg[27], 1 or 2; 1 with teams) consecutive units (xcdplan.hpp).
+constexpr int kElemBits = 8;  // at most 256 units of a one-panel member
+// sums of a slice's later wavefronts, which take the tile's place
+constexpr size_t kTeamLds = kBTx / kTeamMax * (kTeamMax - 1) * sizeof(double2);
+static_assert(kLdsHalf >= 4096 * sizeof(double2) + kTeamLds, "team sums fit beside the largest table");
 
 // LDS bytes of the table: the value zero, then the layout's values
 __host__ __device__ inline size_t tile_tab_bytes(bool real, int ntab) {
@@ -452,15 +455,15 @@ __device__ __forceinline__ void tile_fma(uint32_t e, const char* lds, uint32_t x
     }
 }
 
-// A wavefront's words of one tile: K groups from ent, two groups loaded ahead (a0 and
-// a1 hold the first two).  A row's flagged words come first, so most groups have none.
-template <bool REAL, int G, bool SH>
+// A wavefront's words of one tile: K groups, NP apart, from ent, two groups loaded ahead (a0
+// and a1 hold the first two).  A row's flagged words come first, so most groups have none.
+template <bool REAL, int G, bool SH, int NP>
 __device__ __forceinline__ void tile_sum(const uint4* __restrict__ ent, uint32_t K, uint4 a0, uint4 a1, const char* lds,
                                          uint32_t xbase, uint32_t xstep, const double* ts, double* ar, double* ai) {
     for (uint32_t k = 0; k < K; ++k) {
         const uint4 e = a0;
         a0 = a1;
-        if (k + 2 < K) a1 = ent[(k + 2) * 64];
+        if (k + 2 < K) a1 = ent[(k + 2) * (64 * NP)];
         if (SH && __ballot(((e.x | e.y | e.z | e.w) & 1u) != 0)) {
             tile_fma<REAL, G, true>(e.x, lds, xbase, xstep, ts, ar, ai);
             tile_fma<REAL, G, true>(e.y, lds, xbase, xstep, ts, ar, ai);
@@ -499,16 +502,20 @@ __device__ __forceinline__ T* sgpr(T* p) {
 
 // Problem p0 + g, g < G, of an owner (SH: p0 = owner G; else G = 1, p0 = owner);
 // problem p's item li is item0 + li, as in k_b2 / k_b3.  A stopped problem of a
-// live group is summed along and not written.
-template <bool LZ, int G, bool SH>
+// live group is summed along and not written.  NP: wavefronts of a slice (batch_team); they
+// take its groups of a tile in turn, and the first adds the others' sums in their order.
+template <bool LZ, int G, bool SH, int NP>
 __global__ void __launch_bounds__(kBTx) k_b1x(BState S, const double* __restrict__ tscale, int jrel,
                                               const double2* __restrict__ xs, double2* __restrict__ ys,
                                               double* __restrict__ part) {
+    constexpr int NS = kUnit / NP;       // slices of a unit
+    constexpr int NQ = NP == 1 ? 2 : 1;  // units of an element at most
+    constexpr int NI = kUnitItems / NP;  // items of a unit
     extern __shared__ __align__(16) double ctab[];
-    __shared__ double red[2][G][kUnit];
+    __shared__ double red[NQ][G][NS];
     const int j = LZ ? *S.jbase + jrel : 0;
     if (LZ && j >= S.cap) return;
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, ws = wv / NP, par = wv % NP;
     const char* lds = reinterpret_cast<const char*>(ctab);
     // The XCD's workgroups walk its list side by side (unlike k_b1j's stretches):
     // they stage the x of the same one or two owners, out of the L2.
@@ -534,31 +541,33 @@ __global__ void __launch_bounds__(kBTx) k_b1x(BState S, const double* __restrict
         const uint32_t xbase = (uint32_t)tile_tab_bytes(real, ntab), xstep = (uint32_t)tw * 16u;
         double2* xt = reinterpret_cast<double2*>(reinterpret_cast<char*>(ctab) + xbase);
         const double2* x[G];
-        double ts[G], ar[2][G], ai[2][G];
+        double ts[G], ar[NQ][G], ai[NQ][G];
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             const BProb& Pg = S.probs[p0 + g];
             x[g] = sgpr(LZ ? Pg.W + (int64_t)j * n : xs + Pg.voff);
             ts[g] = SH ? sgpr(tscale[p0 + g]) : 1.0;
-            ar[0][g] = ai[0][g] = ar[1][g] = ai[1][g] = 0.0;
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) ar[q][g] = ai[q][g] = 0.0;
         }
         const int32_t u0 = (id & ((1 << kElemBits) - 1)) * span;  // the element's first unit
-        const int64_t sl0 = (int64_t)u0 * kUnit + wv;             // this wavefront's slices: sl0, sl0 + kUnit
+        const int64_t sl0 = (int64_t)u0 * NS + ws;                // this wavefront's slices: sl0, sl0 + NS
         for (int t = 0; t < nt; ++t) {
             // the first words are on their way while the tile is staged
-            uint32_t K[2];
-            const uint4* ent[2];
-            uint4 a0[2], a1[2];
+            uint32_t K[NQ];
+            const uint4* ent[NQ];
+            uint4 a0[NQ], a1[NQ];
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const int64_t sl = sl0 + q * kUnit;
+            for (int q = 0; q < NQ; ++q) {
+                const int64_t sl = sl0 + q * NS;
                 const bool mine = q < span && sl < nsl;  // uniform over the wavefront
                 const int64_t g0 = mine ? goff[sl * nt + t] : 0;
                 K[q] = mine ? (uint32_t)(goff[sl * nt + t + 1] - g0) : 0u;
-                ent[q] = tent + g0 * 64 + lane;
+                if (NP > 1) K[q] = K[q] > (uint32_t)par ? (K[q] - par + NP - 1) / NP : 0u;
+                ent[q] = tent + (g0 + par) * 64 + lane;
                 a0[q] = a1[q] = make_uint4(0, 0, 0, 0);
                 if (K[q] > 0) a0[q] = ent[q][0];
-                if (K[q] > 1) a1[q] = ent[q][64];
+                if (K[q] > 1) a1[q] = ent[q][64 * NP];
             }
             __syncthreads();  // the previous tile (and table) is no longer read
             if (o != ot) {
@@ -580,16 +589,32 @@ __global__ void __launch_bounds__(kBTx) k_b1x(BState S, const double* __restrict
             wait_vmem();
             __syncthreads();
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                if (real) tile_sum<true, G, SH>(ent[q], K[q], a0[q], a1[q], lds, xbase, xstep, ts, ar[q], ai[q]);
-                else tile_sum<false, G, SH>(ent[q], K[q], a0[q], a1[q], lds, xbase, xstep, ts, ar[q], ai[q]);
+            for (int q = 0; q < NQ; ++q) {
+                if (real) tile_sum<true, G, SH, NP>(ent[q], K[q], a0[q], a1[q], lds, xbase, xstep, ts, ar[q], ai[q]);
+                else tile_sum<false, G, SH, NP>(ent[q], K[q], a0[q], a1[q], lds, xbase, xstep, ts, ar[q], ai[q]);
+            }
+        }
+        if (NP > 1) {  // the team's sums, over the tile (at most 12 KiB, kTeamLds)
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                double2* const sum = xt + (ws * (NP - 1) - 1) * 64 + lane;  // of wavefront par: sum[par * 64]
+                __syncthreads();  // the tile, or the previous sums, are read
+                if (par) sum[par * 64] = make_double2(ar[0][g], ai[0][g]);
+                __syncthreads();
+                if (!par) {
+#pragma unroll
+                    for (int w = 1; w < NP; ++w) {
+                        ar[0][g] += sum[w * 64].x;
+                        ai[0][g] += sum[w * 64].y;
+                    }
+                }
             }
         }
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int64_t sl = sl0 + q * kUnit, row = sl * 64 + lane;
-            const bool mine = q < span && sl < nsl && row < n;
-            if (q < span && sl < nsl) {
+        for (int q = 0; q < NQ; ++q) {
+            const int64_t sl = sl0 + q * NS, row = sl * 64 + lane;
+            const bool slice = q < span && sl < nsl && par == 0, mine = slice && row < n;
+            if (slice) {
                 const int64_t q0 = P.c.rbase[sl];
                 const uint32_t rl = P.c.rlen[row];
                 if (real) tile_rest_sum<true, G, SH>(P.c.rcol + q0, P.c.rval + q0, x, ts, rl, ar[q], ai[q]);
@@ -621,13 +646,13 @@ __global__ void __launch_bounds__(kBTx) k_b1x(BState S, const double* __restrict
                     acc = w.x * yr + w.y * yi;
                 }
                 for (int d = 32; d > 0; d >>= 1) acc += __shfl_xor(acc, d, 64);
-                if (lane == 0) red[q][g][wv] = acc;
+                if (lane == 0 && par == 0) red[q][g][ws] = acc;
             }
         }
         __syncthreads();
-        if (threadIdx.x < 2 * G * kUnitItems) {  // item partials: its four slices in order
-            const int q = threadIdx.x / (G * kUnitItems), g = threadIdx.x / kUnitItems % G, m = threadIdx.x % kUnitItems;
-            const int64_t li = (int64_t)(u0 + q) * kUnitItems + m;
+        if (threadIdx.x < NQ * G * NI) {  // item partials: its four slices in order
+            const int q = threadIdx.x / (G * NI), g = threadIdx.x / NI % G, m = threadIdx.x % NI;
+            const int64_t li = (int64_t)(u0 + q) * NI + m;
             if (q < span && S.active[p0 + g] && li * kItemRows < n) {
                 double t = 0;
                 for (int i = 0; i < kItemRows / 64; ++i) t += red[q][g][m * (kItemRows / 64) + i];
@@ -1026,7 +1051,7 @@ struct blqh_batch {
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     int g_chk = -1, g_lpr = -1, g_cap = -1, g_kinds = -1;
-    std::array<size_t, 2> g_tab{};  // launch shape of the captured K1 (k1_shape)
+    std::array<size_t, 3> g_tab{};  // launch shape of the captured K1 (k1_shape)
     char* pin = nullptr;
     double2* psi_pin = nullptr;  // pinned staging of the ground states (b->rows entries, on first use)
     // pl.u holds every problem's ground state of the last finished solve in
@@ -1049,6 +1074,7 @@ struct blqh_batch {
     DevBuf<int64_t> tgoff;
     size_t x_bytes = 0;           // k_b1x's dynamic LDS
     int x_grid = 0;
+    int x_team = 1;               // wavefronts of a slice (batch_team)
     std::unique_ptr<HostPool> hpool;  // convergence-test threads (batches of 32 or more problems)
     ~blqh_batch() {
         if (gexec) (void)hipGraphExecDestroy(gexec);
@@ -1084,9 +1110,9 @@ SmallShape small_shape(const blqh_batch* b) {
 }
 
 // What the captured K1 launches depend on beside the lanes and the value kinds.
-std::array<size_t, 2> k1_shape(const blqh_batch* b) {
-    if (!use_tiles(b)) return {0, b->tab_bytes};
-    return {(size_t)b->x_grid, b->x_bytes};
+std::array<size_t, 3> k1_shape(const blqh_batch* b) {
+    if (!use_tiles(b)) return {0, b->tab_bytes, 0};
+    return {(size_t)b->x_grid, b->x_bytes, (size_t)b->x_team};
 }
 
 // Work lists (xcd_lists) over the members (all, or those with live[p] set); with
@@ -1097,6 +1123,7 @@ void work_lists(const blqh_batch* b, const std::vector<char>* live, std::vector<
                 std::vector<int32_t>& seg) {
     std::vector<XcdMember> mem;
     const int per = b->G ? b->G : 1, no = (int)b->hs.size() / per;
+    const int64_t unit = (int64_t)kUnit * 64 / b->x_team;  // rows
     mem.reserve(no);
     std::vector<int> on;
     int64_t units = 0;
@@ -1105,15 +1132,15 @@ void work_lists(const blqh_batch* b, const std::vector<char>* live, std::vector<
         for (int g = 0; g < per && !l; ++g) l = (*live)[o * per + g] != 0;
         if (!l) continue;
         on.push_back(o);
-        units += ceil_div(b->h_probs[o * per].n, (int64_t)kUnit * 64);
+        units += ceil_div(b->h_probs[o * per].n, unit);
     }
     const bool tiled = use_tiles(b);
-    const int span = tiled && units >= 8 * (int64_t)b->x_grid ? 2 : 1;
+    const int span = tiled && b->x_team == 1 && units >= 8 * (int64_t)b->x_grid ? 2 : 1;
     for (int o : on) {
         const BProb& d = b->h_probs[o * per];
         if (tiled) {
             const int64_t e0 = (int64_t)o << kElemBits;
-            mem.push_back({e0, e0 + ceil_div(d.n, (int64_t)kUnit * 64 * span), b->hs[o * per]->nnz * per, 1, d.real});
+            mem.push_back({e0, e0 + ceil_div(d.n, unit * span), b->hs[o * per]->nnz * per, 1, d.real});
         } else {
             mem.push_back({b->item0[o], b->item0[o + 1], b->hs[o]->nnz, d.npan, d.real});
         }
@@ -1165,12 +1192,15 @@ void make_tiles(blqh_batch* b) {
     b->tiles.resize(no);
     for (int o = 0; o < no; ++o)
         b->tiles[o] = ColTiles{jobs[o].tw, jobs[o].nt, b->tent.get(), b->tgoff.get() + jobs[o].goff0};
-    int64_t units = 0;
-    for (int o = 0; o < no; ++o) units += ceil_div(jobs[o].c.n, (int64_t)kUnit * 64);
     const int wpc = b->x_bytes <= kLdsHalf ? 2 : 1;  // workgroups of 1024 threads that share a CU's LDS
+    std::vector<int64_t> rows(no);
+    for (int o = 0; o < no; ++o) rows[o] = jobs[o].c.n;
+    b->x_team = batch_team(rows, runtime().num_cus);
+    // an XCD's list holds up to a chunk (xcd_lists) more than its even share: room for all of it at once
+    const int64_t units = batch_units(rows, b->x_team), share = ceil_div(units, kXcds) + ceil_div(units, 64);
     // one of two sizes, so that the next point's tables leave the captured launches as they are
     b->x_bytes = wpc == 2 ? kLdsHalf : kLdsMax;
-    b->x_grid = (int)(8 * ceil_div(std::min<int64_t>(units, (int64_t)runtime().num_cus * wpc), 8));
+    b->x_grid = (int)(kXcds * std::min(share, ceil_div((int64_t)runtime().num_cus * wpc, kXcds)));
     b->tiles_ok = true;
 }
 
@@ -1235,14 +1265,22 @@ void allow_lds(K kern, size_t bytes) {
     BLQH_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
 }
 
+template <bool LZ, int G, bool SH, int NP>
+void launch_b1x_team(const blqh_batch* b, const BState& S, int jrel, const double2* xs, double2* ys, double* part,
+                     hipStream_t st, bool go) {
+    static const bool attr = (allow_lds(k_b1x<LZ, G, SH, NP>, kLdsMax), true);  // once per instantiation, thread-safe
+    (void)attr;
+    if (!go) return;
+    hipLaunchKernelGGL((k_b1x<LZ, G, SH, NP>), dim3(b->x_grid), dim3(kBTx), b->x_bytes, st, S, b->dtscale.get(), jrel,
+                       xs, ys, part);
+}
+
 template <bool LZ, int G, bool SH>
 void launch_b1x(const blqh_batch* b, const BState& S, int jrel, const double2* xs, double2* ys, double* part,
                 hipStream_t st, bool go) {
-    static const bool attr = (allow_lds(k_b1x<LZ, G, SH>, kLdsMax), true);  // once per instantiation, thread-safe
-    (void)attr;
-    if (!go) return;
-    hipLaunchKernelGGL((k_b1x<LZ, G, SH>), dim3(b->x_grid), dim3(kBTx), b->x_bytes, st, S, b->dtscale.get(), jrel, xs,
-                       ys, part);
+    if (b->x_team == 4) launch_b1x_team<LZ, G, SH, 4>(b, S, jrel, xs, ys, part, st, go);
+    else if (b->x_team == 2) launch_b1x_team<LZ, G, SH, 2>(b, S, jrel, xs, ys, part, st, go);
+    else launch_b1x_team<LZ, G, SH, 1>(b, S, jrel, xs, ys, part, st, go);
 }
 
 template <bool LZ, int KIND>

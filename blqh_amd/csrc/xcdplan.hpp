@@ -14,6 +14,30 @@ namespace blqh {
 
 constexpr int kXcds = 8;
 
+// ---- units of the K1 with x in LDS (k_b1x) --------------------------------------
+// A workgroup of 16 wavefronts takes a unit of kUnit / team 64-row slices of one
+// member, `team` wavefronts to a slice.
+constexpr int kUnit = 16;
+constexpr int kTeamMax = 4;  // a unit holds whole 256-row items
+
+inline int64_t batch_units(const std::vector<int64_t>& rows, int team) {
+    const int64_t per = (int64_t)kUnit * 64 / team;
+    int64_t u = 0;
+    for (int64_t n : rows) u += (n + per - 1) / per;
+    return u;
+}
+
+// Wavefronts of a slice: doubled while the units still find a CU each.  With whole units
+// of 1,024 rows a batch of few members leaves most CUs idle; every unit stages its member's x,
+// so that more of them than CUs only cost.  A step of all kernels, 256 CUs, team 1 / 2 / 4: one
+// member of 1,846 rows 28.7 / 22.7 / 21.0 us, 64 of them 53 / 46 / 56; one of 18,802 rows 53 /
+// - / 34, one of 60,096 rows 75 / - / 47, two 141 / - / 64 (the larger team each time by this rule).
+inline int batch_team(const std::vector<int64_t>& rows, int64_t cus) {
+    int team = 1;
+    while (team < kTeamMax && batch_units(rows, 2 * team) <= cus) team *= 2;
+    return team;
+}
+
 // One batch member as the planner sees it: its work items [item0, item1),
 // its nonzeros, its column panels and its value kind.
 struct XcdMember {

@@ -424,6 +424,12 @@ int64_t hc_hop_forms_diff(const blqh_sector* s) {
 
 // Whether one workgroup steps a matrix of n rows and nnz entries.
 int hc_small_matrix(int64_t n, int64_t nnz) { return small_matrix(n, nnz) ? 1 : 0; }
+// Plan of the batched K1 with x in LDS on `cus` CUs: out = team, units.
+void hc_batch_team(int count, const int64_t* rows, int64_t cus, int64_t* out) {
+    const std::vector<int64_t> r(rows, rows + count);
+    out[0] = batch_team(r, cus);
+    out[1] = batch_units(r, (int)out[0]);
+}
 
 // Largest difference between the split ranks (rank_share) and rank_word over a sector's words.
 int64_t hc_split_rank_diff(const blqh_sector* s) {

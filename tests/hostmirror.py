@@ -36,6 +36,8 @@ def lib():
         _L.hc_split_rank_diff.argtypes = [C.POINTER(blqh_amd.Sector)]
         _L.hc_split_rank_diff.restype = C.c_int64
         _L.hc_small_matrix.argtypes = [C.c_int64, C.c_int64]
+        _L.hc_batch_team.argtypes = [C.c_int, C.c_void_p, C.c_int64, C.c_void_p]
+        _L.hc_batch_team.restype = None
         _L.hc_hop_forms_diff.argtypes = [C.POINTER(blqh_amd.Sector)]
         _L.hc_hop_forms_diff.restype = C.c_int64
         _L.hc_hop_images.argtypes = [C.POINTER(blqh_amd.Sector)]
@@ -152,6 +154,11 @@ def hop_forms_diff(sec):
 def small_matrix(n, nnz):
     """Whether one workgroup steps a matrix of n rows and nnz entries."""
     return bool(lib().hc_small_matrix(n, nnz))
+def batch_team(rows, cus=256):
+    """(wavefronts of a slice, units) of the batched K1 with x in LDS."""
+    r, out = np.asarray(rows, np.int64), np.empty(2, np.int64)
+    lib().hc_batch_team(r.size, r.ctypes.data, cus, out.ctypes.data)
+    return tuple(int(v) for v in out)
 
 
 def hop_images(sec):

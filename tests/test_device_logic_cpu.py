@@ -326,3 +326,15 @@ def test_one_workgroup_only_where_it_is_faster(n, nnz, one):
     """Steps go to one workgroup by the entries it has to walk on its one CU: from about 20,000
     on the kernels over the whole chip take less."""
     assert hostmirror.small_matrix(n, nnz) == one
+
+
+@pytest.mark.parametrize("rows", [[1], [64], [1846], [18802], [60096], [60096] * 2, [1846] * 64, [18802] * 16, [604] * 85,
+                                  [604] * 86, [604] * 128, [604] * 129, [65536] * 4, [5, 70000 // 2, 256, 257]])
+def test_batch_units_fill_the_chip(rows):
+    """The batched K1 never runs 1,024-row units on a few CUs while finer ones would still
+    find a CU each, and never takes finer ones than that."""
+    cus = 256
+    team, units = hostmirror.batch_team(rows, cus)
+    of = lambda t: sum(-(-n * t // 1024) for n in rows)  # noqa: E731
+    assert units == of(team)
+    assert team == max([t for t in (2, 4) if of(t) <= cus], default=1)

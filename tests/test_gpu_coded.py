@@ -138,3 +138,40 @@ def test_one_workgroup_steps_equal_kernel_steps(case):
         np.testing.assert_array_equal(a["alpha"], b["alpha"])
         np.testing.assert_array_equal(a["beta"], b["beta"])
         assert a["E0"] == b["E0"]
+
+
+@pytest.mark.parametrize("copies", [2, 90, 130])
+@pytest.mark.parametrize("K", [0, 2], ids=["real", "complex"])
+def test_batch_teams_against_single_solves(copies, K):
+    """One, two and four wavefronts to a slice (by the number of members: 604 rows are three
+    256-row, two 512-row units or one of 1,024), beside members with fewer slices than a unit:
+    eight steps against the single solver's."""
+    par = blqh_amd.params(9, d=0.7, delta_sas=0.05)
+    big = blqh_amd.Hamiltonian(blqh_amd.Basis(9, 9, -1, 3, K), par)
+    tiny = blqh_amd.Hamiltonian(blqh_amd.Basis(8, 8, 4, 4, 4), blqh_amd.params(8, d=3.0))
+    hams = [big] * (copies - 1) + [tiny]
+    print(f"rows {big.n} and {tiny.n}, {copies} members", flush=True)
+    steps = dict(lam=8, tol=0.0, res_tol=0.0)
+    r = blqh_amd.Batch(hams).lanczos(seeds=list(range(copies)), check_every=3, **steps)
+    for p in (0, copies // 2, copies - 2, copies - 1):
+        one = hams[p].lanczos(seed=p, **steps)
+        assert r[p]["E0"] == pytest.approx(one["E0"], rel=1e-11, abs=1e-11)
+        np.testing.assert_allclose(r[p]["psi"], one["psi"], rtol=0, atol=1e-9)
+
+
+@pytest.mark.parametrize("G", [1, 4])
+@pytest.mark.parametrize("copies", [1, 90, 130])
+def test_shared_scale_teams_against_combined(copies, G):
+    """The same for shared-scale groups: sums of one, two and four wavefronts for up to four vectors."""
+    par = blqh_amd.params(9, d=0.7)
+    B = blqh_amd.Basis(9, 9, -1, 3, 2)
+    h0, t = blqh_amd.Hamiltonian(B, par, terms=1), blqh_amd.Hamiltonian(B, par, terms=2)
+    scales = [0.05, 0.1, 0.2, 0.0][:G]
+    print(f"rows {h0.n}, {copies} sectors, {G} scales", flush=True)
+    steps = dict(lam=8, tol=0.0, res_tol=0.0)
+    r = blqh_amd.Batch.scaled([h0] * copies, [t] * copies, scales).lanczos(seeds=list(range(copies * G)), check_every=3,
+                                                                           **steps)
+    for p in {0, G - 1, copies * G // 2, copies * G - 1}:
+        one = blqh_amd.Hamiltonian.combine(h0, t, scales[p % G]).lanczos(seed=p, **steps)
+        assert r[p]["E0"] == pytest.approx(one["E0"], rel=1e-11, abs=1e-11)
+        np.testing.assert_allclose(r[p]["psi"], one["psi"], rtol=0, atol=1e-9)
