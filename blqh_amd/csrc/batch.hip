@@ -255,6 +255,7 @@ __global__ void __launch_bounds__(kBTj) k_b1j(BState S, int jrel, const double2*
             __syncthreads();  // the previous member's table is no longer read
             if (real) cod_stage<true>(P.c.tab, P.c.ntab, ctab, kBTj);
             else cod_stage<false>(P.c.tab, P.c.ntab, ctab, kBTj);
+            wait_vmem();
             __syncthreads();
             pt = p;
         }
@@ -479,14 +480,6 @@ __device__ __forceinline__ void tile_sum(const uint4* __restrict__ ent, uint32_t
         }
     }
 }
-
-// 16 bytes a lane from global memory straight to LDS, lane l to dst + l; complete
-// after wait_vmem.  dst: uniform over the wavefront.
-__device__ __forceinline__ void load_lds16(const double2* src, double2* dst) {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
-}
-__device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // Values that are the same on every lane, into scalar registers (the kernel writes
 // memory, so the compiler keeps what it loads per owner in vector ones).

@@ -481,7 +481,7 @@ void build_coded(blqh_hamil* H, const uint8_t* nu, int64_t* ntun) {
     C.ent.alloc(std::max<int64_t>(C.ncod, 1));
     C.rcol.alloc(std::max<int64_t>(C.nrest, 1));
     C.rval.alloc(std::max<int64_t>(C.nrest, 1) * (C.real ? 1 : 2));
-    C.tab.alloc(std::max(C.ntab, 1) * (C.real ? 1 : 2));
+    C.tab.alloc(cod_lds_bytes(C.real, C.ntab) / sizeof(double));
     BLQH_HIP(hipMemcpyAsync(C.tab.get(), tab.get(), C.tab.bytes(), hipMemcpyDeviceToDevice, st));
     hipLaunchKernelGGL(k_cod_fill, dim3(grid_waves(nsl)), dim3(kBlk), 0, st, n, nsl, C.npan, iperm,
                        H->rowptr.get(), skey.get(), C.len.get(), C.base.get(), C.ent.get());

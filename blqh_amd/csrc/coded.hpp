@@ -34,7 +34,7 @@ struct Coded {
     int npan = 0;
     int ntab = 0;
     int64_t ncod = 0, nrest = 0;
-    DevBuf<double> tab;      // [ntab] |v|, or [2 ntab] (|re|, |im|)
+    DevBuf<double> tab;      // [ntab] |v| (an even number of places), or [2 ntab] (|re|, |im|)
     DevBuf<int64_t> base;    // [npan * nslices + 1] first word of run p * nslices + s
     DevBuf<uint16_t> len;    // [npan][nslices * 64] words of the row in the run
     DevBuf<uint32_t> ent;    // [ncod]
@@ -65,7 +65,18 @@ inline CodView cview(const Coded& C, int64_t n) {
                    C.diag.get()};
 }
 
-inline size_t cod_lds_bytes(bool real, int ntab) { return (size_t)(ntab > 0 ? ntab : 1) * (real ? 8 : 16); }
+__host__ __device__ inline size_t cod_lds_bytes(bool real, int ntab) {
+    const size_t n = ntab > 0 ? ntab : 1;
+    return real ? (n + 1) / 2 * 16 : n * 16;
+}
+
+// 16 bytes a lane from global memory straight to LDS, lane l to dst + l; complete
+// after wait_vmem.  dst: uniform over the wavefront.
+__device__ __forceinline__ void load_lds16(const double2* src, double2* dst) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+__device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // The value of word e: magnitudes from the LDS table, signs from the top bits.
 __device__ __forceinline__ double cod_sign(double v, uint32_t top) {  // top: sign in bit 31
@@ -93,16 +104,29 @@ __device__ __forceinline__ double2 cod_diag(const CodView& C, bool real, int64_t
     return real ? make_double2(C.diag[row], 0.0) : reinterpret_cast<const double2*>(C.diag)[row];
 }
 
-// Table to LDS (the caller synchronises the workgroup).
+// Table to LDS, every load of a wavefront in flight at once (the caller waits, wait_vmem, and
+// synchronises the workgroup).
 template <bool REAL>
 __device__ __forceinline__ void cod_stage(const double* __restrict__ tab, int ntab, double* lds, int nthreads) {
-    if (REAL) {
-        for (int i = threadIdx.x; i < ntab; i += nthreads) lds[i] = tab[i];
-    } else {
-        const double2* t = reinterpret_cast<const double2*>(tab);
-        double2* l = reinterpret_cast<double2*>(lds);
-        for (int i = threadIdx.x; i < ntab; i += nthreads) l[i] = t[i];
-    }
+    const double2* t = reinterpret_cast<const double2*>(tab);
+    double2* l = reinterpret_cast<double2*>(lds);
+    const int n = REAL ? (ntab + 1) >> 1 : ntab, lane = threadIdx.x & 63;
+    for (int i = threadIdx.x; i < n; i += nthreads) load_lds16(t + i, l + (i - lane));
+}
+
+// Sum of v over the wavefront's lanes (all active), the same on every lane.  A step's place in
+// a run is such a sum; counted ballot by ballot over the other wavefronts' steps, those
+// were half of the kernels' instructions, and a launch on a small matrix is as long as its
+// instructions take to arrive: k_cod at 1,855 rows 8.5 -> 7.0 us, k_small's step at 205
+// rows 10.9 -> 7.6.
+__device__ __forceinline__ uint32_t lane_total(uint32_t v) {
+    int t = (int)v;
+    t += __builtin_amdgcn_update_dpp(0, t, 0x128, 0xf, 0xf, false);  // row_ror:8, 4, 2, 1
+    t += __builtin_amdgcn_update_dpp(0, t, 0x124, 0xf, 0xf, false);
+    t += __builtin_amdgcn_update_dpp(0, t, 0x122, 0xf, 0xf, false);
+    t += __builtin_amdgcn_update_dpp(0, t, 0x121, 0xf, 0xf, false);
+    return (uint32_t)(__builtin_amdgcn_readlane(t, 0) + __builtin_amdgcn_readlane(t, 16) +
+                      __builtin_amdgcn_readlane(t, 32) + __builtin_amdgcn_readlane(t, 48));
 }
 
 // Row sums of one run: lane l owns row l (`len` words); the step groups (U
@@ -128,19 +152,14 @@ __device__ __forceinline__ void cod_run_sum(const uint32_t* __restrict__ er, con
             e[u] = t + u < len ? (KEEP ? er[q] : __builtin_nontemporal_load(&er[q])) : 0u;
         }
     };
-    auto skip = [&](uint32_t t) {  // another wave's group: advance the offset only
-#pragma unroll
-        for (int u = 0; u < U; ++u) off += (uint32_t)__popcll(__ballot(t + u < len));
-    };
     uint32_t e0[U], e1[U];
     bool any0, any1;
-    for (int g = 0; g < par; ++g) skip((uint32_t)(U * g));
     uint32_t t0 = (uint32_t)(U * par);
+    if (NP > 1) off = lane_total(t0 < len ? t0 : len);  // words of the steps before: the other wavefronts' groups
     issue(t0, e0, any0);
     while (any0) {
         const uint32_t t = t0 + (uint32_t)(U * NP);
-#pragma unroll
-        for (int g = NP - 1; g > 0; --g) skip(t - (uint32_t)(U * g));
+        if (NP > 1) off = lane_total(t < len ? t : len);
         issue(t, e1, any1);
         double2 xv[U];
 #pragma unroll

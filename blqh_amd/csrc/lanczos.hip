@@ -807,6 +807,7 @@ __global__ void __launch_bounds__(WPB * 64) k_cod(CodView P, const double2* __re
     const int64_t blk = NP > 1 ? (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
     const int64_t sl = blk * TM + wv / NP, row = sl * 64 + lane;
     cod_stage<REAL>(P.tab, P.ntab, ctab, WPB * 64);
+    wait_vmem();
     __syncthreads();
     double2 y = make_double2(0.0, 0.0);
     for (int p = 0; p < P.npan; ++p) {

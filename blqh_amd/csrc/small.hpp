@@ -54,7 +54,7 @@ constexpr int kSmallLaunch = 64;   // steps of a launch at most (the mailbox's e
 // and rest)
 inline size_t small_lds_bytes(bool real, int ntab, int64_t n, int64_t ncod = 0, int64_t nrest = 0) {
     const auto up = [](size_t b) { return (b + 15) & ~(size_t)15; };
-    return up(cod_lds_bytes(real, ntab)) + (size_t)(2 * n + kSmallT) * sizeof(double2) + (size_t)((n + 63) >> 6) * 256 +
+    return cod_lds_bytes(real, ntab) + (size_t)(2 * n + kSmallT) * sizeof(double2) + (size_t)((n + 63) >> 6) * 256 +
            up((size_t)ncod * 4) + up((size_t)nrest * 4) + (size_t)nrest * (real ? 8 : 16);
 }
 constexpr size_t kSmallLdsMax = 152 * 1024;  // dynamic; a static part of 2 KiB an instantiation
@@ -98,7 +98,7 @@ __device__ __forceinline__ void small_steps(const CodView& P, int64_t ncod, int6
     constexpr int TM = kSmallT / 64 / kSmallTeam;
     const int n = (int)P.n, nsl = (int)P.nslices, gv = (n + 255) >> 8;
     const auto up = [](size_t b) { return (b + 15) & ~(size_t)15; };
-    char* at = reinterpret_cast<char*>(lds) + up((size_t)(P.ntab > 0 ? P.ntab : 1) * (REAL ? 8 : 16));
+    char* at = reinterpret_cast<char*>(lds) + cod_lds_bytes(REAL, P.ntab);
     double2* xs = reinterpret_cast<double2*>(at);
     double2* ys = xs + n;
     double2* red = ys + n;
@@ -136,6 +136,7 @@ __device__ __forceinline__ void small_steps(const CodView& P, int64_t ncod, int6
         }
     }
     double ib = invb[j0], bj = beta[j0], ibp = j0 > 0 ? invb[j0 - 1] : 0.0;
+    wait_vmem();
     __syncthreads();
     for (int j = j0; j < j1; ++j) {
         for (int s0 = 0; s0 < nsl; s0 += TM) {
