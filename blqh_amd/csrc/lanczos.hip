@@ -188,16 +188,19 @@ __global__ void __launch_bounds__(kThreads) k_lz2(int64_t n, const double2* __re
     block_partial(acc, part2);
 }
 
-// K3: beta[j+1] = sqrt(sum of K2's partials), invb[j+1]; one workgroup.  mail: null in a
-// replay.
+// K3: beta[j+1] = sqrt(sum of K2's partials), invb[j+1]; one workgroup.  The last `post`
+// steps' coefficients go to the mailbox, those of a convergence test together: the
+// step ends when they have reached the host's memory.
 __global__ void __launch_bounds__(kThreads) k_lz3(Scal sc, int j, const double* __restrict__ part2, int npart2,
-                                                  StepMail* mail, uint64_t tag) {
-    const double t = block_total(part2, npart2);
+                                                  StepMail* mail, int post, uint64_t tag0) {
+    const double t = block_total(part2, npart2), b = sqrt(t);
     if (threadIdx.x == 0) {
-        const double b = sqrt(t);
         sc.beta[j + 1] = b;
         sc.invb[j + 1] = 1.0 / b;
-        if (mail) post_mail(mail, j, sc.alpha[j], b, tag);
+    }
+    if ((int)threadIdx.x < post) {
+        const int k = j - (int)threadIdx.x;
+        post_mail(mail, k, sc.alpha[k], k == j ? b : sc.beta[k + 1], tag0 | (uint64_t)(uint32_t)(k + 1));
     }
 }
 
@@ -1625,11 +1628,11 @@ struct DevWork {
 // K2 and K3 of one step after the K1 launched with grid `g1` wrote part1.
 void launch_lz23(int64_t n, const double2* u, const double2* W, double2* Wn, const Scal& sc, int j, int ns,
                  double2* psi, const double* coef, int ldc, const double* part1, int g1, double* part2,
-                 hipStream_t st, StepMail* mail = nullptr, uint64_t tag = 0) {
+                 hipStream_t st, StepMail* mail = nullptr, int post = 0, uint64_t tag0 = 0) {
     const int gv = vec_grid(n);
     hipLaunchKernelGGL(k_lz2, dim3(gv), dim3(kThreads), 0, st, n, u, W, Wn, sc, j, ns, psi, coef, ldc, part1, g1,
                        part2);
-    hipLaunchKernelGGL(k_lz3, dim3(1), dim3(kThreads), 0, st, sc, j, part2, gv, mail, tag);
+    hipLaunchKernelGGL(k_lz3, dim3(1), dim3(kThreads), 0, st, sc, j, part2, gv, mail, post, tag0);
 }
 
 // *out = |x|^2 and *out = Re<x|y>: block partials, then one wavefront sums them
@@ -1748,6 +1751,7 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
     const bool prof_on = timed && prof.on;
     int ntimed = 0;
     const uint64_t tag0 = ++hw.mail->solve << 32;
+    int posted = 0;  // steps whose coefficients a queued K3 posts
     auto step = [&](int j, double2* psi_acc, const double* cf) {
         double2* W = slot(j);
         double2* Wp = j > 0 ? slot(j - 1) : slot(j);
@@ -1761,8 +1765,14 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
         }
         launch_lz1(H, plan, W, Wp, D.u, sc, j, D.partials, st);
         if (prof_on) BLQH_HIP(hipEventRecord(prof.ev[2 * ntimed++ + 1], st));
+        // pass 1 posts for every convergence test, and by half a mailbox within a long interval
+        int post = 0;
+        if (!psi_acc && ((j + 1) % chk == 0 || j + 1 == cap || j + 1 - posted == kMail / 2)) {
+            post = j + 1 - posted;
+            posted = j + 1;
+        }
         launch_lz23(n, D.u, W, slot(j + 1), sc, j, psi_acc ? 1 : 0, psi_acc, cf, cap, D.partials, g1, D.partials2,
-                    st, psi_acc ? nullptr : hw.mail->m, tag0 | (uint32_t)(j + 1));
+                    st, hw.mail->m, post, tag0);
     };
     auto account = [&]() {
         if (!prof_on) return;

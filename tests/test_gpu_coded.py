@@ -175,3 +175,20 @@ def test_shared_scale_teams_against_combined(copies, G):
         one = blqh_amd.Hamiltonian.combine(h0, t, scales[p % G]).lanczos(seed=p, **steps)
         assert r[p]["E0"] == pytest.approx(one["E0"], rel=1e-11, abs=1e-11)
         np.testing.assert_allclose(r[p]["psi"], one["psi"], rtol=0, atol=1e-9)
+
+
+@pytest.mark.parametrize("store", [0, 1], ids=["replay", "kept"])
+def test_coefficients_for_every_test_interval(store):
+    """Coefficients reach the host in groups, one for each convergence test and one for half a
+    mailbox (32 steps): the same bits whatever the interval, also past the mailbox's 64 entries."""
+    B = blqh_amd.Basis(9, 9, -1, 2, 1)
+    H = blqh_amd.Hamiltonian(B, blqh_amd.params(9, d=0.8, delta_sas=0.05))
+    steps = dict(lam=150, tol=0.0, res_tol=0.0, seed=3, store_basis=store)
+    first = H.lanczos(check_every=1, **steps)
+    assert first["iterations"] == 150
+    for chk in (2, 31, 32, 33, 63, 64, 65, 149, 150, 1000):
+        print(f"interval {chk}", flush=True)
+        r = H.lanczos(check_every=chk, **steps)
+        np.testing.assert_array_equal(r["alpha"], first["alpha"])
+        np.testing.assert_array_equal(r["beta"], first["beta"])
+        np.testing.assert_array_equal(r["psi"], first["psi"])
