@@ -134,8 +134,10 @@ __device__ __forceinline__ uint32_t lane_total(uint32_t v) {
 // == par.  The words of the next group are loaded before the x gathers of the
 // current one, so a wavefront always has loads in flight.
 // KEEP: the words are read again soon (small.hpp), leave them in the caches.  SH: values of
-// words with the tunnelling flag are scaled by ts (columns have 15 bits).
-template <bool REAL, int NP, int U, bool KEEP = false, bool SH = false>
+// words with the tunnelling flag are scaled by ts (columns have 15 bits).  ANY: x may hold
+// infinities and NaN (the public product's), which a lane past its row's end, reading the
+// panel's first entry, is not to multiply with its zero; the solvers' vectors are finite.
+template <bool REAL, int NP, int U, bool KEEP = false, bool SH = false, bool ANY = false>
 __device__ __forceinline__ void cod_run_sum(const uint32_t* __restrict__ er, const double* tab,
                                             const double2* __restrict__ xp, uint32_t len, int par, double& ar,
                                             double& ai, double ts = 1.0) {
@@ -163,7 +165,10 @@ __device__ __forceinline__ void cod_run_sum(const uint32_t* __restrict__ er, con
         issue(t, e1, any1);
         double2 xv[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) xv[u] = xp[e0[u] & (SH ? kCodTun - 1 : 0xffffu)];
+        for (int u = 0; u < U; ++u) {
+            xv[u] = xp[e0[u] & (SH ? kCodTun - 1 : 0xffffu)];
+            if (ANY && !(t0 + u < len)) xv[u] = make_double2(0.0, 0.0);
+        }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const bool act = t0 + u < len;

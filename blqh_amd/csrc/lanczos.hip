@@ -817,8 +817,8 @@ __global__ void __launch_bounds__(WPB * 64) k_cod(CodView P, const double2* __re
         if (P.npan > 1) __syncthreads();  // keep the workgroup on one panel
         if (sl >= nsl) continue;      // uniform over the wavefront
         const int64_t run = (int64_t)p * nsl + sl;
-        cod_run_sum<REAL, NP, U>(P.ent + P.base[run], ctab, x + (int64_t)p * kPanelWidth,
-                                 P.len[run * 64 + lane], par, y.x, y.y);
+        cod_run_sum<REAL, NP, U, false, false, !LZ>(P.ent + P.base[run], ctab, x + (int64_t)p * kPanelWidth,
+                                                    P.len[run * 64 + lane], par, y.x, y.y);
     }
     if (sl < nsl) {
         const int64_t q0 = P.rbase[sl];

@@ -192,3 +192,30 @@ def test_coefficients_for_every_test_interval(store):
         np.testing.assert_array_equal(r["alpha"], first["alpha"])
         np.testing.assert_array_equal(r["beta"], first["beta"])
         np.testing.assert_array_equal(r["psi"], first["psi"])
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf], ids=["nan", "inf"])
+def test_non_finite_entries_reach_their_rows_only(built, bad):
+    """A NaN or an infinity in x shows in the rows that hold its column and in no other: the lanes
+    past their row's end multiply nothing.  Tried at the first internal row of every panel, which
+    those lanes read, and at others."""
+    from tests import hostmirror
+    name, B, H, A = built
+    pos = hostmirror.internal_order(B.sector, B.id)
+    at = np.argsort(pos) if pos is not None else np.arange(H.n)  # reference row of an internal one
+    cols = A.tocsc()
+    rng = np.random.default_rng(2)
+    x = rng.normal(size=H.n) + 1j * rng.normal(size=H.n)
+    rows = list(at[::65536]) + list(rng.integers(0, H.n, 2))
+    for plan in ((-1, 0, 0, 0, 0), (6, 64, 512, 0, 1), (6, 64, 512, 0, 8), (6, 64, 1024, 0, 16)):
+        H.set_spmv(*plan)
+        good = H.spmv(x)
+        for i in rows:
+            print(f"{name} plan {plan} entry {i}", flush=True)
+            z = x.copy()
+            z[i] = bad
+            y = H.spmv(z)
+            hit = np.zeros(H.n, bool)
+            hit[cols.indices[cols.indptr[i]:cols.indptr[i + 1]]] = True
+            np.testing.assert_array_equal(np.isfinite(y), ~hit)
+            np.testing.assert_array_equal(y[~hit], good[~hit])
