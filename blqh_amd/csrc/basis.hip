@@ -190,10 +190,13 @@ __global__ void k_period(int64_t n, const uint64_t* __restrict__ id, Geo g, int1
     }
 }
 
-__global__ void k_rank_split(RankSpec s, const uint32_t* __restrict__ cnt, int rbits, uint32_t total,
-                             uint32_t* __restrict__ out) {
-    for (uint32_t x = blockIdx.x * blockDim.x + threadIdx.x; x < total; x += gridDim.x * blockDim.x)
-        out[x] = rank_share(s, cnt, rbits, x);
+// The M places of the lookup table set to -1, and the `total` rank shares: one launch, since
+// a small basis is as long as its launches.
+__global__ void k_lut_init(RankSpec s, const uint32_t* __restrict__ cnt, int rbits, uint32_t total,
+                           uint32_t* __restrict__ rsplit, int64_t M, int32_t* __restrict__ lut) {
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, nt = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t x = t; x < total; x += nt) rsplit[x] = rank_share(s, cnt, rbits, (uint32_t)x);
+    for (int64_t i = t; i < M; i += nt) lut[i] = -1;
 }
 
 __global__ void k_fill_i32(int32_t* __restrict__ p, int64_t n, int32_t v) {
@@ -583,17 +586,17 @@ void blqh_basis_build_impl(const blqh_sector& s, blqh_basis* B) {
     // lookup table over the (spin-constrained) sector
     B->spec = make_rank_spec(s, true);
     std::vector<uint32_t> tsec = make_rank_table(B->spec, &B->M);
-    B->cnt.alloc(tsec.size());
-    BLQH_HIP(hipMemcpyAsync(B->cnt.get(), tsec.data(), tsec.size() * 4, hipMemcpyHostToDevice, st));
+    uint32_t total = 0;  // rank shares
     if (B->spec.nbits <= 32) {  // both halves' tables in half a megabyte, inside an XCD's L2
         B->rbits = B->spec.nbits / 2;
-        const uint32_t total = (1u << B->rbits) + (1u << (B->spec.nbits - B->rbits));
-        B->rsplit.alloc(total);
-        hipLaunchKernelGGL(k_rank_split, dim3(grid_for(total)), dim3(kBlock), 0, st, B->spec, B->cnt.get(), B->rbits,
-                           total, B->rsplit.get());
+        total = (1u << B->rbits) + (1u << (B->spec.nbits - B->rbits));
     }
+    B->cnt.alloc(tsec.size() + total);
+    if (total) B->rsplit = B->cnt.get() + tsec.size();
+    BLQH_HIP(hipMemcpyAsync(B->cnt.get(), tsec.data(), tsec.size() * 4, hipMemcpyHostToDevice, st));
     B->lut.alloc(B->M);
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(B->M)), dim3(kBlock), 0, st, B->lut.get(), B->M, -1);
+    hipLaunchKernelGGL(k_lut_init, dim3(grid_for(std::max<int64_t>(B->M, total))), dim3(kBlock), 0, st, B->spec,
+                       B->cnt.get(), B->rbits, total, B->rsplit, B->M, B->lut.get());
     hipLaunchKernelGGL(k_lut, dim3(grid_for(n)), dim3(kBlock), 0, st, n, B->id.get(), B->period.get(), B->geo,
                        B->spec, B->cnt.get(), reduce ? 0 : 1, B->lut.get());
     BLQH_HIP(hipGetLastError());

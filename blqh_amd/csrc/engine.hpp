@@ -18,8 +18,8 @@ struct blqh_basis {
     blqh_sector sec{};
     blqh::Geo geo{};
     blqh::RankSpec spec{};           // the sector (with the spin-up constraint)
-    blqh::DevBuf<uint32_t> cnt;      // rank table of spec
-    blqh::DevBuf<uint32_t> rsplit;   // rank shares of the word halves (sector_rank); empty above 32 bits
+    blqh::DevBuf<uint32_t> cnt;      // rank table of spec, then rsplit
+    uint32_t* rsplit = nullptr;      // rank shares of the word halves (sector_rank); null above 32 bits
     int rbits = 0;                   // bits of the lower half
     int64_t M = 0;                   // sector words
     int64_t n = 0;                   // basis states (orbit representatives)
@@ -188,7 +188,7 @@ inline RowCtx make_row_ctx(const blqh_basis* B) {
     c.period = B->period.get();
     c.lut = B->lut.get();
     c.cnt = B->cnt.get();
-    c.rsplit = B->rsplit.get();
+    c.rsplit = B->rsplit;
     c.rbits = B->rbits;
     return c;
 }

@@ -48,3 +48,24 @@ def test_large_basis_checksum(key):
     h.update(np.ascontiguousarray(B.id).astype("<u8").tobytes())
     h.update(np.ascontiguousarray(B.period).astype("<i2").tobytes())
     assert h.hexdigest() == LARGE[key]["sha256"]
+
+
+@pytest.mark.parametrize("case", [(2, 2, 1, -1, -1, 0, 0), (2, 2, 1, -1, -1, -1, -1), (2, 16, 3, -1, -1, 1, 2),
+                                  (4, 8, 2, 1, -1, 1, 1), (2, 17, 3, -1, -1, 1, 2), (2, 8, 8, -1, -1, -1, 3)],
+                         ids=lambda c: "_".join(map(str, c)))
+def test_lookup_tables_by_word_size(oracle_mod, case):
+    """The lookup table and the halves' rank shares come from one launch: fewer table places than
+    shares and more, words of 4 to 32 bits, and of 34, which have no shares.  Rows against the
+    oracle's."""
+    O = oracle_mod
+    S, nphi, nel, nu, nsu, J, K = case
+    B = blqh_amd.Basis(nphi, nel, nu, J, K, nspecies=S, nel_su=nsu)
+    H = blqh_amd.Hamiltonian(B, blqh_amd.params(nphi, d=0.7, delta_sas=0.1))
+    print(f"{case} n {H.n}", flush=True)
+    OB = O.Basis(O.sector(*case))
+    OH = O.Hamiltonian(OB, O.params(nphi, d=0.7, dsas=0.1))
+    np.testing.assert_array_equal(B.id, OB.id)
+    rp, col, val = H.export()
+    np.testing.assert_array_equal(rp, OH.rowptr)
+    np.testing.assert_array_equal(col.astype(np.int64), OH.col)
+    np.testing.assert_allclose(val, OH.val, rtol=0, atol=1e-13 * np.abs(OH.val).max())
