@@ -1583,6 +1583,7 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
         tp = now;
     };
     hipStream_t st = stream();
+    DrainGuard drain{st};  // of the batch's own pools and pinned memory
     const int P = (int)b->hs.size();
     const int cap = o.lambda;
     BLQH_REQUIRE(cap >= 2 && cap <= 100000, BLQH_EINVAL, "lambda out of range");
@@ -2076,6 +2077,7 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
         BLQH_HIP(hipMemcpyAsync(b->psi_pin, pl.u.get(), (size_t)b->rows * sizeof(double2), hipMemcpyDeviceToHost, st));
     }
     BLQH_HIP(hipStreamSynchronize(st));
+    drain.finished = true;
     b->cont_ok = true;
     if (want) {
         auto put = [&](int p) {

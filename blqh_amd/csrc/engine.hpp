@@ -108,6 +108,17 @@ std::vector<uint64_t> hash_iteration_order_map(const blqh_sector& s);  // from a
 std::vector<std::pair<int64_t, uint64_t>> hash_levels(int64_t n);
 RankSpec reversed_rank_spec(const blqh_sector& s, const RankSpec& smap);  // bit-reversed words
 
+// Waits for the stream on every way out of a solve but the finished one: a solve that ends
+// in an error has steps queued ahead, which write its vectors, scalars and mailbox, and those
+// go to other solves, also on other threads' streams.
+struct DrainGuard {
+    hipStream_t st;
+    bool finished = false;
+    ~DrainGuard() {
+        if (!finished) (void)hipStreamSynchronize(st);
+    }
+};
+
 // Event timing of the fused Lanczos SpMV (blqh_profile_*).
 struct Profile {
     bool on = false;

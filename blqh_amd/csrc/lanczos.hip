@@ -1647,8 +1647,8 @@ void reduce_redot(int64_t n, const double2* x, const double2* y, double* out, do
     hipLaunchKernelGGL(k_psum, dim3(1), dim3(kThreads), 0, st, part, gv, out);
 }
 // Mailboxes (pinned, kMail entries): one per host thread, taken on its first solve and
-// handed back when it ends; never freed, since an abandoned solve's kernels may still
-// write there.  `solve` numbers the solves that used it, so a tag is never met twice.
+// handed back when it ends, with no kernel left that writes there (DrainGuard); never freed.
+// `solve` numbers the solves that used it, so a tag is never met twice.
 struct Mailbox {
     StepMail* m = nullptr;
     uint64_t solve = 0;
@@ -1727,6 +1727,7 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
                   const HostWork& hw, Start&& start, bool timed, blqh_lanczos_result& res, double* psi_out,
                   double* alpha_out, double* beta_out, std::chrono::steady_clock::time_point t0) {
     hipStream_t st = stream();
+    DrainGuard drain{st};
     const int64_t n = H->n;
     const int cap = o.lambda;
     const int chk = std::max(1, o.check_every);
@@ -1856,6 +1857,7 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
         res.E_rq = NAN;
         res.passes = 1;
         BLQH_HIP(hipStreamSynchronize(st));
+        drain.finished = true;
         account();
         res.seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
         return;
@@ -1901,6 +1903,7 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
         BLQH_HIP(hipMemcpyAsync(psi_out, out, n * sizeof(double2), hipMemcpyDeviceToHost, st));
     }
     BLQH_HIP(hipStreamSynchronize(st));
+    drain.finished = true;
     account();
     res.E_rq = erq;
     res.seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();

@@ -65,3 +65,44 @@ def test_builds_on_a_worker_thread_overlap_solves():
             assert all(r["converged"] == 1 for r in res)
             np.testing.assert_allclose([r["E0"] for r in res], ref_e[d], rtol=1e-12, atol=0)
     assert ids and main_id not in ids
+
+def _run(f):
+    """f() on a thread of its own, with a stream of its own; its result or exception."""
+    out = []
+
+    def go():
+        try:
+            out.append(f())
+        except Exception as e:  # noqa: BLE001
+            out.append(e)
+
+    t = threading.Thread(target=go)
+    t.start()
+    t.join()
+    return out[0]
+
+
+@pytest.mark.parametrize("how", ["noalloc", "replay", "kept", "batch"])
+def test_solve_after_an_abandoned_one(how):
+    """A solve that ends in an error (a layer bias that overflows: no finite coefficient) has steps
+    queued ahead. It waits for them, so that the next solve, on another thread's stream and with
+    the scratch or the mailbox of the first, has the bits that it has by itself."""
+    B = blqh_amd.Basis(11, 11, -1, 1, 2)
+    bad = blqh_amd.Hamiltonian(B, blqh_amd.params(11, d=0.7, delta_sas=0.05, delta_v=1e308))
+    good = blqh_amd.Hamiltonian(B, blqh_amd.params(11, d=0.7, delta_sas=0.05))
+    steps = dict(lam=30, seed=2, tol=0.0, res_tol=0.0)
+
+    def solve(H):
+        if how == "noalloc":
+            return H.lanczos_noalloc(**steps)
+        if how == "batch":
+            return blqh_amd.Batch([H]).lanczos(lam=30, seeds=2, tol=0.0, res_tol=0.0, check_every=1)[0]
+        return H.lanczos(store_basis=1 if how == "kept" else 0, **steps)
+
+    ref = solve(good)
+    for k in range(5):
+        print(f"{how} {k}", flush=True)
+        assert isinstance(_run(lambda: solve(bad)), blqh_amd.BlqhError)
+        r = _run(lambda: solve(good))
+        assert r["E0"] == ref["E0"] and r["E_rq"] == ref["E_rq"]
+        np.testing.assert_array_equal(r["psi"], ref["psi"])
