@@ -1789,20 +1789,26 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
     Profile& prof = profile();
     const bool timed = prof.on;  // per-kernel events need plain launches
     std::vector<hipEvent_t> ev;
-    int ntimed = 0;
+    int ntimed = 0;             // timed launches
+    int64_t timed_steps = 0;    // and the steps in them
+    auto event_before = [&] {
+        while ((int)ev.size() < 2 * (ntimed + 1)) {
+            hipEvent_t e;
+            BLQH_HIP(hipEventCreate(&e));
+            ev.push_back(e);
+        }
+        BLQH_HIP(hipEventRecord(ev[2 * ntimed], st));
+    };
+    auto event_after = [&](int steps) {
+        BLQH_HIP(hipEventRecord(ev[2 * ntimed++ + 1], st));
+        timed_steps += steps;
+    };
     auto chunk = [&](bool record, int first) {
         for (int k = 0; k < chk; ++k) {
             const bool t = record && first + k < cap;
-            if (t) {
-                while ((int)ev.size() < 2 * (ntimed + 1)) {
-                    hipEvent_t e;
-                    BLQH_HIP(hipEventCreate(&e));
-                    ev.push_back(e);
-                }
-                BLQH_HIP(hipEventRecord(ev[2 * ntimed], st));
-            }
+            if (t) event_before();
             launch_b1<true>(b, S, k, nullptr, nullptr, pl.part1.get(), st);
-            if (t) BLQH_HIP(hipEventRecord(ev[2 * ntimed++ + 1], st));
+            if (t) event_after(1);
             hipLaunchKernelGGL(k_b2, dim3(b->grid), dim3(kBT), 0, st, S, k);
             hipLaunchKernelGGL(k_b3, dim3(P), dim3(64), 0, st, S, k, P);
         }
@@ -1815,7 +1821,7 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
         }
     } evguard{ev};
     const int kinds = (b->has_real ? 2 : 0) | (b->has_complex ? 1 : 0);  // which K1 launches a step has
-    const SmallShape shape = timed ? SmallShape{} : small_shape(b);
+    const SmallShape shape = small_shape(b);
     const bool small = shape.lds > 0;  // k_bsmall takes the steps
     void (*const bsmall)(BState, const double*, int, int) = b->G ? (shape.res ? k_bsmall<true, true> : k_bsmall<false, true>)
                                                                  : (shape.res ? k_bsmall<true, false> : k_bsmall<false, false>);
@@ -1893,9 +1899,12 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
     int queued = 0;  // steps queued so far
     auto enqueue = [&](int first) {
         if (small)
-            for (int j = first; j < std::min(cap, first + stride); j += kSmallLaunch)
-                hipLaunchKernelGGL(bsmall, dim3(P), dim3(kSmallT), shape.lds, st, S, b->dtscale.get(), j,
-                                   std::min({cap, first + stride, j + kSmallLaunch}));
+            for (int j = first; j < std::min(cap, first + stride); j += kSmallLaunch) {
+                const int to = std::min({cap, first + stride, j + kSmallLaunch});
+                if (timed) event_before();
+                hipLaunchKernelGGL(bsmall, dim3(P), dim3(kSmallT), shape.lds, st, S, b->dtscale.get(), j, to);
+                if (timed) event_after(to - j);
+            }
         else if (timed || !gexec) chunk(timed, first);
         else BLQH_HIP(hipGraphLaunch(gexec, st));
         BLQH_HIP(hipGetLastError());
@@ -2098,7 +2107,7 @@ void blqh_batch_lanczos_impl(blqh_batch* b, const blqh_lanczos_opts& o, const ui
             BLQH_HIP(hipEventElapsedTime(&ms, ev[2 * k], ev[2 * k + 1]));
             prof.ms += ms;
         }
-        prof.launches += ntimed;
+        prof.launches += timed_steps;
     }
     phase("finish");
     const double secs = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();

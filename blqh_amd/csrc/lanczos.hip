@@ -1750,22 +1750,27 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
 
     Profile& prof = profile();
     const bool prof_on = timed && prof.on;
-    int ntimed = 0;
+    int ntimed = 0, timed_steps = 0;  // timed launches, and the steps in them
+    auto event_before = [&] {
+        while ((int)prof.ev.size() < 2 * (ntimed + 1)) {
+            hipEvent_t e;
+            BLQH_HIP(hipEventCreate(&e));
+            prof.ev.push_back(e);
+        }
+        BLQH_HIP(hipEventRecord(prof.ev[2 * ntimed], st));
+    };
+    auto event_after = [&](int steps) {
+        BLQH_HIP(hipEventRecord(prof.ev[2 * ntimed++ + 1], st));
+        timed_steps += steps;
+    };
     const uint64_t tag0 = ++hw.mail->solve << 32;
     int posted = 0;  // steps whose coefficients a queued K3 posts
     auto step = [&](int j, double2* psi_acc, const double* cf) {
         double2* W = slot(j);
         double2* Wp = j > 0 ? slot(j - 1) : slot(j);
-        if (prof_on) {
-            while ((int)prof.ev.size() < 2 * (ntimed + 1)) {
-                hipEvent_t e;
-                BLQH_HIP(hipEventCreate(&e));
-                prof.ev.push_back(e);
-            }
-            BLQH_HIP(hipEventRecord(prof.ev[2 * ntimed], st));
-        }
+        if (prof_on) event_before();
         launch_lz1(H, plan, W, Wp, D.u, sc, j, D.partials, st);
-        if (prof_on) BLQH_HIP(hipEventRecord(prof.ev[2 * ntimed++ + 1], st));
+        if (prof_on) event_after(1);
         // pass 1 posts for every convergence test, and by half a mailbox within a long interval
         int post = 0;
         if (!psi_acc && ((j + 1) % chk == 0 || j + 1 == cap || j + 1 - posted == kMail / 2)) {
@@ -1782,8 +1787,8 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
             BLQH_HIP(hipEventElapsedTime(&ms, prof.ev[2 * k], prof.ev[2 * k + 1]));
             prof.ms += ms;
         }
-        prof.launches += ntimed;
-        prof.bytes += (double)ntimed * (20.0 * H->nnz + 56.0 * n + 8.0);
+        prof.launches += timed_steps;
+        prof.bytes += (double)timed_steps * (20.0 * H->nnz + 56.0 * n + 8.0);
     };
 
     // pass 1
@@ -1793,7 +1798,7 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
     bool conv = false;
     double dE = INFINITY, resid = INFINITY;
     int done = 0, queued = 0;
-    const bool small = store && !prof_on && small_plan(H, plan);
+    const bool small = store && small_plan(H, plan);
     const int ahead = small ? kSmallChunk : steps_ahead(H->nnz, chk);
     hb[0] = 1.0;
     while (done < cap && !conv) {
@@ -1810,8 +1815,13 @@ void lanczos_core(blqh_hamil* H, const Plan& plan, const blqh_lanczos_opts& o, b
         while (queued < std::min(cap, upto + ahead)) {
             const int to = small ? std::min(cap, queued + kSmallChunk) : queued + 1;
             read_to(std::min(upto, to - kMail));  // the entries' last tenants have been read
-            if (!small) step(queued, nullptr, nullptr);
-            else launch_small(H, D.Wb, sc, queued, to, hw.mail->m, tag0, st);
+            if (!small) {
+                step(queued, nullptr, nullptr);
+            } else {
+                if (prof_on) event_before();
+                launch_small(H, D.Wb, sc, queued, to, hw.mail->m, tag0, st);
+                if (prof_on) event_after(to - queued);
+            }
             queued = to;
         }
         BLQH_HIP(hipGetLastError());

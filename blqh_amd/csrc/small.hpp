@@ -4,7 +4,9 @@
 // work.  Here one workgroup of 16 wavefronts keeps the value table, the vector and the
 // row sums in LDS and runs the steps back to back; only the new vector goes to memory, for
 // the states.  The sums are taken in the order of k_cod (teams of eight wavefronts on
-// 64-row slices), k_lz2 and k_lz3, so the coefficients have the same bits whichever runs.
+// 64-row slices), k_lz2 and k_lz3, so the coefficients of a single solve have the same bits
+// whichever runs.  A batch's kernels (k_b1x, k_b2, k_b3) sum in another order: the last bits
+// of its members depend on whether all of them are small.
 // Bound by the instructions of the step's chain (sums, two reductions, a root and a division)
 // on one CU: 5.6 us a step at 79 rows (three launches: 12), 12 us at 176 rows (108 such
 // problems at once, kernels over all of them: 27).

@@ -237,6 +237,9 @@ int blqh_lanczos_reconstruct(const blqh_hamil* h, int32_t m, uint32_t seed, cons
  * every `check_every` steps), stops each problem by the rule of blqh_lanczos,
  * keeps all Krylov vectors in HBM ((lambda+1) * nrows * 16 bytes per problem;
  * BLQH_ENOMEM when they do not fit) and reconstructs each ground state.
+ * The kernels, and with them the order of sums, are chosen for the batch as a
+ * whole (the sizes and the number of its members): the last bits of a member's
+ * results depend on the company it is solved in, and are the same on every call.
  * seeds: per-problem mt19937 seeds (NULL: o->seed for all); starts: per-problem
  * start vectors (NULL array or NULL entry: seeded); psi: per-problem outputs
  * (2*nrows doubles; NULL array or entry: not copied); res[count]. ---- */
@@ -389,7 +392,9 @@ int blqh_record_load(const char* path, int32_t cap, int64_t* nhilbert, int32_t* 
  * is bracketed by HIP events on the library stream; blqh_profile_read returns
  * the launch count, the summed kernel time and the algorithmic bytes summed
  * over those launches (20 nnz + 56 n + 8 per launch: CSR values, columns,
- * row pointers, x read once, previous vector read, output written). */
+ * row pointers, x read once, previous vector read, output written).  The steps
+ * of a small matrix run many to a launch: that launch's whole time, and as many
+ * launches as it holds steps.  Timed solves run the kernels of untimed ones. */
 /* Plain device-to-device copy kernel of `bytes` bytes (multiple of 16) on the
  * library stream: the reference point for scaling hardware byte counters. */
 int blqh_device_copy(const void* src_dev, void* dst_dev, int64_t bytes);

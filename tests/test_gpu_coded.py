@@ -219,3 +219,48 @@ def test_non_finite_entries_reach_their_rows_only(built, bad):
             hit[cols.indices[cols.indptr[i]:cols.indptr[i + 1]]] = True
             np.testing.assert_array_equal(np.isfinite(y), ~hit)
             np.testing.assert_array_equal(y[~hit], good[~hit])
+
+
+@pytest.mark.parametrize("name", ["tiny", "mixed_kinds", "scaled", "single"])
+def test_event_timing_runs_the_same_kernels(name):
+    """With the kernel timing on, solves run the kernels that they run without it: the same bits,
+    the steps of one workgroup among them, and every step counted."""
+    steps = dict(lam=30, tol=0.0, res_tol=0.0)
+    if name == "single":
+        H = blqh_amd.Hamiltonian(blqh_amd.Basis(8, 8, 4, 4, 4), blqh_amd.params(8, d=3.0))
+        count = 1
+
+        def solve():
+            return [H.lanczos(seed=1, **steps)]
+    elif name == "scaled":
+        B = blqh_amd.Basis(8, 8, -1, 1, 3)
+        par = blqh_amd.params(8, d=0.6)
+        h0, t = blqh_amd.Hamiltonian(B, par, terms=1), blqh_amd.Hamiltonian(B, par, terms=2)
+        batch = blqh_amd.Batch.scaled([h0], [t], [0.05, 0.1])
+        count = 2
+
+        def solve():
+            return batch.lanczos(seeds=[1, 2], check_every=3, **steps)
+    else:
+        hams = []
+        for S, nphi, nel, nu, nsu, J, K in BATCHES[name]:
+            B = blqh_amd.Basis(nphi, nel, nu, J, K, nspecies=S, nel_su=nsu)
+            hams.append(blqh_amd.Hamiltonian(B, blqh_amd.params(nphi, d=0.9, delta_sas=0.05 if nu < 0 else 0.0)))
+        batch = blqh_amd.Batch(hams)
+        count = len(hams)
+
+        def solve():
+            return batch.lanczos(seeds=list(range(count)), check_every=3, **steps)
+    print(name, flush=True)
+    plain = solve()
+    blqh_amd.profile_reset()
+    blqh_amd.profile_enable(True)
+    try:
+        timed = solve()
+        launches, ms, nbytes = blqh_amd.profile_read()
+    finally:
+        blqh_amd.profile_enable(False)
+    for u, v in zip(plain, timed):
+        assert u["E0"] == v["E0"] and u["iterations"] == v["iterations"] and u["residual"] == v["residual"]
+        np.testing.assert_array_equal(u["psi"], v["psi"])
+    assert launches >= max(r["iterations"] for r in timed) and ms > 0 and nbytes > 0
