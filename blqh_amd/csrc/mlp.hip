@@ -70,7 +70,7 @@ __device__ __forceinline__ float feature(const Dims& D, uint64_t w, float pd, fl
     return k == D.nbits ? pd * (1.0f / 3.0f) : ps * 10.0f;
 }
 
-// A workgroup of kT threads evaluates a tile of kTile states.  LDS holds the
+// Inference: a workgroup of kT threads evaluates a tile of kTile states.  LDS holds the
 // parameters (W2 with a padded row stride so that a wavefront reading one
 // column touches 64 different banks), the tile's inputs and activations.
 constexpr int kTile = 64;
@@ -78,7 +78,7 @@ constexpr int kLd = kH + 1;  // padded row stride of the 64-wide LDS matrices
 struct Lds {
     float W1[kMaxIn * kH], b1[kH], W2[kH * kLd], b2[kH], W3[kH * 2], b3[2];
     float X[kTile * (kMaxIn + 1)];  // inputs, row stride nin + 1
-    float H1[kTile * kLd], H2[kTile * kLd], D2[kTile * kLd];
+    float H1[kTile * kLd], H2[kTile * kLd];
     float O[kTile * 2];
 };
 
