@@ -44,29 +44,36 @@ def build_map(f, xs):
         _BUILD_POOL = ThreadPoolExecutor(4)
     return list(_BUILD_POOL.map(f, xs))
 
-# HBM bytes per launch of the fused SpMV from rocprofv3 FETCH_SIZE / WRITE_SIZE
+# HBM bytes per launch of the fused SpMV, recorded by rocprofv3 FETCH_SIZE / WRITE_SIZE
 # passes, scaled by the same counters on a plain 1 GiB copy (profiles/);
-# reported only when the live run uses the profiled workload and variant
-MEASURED_TRAFFIC = {
+# used only when the live run has the profiled workload and variant
+RECORDED_TRAFFIC = {
     # k_cod<true, true, 8, 1>: 4,289,286.9 KiB FETCH_SIZE x 2.0 + 36,841.3 KiB WRITE_SIZE x 1.0 per dispatch
     ("nphi16_all", (6, 64, 512, 0, 1)): (4289286.9 * 2.0 * 1024 + 36841.3 * 1024, "profiles/k1_counters.md"),
 }
-# HBM bytes per batched K1 launch of the sweeps (FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 KiB, mean over a
-# solve's K1 dispatches), reported for the same batching mode
-MEASURED_SWEEP_TRAFFIC = {
-    ("sweep_spin_nphi8", "per-point"): (215688.2 * 2.0 * 1024 + 11307.8 * 1024, "profiles/k1_counters.md"),
-    ("sweep_nphi12", "shared"): (1159919.4 * 2.0 * 1024 + 90652.6 * 1024, "profiles/k1_counters.md"),
+# The same per batched K1 launch of the sweeps: the mean over one solve's dispatches, with fewer
+# and fewer problems live, so it holds only for what was profiled: (workload, problems to a
+# group, lanes, steps between convergence checks, step limit)
+RECORDED_SWEEP_TRAFFIC = {
+    ("sweep_spin_nphi8", 1, 64, 2, 200): (215688.2 * 2.0 * 1024 + 11307.8 * 1024, "profiles/k1_counters.md"),
+    ("sweep_nphi12", 3, 64, 2, 200): (1159919.4 * 2.0 * 1024 + 90652.6 * 1024, "profiles/k1_counters.md"),
 }
+
+
+def one_workgroup(H, rows):
+    """Whether one workgroup runs the steps (the timing is then that of whole steps)."""
+    return H.n <= rows and H.nnz <= 16384
 
 
 def roofline_rate(achieved, traffic, avg_ms):
     """The SpMV's rates.  "achieved" charges the CSR's bytes (20 per nonzero), the measure that
     formats are compared by; the coded layout moves fewer, so the share of the peak is that of
-    the measured traffic where there is one."""
+    the traffic recorded for this kernel in the named profile, over this run's time, where there is
+    one.  (A kernel that moves other bytes needs the profile taken anew.)"""
     moved = traffic[0] / (avg_ms * 1e-3) / 1e9 if traffic and avg_ms > 0 else None
     return {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": (moved if moved is not None else achieved) / HBM_PEAK_GBS,
-            "frac_of": "measured traffic" if moved is not None else "CSR bytes",
+            "frac_of": f"traffic recorded in {traffic[1]}" if moved is not None else "CSR bytes",
             "achieved_definition": "CSR bytes (20 per nonzero) over the kernel's time", "moved": moved,
             "traffic": traffic[0] if traffic else None, "traffic_source": traffic[1] if traffic else None}
 
@@ -416,8 +423,11 @@ def run_sweep(args):
             "batched_spmv_lanes": batch.lanes,
         },
         "roofline": {
-            **roofline_rate(achieved, MEASURED_SWEEP_TRAFFIC.get((args.workload, "per-point")), avg_ms),
-            "kernel": ("k_b1x<LZ=true> (batched fused SpMV + Lanczos K1, coded layout, x tiles in LDS)" if batch.lanes == 64 else
+            **roofline_rate(achieved, RECORDED_SWEEP_TRAFFIC.get((args.workload, 1, batch.lanes, bchk, args.lam)),
+                            avg_ms),
+            "kernel": ("k_bsmall (whole steps, one workgroup a problem)"
+                       if batch.lanes == 64 and all(one_workgroup(H, 2048) for H in batch.hams) else
+                       "k_b1x<LZ=true> (batched fused SpMV + Lanczos K1, coded layout, x tiles in LDS)" if batch.lanes == 64 else
                        f"k_b1<{batch.lanes}, LZ=true> (batched fused SpMV + Lanczos K1, row-major panels)"),
             "avg_launch_ms": avg_ms,
             "launches": launches,
@@ -638,7 +648,7 @@ def run_sweep_shared(args):
             "basis_s_once": round(t_basis, 2),
         },
         "roofline": {
-            **roofline_rate(achieved, MEASURED_SWEEP_TRAFFIC.get((args.workload, "shared")), avg_ms),
+            **roofline_rate(achieved, RECORDED_SWEEP_TRAFFIC.get((args.workload, G, batch.lanes, bchk, args.lam)), avg_ms),
             "kernel": f"k_b1x<LZ=true, G={G}, shared> (shared-scale batched fused SpMV + Lanczos K1: each sector's "
                       f"entries read once for its {G} DSAS problems)",
             "avg_launch_ms": avg_ms,
@@ -903,7 +913,7 @@ def main():
     avg_ms = kms / max(launches, 1)
     achieved = (kbytes / max(launches, 1)) / (avg_ms * 1e-3) / 1e9 if launches else 0.0
     spread = (max(energies) - min(energies)) / abs(np.mean(energies))
-    traffic = MEASURED_TRAFFIC.get((args.workload, tuple(H.get_spmv())))
+    traffic = RECORDED_TRAFFIC.get((args.workload, tuple(H.get_spmv())))
 
     out = {
         "metric": METRIC,
@@ -933,7 +943,8 @@ def main():
         },
         "roofline": {
             **roofline_rate(achieved, traffic, avg_ms),
-            "kernel": KERNEL_NAMES.get(H.get_spmv()[0], "?") + " (fused complex-FP64 SpMV + Lanczos K1 epilogue)",
+            "kernel": "k_small (whole steps in one workgroup)" if one_workgroup(H, 1024) else
+                      KERNEL_NAMES.get(H.get_spmv()[0], "?") + " (fused complex-FP64 SpMV + Lanczos K1 epilogue)",
             "avg_launch_ms": avg_ms,
             "launches": launches,
             "algorithmic_bytes_per_launch": kbytes / max(launches, 1),
