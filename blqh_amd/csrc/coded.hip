@@ -3,7 +3,7 @@
 //
 // The reference's SpMV walks CSR rows (Mat::operator*,
 // BLQH_without_spin/matrix.cpp:244-267); this copy is what the hot loops read.
-// Stages, all on the device, two host waits:
+// Stages, all on the device, two host waits and three blocks of memory:
 //   k_dict_sample   counts the values of a strided sample in a hash table
 //   k_dict_select   keeps the most frequent ones: the table and its lookup hash
 //   k_cod_rows      a wavefront per row: columns to the internal order, sorted in
@@ -390,6 +390,21 @@ __global__ void __launch_bounds__(kBlk) k_cod_rest(int64_t n, int64_t nslices, i
     }
 }
 
+__global__ void k_cod_totals(const int64_t* __restrict__ a, const int64_t* __restrict__ b, int64_t* __restrict__ out) {
+    out[0] = *a;
+    out[1] = *b;
+}
+
+// arrays of one device block, 256 bytes apart at least
+struct Blocks {
+    size_t bytes = 0;
+    size_t add(size_t b) {
+        const size_t at = bytes;
+        bytes += (b + 255) / 256 * 256 + (b == 0 ? 256 : 0);
+        return at;
+    }
+};
+
 __global__ void k_fill64(uint64_t* __restrict__ p, int64_t n, uint64_t v) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         p[i] = v;
@@ -416,13 +431,18 @@ void build_coded(blqh_hamil* H, const uint8_t* nu, int64_t* ntun) {
     uint32_t slots = 1024;
     while (slots < 2 * samples) slots <<= 1;
     constexpr uint32_t kLook = 2 * (kCodCplx + 1);
-    // one block: maxima (2 words), info and counters (4 + 4 ints), histogram, the
-    // sample's hash, the lookup hash
+    // one block: maxima (2 words), info and counters (4 + 4 ints), totals (2 words), histogram,
+    // the sample's hash, the lookup hash, the table in the making, sorted keys, run totals and
+    // the scans' scratch
     constexpr size_t kHead = 8 + kHist;
-    DevBuf<uint64_t> work(kHead + 3 * (size_t)slots + slots / 2 + 2 * (size_t)kLook + kLook / 2);
+    const int64_t runs = (int64_t)C.npan * nsl, rows = nsl * 64;
+    const size_t hash = 3 * (size_t)slots + slots / 2, lookw = 2 * (size_t)kLook + kLook / 2, tabw = 2 * kCodCplx;
+    DevBuf<uint64_t> work(kHead + hash + lookw + tabw + (size_t)std::max<int64_t>(nnz, 1) + (runs + nsl + 1) / 2 +
+                          scan_scratch(std::max(runs, nsl)));
     unsigned long long* mx = (unsigned long long*)work.get();
     int32_t* info = (int32_t*)(work.get() + 2);
     int32_t* ctr = (int32_t*)(work.get() + 4);
+    int64_t* totals = (int64_t*)(work.get() + 6);
     int32_t* hist = (int32_t*)(work.get() + 8);
     uint64_t* tag = work.get() + kHead;
     uint64_t* skr = tag + slots;
@@ -430,12 +450,15 @@ void build_coded(blqh_hamil* H, const uint8_t* nu, int64_t* ntun) {
     int32_t* cnt = (int32_t*)(ski + slots);
     uint64_t* look = ski + slots + slots / 2;
     const DictHash L{look, look + kLook, (int32_t*)(look + 2 * kLook), 2 * (kCodReal + 1) - 1, kLook - 1};
-    DevBuf<double> tab(2 * kCodCplx);
+    double* tab = (double*)(look + lookw);
+    uint64_t* skey = (uint64_t*)tab + tabw;
+    int32_t* tot = (int32_t*)(skey + std::max<int64_t>(nnz, 1));
+    int64_t* scan = (int64_t*)(skey + std::max<int64_t>(nnz, 1) + (runs + nsl + 1) / 2);
     auto fill = [&](void* p, int64_t words, uint64_t v) {
         hipLaunchKernelGGL(k_fill64, dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>(ceil_div(words, kBlk), 2048))),
                            dim3(kBlk), 0, st, (uint64_t*)p, words, v);
     };
-    fill(work.get(), (int64_t)(kHead + 3 * (size_t)slots + slots / 2), 0);
+    fill(work.get(), (int64_t)(kHead + hash), 0);
     fill(L.id, kLook / 2, ~0ull);
     launch_absmax(nnz, H->val.get(), mx, st);
     const unsigned gs = (unsigned)std::max<int64_t>(1, std::min<int64_t>(ceil_div(samples, kBlk), 2048));
@@ -443,52 +466,57 @@ void build_coded(blqh_hamil* H, const uint8_t* nu, int64_t* ntun) {
                        slots - 1);
     hipLaunchKernelGGL(k_dict_hist, dim3(slots / kHist), dim3(kHist), 0, st, tag, cnt, slots, hist);
     hipLaunchKernelGGL(k_dict_select, dim3(slots / kHist), dim3(kHist), 0, st, tag, skr, ski, cnt, slots, mx,
-                       (int)samples, hist, tab.get(), L, info);
+                       (int)samples, hist, tab, L, info);
     BLQH_HIP(hipGetLastError());
     // rows
-    const int64_t runs = (int64_t)C.npan * nsl;
-    DevBuf<uint64_t> skey(std::max<int64_t>(nnz, 1));
-    C.len.alloc((size_t)runs * 64);
-    C.rlen.alloc((size_t)nsl * 64);
-    C.diag.alloc(2 * (size_t)std::max<int64_t>(n, 1));
-    const int64_t rows = nsl * 64;
+    Blocks A;
+    const size_t obase = A.add((runs + 1) * 8), orbase = A.add((nsl + 1) * 8),
+                 odiag = A.add(2 * (size_t)std::max<int64_t>(n, 1) * 8), olen = A.add((size_t)(runs + nsl) * 64 * 2);
+    C.rows.alloc(A.bytes);
+    C.base = (int64_t*)(C.rows.get() + obase);
+    C.rbase = (int64_t*)(C.rows.get() + orbase);
+    C.diag = (double*)(C.rows.get() + odiag);
+    C.len = (uint16_t*)(C.rows.get() + olen);
+    C.rlen = C.len + (size_t)runs * 64;
     const int gr = (int)std::min<int64_t>(rows, (int64_t)runtime().num_cus * 40);
     int P = 64;  // LDS for the longest row the build can have kept
     const int rmax = std::min<int>(kMaxRow, H->row_max > 0 ? H->row_max : kMaxRow);
     while (P < rmax) P <<= 1;
     hipLaunchKernelGGL(k_cod_rows, dim3(gr), dim3(64), (size_t)P * 8, st, n, rows, C.npan, P, iperm, perm,
-                       H->rowptr.get(), H->col.get(), H->val.get(), L, info, nu, skey.get(), C.len.get(),
-                       C.rlen.get(), C.diag.get(), ctr);
+                       H->rowptr.get(), H->col.get(), H->val.get(), L, info, nu, skey, C.len, C.rlen, C.diag, ctr);
+    hipLaunchKernelGGL(k_cod_runs, dim3(grid_waves(runs + nsl)), dim3(kBlk), 0, st, runs + nsl, C.len, tot);
+    exclusive_scan(tot, C.base, runs, st, scan);
+    exclusive_scan(tot + runs, C.rbase, nsl, st, scan);
+    hipLaunchKernelGGL(k_cod_totals, dim3(1), dim3(1), 0, st, C.base + runs, C.rbase + nsl, totals);
     BLQH_HIP(hipGetLastError());
-    DevBuf<int32_t> tot(runs + nsl);
-    hipLaunchKernelGGL(k_cod_runs, dim3(grid_waves(runs)), dim3(kBlk), 0, st, runs, C.len.get(), tot.get());
-    hipLaunchKernelGGL(k_cod_runs, dim3(grid_waves(nsl)), dim3(kBlk), 0, st, nsl, C.rlen.get(), tot.get() + runs);
-    BLQH_HIP(hipGetLastError());
-    C.base.alloc(runs + 1);
-    C.rbase.alloc(nsl + 1);
-    exclusive_scan(tot.get(), C.base.get(), runs, st);
-    exclusive_scan(tot.get() + runs, C.rbase.get(), nsl, st);
-    int32_t hw[8];
-    BLQH_HIP(hipMemcpyAsync(hw, work.get() + 2, 32, hipMemcpyDeviceToHost, st));
-    BLQH_HIP(hipMemcpyAsync(&C.ncod, C.base.get() + runs, 8, hipMemcpyDeviceToHost, st));
-    BLQH_HIP(hipMemcpyAsync(&C.nrest, C.rbase.get() + nsl, 8, hipMemcpyDeviceToHost, st));
+    int32_t hw[12];
+    BLQH_HIP(hipMemcpyAsync(hw, work.get() + 2, 48, hipMemcpyDeviceToHost, st));
     BLQH_HIP(hipStreamSynchronize(st));
+    std::memcpy(&C.ncod, hw + 8, 8);
+    std::memcpy(&C.nrest, hw + 10, 8);
     C.ntab = hw[0];
     C.real = hw[1] != 0;
     BLQH_REQUIRE(hw[4] == 0, BLQH_EINTERNAL, "a CSR row is longer than the coded layout handles");
     BLQH_REQUIRE(C.ncod + C.nrest + hw[6] == nnz, BLQH_EINTERNAL, "coded layout lost entries");
     if (ntun) *ntun = hw[5];
-    C.ent.alloc(std::max<int64_t>(C.ncod, 1));
-    C.rcol.alloc(std::max<int64_t>(C.nrest, 1));
-    C.rval.alloc(std::max<int64_t>(C.nrest, 1) * (C.real ? 1 : 2));
-    C.tab.alloc(cod_lds_bytes(C.real, C.ntab) / sizeof(double));
-    BLQH_HIP(hipMemcpyAsync(C.tab.get(), tab.get(), C.tab.bytes(), hipMemcpyDeviceToDevice, st));
+    Blocks E;
+    const size_t oent = E.add((size_t)C.ncod * 4), orval = E.add((size_t)C.nrest * (C.real ? 8 : 16)),
+                 orcol = E.add((size_t)C.nrest * 4), otab = E.add(cod_lds_bytes(C.real, C.ntab));
+    // a multiple of a 16th of its size, so that the next parameter point's layout, whose split
+    // differs by a few entries, finds the block again
+    size_t step = 256;
+    while (step * 32 <= E.bytes) step *= 2;
+    C.words.alloc((E.bytes + step - 1) / step * step);
+    C.ent = (uint32_t*)(C.words.get() + oent);
+    C.rval = (double*)(C.words.get() + orval);
+    C.rcol = (uint32_t*)(C.words.get() + orcol);
+    C.tab = (double*)(C.words.get() + otab);
+    BLQH_HIP(hipMemcpyAsync(C.tab, tab, cod_lds_bytes(C.real, C.ntab), hipMemcpyDeviceToDevice, st));
     hipLaunchKernelGGL(k_cod_fill, dim3(grid_waves(nsl)), dim3(kBlk), 0, st, n, nsl, C.npan, iperm,
-                       H->rowptr.get(), skey.get(), C.len.get(), C.base.get(), C.ent.get());
+                       H->rowptr.get(), skey, C.len, C.base, C.ent);
     if (C.nrest > 0)
-        hipLaunchKernelGGL(k_cod_rest, dim3(grid_waves(nsl)), dim3(kBlk), 0, st, n, nsl, C.npan,
-                           C.real ? 1 : 0, iperm, H->rowptr.get(), H->val.get(), skey.get(), C.len.get(), C.rlen.get(), C.rbase.get(), C.rcol.get(),
-                           C.rval.get());
+        hipLaunchKernelGGL(k_cod_rest, dim3(grid_waves(nsl)), dim3(kBlk), 0, st, n, nsl, C.npan, C.real ? 1 : 0, iperm,
+                           H->rowptr.get(), H->val.get(), skey, C.len, C.rlen, C.rbase, C.rcol, C.rval);
     BLQH_HIP(hipGetLastError());
     BLQH_HIP(hipStreamSynchronize(st));  // complete for solves on other threads' streams
     C.built = true;

@@ -34,15 +34,18 @@ struct Coded {
     int npan = 0;
     int ntab = 0;
     int64_t ncod = 0, nrest = 0;
-    DevBuf<double> tab;      // [ntab] |v| (an even number of places), or [2 ntab] (|re|, |im|)
-    DevBuf<int64_t> base;    // [npan * nslices + 1] first word of run p * nslices + s
-    DevBuf<uint16_t> len;    // [npan][nslices * 64] words of the row in the run
-    DevBuf<uint32_t> ent;    // [ncod]
-    DevBuf<int64_t> rbase;   // [nslices + 1]
-    DevBuf<uint16_t> rlen;   // [nslices * 64]
-    DevBuf<uint32_t> rcol;   // [nrest]
-    DevBuf<double> rval;     // [nrest] or [2 nrest]
-    DevBuf<double> diag;     // [n] or [2 n]
+    double* tab = nullptr;      // [ntab] |v| (an even number of places), or [2 ntab] (|re|, |im|)
+    int64_t* base = nullptr;    // [npan * nslices + 1] first word of run p * nslices + s
+    uint16_t* len = nullptr;    // [npan][nslices * 64] words of the row in the run
+    uint32_t* ent = nullptr;    // [ncod]
+    int64_t* rbase = nullptr;   // [nslices + 1]
+    uint16_t* rlen = nullptr;   // [nslices * 64], behind len
+    uint32_t* rcol = nullptr;   // [nrest]
+    double* rval = nullptr;     // [nrest] or [2 nrest]
+    double* diag = nullptr;     // [n] or [2 n]
+    // where they lie: what the rows' number sizes, and what the entries' split does.  Two blocks,
+    // since a block costs the build of a small matrix some 10 us to take and give back.
+    DevBuf<char> rows, words;
 };
 
 struct CodView {
@@ -60,9 +63,8 @@ struct CodView {
 };
 
 inline CodView cview(const Coded& C, int64_t n) {
-    return CodView{n,           (n + 63) >> 6, C.npan,        C.ntab,       C.tab.get(),  C.base.get(),
-                   C.len.get(), C.ent.get(),   C.rbase.get(), C.rlen.get(), C.rcol.get(), C.rval.get(),
-                   C.diag.get()};
+    return CodView{n,     (n + 63) >> 6, C.npan, C.ntab, C.tab,  C.base, C.len,
+                   C.ent, C.rbase,       C.rlen, C.rcol, C.rval, C.diag};
 }
 
 __host__ __device__ inline size_t cod_lds_bytes(bool real, int ntab) {

@@ -264,3 +264,23 @@ def test_event_timing_runs_the_same_kernels(name):
         assert u["E0"] == v["E0"] and u["iterations"] == v["iterations"] and u["residual"] == v["residual"]
         np.testing.assert_array_equal(u["psi"], v["psi"])
     assert launches >= max(r["iterations"] for r in timed) and ms > 0 and nbytes > 0
+
+
+@pytest.mark.parametrize("case,kw", [((2, 2, 1, 1, -1, 0, 0), {}), ((2, 2, 1, -1, -1, 1, 1), dict(delta_sas=0.1)),
+                                     ((1, 4, 1, -1, -1, 0, 0), None), ((2, 3, 2, -1, -1, 1, 2), dict(delta_sas=0.1)),
+                                     ((2, 5, 5, -1, -1, 1, 2), dict(theta_x=0.31, theta_y=0.17, delta_sas=0.1)),
+                                     ((4, 2, 2, -1, -1, 0, 1), dict(delta_sas=0.1))], ids=lambda c: str(c))
+def test_layouts_of_a_few_rows(case, kw):
+    """Layouts whose parts are empty or tiny (no entry beside the diagonal, no value met twice, no
+    rest): the product against scipy's, for real and complex."""
+    S, nphi, nel, nu, nsu, J, K = case
+    B = blqh_amd.Basis(nphi, nel, nu, J, K, nspecies=S, nel_su=nsu)
+    H = blqh_amd.Hamiltonian(B, blqh_amd.params(nphi) if S == 1 else blqh_amd.params(nphi, d=0.7, **kw))
+    rp, col, val = H.export()
+    A = sp.csr_matrix((val, col, rp), shape=(H.n, H.n))
+    x = np.arange(1, H.n + 1) * (1 - 0.5j)
+    for plan in ((6, 64, 512, 0, 8), (6, 64, 256, 0, 1)):
+        print(f"{case} n {H.n} entries {H.nnz} plan {plan}", flush=True)
+        H.set_spmv(*plan)
+        scale = max(np.abs(val).max(initial=0) * np.abs(x).max() * np.diff(rp).max(initial=1), 1e-300)
+        np.testing.assert_allclose(H.spmv(x), A @ x, rtol=0, atol=2e-15 * scale)
