@@ -284,3 +284,24 @@ def test_layouts_of_a_few_rows(case, kw):
         H.set_spmv(*plan)
         scale = max(np.abs(val).max(initial=0) * np.abs(x).max() * np.diff(rp).max(initial=1), 1e-300)
         np.testing.assert_allclose(H.spmv(x), A @ x, rtol=0, atol=2e-15 * scale)
+
+
+def test_default_states_match_csr_solver(built):
+    """Eight steps from one start (before rounding can pick another state of a level): the default
+    plan's state and coefficients are the CSR kernel's up to the order of the sums."""
+    name, B, H, A = built
+    if H.n < 16:
+        pytest.skip("too few states for a set number of steps")
+    print(f"{name} n={H.n}", flush=True)
+    steps = dict(lam=8, seed=5, tol=0.0, res_tol=0.0)
+    H.set_spmv(-1)
+    a = H.lanczos(**steps)
+    H.set_spmv(0, 16)
+    b = H.lanczos(**steps)
+    # a row sum's rounding, grown by at most the spread of the spectrum over beta in each step
+    top = np.abs(a["alpha"]).max() + 2 * a["beta"].max()
+    grown = 2.0 ** -52 * np.diff(A.indptr).max() * (top / a["beta"][1:].min()) ** 8
+    tol = min(max(grown, 1e-13), 1e-6)
+    np.testing.assert_allclose(a["alpha"], b["alpha"], rtol=0, atol=tol * top)
+    np.testing.assert_allclose(a["beta"], b["beta"], rtol=0, atol=tol * top)
+    np.testing.assert_allclose(a["psi"], b["psi"], rtol=0, atol=tol)
