@@ -62,7 +62,7 @@ RECORDED_SWEEP_TRAFFIC = {
 
 def one_workgroup(H, rows):
     """Whether one workgroup runs the steps (the timing is then that of whole steps)."""
-    return H.n <= rows and H.nnz <= 16384
+    return H.n <= rows and H.nnz <= 24576
 
 
 def roofline_rate(achieved, traffic, avg_ms):

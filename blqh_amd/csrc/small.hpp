@@ -8,8 +8,7 @@
 // whichever runs.  A batch's kernels (k_b1x, k_b2, k_b3) sum in another order: the last bits
 // of its members depend on whether all of them are small.
 // Bound by the instructions of the step's chain (sums, two reductions, a root and a division)
-// on one CU: 5.6 us a step at 79 rows (three launches: 12), 12 us at 176 rows (108 such
-// problems at once, kernels over all of them: 27).
+// on one CU: 5.9 us a step at 79 rows (three launches: 15), 8.4 us at 172 rows (16).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cstdint>
@@ -42,12 +41,13 @@ constexpr int kSmallTeam = 8;      // wavefronts of a slice, as k_cod's of a sma
 constexpr int kSmallRows = 2048;   // rows at most: two a thread
 constexpr int kSmallSlices = kSmallRows / 64;
 
-// A matrix of n rows and nnz entries is stepped by one workgroup.  Its step takes 5.3 us and
-// 0.6 us for every 1,000 entries, on its one CU; the kernels' takes 14 to 18 us for one
+// A matrix of n rows and nnz entries is stepped by one workgroup.  Its step takes 5 us and
+// 0.4 us for every 1,000 entries, on its one CU; the kernels' takes 15 to 18 us for one
 // matrix of up to 60,000 entries.  Batch of 1 / 8 / 36 members, this against the kernels: 9,400
-// entries 12 / 21 / 20 us against 16 / 26 / 29; 23,800 entries 20 / 28 / 28 against 17 / 28 / 29;
-// 36,000 entries (1 / 4 / 32 members) 26 / 34 / 38 against 18 / 23 / 31.
-constexpr int64_t kSmallWords = 1 << 14;
+// entries 8.6 / 20 / 17 us against 16 / 27 / 30; 23,800 entries 12 / 24 / 20 us against 17 / 29 /
+// 28; 36,000 entries (1 / 4 / 32 members) 19 / 25 / 29 against 18 / 23 / 31.  Single solves of 60
+// steps: 23,800 entries 0.80 ms against 0.91, 36,000 entries 1.17 against 0.94.
+constexpr int64_t kSmallWords = (int64_t)3 << 13;
 inline bool small_matrix(int64_t n, int64_t nnz) { return n <= kSmallRows && nnz <= kSmallWords; }
 
 constexpr int kSmallLaunch = 64;   // steps of a launch at most (the mailbox's entries)

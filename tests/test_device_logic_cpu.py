@@ -319,11 +319,11 @@ def test_hop_term_with_and_without_the_period(case):
     assert hostmirror.hop_forms_diff(blqh_amd.Sector(*case)) == 0
 
 
-@pytest.mark.parametrize("n,nnz,one", [(79, 3147, True), (205, 7585, True), (176, 9428, True), (2048, 16384, True),
+@pytest.mark.parametrize("n,nnz,one", [(79, 3147, True), (205, 7585, True), (176, 9428, True), (2048, 24576, True),
                                        (604, 36150, False), (636, 58544, False), (936, 83878, False),
-                                       (300, 16385, False), (2049, 9000, False)])
+                                       (474, 23814, True), (300, 24577, False), (2049, 9000, False)])
 def test_one_workgroup_only_where_it_is_faster(n, nnz, one):
-    """Steps go to one workgroup by the entries it has to walk on its one CU: from about 20,000
+    """Steps go to one workgroup by the entries it has to walk on its one CU: from about 30,000
     on the kernels over the whole chip take less."""
     assert hostmirror.small_matrix(n, nnz) == one
 
