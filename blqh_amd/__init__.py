@@ -308,7 +308,7 @@ class Hamiltonian:
         return rowptr, col, val
 
     def get_spmv(self):
-        """(kind, lanes, threads, wgs_per_cu, rows) of the SpMV variant in use (kind -1: not tuned yet)."""
+        """(kind, lanes, threads, wgs_per_cu, rows) of the SpMV variant in use (kind -1: none yet)."""
         v = [C.c_int32() for _ in range(5)]
         _check(lib().blqh_hamil_get_spmv(self.h, *[C.byref(x) for x in v]))
         return tuple(x.value for x in v)

@@ -1499,7 +1499,7 @@ blqh_batch* blqh_batch_create_scaled_impl(const blqh_hamil* const* base, const b
                 BProb d{};
                 d.n = H->n;
                 d.npan = 1;
-                    d.item0 = b->nitems;
+                d.item0 = b->nitems;
                 d.voff = b->rows;
                 for (int64_t i = 0; i < nit; ++i) ip.push_back(p);
                 b->nitems += nit;

@@ -5,10 +5,14 @@
 // phase, so a sector's entries take few distinct values: the 1,023 most
 // frequent magnitudes of a real sector and the 4,095 most frequent (|re|, |im|)
 // pairs of a complex one cover 99 % of the entries and more (N_phi = 12: 99.2 /
-// 99.4 %, N_phi = 14: 99.6 / 99.5 %, N_phi = 16 at half filling: 99.7 %).  Those values sit in a table that every workgroup
-// holds in LDS, and an entry is one 32-bit word: column within its panel in the
-// low 16 bits, table index above, sign of the real (and imaginary) part on top.  The matrix stream is 4 bytes an entry instead of 10 (real) or 18
-// (complex), bit for bit the same values.  Entries whose value is not in the
+// 99.4 %, N_phi = 14: 99.6 / 99.5 %, N_phi = 16 at half filling: 99.7 %).  Those
+// values sit in a table that every workgroup holds in LDS, and an entry is one
+// 32-bit word: column within its panel in the low 16 bits, table index above,
+// sign of the real (and imaginary) part on top.  The matrix stream is 4 bytes an
+// entry instead of 10 (real) or 18 (complex), and the values are the CSR's bit for
+// bit, but for one case: a matrix whose imaginary parts are all at most 1e-14 of
+// its largest entry is a real one (as for the panels), and those parts, the
+// rounding of its phases, are left out.  Entries whose value is not in the
 // table form the rest: 32-bit column and value, one run per 64-row slice.  The
 // diagonal, whose values are nearly all different, is an array of its own.
 //

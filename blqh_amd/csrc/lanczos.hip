@@ -793,8 +793,8 @@ __global__ void __launch_bounds__(kT4Threads) k_t4(TileView V, const double2* __
 // (four: 2,050 us).  Wider panels, 4 or 16 wavefronts a workgroup and persistent
 // grids gave nothing.  Step of one Lanczos iteration, K1 only, against the
 // jagged panels of 10 (real) or 18 (complex) bytes an entry: N_phi = 16 all
-// densities 2,907 -> 1,880 us, nel_up = 8 811 -> 475, N_phi = 14 real 209 -> 124 and
-// complex 265 -> 140, N_phi = 12 complex 24 -> 17.
+// densities 2,907 -> 1,865 us, nel_up = 8 811 -> 468, N_phi = 14 real 209 -> 119 and
+// complex 265 -> 130, N_phi = 12 complex 24 -> 14.
 template <bool REAL, bool LZ, int WPB, int NP>
 __global__ void __launch_bounds__(WPB * 64) k_cod(CodView P, const double2* __restrict__ x, double2* __restrict__ out,
                                                   const double2* __restrict__ Wp, Scal sc, int j, double* partials) {

@@ -203,8 +203,8 @@ __device__ __forceinline__ uint64_t scalar(uint64_t w) {
 // holds only W2 (padded: the backward pass reads it across) and what the gradient sums
 // share.  Bound by latency: a minibatch of 4,096 states is 256 tiles, one for each CU;
 // with tiles of 64 states, every product through LDS and a quarter of the CUs busy the
-// forward and backward of that took 66 us, 46 now, and the sums 16, 4 now.  Past kMaxWgs tiles a workgroup takes
-// several and keeps their sums in registers.
+// forward and backward of that took 66 us, 50 now, and the sums 16, 4 now.
+// Past kMaxWgs tiles a workgroup takes several and keeps their sums in registers.
 constexpr int kSt = 16, kSw = kSt / (kT / 64), kMaxWgs = 512;
 constexpr int kR1 = (kMaxIn + kT / 64 - 1) / (kT / 64);  // rows of W1 a wavefront sums
 

@@ -200,9 +200,10 @@ int blqh_lanczos(const blqh_hamil* h, const blqh_lanczos_opts* o, blqh_lanczos_r
  * bit-identical replay); every device array of the solve lives in one static
  * array per GPU of about 12.3 MiB, held until the process ends.  Limits
  * (BLQH_ERANGE beyond them): at most 131072 rows and lambda <= 1024;
- * start_mix must be 0 (BLQH_EINVAL).  The SpMV is the tuned variant when the
- * Hamiltonian's layout is already in place for it (after a blqh_lanczos or
- * blqh_spmv on it), else the CSR kernel.  Calls in one process are serialised
+ * start_mix must be 0 (BLQH_EINVAL).  The SpMV is the one that blqh_lanczos uses
+ * (the coded layout, or the variant pinned with blqh_hamil_set_spmv) if its layout
+ * is in place, else the coded layout, else, for a part of a merge whose formats
+ * were not built, the CSR kernel.  Calls in one process are serialised
  * (they share the array, whose contents each call re-initialises). */
 int blqh_lanczos_noalloc(const blqh_hamil* h, const blqh_lanczos_opts* o, blqh_lanczos_result* r, double* psi,
                          double* alpha, double* beta);
